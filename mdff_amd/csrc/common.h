@@ -205,6 +205,8 @@ struct alignas(16) AtomRec {
   double x, y, z, q;
 };
 
+struct MeshRecip;
+
 struct mdff_ctx {
   mdff_desc d;
   int n = 0, ntype = 0;
@@ -230,6 +232,7 @@ struct mdff_ctx {
   // reciprocal sums run in FP64): without that box the FP32-class dipole
   // structure factors set the force error above 1e-5
   int rec_f32 = 0;
+  MeshRecip* mesh = nullptr;              // reciprocal sums as fast transforms (mesh.hip); null: the direct kernels
   // LJ together with BMHFT(D) (src/engforce_driver.f90:130-141): the BMHFT(D)
   // pass gives the forces (each reference routine zeroes them first), an LJ
   // pass its energy, virial and stress into peratom_lj (forces into f_lj,
@@ -470,6 +473,12 @@ int recip_tables_from_r(mdff_ctx* c, bool pack);
 int recip_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool use_mu,
                bool forces, bool field, double* ef_out, double* f_out, double* e_out);
 void recip_free(mdff_ctx* c);
+// the same sums as non-uniform fast transforms (mesh.hip)
+int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<double>& kv);
+int mesh_bin(mdff_ctx* c, bool from_r, bool pack);
+int mesh_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool use_mu, int mom, double* e_out,
+              const double** out);
+void mesh_free(mdff_ctx* c);
 // electric field gradient (efg.hip; its real-space part in realspace.hip)
 int realspace_efg(mdff_ctx* c, double* out);
 int efg_alloc(mdff_ctx* c);

@@ -1,0 +1,1345 @@
+// mesh.hip -- the reciprocal Ewald sums as non-uniform fast transforms in
+// FP64 (gfx950).
+//
+// The sums are the reference's: S(k) over the whole half-space k mesh with
+// its A(k) (multipole_ES_rec, src/ewald_rec.f90:38-365; mesh of
+// src/kspace.f90:143-207), and per atom the sums over k of its fields and
+// forces.  Evaluated term by term they cost N x nk; here each is a
+// non-uniform Fourier transform to rounding accuracy, N w^3 + mesh work:
+// the atoms are spread onto a regular grid with a kernel phi of w points a
+// direction, the grid is transformed, and the kernel's own transform is
+// divided out,
+//   S(n) = sum_i a_i e^{2 pi i n.s_i} = 1/phih(n) sum_l b[l] e^{2 pi i n.l/G},
+//   b[l] = sum_i a_i phi(l - G s_i),
+// and the potential V(s) = Re sum_n W(n) e^{2 pi i n.s}, W = A conj(S), comes
+// back the same way: sum_n n_d Im(W e_i) = -dV/ds_d / 2 pi and
+// sum_n n_d n_e Re(W e_i) = -d2V/ds_d ds_e / 4 pi^2, with derivatives of phi.
+// A dipole is the derivative of a charge: its amplitude i 2 pi n.m is
+// m.d/ds on phi.
+//
+// phi(x) = s I1(beta s), s = sqrt(1 - (2x/w)^2): the Kaiser-Bessel family
+// (R. M. Lewitt, J. Opt. Soc. Am. A 7, 1834 (1990)), continuous at its edge,
+// which the derivatives need.  Its transform is elementary
+// (2 h beta (z cosh z - sinh z) / z^3, z^2 = beta^2 - (2 pi f h)^2, h = w/2).
+// The grid G and beta are chosen per direction from the alias error weighted
+// with the decay of A(k) (mesh_error): below 4e-15 with w = 16 in the FP64
+// form, which measured 1e-14 of the reciprocal force (its rounding), below
+// 1e-9 with w = 12 in the mixed form, whose FP32 pair terms carry 1e-7.
+//
+// Launches of one evaluation: k_mesh_bin (s = B^T r, count per bin),
+// k_mesh_scan, k_mesh_scatter, k_mesh_phi (order within the bins, phi
+// values), k_mesh_spread, k_mesh_zy (z and y transforms), k_mesh_x (x
+// transform, W, energy and stress, x transform back), k_mesh_yz, k_mesh_gather.
+// Every sum has a fixed order.
+#include <algorithm>
+#include <cmath>
+
+#include "common.h"
+#include "reduce.h"
+
+namespace {
+
+constexpr int kDeg = 15;        // degree of the piecewise polynomials of phi
+constexpr int kPair = 8;        // even (odd) coefficients of a piece
+constexpr int kTile = 16;       // grid points of a spread tile (and of a bin) a direction
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f64x4 mma64(double a, double b, f64x4 c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ int div_up_dev(int a, int b) { return (a + b - 1) / b; }
+
+// the wave's number in the block, as a scalar
+__device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+
+struct MeshGrid {
+  int G[3];
+  int nyb, nzb;                 // bins (tiles) of y and z
+};
+
+// Grid coordinate of a fractional coordinate s: the first point l (in
+// [0, G)) of the window of w points and t = l - (G s - w/2) in [0, 1).
+// Rounded operation by operation, so that every kernel finds the same l.
+template <int W>
+__device__ __forceinline__ void mesh_coord(double s, int G, int& l, double& t) {
+  const double f = s - floor(s);
+  const double x = __dsub_rn(__dmul_rn(f, (double)G), 0.5 * W);
+  const double c = ceil(x);
+  t = c - x;
+  l = 0;
+  if (f >= 0.0 && f <= 1.0) {     // not NaN
+    l = (int)c;
+    l = l < 0 ? l + G : (l >= G ? l - G : l);
+  }
+}
+
+// bin of a window start: x exactly, y and z by tiles, x fastest
+__device__ __forceinline__ int mesh_bin(const MeshGrid& m, int lx, int ly, int lz) {
+  return ((ly / kTile) * m.nzb + lz / kTile) * m.G[0] + lx;
+}
+
+// ---- atoms into bins -------------------------------------------------------
+
+struct BinArgs {
+  int n, from_r, pack;
+  MeshGrid m;
+  const double *rx, *ry, *rz;
+  double b[9];                   // B column-major
+  double *sx, *sy, *sz;          // written from r, or read
+  int32_t* key;                  // bin of every atom
+  int32_t* slot;                 // its arrival number in the bin (any order)
+  int32_t* cnt;                  // atoms per bin (zero on entry)
+  // pack: the atoms in the cell order of the last list build (pack_atoms)
+  const int32_t* order;
+  const double* q;
+  const int32_t* itype;
+  AtomRec* rec;
+  int2* meta;
+};
+
+// One thread per atom.  fin_row >= 0: the blocks of that row run the queued
+// final sums of the previous MD step (block x: sum x).  s = B^T r is rounded
+// as kardir does (src/lattice.f90:183-216).
+template <int W>
+__global__ void __launch_bounds__(256) k_mesh_bin(BinArgs a, FinalBatch fb, int fin_row) {
+  if ((int)blockIdx.y == fin_row) {
+    __shared__ double sh[4 * kRedMaxCols];
+    run_final_batch(fb, blockIdx.x, sh);
+    return;
+  }
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= a.n) return;
+  const double* b = a.b;
+  auto dot = [](double x, double y, double z, double u, double v, double w) {
+    return __dadd_rn(__dadd_rn(__dmul_rn(x, u), __dmul_rn(y, v)), __dmul_rn(z, w));
+  };
+  double s0, s1, s2;
+  if (a.from_r) {
+    const double x = a.rx[i], y = a.ry[i], z = a.rz[i];
+    s0 = dot(x, y, z, b[0], b[1], b[2]);
+    s1 = dot(x, y, z, b[3], b[4], b[5]);
+    s2 = dot(x, y, z, b[6], b[7], b[8]);
+    a.sx[i] = s0;
+    a.sy[i] = s1;
+    a.sz[i] = s2;
+  } else {
+    s0 = a.sx[i];
+    s1 = a.sy[i];
+    s2 = a.sz[i];
+  }
+  int lx, ly, lz;
+  double t;
+  mesh_coord<W>(s0, a.m.G[0], lx, t);
+  mesh_coord<W>(s1, a.m.G[1], ly, t);
+  mesh_coord<W>(s2, a.m.G[2], lz, t);
+  const int bin = mesh_bin(a.m, lx, ly, lz);
+  a.key[i] = bin;
+  a.slot[i] = atomicAdd(a.cnt + bin, 1);
+  if (a.pack) {
+    const int j = a.order[i];
+    const double xj = a.rx[j], yj = a.ry[j], zj = a.rz[j];
+    a.rec[i] = AtomRec{dot(xj, yj, zj, b[0], b[1], b[2]), dot(xj, yj, zj, b[3], b[4], b[5]),
+                       dot(xj, yj, zj, b[6], b[7], b[8]), a.q[j]};
+    a.meta[i] = make_int2(a.itype[j], j);
+  }
+}
+
+// start[0..nb] = prefix sums of cnt[0..nb), one block; cnt is left zero for
+// the next evaluation
+__global__ void __launch_bounds__(1024) k_mesh_scan(int nb, int32_t* __restrict__ cnt, int32_t* __restrict__ start) {
+  __shared__ int ws[16];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int base = 0;
+  for (int t0 = 0; t0 < nb; t0 += 4096) {
+    const int k0 = t0 + 4 * threadIdx.x;
+    int c[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) c[u] = k0 + u < nb ? cnt[k0 + u] : 0;
+    const int mine = c[0] + c[1] + c[2] + c[3];
+    int v = mine;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int x = __shfl_up(v, o, 64);
+      if (lane >= o) v += x;
+    }
+    if (lane == 63) ws[w] = v;
+    __syncthreads();
+    int before = 0, all = 0;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      before += u < w ? ws[u] : 0;
+      all += ws[u];
+    }
+    int at = base + before + v - mine;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (k0 + u < nb) {
+        start[k0 + u] = at;
+        cnt[k0 + u] = 0;
+        at += c[u];
+      }
+    base += all;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) start[nb] = base;
+}
+
+__global__ void __launch_bounds__(256) k_mesh_scatter(int n, const int32_t* __restrict__ key,
+                                                      const int32_t* __restrict__ slot,
+                                                      const int32_t* __restrict__ start, int32_t* __restrict__ order) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) order[start[key[i]] + slot[i]] = i;
+}
+
+struct PhiArgs {
+  int n;
+  MeshGrid m;
+  const double *sx, *sy, *sz;
+  const int32_t *key, *start, *order;
+  const double* coef;            // [W/2][2][kPair] pieces of phi, even and odd coefficients
+  int4* at;                      // per sorted atom: window start (x, y, z), atom index
+  double* phi;                   // [atom][3][W], with dip [atom][6][W]: phi, then dphi/dv
+};
+
+// Sixteen lanes an atom.  Its place within the bin is the number of smaller
+// indices there (the arrival order is not reproducible); then lane j
+// evaluates window point j of each direction.  Piece W-1-j mirrors piece j
+// (phi is even), so the upper lanes take the lower pieces at -v; the
+// coefficients of a lane's piece stay in registers over the atoms.
+template <int W>
+__device__ __forceinline__ void load_piece(const double* coef, int j, double c[2 * kPair]) {
+  const int jj = j < W / 2 ? j : W - 1 - j;
+#pragma unroll
+  for (int k = 0; k < 2 * kPair; ++k) c[k] = j < W ? coef[jj * 2 * kPair + k] : 0.0;
+}
+
+// E(v^2) + v O(v^2) at v (v times sg for a mirrored piece), its first
+// derivative in v and, SECOND, its second
+template <bool FIRST, bool SECOND>
+__device__ __forceinline__ void piece(const double c[2 * kPair], double v, double sg, double& f, double& df,
+                                      double& d2) {
+  v *= sg;
+  const double v2 = v * v;
+  double e = c[kPair - 1], h = c[2 * kPair - 1], de = 0.0, dh = 0.0, ee = 0.0, hh = 0.0;
+#pragma unroll
+  for (int k = kPair - 2; k >= 0; --k) {
+    if (SECOND) {
+      ee = ee * v2 + de;
+      hh = hh * v2 + dh;
+    }
+    if (FIRST) {
+      de = de * v2 + e;
+      dh = dh * v2 + h;
+    }
+    e = e * v2 + c[k];
+    h = h * v2 + c[kPair + k];
+  }
+  f = e + v * h;
+  if (FIRST) df = sg * (2.0 * v * de + h + 2.0 * v2 * dh);
+  // ee, hh: half the second derivatives of E and O in v^2
+  if (SECOND) d2 = 2.0 * de + 8.0 * v2 * ee + v * (6.0 * dh + 8.0 * v2 * hh);
+}
+
+template <int W, bool DIP>
+__global__ void __launch_bounds__(256) k_mesh_phi(PhiArgs a) {
+  constexpr int NR = DIP ? 6 : 3;
+  const int j = threadIdx.x & 15, step = gridDim.x * 16;
+  double c[2 * kPair];
+  load_piece<W>(a.coef, j, c);
+  const double sg = j < W / 2 ? 1.0 : -1.0;
+  for (int p0 = blockIdx.x * 16 + (threadIdx.x >> 4); p0 < a.n; p0 += step) {
+    const int i = a.order[p0];
+    const int bin = a.key[i];
+    const double s[3] = {a.sx[i], a.sy[i], a.sz[i]};
+    const int b0 = a.start[bin], b1 = a.start[bin + 1];
+    int rank = 0;
+    for (int k = b0 + j; k < b1; k += 16) rank += a.order[k] < i ? 1 : 0;
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) rank += __shfl_xor(rank, o, 16);
+    const size_t p = (size_t)b0 + rank;
+    double* out = a.phi + p * (NR * W) + j;
+    int l[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      double t, f, df = 0.0, d2 = 0.0;
+      mesh_coord<W>(s[d], a.m.G[d], l[d], t);
+      piece<DIP, false>(c, 2.0 * t - 1.0, sg, f, df, d2);
+      if (j < W) {
+        out[d * W] = f;
+        if (DIP) out[(3 + d) * W] = df;
+      }
+    }
+    if (j == 0) a.at[p] = make_int4(l[0], l[1], l[2], i);
+  }
+}
+
+// charge and -2 G m (m = B^T mu) of every sorted atom: the amplitudes of phi
+// and of its derivatives dphi/ds_d = -2 G_d dphi/dv
+__global__ void __launch_bounds__(256) k_mesh_amp(int n, const int4* __restrict__ at, const double* __restrict__ q,
+                                                  int use_q, const double* __restrict__ mu, double b0, double b1,
+                                                  double b2, double b3, double b4, double b5, double b6, double b7,
+                                                  double b8, double gx, double gy, double gz, double4* __restrict__ amp) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n) return;
+  const int i = at[p].w;
+  const double u0 = mu[3 * i], u1 = mu[3 * i + 1], u2 = mu[3 * i + 2];
+  amp[p] = make_double4(use_q ? q[i] : 0.0, gx * (u0 * b0 + u1 * b1 + u2 * b2), gy * (u0 * b3 + u1 * b4 + u2 * b5),
+                        gz * (u0 * b6 + u1 * b7 + u2 * b8));
+}
+
+// ---- spread ------------------------------------------------------------------
+// One block per tile of 16^3 grid points (and share of the bin columns), one
+// wave per x plane of the tile.  The atoms whose window touches the tile are
+// in the four bin columns (its y and z tile and the ones before them), lx from
+// x0 - W + 1 to x0 + 15: x is the fastest index of the bins, so each column
+// has one contiguous range of atoms (two where x wraps).  A chunk of them
+// enters LDS as rows of 16 already in the tile's coordinates, zero outside
+// the window: four atoms a step then cost two reads of 16 values, one product
+// and one v_mfma_f64_16x16x4, D(y, z) += [q phi(x) phi(y)] phi(z).  A wave
+// takes the steps of its own plane's range.  The windows' zeros in y and z are
+// multiplied along (W/32 of each direction is used); no atomics, fixed order.
+struct SpreadArgs {
+  int n, shares, pstride;        // pstride: doubles per atom of phi
+  MeshGrid m;
+  const int32_t* start;
+  const int4* at;
+  const double* phi;
+  const double* q;               // without dipoles
+  const double4* amp;            // with dipoles
+  double* out;                   // [share][Gx][Gy][Gz]
+};
+
+template <int W, bool DIP>
+__global__ void __launch_bounds__(1024) k_mesh_spread(SpreadArgs a) {
+  constexpr int NA = DIP ? 64 : 128;                      // atoms of a chunk
+  constexpr int NR = DIP ? 6 : 3;                         // rows per atom: x, y, z (times q), and for dipoles
+                                                          // x: q phi + m phi', phi; y: phi, m phi'; z: phi, m phi'
+  __shared__ double rows[NR][NA][kTile];
+  const int Gx = a.m.G[0], Gy = a.m.G[1], Gz = a.m.G[2];
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int wave = wave_id();
+  const int tile = blockIdx.x, share = blockIdx.y;
+  const int tz = tile % a.m.nzb, ty = (tile / a.m.nzb) % a.m.nyb, tx = tile / (a.m.nzb * a.m.nyb);
+  const int x0 = kTile * tx, x = x0 + wave;
+  f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+  for (int col = share; col < 4; col += a.shares) {
+    if (((col & 1) && a.m.nyb == 1) || ((col & 2) && a.m.nzb == 1)) continue;
+    int by = ty - (col & 1), bz = tz - (col >> 1);
+    by = by < 0 ? by + a.m.nyb : by;
+    bz = bz < 0 ? bz + a.m.nzb : bz;
+    const int32_t* st = a.start + (size_t)(by * a.m.nzb + bz) * Gx;
+    // lx in [x0 - W + 1, x0 + 15]; below zero they are at the other end of
+    // the row, from x0 + 16 at the earliest (part 1)
+    for (int part = 0; part < 2; ++part) {
+      const int lo = x0 - W + 1;
+      if (part == 1 && lo >= 0) break;
+      const int f0 = part == 0 ? max(lo, 0) : max(Gx + lo, x0 + kTile), f1 = part == 0 ? x0 + kTile : Gx;
+      // the wave's own starts in this part
+      const int wl = x - W + 1 + (part == 0 ? 0 : Gx);
+      const int w0 = max(wl, f0), w1 = part == 0 ? x + 1 : Gx;
+      const int q0 = st[f0], q1 = st[f1];
+      // (a grid of one tile wraps onto itself: every atom, for every plane)
+      const bool whole = Gx == kTile;
+      const int own0 = whole ? q0 : (w0 < w1 ? st[w0] : 0), own1 = whole ? q1 : (w0 < w1 ? st[w1] : 0);
+      for (int p0 = q0; p0 < q1; p0 += NA) {
+        const int na = min(NA, q1 - p0);
+        __syncthreads();
+        // rows: thread -> point c of atom (threadIdx.x >> 4) + 64 k
+        for (int at0 = threadIdx.x >> 4; at0 < ((na + 3) & ~3); at0 += 64) {
+          const int pc = p0 + min(at0, na - 1);
+          const int4 at = a.at[pc];
+          const double* f = a.phi + (size_t)pc * a.pstride;
+          int dx = x0 + c - at.x, dy = kTile * ty + c - at.y, dz = kTile * tz + c - at.z;
+          dx = dx < 0 ? dx + Gx : dx;
+          dy = dy < 0 ? dy + Gy : dy;
+          dz = dz < 0 ? dz + Gz : dz;
+          const bool ok = at0 < na;
+          const bool okx = ok && dx < W, oky = dy < W, okz = dz < W;
+          dx = min(dx, W - 1);
+          dy = min(dy, W - 1);
+          dz = min(dz, W - 1);
+          const double fx = f[dx], fy = f[W + dy], fz = f[2 * W + dz];
+          if constexpr (DIP) {
+            const double4 m = a.amp[pc];
+            const double gx = f[3 * W + dx], gy = f[4 * W + dy], gz = f[5 * W + dz];
+            rows[0][at0][c] = okx ? m.x * fx + m.y * gx : 0.0;
+            rows[1][at0][c] = oky ? fy : 0.0;
+            rows[2][at0][c] = okz ? fz : 0.0;
+            rows[3][at0][c] = okx ? fx : 0.0;
+            rows[4][at0][c] = oky ? m.z * gy : 0.0;
+            rows[5][at0][c] = okz ? m.w * gz : 0.0;
+          } else {
+            rows[0][at0][c] = okx ? a.q[at.w] * fx : 0.0;
+            rows[1][at0][c] = oky ? fy : 0.0;
+            rows[2][at0][c] = okz ? fz : 0.0;
+          }
+        }
+        __syncthreads();
+        const int s0 = max(own0 - p0, 0) >> 2, s1 = (min(own1 - p0, na) + 3) >> 2;
+        for (int t0 = s0; t0 < s1; t0 += 4) {
+          double av[4], bv[4], cv[4], dv[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int k = 4 * min(t0 + u, s1 - 1) + g;
+            const double ax = rows[0][k][wave], ay = rows[1][k][c];
+            bv[u] = rows[2][k][c];
+            if constexpr (DIP) {
+              const double cx = rows[3][k][wave], cy = rows[4][k][c];
+              av[u] = ax * ay + cx * cy;
+              cv[u] = cx * ay;
+              dv[u] = rows[5][k][c];
+            } else {
+              av[u] = ax * ay;
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            if (t0 + u >= s1) break;
+            acc = mma64(av[u], bv[u], acc);
+            if constexpr (DIP) acc = mma64(cv[u], dv[u], acc);
+          }
+        }
+      }
+    }
+  }
+  double* o = a.out + (((size_t)share * Gx + x) * Gy + kTile * ty) * Gz + kTile * tz + c;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) o[(size_t)(4 * r + g) * Gz] = acc[r];
+}
+
+// ---- transforms --------------------------------------------------------------
+// Each direction is a product with its Fourier matrix on
+// v_mfma_f64_16x16x4 (the matrices carry 1 / phih).  A block takes one x
+// plane (k_mesh_zy, k_mesh_yz) or 16 columns (k_mesh_x) through two
+// transforms with the data between them in LDS.  The matrices are stored in
+// the order of the instruction's operands:
+//  - "row" products (real: z), out[row][col] = sum_k in[row][k] M[k][col]: M as
+//    [k / 16][column tile][step][lane]; lane group g takes k = 16 kc + 4 g +
+//    step, so its four values of in are consecutive;
+//  - "mid" products (complex: x, y), out[n][c] = sum_l E[n][l] in[l][c]: E as
+//    [l / 4][n tile of 8][re in, im in][lane]; tile row R holds n = 4 (R >> 3)
+//    + (R & 3) and part (R >> 2) & 1, so a lane ends with re and im of its two
+//    n.  The re and im inputs go to neighbouring waves, which halves the chain
+//    of a wave; their sums meet in LDS.
+constexpr int kFtThreads = 1024, kFtWaves = 16;
+
+// in: LDS planes [re, im][l][16], rows up to the next 16 finite; out(n, c, value)
+template <typename Out>
+__device__ __forceinline__ void mid_product(const double* in, int lrows, int L, int ntiles, int N, const double* E,
+                                            double* xb, Out out) {
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15, wave = wave_id();
+  const int sp = wave & 1;
+  const double* v = in + (size_t)sp * lrows * 16 + 16 * g + c;
+  double* x = xb + (wave >> 1) * 256 + lane;
+  for (int t0 = 0; t0 < ntiles; t0 += kFtWaves / 2) {
+    const int t = t0 + (wave >> 1);
+    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+    if (t < ntiles) {
+      const double* e = E + ((size_t)t * 2 + sp) * 64 + lane;
+      const size_t es = (size_t)ntiles * 128;
+      for (int l = 0; l < L; l += 16) {
+        double ev[4], vv[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          ev[u] = e[(size_t)(l / 4 + u) * es];
+          vv[u] = v[(size_t)(l + 4 * u) * 16];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc = mma64(ev[u], vv[u], acc);
+      }
+    }
+    if (sp == 1) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x[64 * r] = acc[r];
+    }
+    __syncthreads();
+    if (sp == 0 && t < ntiles) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int n = 8 * t + 4 * h + g;
+        if (n < N) out(n, c, acc[2 * h] + x[128 * h], acc[2 * h + 1] + x[128 * h + 64]);
+      }
+    }
+    __syncthreads();
+  }
+}
+
+struct ZyArgs {
+  int Gy, Gz, CN, NY, ctiles, shares;
+  size_t sstride;                // between the shares of the grid, which are added
+  const double* grid;
+  const double* zf;              // row operand: column tile 2 ct + part
+  const double* yf;
+  double2* out;                  // [x][ny][nz]
+};
+
+// Block (nz tile, x): z transform of the plane's rows at 16 nz into LDS, then
+// their y transform
+__global__ void __launch_bounds__(kFtThreads) k_mesh_zy(ZyArgs a) {
+  extern __shared__ double lds[];
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15, wave = wave_id();
+  const int ct = blockIdx.x, x = blockIdx.y;
+  const int ytiles = a.Gy / 16;
+  double* pl = lds;                                       // [part][Gy][16]
+  double* xb = lds + 2 * (size_t)a.Gy * 16;
+  for (int u = wave; u < 2 * ytiles; u += kFtWaves) {
+    const int rt = u >> 1, part = u & 1;
+    const double* in = a.grid + ((size_t)x * a.Gy + 16 * rt + c) * a.Gz + 4 * g;
+    const double* m = a.zf + ((size_t)2 * ct + part) * 256 + lane;
+    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+    for (int k0 = 0; k0 < a.Gz; k0 += 16) {
+      double2 v0 = *reinterpret_cast<const double2*>(in + k0);
+      double2 v1 = *reinterpret_cast<const double2*>(in + k0 + 2);
+      double b[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) b[s] = m[(size_t)(k0 / 16) * a.ctiles * 512 + 64 * s];
+      if (a.shares == 4) {
+        double2 w0[3], w1[3];
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+          w0[s] = *reinterpret_cast<const double2*>(in + (s + 1) * a.sstride + k0);
+          w1[s] = *reinterpret_cast<const double2*>(in + (s + 1) * a.sstride + k0 + 2);
+        }
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+          v0.x += w0[s].x; v0.y += w0[s].y;
+          v1.x += w1[s].x; v1.y += w1[s].y;
+        }
+      } else if (a.shares == 2) {
+        const double2 w0 = *reinterpret_cast<const double2*>(in + a.sstride + k0);
+        const double2 w1 = *reinterpret_cast<const double2*>(in + a.sstride + k0 + 2);
+        v0.x += w0.x; v0.y += w0.y;
+        v1.x += w1.x; v1.y += w1.y;
+      }
+      acc = mma64(v0.x, b[0], acc);
+      acc = mma64(v0.y, b[1], acc);
+      acc = mma64(v1.x, b[2], acc);
+      acc = mma64(v1.y, b[3], acc);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) pl[((size_t)part * a.Gy + 16 * rt + 4 * r + g) * 16 + c] = acc[r];
+  }
+  __syncthreads();
+  double2* out = a.out + (size_t)x * a.NY * a.CN;
+  const int cc = 16 * ct + c;
+  mid_product(pl, a.Gy, a.Gy, div_up_dev(a.NY, 8), a.NY, a.yf, xb, [&](int n, int, double re, double im) {
+    if (cc < a.CN) out[(size_t)n * a.CN + cc] = make_double2(re, im);
+  });
+}
+
+struct XArgs {
+  int Gx, NX, C, back;           // C = NY CN columns
+  const double* xf;
+  const double* xb;
+  double2* t;                    // [x][C], in place
+  const double* A;               // [nx][C]
+  const double* kvec;            // kx, ky, kz, kcoe per (nx, c)
+  double* blk;                   // 7 per block
+};
+
+// Block: 16 columns (ny, nz).  S(n); W = A conj(S); the energy and stress
+// partials ((delta_ab - kcoe k_a k_b) A |S|^2, src/ewald_rec.f90:173-174,
+// 252-263); W's x transform back in place (back).
+__global__ void __launch_bounds__(kFtThreads) k_mesh_x(XArgs a) {
+  extern __shared__ double lds[];
+  const int lane = threadIdx.x & 63, wave = wave_id(), c = lane & 15;
+  const int nxp = (a.NX + 15) & ~15;
+  double* pl = lds;                                       // [part][Gx][16]
+  double* wl = pl + 2 * (size_t)a.Gx * 16;                // [part][nxp][16]
+  double* xb = wl + 2 * (size_t)nxp * 16;
+  const int c0 = blockIdx.x * 16;
+  for (int k = threadIdx.x; k < a.Gx * 16; k += kFtThreads) {
+    const double2 v = a.t[(size_t)(k >> 4) * a.C + min(c0 + (k & 15), a.C - 1)];
+    pl[k] = v.x;
+    pl[(size_t)a.Gx * 16 + k] = v.y;
+  }
+  for (int k = a.NX * 16 + threadIdx.x; k < nxp * 16; k += kFtThreads) {
+    wl[k] = 0.0;
+    wl[(size_t)nxp * 16 + k] = 0.0;
+  }
+  __syncthreads();
+  double sum[7] = {0, 0, 0, 0, 0, 0, 0};
+  const int cc = c0 + c;
+  mid_product(pl, a.Gx, a.Gx, div_up_dev(a.NX, 8), a.NX, a.xf, xb, [&](int n, int, double re, double im) {
+    double wr = 0.0, wi = 0.0;
+    if (cc < a.C) {
+      const size_t at = (size_t)n * a.C + cc;
+      const double Ak = a.A[at];
+      const double* k = a.kvec + 4 * at;
+      const double str = (re * re + im * im) * Ak;
+      const double kx = k[0], ky = k[1], kz = k[2], kc = k[3];
+      sum[0] += str;
+      sum[1] += (1.0 - kc * kx * kx) * str;
+      sum[2] += (1.0 - kc * ky * ky) * str;
+      sum[3] += (1.0 - kc * kz * kz) * str;
+      sum[4] += -kc * kx * ky * str;
+      sum[5] += -kc * kx * kz * str;
+      sum[6] += -kc * ky * kz * str;
+      wr = Ak * re;
+      wi = -Ak * im;
+    }
+    wl[n * 16 + c] = wr;
+    wl[(size_t)nxp * 16 + n * 16 + c] = wi;
+  });
+  // wave sums, then the waves in order
+#pragma unroll
+  for (int k = 0; k < 7; ++k) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) sum[k] += __shfl_down(sum[k], o, 64);
+    if (lane == 0) xb[wave * 8 + k] = sum[k];
+  }
+  __syncthreads();
+  if (threadIdx.x < 7) {
+    double r = 0.0;
+    for (int w = 0; w < kFtWaves; ++w) r += xb[w * 8 + threadIdx.x];
+    a.blk[(size_t)blockIdx.x * 7 + threadIdx.x] = r;
+  }
+  if (!a.back) return;
+  __syncthreads();
+  mid_product(wl, nxp, a.NX, a.Gx / 8, a.Gx, a.xb, xb, [&](int n, int, double re, double im) {
+    if (cc < a.C) a.t[(size_t)n * a.C + cc] = make_double2(re, im);
+  });
+}
+
+constexpr int kYzRows = 32;      // y rows of a k_mesh_yz block
+
+struct YzArgs {
+  int Gy, Gz, CN, NY, ctiles, ld;
+  const double2* in;             // [x][ny][nz]
+  const double* yb;
+  const double* zb;
+  double* grid;
+};
+
+// Block (32 y, x): y transform back of those rows, 16 nz at a time, into LDS
+// rows of (nz, re / im), then their z transform back
+__global__ void __launch_bounds__(kFtThreads) k_mesh_yz(YzArgs a) {
+  extern __shared__ double lds[];
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15, wave = wave_id();
+  const int y0 = blockIdx.x * kYzRows, x = blockIdx.y;
+  const int nyp = (a.NY + 15) & ~15;
+  const int ny = min(kYzRows, a.Gy - y0);
+  double* rows = lds;                                     // [kYzRows][ld]
+  double* pl = rows + (size_t)kYzRows * a.ld;             // [part][nyp][16]
+  double* xb = pl + 2 * (size_t)nyp * 16;
+  const double2* in = a.in + (size_t)x * a.NY * a.CN;
+  // the whole y operand has Gy / 8 tiles a step; this block's start at y0 / 8
+  for (int ct = 0; ct < a.ctiles; ++ct) {
+    for (int k = threadIdx.x; k < nyp * 16; k += kFtThreads) {
+      const int cc = 16 * ct + (k & 15), l = k >> 4;
+      double2 v = in[(size_t)min(l, a.NY - 1) * a.CN + min(cc, a.CN - 1)];
+      if (l >= a.NY || cc >= a.CN) v = make_double2(0.0, 0.0);
+      pl[k] = v.x;
+      pl[(size_t)nyp * 16 + k] = v.y;
+    }
+    __syncthreads();
+    const int sp = wave & 1, t = (wave >> 1);
+    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+    double* xw = xb + (wave >> 1) * 256 + lane;
+    if (8 * t < ny) {
+      const double* e = a.yb + ((size_t)(y0 / 8 + t) * 2 + sp) * 64 + lane;
+      const size_t es = (size_t)(a.Gy / 8) * 128;
+      const double* v = pl + (size_t)sp * nyp * 16 + 16 * g + c;
+      for (int l = 0; l < a.NY; l += 16) {
+        double ev[4], vv[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          ev[u] = e[(size_t)(l / 4 + u) * es];
+          vv[u] = v[(size_t)(l + 4 * u) * 16];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc = mma64(ev[u], vv[u], acc);
+      }
+      if (sp == 1) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) xw[64 * r] = acc[r];
+      }
+    }
+    __syncthreads();
+    if (sp == 0 && 8 * t < ny) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        double* o = rows + (size_t)(8 * t + 4 * h + g) * a.ld + 2 * (16 * ct + c);
+        o[0] = acc[2 * h] + xw[128 * h];
+        o[1] = acc[2 * h + 1] + xw[128 * h + 64];
+      }
+    }
+    __syncthreads();
+  }
+  const int ztiles = a.Gz / 16, units = (ny / 16) * ztiles;
+  for (int u = wave; u < units; u += kFtWaves) {
+    const int rt = u / ztiles, zt = u - rt * ztiles;
+    const double* r = rows + (size_t)(16 * rt + c) * a.ld + 4 * g;
+    const double* m = a.zb + (size_t)zt * 256 + lane;
+    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+    for (int k0 = 0; k0 < 32 * a.ctiles; k0 += 16) {
+      double b[4], v[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        b[s] = m[(size_t)(k0 / 16) * ztiles * 256 + 64 * s];
+        v[s] = r[k0 + s];
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s) acc = mma64(v[s], b[s], acc);
+    }
+    double* o = a.grid + ((size_t)x * a.Gy + y0 + 16 * rt) * a.Gz + 16 * zt + c;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) o[(size_t)(4 * q + g) * a.Gz] = acc[q];
+  }
+}
+
+// ---- gather -------------------------------------------------------------------
+// V's derivatives at the atoms.  One block per bin column (y tile, z tile) and
+// run of X window starts; the grid planes that its atoms' windows touch pass
+// through LDS kPlanes at a time, sixteen lanes an atom, lane = z point of the
+// window, so a group's reads are consecutive.  Each value serves phi and
+// dphi/dv of y, which lane j holds for row j and broadcasts within its row of
+// 16 lanes; x is applied per plane, z at the end.
+constexpr int kGatherThreads = 512;
+constexpr int kGatherAtoms = 2;  // atoms of a group in flight
+constexpr int kPlanes = 8;
+
+struct GatherArgs {
+  int n, X;
+  MeshGrid m;
+  const int32_t* start;
+  const int4* at;
+  const double *sx, *sy, *sz;
+  const double* coef;
+  const double* grid;
+  double* out;                   // [moments][n] by atom index
+};
+
+// t += sum over rows K .. K+3 of f(lane K of the row of 16 lanes) v: the
+// broadcast is part of the multiply.  The wait states that it needs after a
+// write of f's register are in the string.
+#define MESH_ROW4(t, f, v, K0, K1, K2, K3)                                      \
+  asm("s_nop 1\n\t"                                                             \
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #K0 " row_mask:0xf bank_mask:0xf\n\t" \
+      "v_fmac_f64_dpp %0, %1, %3 row_newbcast:" #K1 " row_mask:0xf bank_mask:0xf\n\t" \
+      "v_fmac_f64_dpp %0, %1, %4 row_newbcast:" #K2 " row_mask:0xf bank_mask:0xf\n\t" \
+      "v_fmac_f64_dpp %0, %1, %5 row_newbcast:" #K3 " row_mask:0xf bank_mask:0xf"     \
+      : "+v"(t)                                                                 \
+      : "v"(f), "v"((v)[K0]), "v"((v)[K1]), "v"((v)[K2]), "v"((v)[K3]))
+
+// sums over the W window rows of a plane: phi, dphi/dv and (SECOND)
+// d2phi/dv2 of y times the plane's values at the lane's z
+template <int W, int RZ, bool SECOND>
+__device__ __forceinline__ void row_sums(const double* p, double f, double d, double dd, double& t0, double& t1,
+                                         double& t2) {
+  double v[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) v[k] = k < W ? p[k * RZ] : 0.0;
+#define MESH_ROWS(K0, K1, K2, K3)     \
+  MESH_ROW4(t0, f, v, K0, K1, K2, K3); \
+  MESH_ROW4(t1, d, v, K0, K1, K2, K3); \
+  if constexpr (SECOND) MESH_ROW4(t2, dd, v, K0, K1, K2, K3)
+  MESH_ROWS(0, 1, 2, 3);
+  MESH_ROWS(4, 5, 6, 7);
+  MESH_ROWS(8, 9, 10, 11);
+  if constexpr (W == 16) {
+    MESH_ROWS(12, 13, 14, 15);
+  }
+#undef MESH_ROWS
+}
+#undef MESH_ROW4
+
+template <int W, int MOM>
+__global__ void __launch_bounds__(kGatherThreads) __attribute__((amdgpu_waves_per_eu(MOM == 9 ? 2 : 4)))
+k_mesh_gather(GatherArgs a) {
+  constexpr bool SECOND = MOM == 9;
+  constexpr int RY = kTile + W - 1, RZ = kTile + W;       // rows and padded row length of a staged plane
+  constexpr int GRP = kGatherThreads / 16, NS = GRP * kGatherAtoms;
+  __shared__ double plane[kPlanes][RY * RZ];
+  __shared__ double px[NS][W][SECOND ? 4 : 2];            // phi, dphi/dv (, d2phi/dv2) of x per atom in flight
+  const int Gx = a.m.G[0], Gy = a.m.G[1], Gz = a.m.G[2];
+  const int col = blockIdx.y, x0 = blockIdx.x * a.X, x1 = min(Gx, x0 + a.X);
+  const int ty = col / a.m.nzb, tz = col % a.m.nzb;
+  const int32_t* st = a.start + (size_t)col * Gx;
+  const int p0 = st[x0], p1 = st[x1];
+  if (p0 >= p1) return;
+  const int grp = threadIdx.x >> 4, j = threadIdx.x & 15;
+  const double sg = j < W / 2 ? 1.0 : -1.0;
+  const double fx = (double)Gx / MDFF_PI, fy = (double)Gy / MDFF_PI, fz = (double)Gz / MDFF_PI;
+  // staging: half a wave per row of a plane, lane = z
+  const int hz = threadIdx.x & 31;
+  int gz = kTile * tz + min(hz, RZ - 1);
+  gz = gz >= Gz ? gz - Gz : gz;
+  for (int base = p0; base < p1; base += NS) {
+    double py[kGatherAtoms], dy[kGatherAtoms], ey[kGatherAtoms], pz[kGatherAtoms], dz[kGatherAtoms], ez[kGatherAtoms];
+    double s0[kGatherAtoms], s1[kGatherAtoms], s2[kGatherAtoms], s3[kGatherAtoms], s4[kGatherAtoms], s5[kGatherAtoms];
+    int off[kGatherAtoms], xs[kGatherAtoms], idx[kGatherAtoms];
+    __syncthreads();
+    {
+      double c[2 * kPair];
+      load_piece<W>(a.coef, j, c);
+#pragma unroll
+      for (int r = 0; r < kGatherAtoms; ++r) {
+        const int p = base + r * GRP + grp;
+        const int4 at = a.at[min(p, p1 - 1)];
+        const int i = at.w;
+        idx[r] = p < p1 ? i : -1;
+        xs[r] = p < p1 ? at.x - x0 : -4 * kTile;          // no plane of the block touches an atom that is not there
+        off[r] = (at.y - kTile * ty) * RZ + (at.z - kTile * tz) + min(j, W - 1);
+        s0[r] = s1[r] = s2[r] = s3[r] = s4[r] = s5[r] = 0.0;
+        double f[3], df[3], d2[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          int l;
+          double t;
+          mesh_coord<W>(d == 0 ? a.sx[i] : (d == 1 ? a.sy[i] : a.sz[i]), a.m.G[d], l, t);
+          piece<true, SECOND>(c, 2.0 * t - 1.0, sg, f[d], df[d], d2[d]);
+        }
+        if (j < W) {
+          const int slot = r * GRP + grp;
+          px[slot][j][0] = f[0];
+          px[slot][j][1] = df[0];
+          if constexpr (SECOND) px[slot][j][2] = d2[0];
+        }
+        // lanes beyond the window hold zeros (their pieces have none)
+        py[r] = f[1]; dy[r] = df[1]; ey[r] = SECOND ? d2[1] : 0.0;
+        pz[r] = f[2]; dz[r] = df[2]; ez[r] = SECOND ? d2[2] : 0.0;
+      }
+    }
+    const int xend = x1 - x0 + W - 1;                     // planes x0 .. x0 + xend - 1
+    for (int c0 = 0; c0 < xend; c0 += kPlanes) {
+      const int np = min(kPlanes, xend - c0);
+      __syncthreads();
+      for (int row = threadIdx.x >> 5; row < np * RY; row += kGatherThreads / 32) {
+        const int pl = row / RY, yy = row - pl * RY;
+        int gx = x0 + c0 + pl, gy = kTile * ty + yy;
+        gx = gx >= 2 * Gx ? gx - 2 * Gx : (gx >= Gx ? gx - Gx : gx);
+        gy = gy >= Gy ? gy - Gy : gy;
+        const double v = a.grid[((size_t)gx * Gy + gy) * Gz + gz];
+        if (hz < RZ) plane[pl][yy * RZ + hz] = v;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < kGatherAtoms; ++r) {
+        const int slot = r * GRP + grp;
+        const int pb = max(0, xs[r] - c0), pe = min(np, xs[r] + W - c0);
+        for (int pl = pb; pl < pe; ++pl) {
+          const int xi = c0 + pl - xs[r];
+          double t0 = 0.0, t1 = 0.0, t2 = 0.0;
+          row_sums<W, RZ, SECOND>(plane[pl] + off[r], py[r], dy[r], ey[r], t0, t1, t2);
+          const double ax = px[slot][xi][0], bx = px[slot][xi][1];
+          s0[r] = fma(bx, t0, s0[r]);                     // phi' phi
+          s1[r] = fma(ax, t1, s1[r]);                     // phi  phi'
+          s2[r] = fma(ax, t0, s2[r]);                     // phi  phi
+          if constexpr (SECOND) {
+            const double cx = px[slot][xi][2];
+            s3[r] = fma(cx, t0, s3[r]);                   // phi'' phi
+            s4[r] = fma(ax, t2, s4[r]);                   // phi  phi''
+            s5[r] = fma(bx, t1, s5[r]);                   // phi' phi'
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < kGatherAtoms; ++r) {
+      double m[9] = {fx * (pz[r] * s0[r]), fy * (pz[r] * s1[r]), fz * (dz[r] * s2[r])};
+      if constexpr (SECOND) {
+        m[3] = -(fx * fx) * (pz[r] * s3[r]);
+        m[4] = -(fy * fy) * (pz[r] * s4[r]);
+        m[5] = -(fz * fz) * (ez[r] * s2[r]);
+        m[6] = -(fx * fy) * (pz[r] * s5[r]);
+        m[7] = -(fx * fz) * (dz[r] * s0[r]);
+        m[8] = -(fy * fz) * (dz[r] * s1[r]);
+      }
+#pragma unroll
+      for (int k = 0; k < MOM; ++k) {
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) m[k] += __shfl_xor(m[k], o, 16);
+        if (j == 0 && idx[r] >= 0) a.out[(size_t)k * a.n + idx[r]] = m[k];
+      }
+    }
+  }
+}
+
+// ---- host: kernel, grid and tables ------------------------------------------
+
+typedef long double ld;
+const ld kPiL = 3.14159265358979323846264338327950288L;
+
+// x I1(x): the kernel's profile up to a constant, by its series
+ld bessel_xi1(ld x) {
+  const ld y = x * x / 4;
+  ld t = x * x / 2, s = t;
+  for (int k = 1; k < 400 && t > s * 1e-22L; ++k) {
+    t *= y / ((ld)k * (k + 1));
+    s += t;
+  }
+  return s;
+}
+
+// transform of the kernel at frequency f (cycles per grid spacing), times a
+// constant common to all f
+template <typename R>
+R kernel_hat(int w, R beta, R f) {
+  const R h = (R)w / 2, a = 2 * (R)kPiL * f * h, z2 = beta * beta - a * a;
+  if (std::fabs(z2) < (R)1e-6) return (R)1 / 3 + z2 / 30;
+  const R z = std::sqrt(std::fabs(z2));
+  if (z2 > 0) return (z * std::cosh(z) - std::sinh(z)) / (z * z2);
+  return (std::sin(z) - z * std::cos(z)) / (z * -z2);
+}
+
+// The alias error of the gradient of V from one direction, relative to the
+// terms that carry the force: mode n of weight a(n) >= A(n)/A(0) comes with
+// modes n + jG of weight phih(n + jG) / phih(n), each differentiated.  The
+// force itself sits at n* = alpha |a| / (pi sqrt 2).  Measured errors are
+// about 3 times this.  Stops where it exceeds `enough`.
+double mesh_error(int K, double aL, int G, int w, double beta, double enough) {
+  const double pi = MDFF_PI, nstar = std::max(1.0, aL / (pi * sqrt(2.0)));
+  double worst = 0.0;
+  for (int n = K; n >= 0 && worst <= enough * nstar; --n) {
+    double e = 0.0;
+    for (int j = 1; j <= 2; ++j)
+      for (int sg = -1; sg <= 1; sg += 2) {
+        const double m = n + (double)sg * j * G;
+        e += fabs(kernel_hat<double>(w, beta, m / G)) * fabs(m);
+      }
+    const double an = exp(-(pi * n / aL) * (pi * n / aL));
+    worst = std::max(worst, an * e / kernel_hat<double>(w, beta, (double)n / G));
+  }
+  return worst / nstar;
+}
+
+// Grids (multiples of the tile, at least the 2K + 1 modes and w) and the beta
+// they share, with an error below tol in every direction: the beta whose
+// grids have the fewest points.  false: none up to 4 (2K + 1) points.
+bool choose_grid(const int* K, const double* aL, int w, double tol, int* G, double& beta) {
+  double best = 0.0;
+  for (double r = 1.5; r < 3.0; r += 0.05) {
+    int g[3];
+    double cells = 1.0;
+    for (int d = 0; d < 3 && cells > 0.0; ++d) {
+      if (d > 0 && K[d] == K[d - 1] && aL[d] == aL[d - 1]) {
+        g[d] = g[d - 1];
+      } else {
+        const int lo = std::max(w, 2 * K[d] + 1), hi = 4 * lo + 2 * kTile;
+        g[d] = div_up(lo, kTile) * kTile;
+        while (g[d] <= hi && mesh_error(K[d], aL[d], g[d], w, r * w, tol) > tol) g[d] += kTile;
+        if (g[d] > hi) cells = 0.0;
+      }
+      cells *= g[d];
+      if (best > 0.0 && cells > best) cells = 0.0;
+    }
+    if (cells > 0.0 && (best == 0.0 || cells < best)) {
+      best = cells;
+      beta = r * w;
+      for (int d = 0; d < 3; ++d) G[d] = g[d];
+    }
+  }
+  return best > 0.0;
+}
+
+// pieces of phi on v in [-1, 1] (piece j: x = j - w/2 + (v + 1)/2) as
+// polynomials through the Chebyshev nodes; coef[j][even | odd]
+void kernel_pieces(int w, double beta, std::vector<double>& coef) {
+  constexpr int M = kDeg + 1;
+  ld T[M][M] = {};
+  T[0][0] = 1;
+  T[1][1] = 1;
+  for (int k = 2; k < M; ++k)
+    for (int c = 0; c < M; ++c) T[k][c] = (c ? 2 * T[k - 1][c - 1] : 0) - T[k - 2][c];
+  const ld top = bessel_xi1(beta);
+  coef.assign((size_t)(w / 2) * M, 0.0);
+  for (int j = 0; j < w / 2; ++j) {
+    ld y[M], mono[M] = {};
+    for (int a = 0; a < M; ++a) {
+      const ld v = cosl((a + 0.5L) * kPiL / M);
+      const ld x = (j - (ld)w / 2 + (v + 1) / 2) / ((ld)w / 2);
+      const ld s2 = 1 - x * x;
+      y[a] = s2 > 0 ? bessel_xi1((ld)beta * sqrtl(s2)) / top : 0;
+    }
+    for (int k = 0; k < M; ++k) {
+      ld ck = 0;
+      for (int a = 0; a < M; ++a) ck += y[a] * cosl(k * (a + 0.5L) * kPiL / M);
+      ck *= (k ? 2.0L : 1.0L) / M;
+      for (int c = 0; c <= k; ++c) mono[c] += ck * T[k][c];
+    }
+    for (int k = 0; k < M; ++k) coef[(size_t)j * M + (k & 1) * kPair + k / 2] = (double)mono[k];
+  }
+}
+
+// 1 / phih(n) for n = 0..K, phi as the pieces have it (x I1(x) over its top)
+std::vector<ld> deconv(int w, double beta, int K, int G) {
+  std::vector<ld> d(K + 1);
+  const ld h = (ld)w / 2, b = beta;
+  for (int n = 0; n <= K; ++n) d[n] = bessel_xi1(b) / (2 * h * b * b * kernel_hat<ld>(w, b, (ld)n / G));
+  return d;
+}
+
+// e^{2 pi i a / G} for every a
+struct Roots {
+  std::vector<ld> c, s;
+  explicit Roots(int G) : c(G), s(G) {
+    for (int a = 0; a < G; ++a) {
+      c[a] = cosl(2 * kPiL * a / G);
+      s[a] = sinl(2 * kPiL * a / G);
+    }
+  }
+  size_t at(long long a) const {
+    const long long G = (long long)c.size();
+    return (size_t)(((a % G) + G) % G);
+  }
+};
+
+// operand order of a row product for an M of K rows and N columns
+template <typename F>
+std::vector<double> row_operand(int K, int N, F value) {
+  const int kc = div_up(K, 16), nt = div_up(N, 16);
+  std::vector<double> m((size_t)kc * nt * 256, 0.0);
+  for (int k = 0; k < K; ++k)
+    for (int n = 0; n < N; ++n) {
+      const int g = (k & 15) >> 2, s = k & 3;
+      m[(((size_t)(k / 16) * nt + n / 16) * 4 + s) * 64 + 16 * g + (n & 15)] = value(k, n);
+    }
+  return m;
+}
+
+// operand order of a mid product for E of N rows and L columns (zero up to
+// the next 16 of L)
+template <typename F>
+std::vector<double> mid_operand(int N, int L, F value) {
+  const int lc = 4 * div_up(L, 16), nt = div_up(N, 8);
+  std::vector<double> m((size_t)lc * nt * 128, 0.0);
+  for (int l = 0; l < L; ++l)
+    for (int n = 0; n < N; ++n) {
+      ld re, im;
+      value(n, l, re, im);
+      const int nl = n & 7, g = l & 3;
+      double* t = m.data() + ((size_t)(l / 4) * nt + n / 8) * 128;
+      for (int part = 0; part < 2; ++part) {
+        const int R = 8 * (nl >> 2) + 4 * part + (nl & 3);
+        t[16 * g + R] = (double)(part ? im : re);
+        t[64 + 16 * g + R] = (double)(part ? re : -im);
+      }
+    }
+  return m;
+}
+
+int upload(mdff_ctx* c, const std::vector<double>& v, double** p) {
+  HIP_TRY(c, hipMalloc((void**)p, sizeof(double) * v.size()));
+  HIP_TRY(c, hipMemcpy(*p, v.data(), sizeof(double) * v.size(), hipMemcpyHostToDevice));
+  return MDFF_OK;
+}
+
+}  // namespace
+
+struct MeshRecip {
+  int w = 0, dip = 0, second = 0;
+  MeshGrid m{};
+  int K[3] = {0, 0, 0}, CN = 0;            // CN = Kz + 1 complex columns
+  int nbins = 0, shares = 1, X = 8, nblk = 0, ctiles = 0, ld = 0;
+  size_t lds_zy = 0, lds_x = 0, lds_yz = 0;
+  int sorted = 0;                          // bins and phi belong to the current coordinates
+  int counted = 0;                         // k_mesh_bin has run and the scan has not
+  double *zf = nullptr, *zb = nullptr, *yf = nullptr, *yb = nullptr, *xf = nullptr, *xb = nullptr;
+  double *coef = nullptr, *A = nullptr, *kvec = nullptr;
+  int32_t *key = nullptr, *slot = nullptr, *cnt = nullptr, *start = nullptr, *order = nullptr;
+  int4* at = nullptr;
+  double4* amp = nullptr;
+  double *phi = nullptr, *grid = nullptr, *mom = nullptr, *blk = nullptr;
+  double2* t = nullptr;
+};
+
+void mesh_free(mdff_ctx* c) {
+  MeshRecip* m = c->mesh;
+  if (!m) return;
+  void* ps[] = {m->zf, m->zb, m->yf, m->yb, m->xf, m->xb, m->coef, m->A, m->kvec, m->key, m->slot, m->cnt, m->start,
+                m->order, m->at, m->amp, m->phi, m->grid, m->mom, m->blk, m->t};
+  for (void* p : ps)
+    if (p) (void)hipFree(p);
+  delete m;
+  c->mesh = nullptr;
+}
+
+// A and kvec: the k mesh of recip_setup ([nx][ny][nz], nx >= 0, A = 0 outside
+// the half space).  Leaves c->mesh null where no grid meets the error bound.
+int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<double>& kv) {
+  const int n = c->n;
+  const bool mixed = c->d.precision == MDFF_PREC_MIXED;
+  const int w = mixed ? 12 : 16;
+  const double tol = mixed ? 1e-9 : 4e-15;
+  int G[3];
+  double aL[3], beta = 0.0;
+  for (int d = 0; d < 3; ++d) {
+    const double* a = c->A + 3 * d;
+    aL[d] = c->alpha * sqrt(a[0] * a[0] + a[1] * a[1] + a[2] * a[2]);
+  }
+  if (!choose_grid(c->K, aL, w, tol, G, beta)) return MDFF_OK;
+  if ((double)G[0] * G[1] * G[2] > 536870912.0) return MDFF_OK;   // 4 GiB of grid
+  // LDS of the transforms (doubles: planes and the waves' exchange)
+  const int nyp = (2 * c->K[1] + 16) & ~15, nxp = (2 * c->K[0] + 16) & ~15;
+  const int ctiles = div_up(c->K[2] + 1, 16), yld = 32 * ctiles + 2;
+  const size_t xch = (size_t)kFtWaves / 2 * 256;
+  const size_t lds_zy = 8 * (2 * (size_t)G[1] * 16 + xch), lds_x = 8 * (32 * ((size_t)G[0] + nxp) + xch),
+               lds_yz = 8 * ((size_t)kYzRows * yld + 2 * (size_t)nyp * 16 + xch);
+  int maxlds = 0;
+  HIP_TRY(c, hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device));
+  if (std::max({lds_zy, lds_x, lds_yz}) > (size_t)maxlds) return MDFF_OK;
+  HIP_TRY(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mesh_zy), hipFuncAttributeMaxDynamicSharedMemorySize, maxlds));
+  HIP_TRY(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mesh_x), hipFuncAttributeMaxDynamicSharedMemorySize, maxlds));
+  HIP_TRY(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mesh_yz), hipFuncAttributeMaxDynamicSharedMemorySize, maxlds));
+  MeshRecip* m = new MeshRecip();
+  c->mesh = m;
+  m->w = w;
+  m->ctiles = ctiles;
+  m->ld = yld;
+  m->lds_zy = lds_zy;
+  m->lds_x = lds_x;
+  m->lds_yz = lds_yz;
+  m->dip = (c->task_qd || c->task_dd) ? 1 : 0;
+  for (int d = 0; d < 3; ++d) {
+    m->m.G[d] = G[d];
+    m->K[d] = c->K[d];
+  }
+  m->m.nyb = G[1] / kTile;
+  m->m.nzb = G[2] / kTile;
+  m->nbins = G[0] * m->m.nyb * m->m.nzb;
+  const int tiles = (G[0] / kTile) * m->m.nyb * m->m.nzb;
+  // blocks of the spread: shares of a tile's four bin columns until every
+  // CU has a block
+  m->shares = tiles >= 192 ? 1 : (tiles >= 96 ? 2 : 4);
+  // window starts per gather block: about as many atoms as it has in flight
+  const double per_x = (double)n / m->nbins;
+  const int flight = kGatherThreads / 16 * kGatherAtoms;
+  m->X = std::max(2, std::min(16, (int)(0.9 * flight / std::max(per_x, 1e-3))));
+  m->CN = c->K[2] + 1;
+  const int Kx = c->K[0], Ky = c->K[1], Kz = c->K[2], CN = m->CN, NX = 2 * Kx + 1, NY = 2 * Ky + 1;
+  std::vector<double> coef;
+  kernel_pieces(w, beta, coef);
+  MDFF_TRY(upload(c, coef, &m->coef));
+  const std::vector<ld> dx = deconv(w, beta, Kx, G[0]), dy = deconv(w, beta, Ky, G[1]),
+                        dz = deconv(w, beta, Kz, G[2]);
+  const Roots rz(G[2]);
+  // z: column tile 2 ct + part holds that part of nz = 16 ct ..; back, row
+  // k = 2 nz + part
+  MDFF_TRY(upload(c, row_operand(G[2], 32 * ctiles, [&](int k, int col) {
+                    const int nz = 16 * (col / 32) + (col & 15);
+                    if (nz >= CN) return 0.0;
+                    const size_t a = rz.at((long long)nz * k);
+                    return (double)(((col & 16) ? rz.s[a] : rz.c[a]) * dz[nz]);
+                  }), &m->zf));
+  MDFF_TRY(upload(c, row_operand(32 * ctiles, G[2], [&](int k, int z) {
+                    if (k >= 2 * CN) return 0.0;
+                    const size_t a = rz.at((long long)(k >> 1) * z);
+                    return (double)(((k & 1) ? -rz.s[a] : rz.c[a]) * dz[k >> 1]);
+                  }), &m->zb));
+  auto mid = [&](int K, int g, const std::vector<ld>& dd, double** f, double** b) -> int {
+    const Roots r(g);
+    auto value = [&](int nn, int l, ld& re, ld& im) {
+      const size_t a = r.at((long long)(nn - K) * l);
+      re = r.c[a] * dd[std::abs(nn - K)];
+      im = r.s[a] * dd[std::abs(nn - K)];
+    };
+    MDFF_TRY(upload(c, mid_operand(2 * K + 1, g, value), f));
+    return upload(c, mid_operand(g, 2 * K + 1, [&](int l, int nn, ld& re, ld& im) { value(nn, l, re, im); }), b);
+  };
+  MDFF_TRY(mid(Ky, G[1], dy, &m->yf, &m->yb));
+  MDFF_TRY(mid(Kx, G[0], dx, &m->xf, &m->xb));
+  // A and k on nz >= 0: an entry and its opposite are one term, so nz = 0
+  // keeps half of each of the two
+  const size_t nk = (size_t)NX * NY * CN;
+  std::vector<double> Am(nk), km(4 * nk);
+  for (int x = -Kx; x <= Kx; ++x)
+    for (int y = -Ky; y <= Ky; ++y)
+      for (int z = 0; z <= Kz; ++z) {
+        const size_t o = ((size_t)(x + Kx) * NY + (y + Ky)) * CN + z;
+        auto src = [&](int a, int b, int e) { return ((size_t)a * c->NYk + (b + Ky)) * c->NZk + (e + Kz); };
+        double v, sg = 1.0;
+        size_t at;
+        if (x >= 0 && A[src(x, y, z)] != 0.0) at = src(x, y, z);
+        else if (x <= 0) { at = src(-x, -y, -z); sg = -1.0; }
+        else at = src(x, y, z);
+        v = A[at];
+        Am[o] = z == 0 ? 0.5 * v : v;
+        for (int k = 0; k < 3; ++k) km[4 * o + k] = sg * kv[4 * at + k];
+        km[4 * o + 3] = kv[4 * at + 3];
+      }
+  MDFF_TRY(upload(c, Am, &m->A));
+  MDFF_TRY(upload(c, km, &m->kvec));
+  const int nr = m->dip ? 6 : 3;
+  const size_t gcells = (size_t)G[0] * G[1] * G[2];
+  HIP_TRY(c, hipMalloc((void**)&m->key, sizeof(int32_t) * n));
+  HIP_TRY(c, hipMalloc((void**)&m->slot, sizeof(int32_t) * n));
+  HIP_TRY(c, hipMalloc((void**)&m->order, sizeof(int32_t) * n));
+  HIP_TRY(c, hipMalloc((void**)&m->cnt, sizeof(int32_t) * m->nbins));
+  HIP_TRY(c, hipMemset(m->cnt, 0, sizeof(int32_t) * m->nbins));
+  HIP_TRY(c, hipMalloc((void**)&m->start, sizeof(int32_t) * (m->nbins + 1)));
+  HIP_TRY(c, hipMalloc((void**)&m->at, sizeof(int4) * n));
+  HIP_TRY(c, hipMalloc((void**)&m->phi, sizeof(double) * nr * w * (size_t)n));
+  if (m->dip) HIP_TRY(c, hipMalloc((void**)&m->amp, sizeof(double4) * n));
+  HIP_TRY(c, hipMalloc((void**)&m->grid, sizeof(double) * gcells * m->shares));
+  HIP_TRY(c, hipMalloc((void**)&m->t, sizeof(double2) * (size_t)G[0] * NY * CN));
+  HIP_TRY(c, hipMalloc((void**)&m->mom, sizeof(double) * 9 * (size_t)n));
+  m->nblk = div_up((int64_t)NY * CN, 16);
+  HIP_TRY(c, hipMalloc((void**)&m->blk, sizeof(double) * 7 * m->nblk));
+  return MDFF_OK;
+}
+
+// s = B^T r (from_r) and the bin counts; pack: also the pair kernel's atoms.
+// The previous MD step's queued sums ride along.
+int mesh_bin(mdff_ctx* c, bool from_r, bool pack) {
+  MeshRecip* m = c->mesh;
+  if (m->counted)   // an evaluation that ended early left its counts: the scan clears them
+    hipLaunchKernelGGL(k_mesh_scan, dim3(1), dim3(1024), 0, c->stream, m->nbins, m->cnt, m->start);
+  BinArgs a{};
+  a.n = c->n;
+  a.from_r = from_r ? 1 : 0;
+  a.pack = pack ? 1 : 0;
+  a.m = m->m;
+  a.rx = c->rx; a.ry = c->ry; a.rz = c->rz;
+  for (int k = 0; k < 9; ++k) a.b[k] = c->B[k];
+  a.sx = c->sx; a.sy = c->sy; a.sz = c->sz;
+  a.key = m->key;
+  a.slot = m->slot;
+  a.cnt = m->cnt;
+  a.order = c->cell_atoms;
+  a.q = c->q;
+  a.itype = c->itype;
+  a.rec = c->arec;
+  a.meta = c->ameta;
+  const int nbx = div_up(c->n, 256);
+  if (c->nfin > nbx) MDFF_TRY(flush_finals(c));
+  const FinalBatch fb = from_r ? take_finals(c) : FinalBatch{};
+  const bool extra = fb.nfin > 0 || fb.seq_out;
+  const dim3 grid(nbx, extra ? 2 : 1);
+  m->counted = 1;
+  m->sorted = 0;
+  if (m->w == 16)
+    PROF_LAUNCH(c, PK_TABLES,
+                hipLaunchKernelGGL(k_mesh_bin<16>, grid, dim3(256), 0, c->stream, a, fb, extra ? 1 : -1));
+  else
+    PROF_LAUNCH(c, PK_TABLES,
+                hipLaunchKernelGGL(k_mesh_bin<12>, grid, dim3(256), 0, c->stream, a, fb, extra ? 1 : -1));
+  HIP_TRY(c, hipGetLastError());
+  return MDFF_OK;
+}
+
+// bins to sorted atoms and their kernel values
+static int mesh_sort(mdff_ctx* c) {
+  MeshRecip* m = c->mesh;
+  if (m->sorted) return MDFF_OK;
+  const int n = c->n;
+  PROF_LAUNCH(c, PK_TABLES,
+              hipLaunchKernelGGL(k_mesh_scan, dim3(1), dim3(1024), 0, c->stream, m->nbins, m->cnt, m->start));
+  PROF_LAUNCH(c, PK_TABLES,
+              hipLaunchKernelGGL(k_mesh_scatter, dim3(div_up(n, 256)), dim3(256), 0, c->stream, n, m->key, m->slot,
+                                 m->start, m->order));
+  PhiArgs a{};
+  a.n = n;
+  a.m = m->m;
+  a.sx = c->sx; a.sy = c->sy; a.sz = c->sz;
+  a.key = m->key;
+  a.start = m->start;
+  a.order = m->order;
+  a.coef = m->coef;
+  a.at = m->at;
+  a.phi = m->phi;
+  const dim3 grid(std::min(2048, div_up(n, 16)));
+  if (m->w == 16) {
+    if (m->dip) PROF_LAUNCH(c, PK_TABLES, hipLaunchKernelGGL((k_mesh_phi<16, true>), grid, dim3(256), 0, c->stream, a));
+    else PROF_LAUNCH(c, PK_TABLES, hipLaunchKernelGGL((k_mesh_phi<16, false>), grid, dim3(256), 0, c->stream, a));
+  } else {
+    if (m->dip) PROF_LAUNCH(c, PK_TABLES, hipLaunchKernelGGL((k_mesh_phi<12, true>), grid, dim3(256), 0, c->stream, a));
+    else PROF_LAUNCH(c, PK_TABLES, hipLaunchKernelGGL((k_mesh_phi<12, false>), grid, dim3(256), 0, c->stream, a));
+  }
+  HIP_TRY(c, hipGetLastError());
+  m->counted = 0;
+  m->sorted = 1;
+  return MDFF_OK;
+}
+
+template <int W>
+static void launch_spread(mdff_ctx* c, const SpreadArgs& a, bool dip, dim3 grid) {
+  if (dip) PROF_LAUNCH(c, PK_SK, hipLaunchKernelGGL((k_mesh_spread<W, true>), grid, dim3(1024), 0, c->stream, a));
+  else PROF_LAUNCH(c, PK_SK, hipLaunchKernelGGL((k_mesh_spread<W, false>), grid, dim3(1024), 0, c->stream, a));
+}
+
+template <int W>
+static void launch_gather(mdff_ctx* c, const GatherArgs& a, int mom, dim3 grid) {
+  if (mom == 9)
+    PROF_LAUNCH(c, PK_GATHER, hipLaunchKernelGGL((k_mesh_gather<W, 9>), grid, dim3(kGatherThreads), 0, c->stream, a));
+  else
+    PROF_LAUNCH(c, PK_GATHER, hipLaunchKernelGGL((k_mesh_gather<W, 3>), grid, dim3(kGatherThreads), 0, c->stream, a));
+}
+
+// S, W, the 7 energy / stress sums into e_out (queued), and with mom = 3 or 9
+// the moments of every atom; *out: [mom][n]
+int mesh_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool use_mu, int mom, double* e_out,
+              const double** out) {
+  MeshRecip* m = c->mesh;
+  MDFF_TRY(mesh_sort(c));
+  const int n = c->n;
+  const int Gx = m->m.G[0], Gy = m->m.G[1], Gz = m->m.G[2];
+  const int NX = 2 * m->K[0] + 1, NY = 2 * m->K[1] + 1, CN = m->CN;
+  if (use_mu) {
+    const double* b = c->B;
+    PROF_LAUNCH(c, PK_SK, hipLaunchKernelGGL(k_mesh_amp, dim3(div_up(n, 256)), dim3(256), 0, c->stream, n, m->at, q,
+                                             use_q ? 1 : 0, mu, b[0], b[1], b[2], b[3], b[4], b[5], b[6], b[7], b[8],
+                                             -2.0 * Gx, -2.0 * Gy, -2.0 * Gz, m->amp));
+  }
+  SpreadArgs sa{};
+  sa.n = n;
+  sa.shares = m->shares;
+  sa.pstride = (m->dip ? 6 : 3) * m->w;
+  sa.m = m->m;
+  sa.start = m->start;
+  sa.at = m->at;
+  sa.phi = m->phi;
+  sa.q = use_q ? q : c->zeros;
+  sa.amp = m->amp;
+  sa.out = m->grid;
+  const dim3 sg((Gx / kTile) * m->m.nyb * m->m.nzb, m->shares);
+  if (m->w == 16) launch_spread<16>(c, sa, use_mu, sg);
+  else launch_spread<12>(c, sa, use_mu, sg);
+  ZyArgs za{};
+  za.Gy = Gy; za.Gz = Gz; za.CN = CN; za.NY = NY;
+  za.ctiles = m->ctiles;
+  za.shares = m->shares;
+  za.sstride = (size_t)Gx * Gy * Gz;
+  za.grid = m->grid;
+  za.zf = m->zf; za.yf = m->yf;
+  za.out = m->t;
+  PROF_LAUNCH(c, PK_SKRED, hipLaunchKernelGGL(k_mesh_zy, dim3(m->ctiles, Gx), dim3(kFtThreads), m->lds_zy, c->stream, za));
+  MDFF_TRY(claim_partials(c, m->blk));
+  XArgs xa{};
+  xa.Gx = Gx; xa.NX = NX; xa.C = NY * CN;
+  xa.back = mom > 0 ? 1 : 0;
+  xa.xf = m->xf; xa.xb = m->xb;
+  xa.t = m->t;
+  xa.A = m->A; xa.kvec = m->kvec; xa.blk = m->blk;
+  PROF_LAUNCH(c, PK_SKRED, hipLaunchKernelGGL(k_mesh_x, dim3(m->nblk), dim3(kFtThreads), m->lds_x, c->stream, xa));
+  if (e_out) MDFF_TRY(queue_final(c, m->blk, m->nblk, 7, e_out));
+  if (mom > 0) {
+    YzArgs ya{};
+    ya.Gy = Gy; ya.Gz = Gz; ya.CN = CN; ya.NY = NY;
+    ya.ctiles = m->ctiles;
+    ya.ld = m->ld;
+    ya.in = m->t;
+    ya.yb = m->yb; ya.zb = m->zb;
+    ya.grid = m->grid;
+    PROF_LAUNCH(c, PK_SKRED, hipLaunchKernelGGL(k_mesh_yz, dim3(div_up(Gy, kYzRows), Gx), dim3(kFtThreads), m->lds_yz,
+                                                c->stream, ya));
+    GatherArgs ga{};
+    ga.n = n;
+    ga.X = m->X;
+    ga.m = m->m;
+    ga.start = m->start;
+    ga.at = m->at;
+    ga.sx = c->sx; ga.sy = c->sy; ga.sz = c->sz;
+    ga.coef = m->coef;
+    ga.grid = m->grid;
+    ga.out = m->mom;
+    const dim3 gg(div_up(Gx, m->X), m->m.nyb * m->m.nzb);
+    if (m->w == 16) launch_gather<16>(c, ga, mom, gg);
+    else launch_gather<12>(c, ga, mom, gg);
+    *out = m->mom;
+  }
+  HIP_TRY(c, hipGetLastError());
+  return MDFF_OK;
+}

@@ -2436,6 +2436,15 @@ int recip_setup(mdff_ctx* c) {
   HIP_TRY(c, hipMalloc((void**)&c->kvec, sizeof(double) * 4 * nb));
   HIP_TRY(c, hipMemcpy(c->kA, A.data(), sizeof(double) * nb, hipMemcpyHostToDevice));
   HIP_TRY(c, hipMemcpy(c->kvec, kv.data(), sizeof(double) * 4 * nb, hipMemcpyHostToDevice));
+  {
+    const char* ev = getenv("MDFF_RECIP_MESH");
+    const char* f32 = getenv("MDFF_RECIP_F32MMA");
+    const bool on = ev && ev[0] ? ev[0] != '0' : (double)c->n * nb > 8e7;
+    if (on && c->use_mma && !(f32 && f32[0])) {
+      MDFF_TRY(mesh_setup(c, A, kv));
+      if (c->mesh) return MDFF_OK;
+    }
+  }
   const size_t tsz = c->rec_f32 ? sizeof(cplx<float>) : sizeof(cplx<double>);
   const int ncol = Kx + Ky + Kz + 3;
   HIP_TRY(c, hipMalloc(&c->tab, tsz * ncol * (size_t)c->n));
@@ -2580,6 +2589,7 @@ int recip_setup(mdff_ctx* c) {
 }
 
 void recip_free(mdff_ctx* c) {
+  mesh_free(c);
   void* ps[] = {c->kA, c->kvec, c->tab, c->sk_part, c->sk, c->wk, c->wk_t, c->rec_part, c->amat, c->rec_blk,
                 c->amat_h3, c->ascale_h3, c->kA_mask, c->kA_in, c->kvec_in, c->sk_in_part, c->wk_in, c->tab_in, c->wt_in,
                 c->mu_pscale, c->dip_part};
@@ -2622,6 +2632,7 @@ static void tables_r_t(mdff_ctx* c, bool pack) {
 }
 
 int recip_tables_from_r(mdff_ctx* c, bool pack) {
+  if (c->mesh) return mesh_bin(c, true, pack);
   if (c->rec_f32) tables_r_t<float>(c, pack);
   else tables_r_t<double>(c, pack);
   HIP_TRY(c, hipGetLastError());
@@ -2629,6 +2640,7 @@ int recip_tables_from_r(mdff_ctx* c, bool pack) {
 }
 
 int recip_tables(mdff_ctx* c) {
+  if (c->mesh) return mesh_bin(c, false, false);
   if (c->rec_f32) tables_t<float>(c);
   else tables_t<double>(c);
   HIP_TRY(c, hipGetLastError());
@@ -2651,6 +2663,33 @@ template <typename T>
 static void launch_sk_mma2(int ctm, dim3 grid, size_t lds, hipStream_t st, const Sm2Args& sm) {
   void* args[] = {const_cast<Sm2Args*>(&sm)};
   (void)hipLaunchKernel(sk_kernel<T>(ctm, sm.TA), grid, dim3(256), args, lds, st);
+}
+
+// the fields and forces from the moments of the splits; forces wanted with no
+// output array: the caller's force kernel finishes them (c->rfin)
+static int rec_finish(mdff_ctx* c, const double* part, int nsplit, int moments, const double* q, const double* mu,
+                      bool use_q, bool forces, bool field, double* ef_out, double* f_out) {
+  RecFinal rf{};
+  rf.n = c->n;
+  rf.nsplit = nsplit;
+  rf.moments = moments;
+  rf.use_q = use_q ? 1 : 0;
+  rf.part = part;
+  rf.q = q;
+  rf.mu = mu;
+  for (int k = 0; k < 9; ++k) rf.b[k] = c->B[k];
+  rf.fpi_V = 2.0 * (2.0 * MDFF_PI / c->omega);
+  const bool defer = forces && !f_out;
+  if (defer) {
+    c->rfin = rf;
+    c->rfin_pending = 1;
+  }
+  if (field || !defer)
+    PROF_LAUNCH(c, PK_GFINAL,
+                hipLaunchKernelGGL(k_gather_final, dim3(div_up(c->n, 256)), dim3(256), 0, c->stream, rf,
+                                   field ? 1 : 0, (forces && !defer) ? 1 : 0, ef_out, f_out));
+  HIP_TRY(c, hipGetLastError());
+  return MDFF_OK;
 }
 
 template <typename T>
@@ -2951,33 +2990,17 @@ static int eval_t(mdff_ctx* c, const double* q, const double* mu, bool use_q, bo
     }
     nsplit += c->kin_splits * c->kin_jb;
   }
-  RecFinal rf{};
-  rf.n = c->n;
-  rf.nsplit = nsplit;
-  rf.moments = moments;
-  rf.use_q = use_q ? 1 : 0;
-  rf.part = c->rec_part;
-  rf.q = q;
-  rf.mu = mu;
-  for (int k = 0; k < 9; ++k) rf.b[k] = c->B[k];
-  rf.fpi_V = 2.0 * (2.0 * MDFF_PI / c->omega);
-  // forces wanted with no output array: the caller's force kernel finishes
-  // them from the split partials (c->rfin)
-  const bool defer = forces && !f_out;
-  if (defer) {
-    c->rfin = rf;
-    c->rfin_pending = 1;
-  }
-  if (field || !defer)
-    PROF_LAUNCH(c, PK_GFINAL,
-                hipLaunchKernelGGL(k_gather_final, dim3(div_up(c->n, 256)), dim3(256), 0, c->stream, rf,
-                                   field ? 1 : 0, (forces && !defer) ? 1 : 0, ef_out, f_out));
-  HIP_TRY(c, hipGetLastError());
-  return MDFF_OK;
+  return rec_finish(c, c->rec_part, nsplit, moments, q, mu, use_q, forces, field, ef_out, f_out);
 }
 
 int recip_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool use_mu, bool forces,
                bool field, double* ef_out, double* f_out, double* e_out) {
+  if (c->mesh) {
+    const int moments = !forces && !field ? 0 : (forces && use_mu ? 9 : 3);
+    const double* part = nullptr;
+    MDFF_TRY(mesh_eval(c, q, mu, use_q, use_mu, moments, e_out, &part));
+    return moments ? rec_finish(c, part, 1, moments, q, mu, use_q, forces, field, ef_out, f_out) : MDFF_OK;
+  }
   if (c->rec_f32) return eval_t<float>(c, q, mu, use_q, use_mu, forces, field, ef_out, f_out, e_out);
   return eval_t<double>(c, q, mu, use_q, use_mu, forces, field, ef_out, f_out, e_out);
 }
