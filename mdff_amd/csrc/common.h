@@ -476,8 +476,7 @@ void recip_free(mdff_ctx* c);
 // the same sums as non-uniform fast transforms (mesh.hip)
 int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<double>& kv);
 int mesh_bin(mdff_ctx* c, bool from_r, bool pack);
-int mesh_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool use_mu, int mom, double* e_out,
-              const double** out);
+int mesh_eval(mdff_ctx* c, const double* mu, bool use_q, bool use_mu, int mom, double* e_out, const double** out);
 void mesh_free(mdff_ctx* c);
 // electric field gradient (efg.hip; its real-space part in realspace.hip)
 int realspace_efg(mdff_ctx* c, double* out);

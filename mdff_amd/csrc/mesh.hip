@@ -146,9 +146,9 @@ __global__ void __launch_bounds__(256) k_mesh_bin(BinArgs a, FinalBatch fb, int 
   }
 }
 
-// start[0..nb] = prefix sums of cnt[0..nb), one block; cnt is left zero for
-// the next evaluation
-__global__ void __launch_bounds__(1024) k_mesh_scan(int nb, int32_t* __restrict__ cnt, int32_t* __restrict__ start) {
+// start[0..nb] = prefix sums of cnt[0..nb), one block (many bins; few: the
+// scatter forms them)
+__global__ void __launch_bounds__(1024) k_mesh_scan(int nb, const int32_t* __restrict__ cnt, int32_t* __restrict__ start) {
   __shared__ int ws[16];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   int base = 0;
@@ -177,7 +177,6 @@ __global__ void __launch_bounds__(1024) k_mesh_scan(int nb, int32_t* __restrict_
     for (int u = 0; u < 4; ++u)
       if (k0 + u < nb) {
         start[k0 + u] = at;
-        cnt[k0 + u] = 0;
         at += c[u];
       }
     base += all;
@@ -186,20 +185,86 @@ __global__ void __launch_bounds__(1024) k_mesh_scan(int nb, int32_t* __restrict_
   if (threadIdx.x == 0) start[nb] = base;
 }
 
-__global__ void __launch_bounds__(256) k_mesh_scatter(int n, const int32_t* __restrict__ key,
-                                                      const int32_t* __restrict__ slot,
-                                                      const int32_t* __restrict__ start, int32_t* __restrict__ order) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) order[start[key[i]] + slot[i]] = i;
+__global__ void k_mesh_clear(int nb, int32_t* __restrict__ cnt) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < nb) cnt[k] = 0;
+}
+
+// an atom among those of its bin: fractional coordinates, index, bin
+struct alignas(16) BinAtom {
+  double x, y, z;
+  int32_t i, bin;
+};
+
+struct ScatterArgs {
+  int n, nb;
+  const int32_t *key, *slot, *cnt;
+  int32_t* start;                // prefix sums of cnt: read, or (SCAN) written
+  const double *sx, *sy, *sz;
+  BinAtom* order;
+};
+
+// SCAN: every block forms the prefix sums itself (a launch less: 4.5 us of a
+// 24,000-ion step), 256 runs of bins, then the atom's bin within its run; block
+// 0 stores them.  For up to kScanBins bins, whose counts the blocks can all
+// read in the time of one launch.
+constexpr int kScanBins = 8192;
+template <bool SCAN>
+__global__ void __launch_bounds__(256) k_mesh_scatter(ScatterArgs a) {
+  __shared__ int base[257];
+  __shared__ int ws[4];
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int ic = min(i, a.n - 1);
+  const int bin = a.key[ic], slot = a.slot[ic];
+  const double x = a.sx[ic], y = a.sy[ic], z = a.sz[ic];
+  int first;
+  if constexpr (SCAN) {
+    const int run = (a.nb + 255) / 256, k0 = threadIdx.x * run, k1 = min(a.nb, k0 + run);
+    int mine = 0;
+#pragma unroll 8
+    for (int k = k0; k < k1; ++k) mine += a.cnt[k];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int v = mine;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(v, o, 64);
+      if (lane >= o) v += t;
+    }
+    if (lane == 63) ws[w] = v;
+    __syncthreads();
+    int before = v - mine;
+    for (int u = 0; u < w; ++u) before += ws[u];
+    base[threadIdx.x] = before;
+    __syncthreads();
+    const int r0 = bin / run;
+    first = base[r0];
+#pragma unroll 8
+    for (int k = r0 * run; k < bin; ++k) first += a.cnt[k];
+    if (blockIdx.x == 0) {
+      int at = before;
+      for (int k = k0; k < k1; ++k) {
+        a.start[k] = at;
+        at += a.cnt[k];
+      }
+      if (threadIdx.x == 0) a.start[a.nb] = a.n;
+    }
+  } else {
+    first = a.start[bin];
+  }
+  if (i < a.n) a.order[first + slot] = BinAtom{x, y, z, i, bin};
 }
 
 struct PhiArgs {
   int n;
   MeshGrid m;
-  const double *sx, *sy, *sz;
-  const int32_t *key, *start, *order;
+  const BinAtom* order;
+  const int32_t* start;
+  int32_t* cnt;                  // the bins' counts, cleared for the next evaluation
+  int nb;
+  const double* q;
   const double* coef;            // [W/2][2][kPair] pieces of phi, even and odd coefficients
   int4* at;                      // per sorted atom: window start (x, y, z), atom index
+  double4* vt;                   // v = 2t - 1 of x, y, z, charge
   double* phi;                   // [atom][3][W], with dip [atom][6][W]: phi, then dphi/dv
 };
 
@@ -243,35 +308,41 @@ __device__ __forceinline__ void piece(const double c[2 * kPair], double v, doubl
 }
 
 template <int W, bool DIP>
-__global__ void __launch_bounds__(256) k_mesh_phi(PhiArgs a) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DIP ? 4 : 6))) k_mesh_phi(PhiArgs a) {
   constexpr int NR = DIP ? 6 : 3;
   const int j = threadIdx.x & 15, step = gridDim.x * 16;
   double c[2 * kPair];
   load_piece<W>(a.coef, j, c);
   const double sg = j < W / 2 ? 1.0 : -1.0;
+  for (int k = blockIdx.x * 256 + threadIdx.x; k < a.nb; k += gridDim.x * 256) a.cnt[k] = 0;
   for (int p0 = blockIdx.x * 16 + (threadIdx.x >> 4); p0 < a.n; p0 += step) {
-    const int i = a.order[p0];
-    const int bin = a.key[i];
-    const double s[3] = {a.sx[i], a.sy[i], a.sz[i]};
-    const int b0 = a.start[bin], b1 = a.start[bin + 1];
+    const BinAtom me = a.order[p0];
+    const int i = me.i;
+    const double s[3] = {me.x, me.y, me.z}, qi = a.q[i];
+    const int b0 = a.start[me.bin], b1 = a.start[me.bin + 1];
     int rank = 0;
-    for (int k = b0 + j; k < b1; k += 16) rank += a.order[k] < i ? 1 : 0;
+    for (int k = b0 + j; k < b1; k += 16) rank += a.order[k].i < i ? 1 : 0;
 #pragma unroll
     for (int o = 8; o > 0; o >>= 1) rank += __shfl_xor(rank, o, 16);
     const size_t p = (size_t)b0 + rank;
     double* out = a.phi + p * (NR * W) + j;
     int l[3];
+    double v[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       double t, f, df = 0.0, d2 = 0.0;
       mesh_coord<W>(s[d], a.m.G[d], l[d], t);
-      piece<DIP, false>(c, 2.0 * t - 1.0, sg, f, df, d2);
+      v[d] = 2.0 * t - 1.0;
+      piece<DIP, false>(c, v[d], sg, f, df, d2);
       if (j < W) {
         out[d * W] = f;
         if (DIP) out[(3 + d) * W] = df;
       }
     }
-    if (j == 0) a.at[p] = make_int4(l[0], l[1], l[2], i);
+    if (j == 0) {
+      a.at[p] = make_int4(l[0], l[1], l[2], i);
+      a.vt[p] = make_double4(v[0], v[1], v[2], qi);
+    }
   }
 }
 
@@ -305,23 +376,28 @@ struct SpreadArgs {
   MeshGrid m;
   const int32_t* start;
   const int4* at;
+  const double4* vt;             // .w: charge (without dipoles)
   const double* phi;
-  const double* q;               // without dipoles
   const double4* amp;            // with dipoles
   double* out;                   // [share][Gx][Gy][Gz]
 };
 
 template <int W, bool DIP>
 __global__ void __launch_bounds__(1024) k_mesh_spread(SpreadArgs a) {
-  constexpr int NA = DIP ? 64 : 128;                      // atoms of a chunk
-  constexpr int NR = DIP ? 6 : 3;                         // rows per atom: x, y, z (times q), and for dipoles
-                                                          // x: q phi + m phi', phi; y: phi, m phi'; z: phi, m phi'
-  __shared__ double rows[NR][NA][kTile];
+  constexpr int U = DIP ? 1 : 2;                          // staging passes of a chunk
+  constexpr int NA = 64 * U;                              // atoms of a chunk
+  constexpr int NR = DIP ? 2 : 1;
+  // per atom: y and z rows (phi, and for dipoles m phi'), and by x plane q phi
+  // (+ m phi') and, for dipoles, phi (padded against bank conflicts)
+  __shared__ double ry[NR][NA + 16][kTile], rz[NR][NA + 16][kTile], rx[NR][kTile][NA + 18];
   const int Gx = a.m.G[0], Gy = a.m.G[1], Gz = a.m.G[2];
-  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15, grp = threadIdx.x >> 4;
   const int wave = wave_id();
-  const int tile = blockIdx.x, share = blockIdx.y;
-  const int tz = tile % a.m.nzb, ty = (tile / a.m.nzb) % a.m.nyb, tx = tile / (a.m.nzb * a.m.nyb);
+  // tiles x fastest, in XCD order: an XCD's tiles share bin columns
+  const int ntx = Gx / kTile;
+  const int lin = xcd_order(blockIdx.x, (int)gridDim.x);
+  const int tx = lin % ntx, share = (lin / ntx) % a.shares, yz = lin / (ntx * a.shares);
+  const int tz = yz % a.m.nzb, ty = yz / a.m.nzb;
   const int x0 = kTile * tx, x = x0 + wave;
   f64x4 acc = {0.0, 0.0, 0.0, 0.0};
   for (int col = share; col < 4; col += a.shares) {
@@ -329,6 +405,10 @@ __global__ void __launch_bounds__(1024) k_mesh_spread(SpreadArgs a) {
     int by = ty - (col & 1), bz = tz - (col >> 1);
     by = by < 0 ? by + a.m.nyb : by;
     bz = bz < 0 ? bz + a.m.nzb : bz;
+    // the window's offset in the tile: its own column, or the one before (a
+    // single tile wraps onto itself: both, from one column)
+    const int oy = c + ((col & 1) ? kTile : 0), oz = c + ((col & 2) ? kTile : 0);
+    const bool wy = a.m.nyb == 1, wz = a.m.nzb == 1;
     const int32_t* st = a.start + (size_t)(by * a.m.nzb + bz) * Gx;
     // lx in [x0 - W + 1, x0 + 15]; below zero they are at the other end of
     // the row, from x0 + 16 at the earliest (part 1)
@@ -340,63 +420,87 @@ __global__ void __launch_bounds__(1024) k_mesh_spread(SpreadArgs a) {
       const int wl = x - W + 1 + (part == 0 ? 0 : Gx);
       const int w0 = max(wl, f0), w1 = part == 0 ? x + 1 : Gx;
       const int q0 = st[f0], q1 = st[f1];
+      if (q0 >= q1) continue;
       // (a grid of one tile wraps onto itself: every atom, for every plane)
       const bool whole = Gx == kTile;
       const int own0 = whole ? q0 : (w0 < w1 ? st[w0] : 0), own1 = whole ? q1 : (w0 < w1 ? st[w1] : 0);
-      for (int p0 = q0; p0 < q1; p0 += NA) {
-        const int na = min(NA, q1 - p0);
-        __syncthreads();
-        // rows: thread -> point c of atom (threadIdx.x >> 4) + 64 k
-        for (int at0 = threadIdx.x >> 4; at0 < ((na + 3) & ~3); at0 += 64) {
-          const int pc = p0 + min(at0, na - 1);
-          const int4 at = a.at[pc];
+      const int ox = x0 + c + (part == 0 ? 0 : Gx);
+      // the next chunk's atoms and the chunk after's places are on their way
+      // while a chunk is summed
+      double vx[NR][U], vy[NR][U], vz[NR][U];
+      int4 at[U];
+      auto load_at = [&](int p0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) at[u] = a.at[min(p0 + grp + 64 * u, q1 - 1)];
+      };
+      auto load_phi = [&](int p0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int p = p0 + grp + 64 * u, pc = min(p, q1 - 1);
           const double* f = a.phi + (size_t)pc * a.pstride;
-          int dx = x0 + c - at.x, dy = kTile * ty + c - at.y, dz = kTile * tz + c - at.z;
-          dx = dx < 0 ? dx + Gx : dx;
-          dy = dy < 0 ? dy + Gy : dy;
-          dz = dz < 0 ? dz + Gz : dz;
-          const bool ok = at0 < na;
-          const bool okx = ok && dx < W, oky = dy < W, okz = dz < W;
-          dx = min(dx, W - 1);
-          dy = min(dy, W - 1);
-          dz = min(dz, W - 1);
-          const double fx = f[dx], fy = f[W + dy], fz = f[2 * W + dz];
+          int dx = ox - at[u].x, dy = oy - (at[u].y & (kTile - 1)), dz = oz - (at[u].z & (kTile - 1));
+          if (whole) dx &= kTile - 1;
+          if (wy) dy &= kTile - 1;
+          if (wz) dz &= kTile - 1;
+          const bool okx = p < q1 && (unsigned)dx < (unsigned)W, oky = (unsigned)dy < (unsigned)W,
+                     okz = (unsigned)dz < (unsigned)W;
+          const unsigned ux = min((unsigned)dx, W - 1u), uy = min((unsigned)dy, W - 1u), uz = min((unsigned)dz, W - 1u);
+          const double fx = f[ux], fy = f[W + uy], fz = f[2 * W + uz];
           if constexpr (DIP) {
             const double4 m = a.amp[pc];
-            const double gx = f[3 * W + dx], gy = f[4 * W + dy], gz = f[5 * W + dz];
-            rows[0][at0][c] = okx ? m.x * fx + m.y * gx : 0.0;
-            rows[1][at0][c] = oky ? fy : 0.0;
-            rows[2][at0][c] = okz ? fz : 0.0;
-            rows[3][at0][c] = okx ? fx : 0.0;
-            rows[4][at0][c] = oky ? m.z * gy : 0.0;
-            rows[5][at0][c] = okz ? m.w * gz : 0.0;
+            const double gx = f[3 * W + ux], gy = f[4 * W + uy], gz = f[5 * W + uz];
+            vx[0][u] = okx ? m.x * fx + m.y * gx : 0.0;
+            vx[1][u] = okx ? fx : 0.0;
+            vy[1][u] = oky ? m.z * gy : 0.0;
+            vz[1][u] = okz ? m.w * gz : 0.0;
           } else {
-            rows[0][at0][c] = okx ? a.q[at.w] * fx : 0.0;
-            rows[1][at0][c] = oky ? fy : 0.0;
-            rows[2][at0][c] = okz ? fz : 0.0;
+            vx[0][u] = okx ? a.vt[pc].w * fx : 0.0;
           }
+          vy[0][u] = oky ? fy : 0.0;
+          vz[0][u] = okz ? fz : 0.0;
         }
+      };
+      load_at(q0);
+      load_phi(q0);
+      load_at(q0 + NA);
+      for (int p0 = q0; p0 < q1; p0 += NA) {
         __syncthreads();
-        const int s0 = max(own0 - p0, 0) >> 2, s1 = (min(own1 - p0, na) + 3) >> 2;
-        for (int t0 = s0; t0 < s1; t0 += 4) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int r = 0; r < NR; ++r) {
+            rx[r][c][grp + 64 * u] = vx[r][u];
+            ry[r][grp + 64 * u][c] = vy[r][u];
+            rz[r][grp + 64 * u][c] = vz[r][u];
+          }
+        __syncthreads();
+        if (p0 + NA < q1) {
+          load_phi(p0 + NA);
+          load_at(p0 + 2 * NA);
+        }
+        const int s0 = max(own0 - p0, 0) >> 2, s1 = (min(own1 - p0, NA) + 3) >> 2;
+        const double* px = &rx[0][wave][g];
+        const double* py = &ry[0][g][c];
+        const double* pz = &rz[0][g][c];
+        constexpr int SX = kTile * (NA + 18), SY = (NA + 16) * kTile;   // to the second row set
+        for (int t = s0; t < s1; t += 4) {
           double av[4], bv[4], cv[4], dv[4];
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            const int k = 4 * min(t0 + u, s1 - 1) + g;
-            const double ax = rows[0][k][wave], ay = rows[1][k][c];
-            bv[u] = rows[2][k][c];
+            const double ax = px[4 * (t + u)], ay = py[64 * (t + u)];
+            bv[u] = pz[64 * (t + u)];
             if constexpr (DIP) {
-              const double cx = rows[3][k][wave], cy = rows[4][k][c];
-              av[u] = ax * ay + cx * cy;
+              const double cx = px[SX + 4 * (t + u)];
+              av[u] = ax * ay + cx * py[SY + 64 * (t + u)];
               cv[u] = cx * ay;
-              dv[u] = rows[5][k][c];
+              dv[u] = pz[SY + 64 * (t + u)];
             } else {
               av[u] = ax * ay;
             }
           }
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            if (t0 + u >= s1) break;
+            if (t + u >= s1) break;
             acc = mma64(av[u], bv[u], acc);
             if constexpr (DIP) acc = mma64(cv[u], dv[u], acc);
           }
@@ -425,6 +529,23 @@ __global__ void __launch_bounds__(1024) k_mesh_spread(SpreadArgs a) {
 //    of a wave; their sums meet in LDS.
 constexpr int kFtThreads = 1024, kFtWaves = 16;
 
+// the tile's operand (e, es doubles between steps of 4 l) times the LDS rows v
+// over L (operand and rows up to the next 16)
+__device__ __forceinline__ f64x4 mid_chain(const double* e, size_t es, const double* v, int L) {
+  f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+  for (int l = 0; l < L; l += 16) {
+    double ev[4], vv[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      ev[u] = e[(size_t)(l / 4 + u) * es];
+      vv[u] = v[(size_t)(l + 4 * u) * 16];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) acc = mma64(ev[u], vv[u], acc);
+  }
+  return acc;
+}
+
 // in: LDS planes [re, im][l][16], rows up to the next 16 finite; out(n, c, value)
 template <typename Out>
 __device__ __forceinline__ void mid_product(const double* in, int lrows, int L, int ntiles, int N, const double* E,
@@ -436,20 +557,7 @@ __device__ __forceinline__ void mid_product(const double* in, int lrows, int L, 
   for (int t0 = 0; t0 < ntiles; t0 += kFtWaves / 2) {
     const int t = t0 + (wave >> 1);
     f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-    if (t < ntiles) {
-      const double* e = E + ((size_t)t * 2 + sp) * 64 + lane;
-      const size_t es = (size_t)ntiles * 128;
-      for (int l = 0; l < L; l += 16) {
-        double ev[4], vv[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          ev[u] = e[(size_t)(l / 4 + u) * es];
-          vv[u] = v[(size_t)(l + 4 * u) * 16];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) acc = mma64(ev[u], vv[u], acc);
-      }
-    }
+    if (t < ntiles) acc = mid_chain(E + ((size_t)t * 2 + sp) * 64 + lane, (size_t)ntiles * 128, v, L);
     if (sp == 1) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) x[64 * r] = acc[r];
@@ -467,7 +575,7 @@ __device__ __forceinline__ void mid_product(const double* in, int lrows, int L, 
 }
 
 struct ZyArgs {
-  int Gy, Gz, CN, NY, ctiles, shares;
+  int Gy, Gz, CN, NY, ctiles;
   size_t sstride;                // between the shares of the grid, which are added
   const double* grid;
   const double* zf;              // row operand: column tile 2 ct + part
@@ -476,7 +584,8 @@ struct ZyArgs {
 };
 
 // Block (nz tile, x): z transform of the plane's rows at 16 nz into LDS, then
-// their y transform
+// their y transform.  SH: shares of the grid
+template <int SH>
 __global__ void __launch_bounds__(kFtThreads) k_mesh_zy(ZyArgs a) {
   extern __shared__ double lds[];
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15, wave = wave_id();
@@ -489,34 +598,35 @@ __global__ void __launch_bounds__(kFtThreads) k_mesh_zy(ZyArgs a) {
     const double* in = a.grid + ((size_t)x * a.Gy + 16 * rt + c) * a.Gz + 4 * g;
     const double* m = a.zf + ((size_t)2 * ct + part) * 256 + lane;
     f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-    for (int k0 = 0; k0 < a.Gz; k0 += 16) {
-      double2 v0 = *reinterpret_cast<const double2*>(in + k0);
-      double2 v1 = *reinterpret_cast<const double2*>(in + k0 + 2);
-      double b[4];
+    for (int k0 = 0; k0 < a.Gz; k0 += 32) {
+      // the second of the two steps repeats a valid one when Gz ends before it
+      const int kk[2] = {k0, min(k0 + 16, a.Gz - 16)};
+      double2 v[2][SH][2];
+      double b[2][4];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) b[s] = m[(size_t)(k0 / 16) * a.ctiles * 512 + 64 * s];
-      if (a.shares == 4) {
-        double2 w0[3], w1[3];
+      for (int h = 0; h < 2; ++h) {
 #pragma unroll
-        for (int s = 0; s < 3; ++s) {
-          w0[s] = *reinterpret_cast<const double2*>(in + (s + 1) * a.sstride + k0);
-          w1[s] = *reinterpret_cast<const double2*>(in + (s + 1) * a.sstride + k0 + 2);
+        for (int s = 0; s < SH; ++s) {
+          v[h][s][0] = *reinterpret_cast<const double2*>(in + s * a.sstride + kk[h]);
+          v[h][s][1] = *reinterpret_cast<const double2*>(in + s * a.sstride + kk[h] + 2);
         }
 #pragma unroll
-        for (int s = 0; s < 3; ++s) {
-          v0.x += w0[s].x; v0.y += w0[s].y;
-          v1.x += w1[s].x; v1.y += w1[s].y;
-        }
-      } else if (a.shares == 2) {
-        const double2 w0 = *reinterpret_cast<const double2*>(in + a.sstride + k0);
-        const double2 w1 = *reinterpret_cast<const double2*>(in + a.sstride + k0 + 2);
-        v0.x += w0.x; v0.y += w0.y;
-        v1.x += w1.x; v1.y += w1.y;
+        for (int s = 0; s < 4; ++s) b[h][s] = m[(size_t)(kk[h] / 16) * a.ctiles * 512 + 64 * s];
       }
-      acc = mma64(v0.x, b[0], acc);
-      acc = mma64(v0.y, b[1], acc);
-      acc = mma64(v1.x, b[2], acc);
-      acc = mma64(v1.y, b[3], acc);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (h == 1 && k0 + 16 >= a.Gz) break;
+        double2 v0 = v[h][0][0], v1 = v[h][0][1];
+#pragma unroll
+        for (int s = 1; s < SH; ++s) {
+          v0.x += v[h][s][0].x; v0.y += v[h][s][0].y;
+          v1.x += v[h][s][1].x; v1.y += v[h][s][1].y;
+        }
+        acc = mma64(v0.x, b[h][0], acc);
+        acc = mma64(v0.y, b[h][1], acc);
+        acc = mma64(v1.x, b[h][2], acc);
+        acc = mma64(v1.y, b[h][3], acc);
+      }
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) pl[((size_t)part * a.Gy + 16 * rt + 4 * r + g) * 16 + c] = acc[r];
@@ -622,46 +732,39 @@ __global__ void __launch_bounds__(kFtThreads) k_mesh_yz(YzArgs a) {
   const int nyp = (a.NY + 15) & ~15;
   const int ny = min(kYzRows, a.Gy - y0);
   double* rows = lds;                                     // [kYzRows][ld]
-  double* pl = rows + (size_t)kYzRows * a.ld;             // [part][nyp][16]
-  double* xb = pl + 2 * (size_t)nyp * 16;
+  double* pl = rows + (size_t)kYzRows * a.ld;             // [nz tile][part][nyp][16]
+  double* xb = pl + 4 * (size_t)nyp * 16;
   const double2* in = a.in + (size_t)x * a.NY * a.CN;
-  // the whole y operand has Gy / 8 tiles a step; this block's start at y0 / 8
-  for (int ct = 0; ct < a.ctiles; ++ct) {
-    for (int k = threadIdx.x; k < nyp * 16; k += kFtThreads) {
-      const int cc = 16 * ct + (k & 15), l = k >> 4;
+  // the whole y operand has Gy / 8 tiles a step; this block's start at y0 / 8.
+  // Two nz tiles at a time, eight waves each: (n tile, re / im input)
+  const int sp = wave & 1, t = (wave >> 1) & 3, half = wave >> 3;
+  double* xw = xb + (wave >> 1) * 256 + lane;
+  for (int ct0 = 0; ct0 < a.ctiles; ct0 += 2) {
+    const int nct = min(2, a.ctiles - ct0);
+    for (int k = threadIdx.x; k < nct * nyp * 16; k += kFtThreads) {
+      const int h = k >= nyp * 16 ? 1 : 0, kk = k - h * nyp * 16;
+      const int cc = 16 * (ct0 + h) + (kk & 15), l = kk >> 4;
       double2 v = in[(size_t)min(l, a.NY - 1) * a.CN + min(cc, a.CN - 1)];
       if (l >= a.NY || cc >= a.CN) v = make_double2(0.0, 0.0);
-      pl[k] = v.x;
-      pl[(size_t)nyp * 16 + k] = v.y;
+      pl[(size_t)(2 * h) * nyp * 16 + kk] = v.x;
+      pl[(size_t)(2 * h + 1) * nyp * 16 + kk] = v.y;
     }
     __syncthreads();
-    const int sp = wave & 1, t = (wave >> 1);
     f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-    double* xw = xb + (wave >> 1) * 256 + lane;
-    if (8 * t < ny) {
-      const double* e = a.yb + ((size_t)(y0 / 8 + t) * 2 + sp) * 64 + lane;
-      const size_t es = (size_t)(a.Gy / 8) * 128;
-      const double* v = pl + (size_t)sp * nyp * 16 + 16 * g + c;
-      for (int l = 0; l < a.NY; l += 16) {
-        double ev[4], vv[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          ev[u] = e[(size_t)(l / 4 + u) * es];
-          vv[u] = v[(size_t)(l + 4 * u) * 16];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) acc = mma64(ev[u], vv[u], acc);
-      }
+    const bool on = 8 * t < ny && half < nct;
+    if (on) {
+      acc = mid_chain(a.yb + ((size_t)(y0 / 8 + t) * 2 + sp) * 64 + lane, (size_t)(a.Gy / 8) * 128,
+                      pl + (size_t)(2 * half + sp) * nyp * 16 + 16 * g + c, a.NY);
       if (sp == 1) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) xw[64 * r] = acc[r];
       }
     }
     __syncthreads();
-    if (sp == 0 && 8 * t < ny) {
+    if (sp == 0 && on) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        double* o = rows + (size_t)(8 * t + 4 * h + g) * a.ld + 2 * (16 * ct + c);
+        double* o = rows + (size_t)(8 * t + 4 * h + g) * a.ld + 2 * (16 * (ct0 + half) + c);
         o[0] = acc[2 * h] + xw[128 * h];
         o[1] = acc[2 * h + 1] + xw[128 * h + 64];
       }
@@ -674,15 +777,14 @@ __global__ void __launch_bounds__(kFtThreads) k_mesh_yz(YzArgs a) {
     const double* r = rows + (size_t)(16 * rt + c) * a.ld + 4 * g;
     const double* m = a.zb + (size_t)zt * 256 + lane;
     f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-    for (int k0 = 0; k0 < 32 * a.ctiles; k0 += 16) {
-      double b[4], v[4];
+    for (int k0 = 0; k0 < 32 * a.ctiles; k0 += 32) {
+      double b[8], v[8];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        b[s] = m[(size_t)(k0 / 16) * ztiles * 256 + 64 * s];
-        v[s] = r[k0 + s];
-      }
+      for (int s = 0; s < 8; ++s) b[s] = m[(size_t)(k0 / 16 + (s >> 2)) * ztiles * 256 + 64 * (s & 3)];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) acc = mma64(v[s], b[s], acc);
+      for (int s = 0; s < 8; ++s) v[s] = r[k0 + 16 * (s >> 2) + (s & 3)];
+#pragma unroll
+      for (int s = 0; s < 8; ++s) acc = mma64(v[s], b[s], acc);
     }
     double* o = a.grid + ((size_t)x * a.Gy + y0 + 16 * rt) * a.Gz + 16 * zt + c;
 #pragma unroll
@@ -699,52 +801,106 @@ __global__ void __launch_bounds__(kFtThreads) k_mesh_yz(YzArgs a) {
 // 16 lanes; x is applied per plane, z at the end.
 constexpr int kGatherThreads = 512;
 constexpr int kGatherAtoms = 2;  // atoms of a group in flight
-constexpr int kPlanes = 8;
 
 struct GatherArgs {
   int n, X;
   MeshGrid m;
   const int32_t* start;
   const int4* at;
-  const double *sx, *sy, *sz;
+  const double4* vt;
   const double* coef;
   const double* grid;
   double* out;                   // [moments][n] by atom index
 };
 
-// t += sum over rows K .. K+3 of f(lane K of the row of 16 lanes) v: the
-// broadcast is part of the multiply.  The wait states that it needs after a
-// write of f's register are in the string.
-#define MESH_ROW4(t, f, v, K0, K1, K2, K3)                                      \
-  asm("s_nop 1\n\t"                                                             \
-      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #K0 " row_mask:0xf bank_mask:0xf\n\t" \
-      "v_fmac_f64_dpp %0, %1, %3 row_newbcast:" #K1 " row_mask:0xf bank_mask:0xf\n\t" \
-      "v_fmac_f64_dpp %0, %1, %4 row_newbcast:" #K2 " row_mask:0xf bank_mask:0xf\n\t" \
-      "v_fmac_f64_dpp %0, %1, %5 row_newbcast:" #K3 " row_mask:0xf bank_mask:0xf"     \
-      : "+v"(t)                                                                 \
-      : "v"(f), "v"((v)[K0]), "v"((v)[K1]), "v"((v)[K2]), "v"((v)[K3]))
+// t += sum over the window rows k of f(lane k of the row of 16 lanes) v[k], and
+// u with d: the broadcast is part of the multiply.  The wait states that it
+// needs after a write of f's or d's register are in the string.
+__device__ __forceinline__ void fma_rows12(const double* v, double f, double d, double& t, double& u) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %2, %4 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %4 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %5 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %5 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %6 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %6 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %7 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %7 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %8 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %8 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %9 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %9 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %10 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %10 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %11 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %11 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %12 row_newbcast:8 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %12 row_newbcast:8 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %13 row_newbcast:9 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %13 row_newbcast:9 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %14 row_newbcast:10 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %14 row_newbcast:10 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %15 row_newbcast:11 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %15 row_newbcast:11 row_mask:0xf bank_mask:0xf\n\t"
+      : "+v"(t), "+v"(u)
+      : "v"(f), "v"(d), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]), "v"(v[8]), "v"(v[9]), "v"(v[10]), "v"(v[11]));
+}
+__device__ __forceinline__ void fma_rows16(const double* v, double f, double d, double& t, double& u) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %2, %4 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %4 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %5 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %5 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %6 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %6 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %7 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %7 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %8 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %8 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %9 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %9 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %10 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %10 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %11 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %11 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %12 row_newbcast:8 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %12 row_newbcast:8 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %13 row_newbcast:9 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %13 row_newbcast:9 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %14 row_newbcast:10 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %14 row_newbcast:10 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %15 row_newbcast:11 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %15 row_newbcast:11 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %16 row_newbcast:12 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %16 row_newbcast:12 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %17 row_newbcast:13 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %17 row_newbcast:13 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %18 row_newbcast:14 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %18 row_newbcast:14 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %19 row_newbcast:15 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %3, %19 row_newbcast:15 row_mask:0xf bank_mask:0xf\n\t"
+      : "+v"(t), "+v"(u)
+      : "v"(f), "v"(d), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]), "v"(v[8]), "v"(v[9]), "v"(v[10]), "v"(v[11]), "v"(v[12]), "v"(v[13]), "v"(v[14]), "v"(v[15]));
+}
 
 // sums over the W window rows of a plane: phi, dphi/dv and (SECOND)
 // d2phi/dv2 of y times the plane's values at the lane's z
 template <int W, int RZ, bool SECOND>
 __device__ __forceinline__ void row_sums(const double* p, double f, double d, double dd, double& t0, double& t1,
                                          double& t2) {
-  double v[16];
+  double v[W], unused = 0.0;
 #pragma unroll
-  for (int k = 0; k < 16; ++k) v[k] = k < W ? p[k * RZ] : 0.0;
-#define MESH_ROWS(K0, K1, K2, K3)     \
-  MESH_ROW4(t0, f, v, K0, K1, K2, K3); \
-  MESH_ROW4(t1, d, v, K0, K1, K2, K3); \
-  if constexpr (SECOND) MESH_ROW4(t2, dd, v, K0, K1, K2, K3)
-  MESH_ROWS(0, 1, 2, 3);
-  MESH_ROWS(4, 5, 6, 7);
-  MESH_ROWS(8, 9, 10, 11);
+  for (int k = 0; k < W; ++k) v[k] = p[k * RZ];
   if constexpr (W == 16) {
-    MESH_ROWS(12, 13, 14, 15);
+    fma_rows16(v, f, d, t0, t1);
+    if constexpr (SECOND) fma_rows16(v, dd, dd, t2, unused);
+  } else {
+    fma_rows12(v, f, d, t0, t1);
+    if constexpr (SECOND) fma_rows12(v, dd, dd, t2, unused);
   }
-#undef MESH_ROWS
 }
-#undef MESH_ROW4
+
+constexpr int kPlanes = 8;       // staged planes
 
 template <int W, int MOM>
 __global__ void __launch_bounds__(kGatherThreads) __attribute__((amdgpu_waves_per_eu(MOM == 9 ? 2 : 4)))
@@ -752,10 +908,12 @@ k_mesh_gather(GatherArgs a) {
   constexpr bool SECOND = MOM == 9;
   constexpr int RY = kTile + W - 1, RZ = kTile + W;       // rows and padded row length of a staged plane
   constexpr int GRP = kGatherThreads / 16, NS = GRP * kGatherAtoms;
-  __shared__ double plane[kPlanes][RY * RZ];
+  __shared__ double plane[kPlanes * RY * RZ];
   __shared__ double px[NS][W][SECOND ? 4 : 2];            // phi, dphi/dv (, d2phi/dv2) of x per atom in flight
   const int Gx = a.m.G[0], Gy = a.m.G[1], Gz = a.m.G[2];
-  const int col = blockIdx.y, x0 = blockIdx.x * a.X, x1 = min(Gx, x0 + a.X);
+  // x runs fastest, in XCD order: an XCD's blocks share bin columns and planes
+  const int lin = xcd_order(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
+  const int col = lin / (int)gridDim.x, x0 = (lin % (int)gridDim.x) * a.X, x1 = min(Gx, x0 + a.X);
   const int ty = col / a.m.nzb, tz = col % a.m.nzb;
   const int32_t* st = a.start + (size_t)col * Gx;
   const int p0 = st[x0], p1 = st[x1];
@@ -764,36 +922,32 @@ k_mesh_gather(GatherArgs a) {
   const double sg = j < W / 2 ? 1.0 : -1.0;
   const double fx = (double)Gx / MDFF_PI, fy = (double)Gy / MDFF_PI, fz = (double)Gz / MDFF_PI;
   // staging: half a wave per row of a plane, lane = z
-  const int hz = threadIdx.x & 31;
+  const int hz = threadIdx.x & 31, row0 = threadIdx.x >> 5;
   int gz = kTile * tz + min(hz, RZ - 1);
   gz = gz >= Gz ? gz - Gz : gz;
+  const int xend = x1 - x0 + W - 1;                       // planes x0 .. x0 + xend - 1
   for (int base = p0; base < p1; base += NS) {
     double py[kGatherAtoms], dy[kGatherAtoms], ey[kGatherAtoms], pz[kGatherAtoms], dz[kGatherAtoms], ez[kGatherAtoms];
     double s0[kGatherAtoms], s1[kGatherAtoms], s2[kGatherAtoms], s3[kGatherAtoms], s4[kGatherAtoms], s5[kGatherAtoms];
     int off[kGatherAtoms], xs[kGatherAtoms], idx[kGatherAtoms];
-    __syncthreads();
+    __syncthreads();                                      // the last round's planes and table are done with
     {
       double c[2 * kPair];
       load_piece<W>(a.coef, j, c);
 #pragma unroll
       for (int r = 0; r < kGatherAtoms; ++r) {
-        const int p = base + r * GRP + grp;
+        const int p = base + r * GRP + grp, slot = r * GRP + grp;
         const int4 at = a.at[min(p, p1 - 1)];
-        const int i = at.w;
-        idx[r] = p < p1 ? i : -1;
-        xs[r] = p < p1 ? at.x - x0 : -4 * kTile;          // no plane of the block touches an atom that is not there
+        const double4 vt = a.vt[min(p, p1 - 1)];
+        idx[r] = p < p1 ? at.w : -1;
         off[r] = (at.y - kTile * ty) * RZ + (at.z - kTile * tz) + min(j, W - 1);
         s0[r] = s1[r] = s2[r] = s3[r] = s4[r] = s5[r] = 0.0;
         double f[3], df[3], d2[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          int l;
-          double t;
-          mesh_coord<W>(d == 0 ? a.sx[i] : (d == 1 ? a.sy[i] : a.sz[i]), a.m.G[d], l, t);
-          piece<true, SECOND>(c, 2.0 * t - 1.0, sg, f[d], df[d], d2[d]);
-        }
+        piece<true, SECOND>(c, vt.x, sg, f[0], df[0], d2[0]);
+        piece<true, SECOND>(c, vt.y, sg, f[1], df[1], d2[1]);
+        piece<true, SECOND>(c, vt.z, sg, f[2], df[2], d2[2]);
+        xs[r] = p < p1 ? at.x - x0 : -4 * kTile;          // no plane touches an atom that is not there
         if (j < W) {
-          const int slot = r * GRP + grp;
           px[slot][j][0] = f[0];
           px[slot][j][1] = df[0];
           if constexpr (SECOND) px[slot][j][2] = d2[0];
@@ -803,37 +957,49 @@ k_mesh_gather(GatherArgs a) {
         pz[r] = f[2]; dz[r] = df[2]; ez[r] = SECOND ? d2[2] : 0.0;
       }
     }
-    const int xend = x1 - x0 + W - 1;                     // planes x0 .. x0 + xend - 1
     for (int c0 = 0; c0 < xend; c0 += kPlanes) {
-      const int np = min(kPlanes, xend - c0);
-      __syncthreads();
-      for (int row = threadIdx.x >> 5; row < np * RY; row += kGatherThreads / 32) {
-        const int pl = row / RY, yy = row - pl * RY;
-        int gx = x0 + c0 + pl, gy = kTile * ty + yy;
-        gx = gx >= 2 * Gx ? gx - 2 * Gx : (gx >= Gx ? gx - Gx : gx);
-        gy = gy >= Gy ? gy - Gy : gy;
-        const double v = a.grid[((size_t)gx * Gy + gy) * Gz + gz];
-        if (hz < RZ) plane[pl][yy * RZ + hz] = v;
+      const int nr = min(kPlanes, xend - c0) * RY;
+      if (c0 > 0) __syncthreads();
+      // (eight rows' loads in flight)
+      for (int r0 = row0; r0 < nr; r0 += 8 * (kGatherThreads / 32)) {
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int row = min(r0 + u * (kGatherThreads / 32), nr - 1);
+          const int pl = row / RY, yy = row - pl * RY;
+          int gx = x0 + c0 + pl, gy = kTile * ty + yy;
+          gx = gx >= 2 * Gx ? gx - 2 * Gx : (gx >= Gx ? gx - Gx : gx);
+          gy = gy >= Gy ? gy - Gy : gy;
+          v[u] = a.grid[((size_t)gx * Gy + gy) * Gz + gz];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int row = r0 + u * (kGatherThreads / 32);
+          if (row < nr && hz < RZ) plane[row * RZ + hz] = v[u];
+        }
       }
       __syncthreads();
 #pragma unroll
       for (int r = 0; r < kGatherAtoms; ++r) {
         const int slot = r * GRP + grp;
-        const int pb = max(0, xs[r] - c0), pe = min(np, xs[r] + W - c0);
+        const int pb = max(0, xs[r] - c0), pe = min(min(kPlanes, xend - c0), xs[r] + W - c0);
+        const double* pp = plane + off[r] + pb * (RY * RZ);
+        const double* tx = px[slot][max(0, c0 - xs[r])];
         for (int pl = pb; pl < pe; ++pl) {
-          const int xi = c0 + pl - xs[r];
           double t0 = 0.0, t1 = 0.0, t2 = 0.0;
-          row_sums<W, RZ, SECOND>(plane[pl] + off[r], py[r], dy[r], ey[r], t0, t1, t2);
-          const double ax = px[slot][xi][0], bx = px[slot][xi][1];
+          row_sums<W, RZ, SECOND>(pp, py[r], dy[r], ey[r], t0, t1, t2);
+          const double ax = tx[0], bx = tx[1];
           s0[r] = fma(bx, t0, s0[r]);                     // phi' phi
           s1[r] = fma(ax, t1, s1[r]);                     // phi  phi'
           s2[r] = fma(ax, t0, s2[r]);                     // phi  phi
           if constexpr (SECOND) {
-            const double cx = px[slot][xi][2];
+            const double cx = tx[2];
             s3[r] = fma(cx, t0, s3[r]);                   // phi'' phi
             s4[r] = fma(ax, t2, s4[r]);                   // phi  phi''
             s5[r] = fma(bx, t1, s5[r]);                   // phi' phi'
           }
+          pp += RY * RZ;
+          tx += SECOND ? 4 : 2;
         }
       }
     }
@@ -1039,9 +1205,10 @@ struct MeshRecip {
   int counted = 0;                         // k_mesh_bin has run and the scan has not
   double *zf = nullptr, *zb = nullptr, *yf = nullptr, *yb = nullptr, *xf = nullptr, *xb = nullptr;
   double *coef = nullptr, *A = nullptr, *kvec = nullptr;
-  int32_t *key = nullptr, *slot = nullptr, *cnt = nullptr, *start = nullptr, *order = nullptr;
+  int32_t *key = nullptr, *slot = nullptr, *cnt = nullptr, *start = nullptr;
+  BinAtom* order = nullptr;
   int4* at = nullptr;
-  double4* amp = nullptr;
+  double4 *amp = nullptr, *vt = nullptr;
   double *phi = nullptr, *grid = nullptr, *mom = nullptr, *blk = nullptr;
   double2* t = nullptr;
 };
@@ -1050,7 +1217,7 @@ void mesh_free(mdff_ctx* c) {
   MeshRecip* m = c->mesh;
   if (!m) return;
   void* ps[] = {m->zf, m->zb, m->yf, m->yb, m->xf, m->xb, m->coef, m->A, m->kvec, m->key, m->slot, m->cnt, m->start,
-                m->order, m->at, m->amp, m->phi, m->grid, m->mom, m->blk, m->t};
+                m->order, m->at, m->amp, m->vt, m->phi, m->grid, m->mom, m->blk, m->t};
   for (void* p : ps)
     if (p) (void)hipFree(p);
   delete m;
@@ -1077,13 +1244,14 @@ int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<doub
   const int ctiles = div_up(c->K[2] + 1, 16), yld = 32 * ctiles + 2;
   const size_t xch = (size_t)kFtWaves / 2 * 256;
   const size_t lds_zy = 8 * (2 * (size_t)G[1] * 16 + xch), lds_x = 8 * (32 * ((size_t)G[0] + nxp) + xch),
-               lds_yz = 8 * ((size_t)kYzRows * yld + 2 * (size_t)nyp * 16 + xch);
+               lds_yz = 8 * ((size_t)kYzRows * yld + 4 * (size_t)nyp * 16 + xch);
   int maxlds = 0;
   HIP_TRY(c, hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device));
   if (std::max({lds_zy, lds_x, lds_yz}) > (size_t)maxlds) return MDFF_OK;
-  HIP_TRY(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mesh_zy), hipFuncAttributeMaxDynamicSharedMemorySize, maxlds));
-  HIP_TRY(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mesh_x), hipFuncAttributeMaxDynamicSharedMemorySize, maxlds));
-  HIP_TRY(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mesh_yz), hipFuncAttributeMaxDynamicSharedMemorySize, maxlds));
+  for (const void* fn : {reinterpret_cast<const void*>(&k_mesh_zy<1>), reinterpret_cast<const void*>(&k_mesh_zy<2>),
+                         reinterpret_cast<const void*>(&k_mesh_zy<4>), reinterpret_cast<const void*>(&k_mesh_x),
+                         reinterpret_cast<const void*>(&k_mesh_yz)})
+    HIP_TRY(c, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, maxlds));
   MeshRecip* m = new MeshRecip();
   c->mesh = m;
   m->w = w;
@@ -1166,12 +1334,13 @@ int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<doub
   const size_t gcells = (size_t)G[0] * G[1] * G[2];
   HIP_TRY(c, hipMalloc((void**)&m->key, sizeof(int32_t) * n));
   HIP_TRY(c, hipMalloc((void**)&m->slot, sizeof(int32_t) * n));
-  HIP_TRY(c, hipMalloc((void**)&m->order, sizeof(int32_t) * n));
+  HIP_TRY(c, hipMalloc((void**)&m->order, sizeof(BinAtom) * n));
   HIP_TRY(c, hipMalloc((void**)&m->cnt, sizeof(int32_t) * m->nbins));
   HIP_TRY(c, hipMemset(m->cnt, 0, sizeof(int32_t) * m->nbins));
   HIP_TRY(c, hipMalloc((void**)&m->start, sizeof(int32_t) * (m->nbins + 1)));
   HIP_TRY(c, hipMalloc((void**)&m->at, sizeof(int4) * n));
   HIP_TRY(c, hipMalloc((void**)&m->phi, sizeof(double) * nr * w * (size_t)n));
+  HIP_TRY(c, hipMalloc((void**)&m->vt, sizeof(double4) * n));
   if (m->dip) HIP_TRY(c, hipMalloc((void**)&m->amp, sizeof(double4) * n));
   HIP_TRY(c, hipMalloc((void**)&m->grid, sizeof(double) * gcells * m->shares));
   HIP_TRY(c, hipMalloc((void**)&m->t, sizeof(double2) * (size_t)G[0] * NY * CN));
@@ -1185,8 +1354,8 @@ int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<doub
 // The previous MD step's queued sums ride along.
 int mesh_bin(mdff_ctx* c, bool from_r, bool pack) {
   MeshRecip* m = c->mesh;
-  if (m->counted)   // an evaluation that ended early left its counts: the scan clears them
-    hipLaunchKernelGGL(k_mesh_scan, dim3(1), dim3(1024), 0, c->stream, m->nbins, m->cnt, m->start);
+  if (m->counted)   // an evaluation that ended early left its counts
+    hipLaunchKernelGGL(k_mesh_clear, dim3(div_up(m->nbins, 256)), dim3(256), 0, c->stream, m->nbins, m->cnt);
   BinArgs a{};
   a.n = c->n;
   a.from_r = from_r ? 1 : 0;
@@ -1225,20 +1394,31 @@ static int mesh_sort(mdff_ctx* c) {
   MeshRecip* m = c->mesh;
   if (m->sorted) return MDFF_OK;
   const int n = c->n;
-  PROF_LAUNCH(c, PK_TABLES,
-              hipLaunchKernelGGL(k_mesh_scan, dim3(1), dim3(1024), 0, c->stream, m->nbins, m->cnt, m->start));
-  PROF_LAUNCH(c, PK_TABLES,
-              hipLaunchKernelGGL(k_mesh_scatter, dim3(div_up(n, 256)), dim3(256), 0, c->stream, n, m->key, m->slot,
-                                 m->start, m->order));
+  ScatterArgs sc{};
+  sc.n = n;
+  sc.nb = m->nbins;
+  sc.key = m->key; sc.slot = m->slot; sc.cnt = m->cnt;
+  sc.start = m->start;
+  sc.sx = c->sx; sc.sy = c->sy; sc.sz = c->sz;
+  sc.order = m->order;
+  if (m->nbins <= kScanBins) {
+    PROF_LAUNCH(c, PK_TABLES, hipLaunchKernelGGL(k_mesh_scatter<true>, dim3(div_up(n, 256)), dim3(256), 0, c->stream, sc));
+  } else {
+    PROF_LAUNCH(c, PK_TABLES,
+                hipLaunchKernelGGL(k_mesh_scan, dim3(1), dim3(1024), 0, c->stream, m->nbins, m->cnt, m->start));
+    PROF_LAUNCH(c, PK_TABLES, hipLaunchKernelGGL(k_mesh_scatter<false>, dim3(div_up(n, 256)), dim3(256), 0, c->stream, sc));
+  }
   PhiArgs a{};
   a.n = n;
   a.m = m->m;
-  a.sx = c->sx; a.sy = c->sy; a.sz = c->sz;
-  a.key = m->key;
   a.start = m->start;
+  a.cnt = m->cnt;
+  a.nb = m->nbins;
   a.order = m->order;
+  a.q = c->q;
   a.coef = m->coef;
   a.at = m->at;
+  a.vt = m->vt;
   a.phi = m->phi;
   const dim3 grid(std::min(2048, div_up(n, 16)));
   if (m->w == 16) {
@@ -1268,10 +1448,10 @@ static void launch_gather(mdff_ctx* c, const GatherArgs& a, int mom, dim3 grid) 
     PROF_LAUNCH(c, PK_GATHER, hipLaunchKernelGGL((k_mesh_gather<W, 3>), grid, dim3(kGatherThreads), 0, c->stream, a));
 }
 
-// S, W, the 7 energy / stress sums into e_out (queued), and with mom = 3 or 9
-// the moments of every atom; *out: [mom][n]
-int mesh_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool use_mu, int mom, double* e_out,
-              const double** out) {
+// S of the charges or (use_mu) of the dipoles mu and, use_q, the charges; W, the
+// 7 energy / stress sums into e_out (queued), and with mom = 3 or 9 the moments
+// of every atom; *out: [mom][n]
+int mesh_eval(mdff_ctx* c, const double* mu, bool use_q, bool use_mu, int mom, double* e_out, const double** out) {
   MeshRecip* m = c->mesh;
   MDFF_TRY(mesh_sort(c));
   const int n = c->n;
@@ -1279,33 +1459,33 @@ int mesh_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool u
   const int NX = 2 * m->K[0] + 1, NY = 2 * m->K[1] + 1, CN = m->CN;
   if (use_mu) {
     const double* b = c->B;
-    PROF_LAUNCH(c, PK_SK, hipLaunchKernelGGL(k_mesh_amp, dim3(div_up(n, 256)), dim3(256), 0, c->stream, n, m->at, q,
+    PROF_LAUNCH(c, PK_SK, hipLaunchKernelGGL(k_mesh_amp, dim3(div_up(n, 256)), dim3(256), 0, c->stream, n, m->at, c->q,
                                              use_q ? 1 : 0, mu, b[0], b[1], b[2], b[3], b[4], b[5], b[6], b[7], b[8],
                                              -2.0 * Gx, -2.0 * Gy, -2.0 * Gz, m->amp));
   }
   SpreadArgs sa{};
   sa.n = n;
   sa.shares = m->shares;
-  sa.pstride = (m->dip ? 6 : 3) * m->w;
   sa.m = m->m;
   sa.start = m->start;
   sa.at = m->at;
   sa.phi = m->phi;
-  sa.q = use_q ? q : c->zeros;
+  sa.vt = m->vt;
+  sa.pstride = (m->dip ? 6 : 3) * m->w;
   sa.amp = m->amp;
   sa.out = m->grid;
-  const dim3 sg((Gx / kTile) * m->m.nyb * m->m.nzb, m->shares);
+  const dim3 sg((Gx / kTile) * m->m.nyb * m->m.nzb * m->shares);
   if (m->w == 16) launch_spread<16>(c, sa, use_mu, sg);
   else launch_spread<12>(c, sa, use_mu, sg);
   ZyArgs za{};
   za.Gy = Gy; za.Gz = Gz; za.CN = CN; za.NY = NY;
   za.ctiles = m->ctiles;
-  za.shares = m->shares;
   za.sstride = (size_t)Gx * Gy * Gz;
   za.grid = m->grid;
   za.zf = m->zf; za.yf = m->yf;
   za.out = m->t;
-  PROF_LAUNCH(c, PK_SKRED, hipLaunchKernelGGL(k_mesh_zy, dim3(m->ctiles, Gx), dim3(kFtThreads), m->lds_zy, c->stream, za));
+  const auto zy = m->shares == 1 ? &k_mesh_zy<1> : (m->shares == 2 ? &k_mesh_zy<2> : &k_mesh_zy<4>);
+  PROF_LAUNCH(c, PK_SKRED, hipLaunchKernelGGL(zy, dim3(m->ctiles, Gx), dim3(kFtThreads), m->lds_zy, c->stream, za));
   MDFF_TRY(claim_partials(c, m->blk));
   XArgs xa{};
   xa.Gx = Gx; xa.NX = NX; xa.C = NY * CN;
@@ -1331,7 +1511,7 @@ int mesh_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool u
     ga.m = m->m;
     ga.start = m->start;
     ga.at = m->at;
-    ga.sx = c->sx; ga.sy = c->sy; ga.sz = c->sz;
+    ga.vt = m->vt;
     ga.coef = m->coef;
     ga.grid = m->grid;
     ga.out = m->mom;

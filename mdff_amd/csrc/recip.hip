@@ -2998,7 +2998,7 @@ int recip_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool 
   if (c->mesh) {
     const int moments = !forces && !field ? 0 : (forces && use_mu ? 9 : 3);
     const double* part = nullptr;
-    MDFF_TRY(mesh_eval(c, q, mu, use_q, use_mu, moments, e_out, &part));
+    MDFF_TRY(mesh_eval(c, mu, use_q, use_mu, moments, e_out, &part));
     return moments ? rec_finish(c, part, 1, moments, q, mu, use_q, forces, field, ef_out, f_out) : MDFF_OK;
   }
   if (c->rec_f32) return eval_t<float>(c, q, mu, use_q, use_mu, forces, field, ef_out, f_out, e_out);
