@@ -72,7 +72,8 @@ struct PairParam {
   double epsp, sigsq, pl, ql, uc, uc1, uc2, fc;  // LJ derived (src/non_bonded.f90:563-600)
   double epsmor, rhomor, rs;              // Morse
   double db_i, dc_i, db_j, dc_j;          // TT damping of the field at i (from j) / at j
-  int32_t dk_i, dk_j, ldamp, pad;
+  int32_t dk_i, dk_j, ldamp;
+  int32_t half_pow;                       // LJ: pl/2 | (ql/2) << 8 where both are whole numbers below 128, else -1
 };
 
 // ---------------------------------------------------------------------------

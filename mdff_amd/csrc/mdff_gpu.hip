@@ -579,6 +579,9 @@ static void build_pair_params(mdff_ctx* c, const int32_t* natmi) {
       P.rcutsq = rcsq;
       P.A = d.Abmhftd[p]; P.B = d.Bbmhftd[p]; P.C = d.Cbmhftd[p]; P.D = d.Dbmhftd[p]; P.BD = d.BDbmhftd[p];
       P.pl = pl; P.ql = ql;
+      const double hp = 0.5 * pl, hq = 0.5 * ql;
+      P.half_pow = hp == floor(hp) && hq == floor(hq) && hp >= 0 && hq >= 0 && hp < 128 && hq < 128
+                       ? (int)hp | ((int)hq << 8) : -1;
       P.epsp = d.epslj[p] / (ql - pl);
       P.sigsq = two16 * two16 * d.sigmalj[p] * d.sigmalj[p];
       double sr2 = P.sigsq / rcsq, sr = sqrt(sr2), srp = pow(sr, pl), srq = pow(sr, ql);
