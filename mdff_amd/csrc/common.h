@@ -281,6 +281,10 @@ struct mdff_ctx {
   int chk_seq_wait = 0;
   double chk_seq = 0.0;
   double* red_part = nullptr;             // reduction block partials
+  double* scf_part = nullptr;             // block partials of a dipole iteration's two sums
+  double* h_scf = nullptr;                // mapped pinned host memory: those sums and their sequence number
+  double* d_scf = nullptr;                // its device address
+  double scf_seq = 0.0;
   double* fin_part = nullptr;             // block partials of the pair sums [0, 1024*16) and kinetic energy
   double* nhc_part = nullptr;             // Nose-Hoover chain steps: two sets of kinetic block partials
   double* nhc_st = nullptr;               // Nose-Hoover chain state (xi, vxi, Q, scale)
@@ -473,6 +477,8 @@ int recip_tables_from_r(mdff_ctx* c, bool pack);
 // describes them, for a later kernel that finishes the forces itself
 int recip_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool use_mu,
                bool forces, bool field, double* ef_out, double* f_out, double* e_out);
+// the moments of the dipoles mu (charges off), left for the caller's kernel
+int recip_moments(mdff_ctx* c, const double* mu, RecFinal* rf);
 void recip_free(mdff_ctx* c);
 // the same sums as non-uniform fast transforms (mesh.hip)
 int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<double>& kv);

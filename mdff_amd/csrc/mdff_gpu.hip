@@ -182,6 +182,117 @@ __global__ void k_upol(int n, const double* __restrict__ invpol, const double* _
   upol[i] = u;
 }
 
+// One SCF iteration is two of these small kernels around the two field sums
+// (real space beside the reciprocal chain).  An iteration of few ions is bound
+// by launches and waits: 12 small launches and two copies with a wait each took
+// 40 us of it; now four and one wait on a word in host memory (216 ions
+// converged 2432 -> 2114 us FP64, 2073 -> 1662 mixed; 1,440 ions 3094 -> 2645
+// and 2499 -> 2109).
+// Start of an iteration: mu = alpha E (induced_moment; or, INDUCE = false, the
+// predicted mu as it is) and the block partials of mu.alpha^-1.mu.
+template <bool INDUCE>
+__global__ void __launch_bounds__(256) k_scf_begin(int n, const double* __restrict__ pol,
+                                                   const double* __restrict__ invpol, const double* __restrict__ E,
+                                                   double* __restrict__ mu, double* __restrict__ part) {
+  __shared__ double sh[4 * kRedMaxCols];
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  double v[kRedMaxCols] = {};
+  if (i < n) {
+    double m[3];
+    if (INDUCE) {
+      const double* p = pol + 9 * (size_t)i;
+      for (int a = 0; a < 3; ++a) {
+        double x = 0.0;
+        for (int b = 0; b < 3; ++b) x = x + p[a + 3 * b] * E[3 * i + b];
+        m[a] = x;
+        mu[3 * i + a] = x;
+      }
+    } else {
+      for (int a = 0; a < 3; ++a) m[a] = mu[3 * i + a];
+    }
+    const double* ip = invpol + 9 * (size_t)i;
+    double u = 0.0;
+    for (int a = 0; a < 3; ++a)
+      for (int b = 0; b < 3; ++b) u = u + m[a] * ip[a + 3 * b] * m[b];
+    v[0] = u;
+  }
+  const double r = block_sum_cols(v, 1, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = r;
+}
+
+// End of an iteration: E = E_stat + E_ind, E_ind = real space + reciprocal
+// (from the moments, rec_final_field) + surface + self term of mu; correct:
+// mu = aspc alpha E + (1 - aspc) mu (:579-583); then the block
+// partials of the residual (mu / alpha - E)^2 (get_rmsd_mu, :998-1027).
+struct ScfEndArgs {
+  int n, lsurf;
+  RecFinal rf;
+  const double *edir, *estat, *pol;
+  const int32_t* polar;
+  int correct;                   // the ASPC corrector with weight aspc
+  double self2, fpi_3V, aspc;
+  const double* mom;             // device moments (lsurf)
+  double *mu, *E, *part;
+};
+__global__ void __launch_bounds__(256) k_scf_end(ScfEndArgs a) {
+  __shared__ double sh[4 * kRedMaxCols];
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  double v[kRedMaxCols] = {};
+  if (i < a.n) {
+    double s[9], g[3], er[3], E[3], m[3];
+    rec_final_moments(a.rf, i, s, g);
+    rec_final_field(a.rf, g, er);
+    for (int k = 0; k < 3; ++k) {
+      m[k] = a.mu[3 * i + k];
+      double e = a.edir[3 * i + k] + er[k];
+      if (a.lsurf) e += -a.mom[1 + k] * a.fpi_3V;
+      e += a.self2 * m[k];
+      E[k] = a.estat[3 * i + k] + e;
+      a.E[3 * i + k] = E[k];
+    }
+    const double* p = a.pol + 9 * (size_t)i;
+    if (a.correct) {
+      const double w = a.aspc;
+      double t[3];
+      for (int k = 0; k < 3; ++k) {
+        double x = 0.0;
+        for (int b = 0; b < 3; ++b) x = x + p[k + 3 * b] * E[b];
+        t[k] = w * x + (1.0 - w) * m[k];
+      }
+      for (int k = 0; k < 3; ++k) {
+        m[k] = t[k];
+        a.mu[3 * i + k] = t[k];
+      }
+    }
+    if (a.polar[i])
+      for (int k = 0; k < 3; ++k) {
+        const double pk = p[k + 3 * k];
+        if (pk == 0.0) continue;
+        const double x = m[k] / pk - E[k];
+        v[0] = v[0] + x * x;
+      }
+  }
+  const double r = block_sum_cols(v, 1, sh);
+  if (threadIdx.x == 0) a.part[blockIdx.x] = r;
+}
+
+// both sums of an iteration to the host: out[0] = sum pu, out[1] = sum pr
+// (mapped memory), then the sequence number the host waits for
+__global__ void __launch_bounds__(256) k_scf_sums(int nb, const double* __restrict__ pu, const double* __restrict__ pr,
+                                                  double* __restrict__ out, double seq) {
+  __shared__ double sh[4 * kRedMaxCols];
+  __shared__ double tot[2];
+  sum_block_partials(nb, 1, pu, tot, sh);
+  sum_block_partials(nb, 1, pr, tot + 1, sh);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    out[0] = tot[0];
+    out[1] = tot[1];
+    __threadfence_system();
+    out[2] = seq;
+  }
+}
+
 // ASPC predictor (src/moment_from_pola.f90:566-575) and history shift
 __global__ void k_aspc_predict(size_t n3, int ext, double b0, double b1, double b2, double b3, double b4,
                                double* __restrict__ hist, double* __restrict__ mu) {
@@ -734,6 +845,10 @@ static int ctx_init(mdff_ctx* c, const mdff_desc* d, const int32_t* itype) {
   const size_t nred = std::max<size_t>(64 * 1024, 2 * (size_t)nblk(n) + 2);
   HIP_TRY(c, hipHostMalloc((void**)&c->h_red, sizeof(double) * nred));
   DMALLOC(c->red_part, nred);
+  DMALLOC(c->scf_part, 2 * (size_t)nblk(n));
+  HIP_TRY(c, hipHostMalloc((void**)&c->h_scf, sizeof(double) * 4, hipHostMallocMapped | hipHostMallocCoherent));
+  HIP_TRY(c, hipHostGetDevicePointer((void**)&c->d_scf, c->h_scf, 0));
+  memset(c->h_scf, 0, sizeof(double) * 4);
   DMALLOC(c->red, 64);
   DMALLOC(c->fin_part, 1024 * 16 + (size_t)nblk(n) + 16);
   DMALLOC(c->nhc_part, 2 * (size_t)nblk(n));
@@ -847,27 +962,65 @@ static int scf(mdff_ctx* c, mdff_terms* t) {
     default: Bc[0] = 3.0; Bc[1] = -24.0 / 7.0; Bc[2] = 27.0 / 14.0; Bc[3] = -4.0 / 7.0; Bc[4] = 1.0 / 14.0; w = 5.0 / 9.0; break;
   }
   double upol = 0.0;
+  const int nb = nblk(n);
+  const double alpha2 = c->alpha * c->alpha;
+  const double selfa = c->alpha / sqrt(MDFF_PI), selfa2 = 2.0 * selfa * alpha2 / 3.0;
+  double* pu = c->scf_part;        // block partials: mu.alpha^-1.mu, then the residual
+  double* pr = c->scf_part + nb;
   while ((iscf < d.max_scf_pol_iter && rmsd > d.conv_tol_ind) || iscf < d.min_scf_pol_iter) {
     iscf++;
-    if (iscf != 1 || !d.calc_md) {
-      hipLaunchKernelGGL(k_induced, dim3(nblk(n)), dim3(256), 0, c->stream, n, c->pol, c->invpol, c->e_tot,
-                         c->mu_ind, extra(c));
-    } else {
+    const bool predict = iscf == 1 && d.calc_md;
+    if (predict)
       hipLaunchKernelGGL(k_aspc_predict, dim3(div_up(n3, 256)), dim3(256), 0, c->stream, n3, ext, Bc[0], Bc[1],
                          Bc[2], Bc[3], Bc[4], c->hist, c->mu_ind);
-      hipLaunchKernelGGL(k_upol, dim3(nblk(n)), dim3(256), 0, c->stream, n, c->invpol, c->mu_ind, extra(c));
+    hipLaunchKernelGGL(predict ? &k_scf_begin<false> : &k_scf_begin<true>, dim3(nb), dim3(256), 0, c->stream, n, c->pol,
+                       c->invpol, c->e_tot, c->mu_ind, pu);
+    // the real-space field beside the reciprocal sums (both read mu only);
+    // off with MDFF_PAIR_OVERLAP=0 and while the event profiler runs
+    const bool ov = c->overlap && !c->prof_on;
+    hipStream_t s0 = c->stream;
+    if (ov) {
+      HIP_TRY(c, hipEventRecord(c->ov_tab, c->stream));
+      HIP_TRY(c, hipStreamWaitEvent(c->stream2, c->ov_tab, 0));
+      c->stream = c->stream2;
     }
-    double h[1];
-    MDFF_TRY(reduce_cols(c, extra(c), 1, h));
+    const int rc = realspace_field(c, 1, c->mu_ind, ef_dir(c));
+    c->stream = s0;
+    MDFF_TRY(rc);
+    if (ov) HIP_TRY(c, hipEventRecord(c->ov_pair, c->stream2));
+    ScfEndArgs a{};
+    MDFF_TRY(recip_moments(c, c->mu_ind, &a.rf));
+    a.mom = c->raw + RAW_SCRATCH;
+    if (d.lsurf) MDFF_TRY(moments_dev(c, c->q, c->mu_ind, c->raw + RAW_SCRATCH));
+    if (ov) HIP_TRY(c, hipStreamWaitEvent(c->stream, c->ov_pair, 0));
+    a.n = n;
+    a.lsurf = d.lsurf;
+    a.edir = ef_dir(c);
+    a.estat = c->e_stat;
+    a.pol = c->pol;
+    a.polar = polar;
+    a.self2 = 2.0 * selfa2;
+    a.fpi_3V = 2.0 * (2.0 * MDFF_PI / c->omega / 3.0);
+    a.correct = predict ? 1 : 0;
+    a.aspc = w;
+    a.mu = c->mu_ind;
+    a.E = c->e_tot;
+    a.part = pr;
+    hipLaunchKernelGGL(k_scf_end, dim3(nb), dim3(256), 0, c->stream, a);
+    c->scf_seq += 1.0;
+    hipLaunchKernelGGL(k_scf_sums, dim3(1), dim3(256), 0, c->stream, nb, pu, pr, c->d_scf, c->scf_seq);
+    HIP_TRY(c, hipGetLastError());
+    // wait for the sequence number; a launch that never reports is caught by
+    // the stream
+    volatile const double* h = c->h_scf;
+    bool seen = false;
+    for (long k = 0; k < 20000000L && !seen; ++k) seen = h[2] == c->scf_seq;
+    if (!seen) {
+      HIP_TRY(c, hipStreamSynchronize(c->stream));
+      if (h[2] != c->scf_seq) return fail(c, MDFF_ERR_HIP, "dipole iteration signal missing");
+    }
     upol = 0.5 * h[0];
-    MDFF_TRY(ewald_field(c, false, c->mu_ind, c->e_ind));
-    hipLaunchKernelGGL(k_add3, dim3(div_up(n3, 256)), dim3(256), 0, c->stream, n3, c->e_stat, c->e_ind, c->e_tot);
-    if (iscf == 1 && d.calc_md)
-      hipLaunchKernelGGL(k_aspc_correct, dim3(nblk(n)), dim3(256), 0, c->stream, n, w, c->pol, c->e_tot, c->mu_ind);
-    hipLaunchKernelGGL(k_rmsd_terms, dim3(nblk(n)), dim3(256), 0, c->stream, n, polar, c->pol, c->e_tot, c->mu_ind,
-                       extra(c));
-    MDFF_TRY(reduce_cols(c, extra(c), 1, h));
-    rmsd = sqrt(h[0] / (double)npol);
+    rmsd = sqrt(h[1] / (double)npol);
   }
   HIP_TRY(c, hipMemcpyAsync(c->hist, c->mu_ind, sizeof(double) * n3, hipMemcpyDeviceToDevice, c->stream));
   t->u_pol = upol;
@@ -1383,7 +1536,7 @@ int mdff_ctx_destroy(mdff_ctx* c) {
                 c->hist, c->frec, c->zeros, c->arec, c->ameta, c->peratom, c->red, c->red_part, c->d_pp, c->cell_of, c->cell_key,
                 c->cell_atoms, c->cell_atoms_in, c->cell_start, c->nl_count, c->nl_start, c->nl_j,
                 c->nl_flag, c->nl_count_in, c->nl_j_tmp, c->nl_flag_tmp, c->sort_tmp, c->d_flag, c->raw,
-                c->cx, c->cy, c->cz, c->fin_part, c->nhc_part, c->nhc_st, c->peratom_lj, c->f_lj, c->lj_part};
+                c->cx, c->cy, c->cz, c->fin_part, c->nhc_part, c->nhc_st, c->peratom_lj, c->f_lj, c->lj_part, c->scf_part};
   for (void* p : ps)
     if (p) (void)hipFree(p);
   if (c->polar) (void)hipFree(c->polar);
@@ -1393,6 +1546,7 @@ int mdff_ctx_destroy(mdff_ctx* c) {
   if (c->h_red) (void)hipHostFree(c->h_red);
   if (c->h_raw) (void)hipHostFree(c->h_raw);
   if (c->h_chk) (void)hipHostFree(c->h_chk);
+  if (c->h_scf) (void)hipHostFree(c->h_scf);
   if (c->chk_ev) (void)hipEventDestroy(c->chk_ev);
   if (c->ov_tab) (void)hipEventDestroy(c->ov_tab);
   if (c->ov_pair) (void)hipEventDestroy(c->ov_pair);

@@ -2684,6 +2684,10 @@ static int rec_finish(mdff_ctx* c, const double* part, int nsplit, int moments, 
     c->rfin = rf;
     c->rfin_pending = 1;
   }
+  if (field && !ef_out) {          // recip_moments
+    c->rfin = rf;
+    return MDFF_OK;
+  }
   if (field || !defer)
     PROF_LAUNCH(c, PK_GFINAL,
                 hipLaunchKernelGGL(k_gather_final, dim3(div_up(c->n, 256)), dim3(256), 0, c->stream, rf,
@@ -3003,4 +3007,10 @@ int recip_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool 
   }
   if (c->rec_f32) return eval_t<float>(c, q, mu, use_q, use_mu, forces, field, ef_out, f_out, e_out);
   return eval_t<double>(c, q, mu, use_q, use_mu, forces, field, ef_out, f_out, e_out);
+}
+
+int recip_moments(mdff_ctx* c, const double* mu, RecFinal* rf) {
+  MDFF_TRY(recip_eval(c, c->q, mu, false, true, false, true, nullptr, nullptr, nullptr));
+  *rf = c->rfin;
+  return MDFF_OK;
 }
