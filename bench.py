@@ -38,40 +38,24 @@ PEAK = {"fp32": 157.3, "fp64": 78.6, "fp16": 2500.0}   # MI355X dense TFLOP/s (m
 HBM_PEAK = 8000.0                          # GB/s
 # canonical algorithmic flops per unit (counting FMA = 2, sqrt/exp/sin/cos/div = 1)
 FLOPS_PER_UNIT = {
-    "k_sk": 11.0,          # per (k, i): k.r 5, cos+sin 2, rho accumulate 4 (src/ewald_rec.f90:116-127)
-    "k_gather": 10.0,      # per (k, i): recarg 3 + force 7 (src/ewald_rec.f90:196-224)
+    "k_sk": 2.0,           # per (atom, grid point of its 12^3 window): one multiply-add of the spread
+    "k_gather": 2.7,       # the value and three derivatives, the two inner axes shared: 2 + 8 / 12
     "k_pair_force": 106.0, # per in-cutoff Buckingham + Ewald q-q pair
 }
 # the kernel behind each profiler class of the mixed form, and the unit it
-# is bound by: the reciprocal sums run on split-half FP16 matrix cores
-# (three FP16 products per FP32-class product), the pair kernel on FP32 VALU
-KERNEL_OF = {"k_sk": "k_sk_h3<32,0>", "k_gather": "k_gather_h3<CT,NSH>", "k_pair_force": "k_pair_force<float,false,16,2>"}
-BOUND_OF = {"k_sk": ("mfma", "fp16"), "k_gather": ("mfma", "fp16"), "k_pair_force": ("valu", "fp32")}
-# HBM bytes per launch of the mixed-form kernels on this workload: rocprofv3
-# FETCH_SIZE x 1.987 + WRITE_SIZE x 0.996 (KiB per dispatch x 1024; the factors
-# calibrate the counters on a 256 MiB device-to-device copy), measured with
+# is bound by: the reciprocal sums are FP64 transforms (spread on the FP64
+# matrix cores), the pair kernel runs on the FP32 VALU
+KERNEL_OF = {"k_sk": "k_mesh_spread<12,false>", "k_gather": "k_mesh_gather<12,3>",
+             "k_pair_force": "k_pair_force<float,false,16,2>"}
+BOUND_OF = {"k_sk": ("mfma", "fp64"), "k_gather": ("valu", "fp64"), "k_pair_force": ("valu", "fp32")}
+# HBM bytes per launch on this workload: rocprofv3 FETCH_SIZE x 1.987 +
+# WRITE_SIZE x 0.996 (KiB per dispatch x 1024; the factors calibrate the
+# counters on a 256 MiB device-to-device copy), measured with
 # mdff_amd.profile_workload (profiles/engforce_sio2_24k_hbm_traffic.md)
-TRAFFIC = {"k_gather": 64.46e6, "k_sk": 40.60e6, "k_pair_force": 63.92e6}
+TRAFFIC = {"k_pair_force": 63.92e6}
 
 
-def mfma_issued(kind: str, natm: int, kmax) -> float:
-    """FP16 MFMA flops the split-half kernels issue per launch (32x32x16:
-    32768 flops each): gather 3 NSH per (32-atom tile, 8-m tile), NSH =
-    K steps of 16 over 2 (2 kz + 1) padded to 4, 7, 10 or 15; structure
-    factor 12 per (8 atoms, 32-m wave tile)."""
-    kx, ky, kz = kmax
-    M = (kx + 1) * (2 * ky + 1)
-    nz = 2 * kz + 1
-    nsh = next(b for b in (4, 7, 10, 15) if -(-2 * nz // 16) <= b)
-    if kind == "k_gather":
-        return -(-natm // 32) * -(-M // 8) * 3 * nsh * 32768.0
-    if kind == "k_sk":
-        waves_m = -(-(-(-M // 32)) // 4) * 4
-        return waves_m * -(-natm // 32) * 4 * 12 * -(-nz // 64) * 32768.0
-    return 0.0
-
-
-NKINDS = 10  # kernel classes of the library's event profiler (mdff_profile_name)
+NKINDS = 8  # kernel classes of the library's event profiler (mdff_profile_name)
 
 
 def build_system(natm: int, relax_iters: int):
@@ -362,7 +346,7 @@ def main() -> int:
     # dominant kernel of the mixed form
     prof = r32["prof"]
     dom = max(prof, key=lambda k: prof[k]["ms_total"])
-    units = {"k_sk": nk * s.natm, "k_gather": nk * s.natm, "k_pair_force": npairs}
+    units = {"k_sk": s.natm * 12**3, "k_gather": s.natm * 12**3, "k_pair_force": npairs}
     roof = None
     if dom in FLOPS_PER_UNIT and prof[dom]["ms_avg"] > 0:
         flops = FLOPS_PER_UNIT[dom] * units[dom]
@@ -373,10 +357,6 @@ def main() -> int:
                 "unit": "TFLOP/s", "frac": round(ach / PEAK[kind], 4), "traffic": TRAFFIC.get(dom),
                 "algorithmic_flops_per_launch": flops, "avg_launch_ms": prof[dom]["ms_avg"],
                 "units_per_launch": units[dom], "flops_per_unit": FLOPS_PER_UNIT[dom]}
-        issued = mfma_issued(dom, s.natm, kmax)
-        if issued > 0:
-            roof["mfma_fp16_issued_tflops"] = round(issued / sec / 1e12, 3)
-            roof["mfma_fp16_issued_frac"] = round(issued / sec / 1e12 / PEAK["fp16"], 4)
 
     out = {
         "metric": "ns/day mixed vs FP64 on GPU at <=1e-5 rel force err; fit-gradients/s",
@@ -389,7 +369,7 @@ def main() -> int:
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f32 pair/field math, split-half f16 (f32-class) reciprocal products, f64 accumulation",
+        "dtype": "f32 pair/field math, f64 reciprocal sums and accumulation",
         "data": "synthetic (seeded random packing)",
         "config": {"workload": f"a-SiO2 {s.natm} ions, Buckingham+Ewald rc {rc} alpha {s.desc.alphaES} "
                                f"kmax {kmax[0]}, skin {s.desc.skindiff}, NVE velocity Verlet dt 1 fs",

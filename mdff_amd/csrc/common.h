@@ -85,7 +85,7 @@ struct DevBuf {
 };
 
 // kernel classes timed by the in-library event profiler
-enum ProfKind { PK_PAIR = 0, PK_FIELD, PK_TABLES, PK_SK, PK_SKRED, PK_GATHER, PK_GFINAL, PK_NLIST, PK_AMAT, PK_INNER, PK_COUNT };
+enum ProfKind { PK_PAIR = 0, PK_FIELD, PK_TABLES, PK_SK, PK_SKRED, PK_GATHER, PK_GFINAL, PK_NLIST, PK_COUNT };
 struct ProfRec {
   int kind;
   hipEvent_t a, b;
@@ -207,6 +207,7 @@ struct alignas(16) AtomRec {
 };
 
 struct MeshRecip;
+struct cplx;
 
 struct mdff_ctx {
   mdff_desc d;
@@ -227,12 +228,6 @@ struct mdff_ctx {
   double rc_vdw, rc_coul, alpha;
   int task_qq = 0, task_qd = 0, task_dd = 0, linduced = 0, ldip_static = 0;
   int sr_model = 0;                       // 0 none, 1 LJ, 2 BMH, 3 Morse
-  // reciprocal kernels in the FP32-class form (split-half / FP32 tables): the
-  // mixed form.  A dipole system keeps them only where the FP64 inner k-box
-  // of its force evaluation exists (else, or with MDFF_DIP_RECIP_FP64=1, its
-  // reciprocal sums run in FP64): without that box the FP32-class dipole
-  // structure factors set the force error above 1e-5
-  int rec_f32 = 0;
   MeshRecip* mesh = nullptr;              // reciprocal sums as fast transforms (mesh.hip); null: the direct kernels
   // LJ together with BMHFT(D) (src/engforce_driver.f90:130-141): the BMHFT(D)
   // pass gives the forces (each reference routine zeroes them first), an LJ
@@ -300,7 +295,6 @@ struct mdff_ctx {
   int32_t* polar = nullptr;               // 1 for polarisable ions
   int npol = 0;                           // number of polarisable ions
   double qsq = 0.0;                       // sum of q^2 (self term)
-  double qmax = 0.0;                      // max |q|
   double* zeros = nullptr;                // n zeros (charges switched off)
 
   // neighbour list (full rows, cut = max(rc_vdw, rc_coul) + skin)
@@ -346,50 +340,16 @@ struct mdff_ctx {
   int nk_box = 0, nk = 0;
   double* kA = nullptr;                   // A(n) on the box, 0 where excluded (nk_box)
   double* kvec = nullptr;                 // kx,ky,kz,kcoe per box entry (4 x nk_box)
-  void* tab = nullptr;                    // per-atom phase tables (precision dependent)
-  void* sk_part = nullptr;                // structure-factor partials
-  double* sk = nullptr;                   // S(n) (2 x nk_box) FP64
+  cplx* tab = nullptr;                    // per-atom phase tables
+  double* sk_part = nullptr;              // structure-factor partials
   double* wk = nullptr;                   // W(n) = A(n) conj(S(n)) (2 x nk_box)
-  void* wk_t = nullptr;                   // W in the working precision
   double* rec_part = nullptr;             // per (atom, split) partial moments
   int rec_splits = 1, sk_chunks = 1;
-  void* amat = nullptr;                   // matrix-core gather A operand
+  double* amat = nullptr;                 // matrix-core gather A operand
   int mma_nks = 0, mma_mtiles = 0, mma_ct = 0, mma_splits = 1;
   int use_mma = 1;                        // matrix-core reciprocal kernels
-  int sk_ctm = 1;                         // m-tiles per wave of the structure factor
   int sk_ta = 0;                          // atoms per staged tile of the structure factor
   int sk_mma_ch = 1;                      // atom chunks of the matrix-core structure factor
-  // mixed form: split-half (FP16 hi + lo) matrix-core reciprocal kernels
-  int h3 = 0;                             // split-half gather (and its A operand from the reduction)
-  int h3_sk = 0;                          // split-half structure factor as well
-  int h3_wide = 0;                        // ... in its wide-mesh form (more than 64 staged X / Y columns)
-  int h3_ch = 1, h3_nsh = 0, h3_ct = 1, h3_splits = 1, h3_mt8 = 0;
-  float h3_pscale = 1.f;                  // charge scale of the structure factor's B operand
-  float* mu_pscale = nullptr;             // device: scales of the two dipole passes (k_mu_pscale)
-  // Mixed form, charge-only evaluations: the k-vectors of the inner box
-  // |nx| <= kin[0], |ny| <= kin[1], |nz| <= kin[2] (every k with |k| <=
-  // 2.5 alpha) carry most of the weight of the force sums and run in FP64
-  // (k_in_phase, k_in_sk_s, k_in_reduce_r, k_in_gather_s, or the generic
-  // k_in_sk, k_in_reduce, k_in_gather); the main kernels see A = 0 there
-  // (kA_mask).  kin_on = 0: no inner pass.
-  int kin_on = 0;
-  int kin[3] = {0, 0, 0};
-  int nb_in = 0, in_chunk = 0, in_nch = 0, kin_tile = 0, kin_msplit = 0, kin_splits = 0;
-  int kin_reg = 0;                        // 1: the scalar-operand forms (Kz' small enough)
-  int kin_ts = 0, kin_sg = 0;             // k_in_sk_s: threads per subgroup, subgroups
-  int kin_jb = 1, kin_kb = 0;             // scalar-operand forms: blocks of j = |nz|, KZ (j per block - 1)
-  int kin_zpad = 0;                       // j columns of the phase rows and the W table: kin_jb (kin_kb + 1)
-  size_t kin_lds = 0;                     // LDS bytes of the structure-factor kernel
-  void* tab_in = nullptr;                 // per atom X, Y, q Z rows (FP64 complex)
-  double* wt_in = nullptr;                // per (m, j) sum / difference table of W
-  double* kA_mask = nullptr;              // kA with the inner box zeroed (nk_box)
-  double* kA_in = nullptr;                // A of the inner box, 0 outside the half space (nb_in)
-  double* kvec_in = nullptr;              // kx, ky, kz, kcoe of the inner box (4 x nb_in)
-  double* sk_in_part = nullptr;           // [chunk][2 nb_in] FP64 partials
-  double* wk_in = nullptr;                // W = A conj(S) of the inner box (2 x nb_in)
-  double* dip_part = nullptr;             // dipole systems: [q, mu_x, mu_y, mu_z][chunk][2 nb_in]
-  void* amat_h3 = nullptr;                // gather A operand, split halves
-  float* ascale_h3 = nullptr;             // inverse scale per gather m-tile
   double* kO_ws = nullptr;                // scf_kO_v2 work vectors (11 x 3n)
   AtomRec* arec = nullptr;                // atoms in cell-sorted order (refreshed every evaluation)
   int2* ameta = nullptr;                  // (type, original index) in the same order

@@ -868,21 +868,12 @@ static int ctx_init(mdff_ctx* c, const mdff_desc* d, const int32_t* itype) {
   for (int i = 0; i < n; ++i) {
     c->npol += polar[i] != 0;
     c->qsq = c->qsq + q[i] * q[i];
-    c->qmax = std::max(c->qmax, std::fabs(q[i]));
   }
   // reciprocal kernels: matrix-core by default; MDFF_RECIP_VALU=1 selects the
   // vector-ALU kernels (same sums, kept for comparison and for shapes the
   // matrix-core kernels do not cover)
   const char* ev = getenv("MDFF_RECIP_VALU");
   c->use_mma = (ev && ev[0] == '1') ? 0 : 1;
-  // m-tiles per wave of the matrix-core structure factor: one (two would
-  // exceed 256 VGPRs with the unrolled atom tile)
-  c->sk_ctm = 1;
-  {
-    const char* ev = getenv("MDFF_DIP_RECIP_FP64");
-    const bool dip64 = ev && ev[0] == '1' && (c->task_qd || c->task_dd);
-    c->rec_f32 = (d->precision == MDFF_PREC_MIXED && !dip64) ? 1 : 0;
-  }
   if (d->lcoulomb) MDFF_TRY(recip_setup(c));
   return MDFF_OK;
 }
@@ -1476,8 +1467,7 @@ hipEvent_t prof_event(mdff_ctx* c) {
 }
 
 static const char* kProfNames[PK_COUNT] = {"k_pair_force", "k_pair_field", "k_tables",       "k_sk",
-                                           "k_sk_reduce",  "k_gather",     "k_gather_final", "k_nl_sweep",
-                                           "k_amat",       "k_inner_box"};
+                                           "k_sk_reduce",  "k_gather",     "k_gather_final", "k_nl_sweep"};
 
 // ====================================================================== C-ABI
 
