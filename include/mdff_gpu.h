@@ -65,7 +65,7 @@ typedef enum mdff_precision {
   MDFF_PREC_FP64 = 0,   /* every operation in FP64 (parity form)                         */
   MDFF_PREC_MIXED = 1   /* FP32 pair / dipole-field arithmetic, FP64 force and field
                            accumulation (pair energies / stresses: FP32 within one
-                           lane's row share, FP64 beyond), FP64 minimum image, FP64
+                           lane's row share, FP64 beyond), FP64 minimum image,
                            reciprocal sums and SCF residual in FP64                  */
 } mdff_precision;
 

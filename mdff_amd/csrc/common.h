@@ -346,7 +346,8 @@ struct mdff_ctx {
   double* rec_part = nullptr;             // per (atom, split) partial moments
   int rec_splits = 1, sk_chunks = 1;
   double* amat = nullptr;                 // matrix-core gather A operand
-  int mma_nks = 0, mma_mtiles = 0, mma_ct = 0, mma_splits = 1;
+  int mma_nks = 0, mma_mtiles = 0;
+  int mma_splits[2] = {1, 1};             // of the gathers of 3 and 9 moments
   int use_mma = 1;                        // matrix-core reciprocal kernels
   int sk_ta = 0;                          // atoms per staged tile of the structure factor
   int sk_mma_ch = 1;                      // atom chunks of the matrix-core structure factor
@@ -355,12 +356,9 @@ struct mdff_ctx {
   int2* ameta = nullptr;                  // (type, original index) in the same order
 
   // electric field gradient efg_t (9 x n, column-major per atom) and its
-  // work arrays: real-space part (6 x n), S(k) / reciprocal partials, W = A S
+  // real-space part (6 x n)
   double* efg = nullptr;
   double* efg_dir = nullptr;
-  double* efg_part = nullptr;
-  double* efg_w = nullptr;
-  int efg_sk_nch = 1, efg_sk_chunk = 1, efg_rec_nch = 1, efg_rec_chunk = 1;
 
   double last_ms[8] = {0};
   int n_last = 0;

@@ -450,7 +450,7 @@ __global__ void k_gather_final(RecFinal r, int field, int forces, double* __rest
 
 
 // ---------------------------------------------------------------------------
-// Matrix-core form of phase 2 (field / charge forces).
+// Matrix-core form of phase 2.
 //
 // For one 16-atom tile the contraction over nz is a real GEMM on MFMA
 // 16x16x4: rows R = (m_local, comp) of 4 values of m = (nx, ny) and four
@@ -463,6 +463,11 @@ __global__ void k_gather_final(RecFinal r, int field, int forces, double* __rest
 // accumulator registers, so the (nx, ny) epilogue (multiply by
 // X_i[nx] Y_i[ny], weight by nx, ny) is lane-local; the four m_local lane
 // groups are summed with two cross-lane shuffles at the very end.
+//
+// Second moments (MOM 9) need U2 too: a second product of the same A operand
+// with nz Z has (U1, U2) in its rows, so it costs one multiply a step and no
+// second A operand (a gradient evaluation of 480 ions 339 us with the
+// vector-ALU gather, 217 with this; of 4,096 ions 437 and 364).
 // Lane layouts (checked on gfx950): A(row = l%16, k = l/16), B(k = l/16,
 // col = l%16); D f32: row = 4*(l/16) + r; D f64: row = 4*r + l/16.
 // ---------------------------------------------------------------------------
@@ -478,19 +483,19 @@ struct GmArgs {
   int n, Kx, Ky, Kz, NY, NZ, M, nks, mt_per_split, mtiles;
   const cplx* tab;
   const double* amat;
-  double* out;                   // [split][3][n]
+  double* out;                   // [split][moments][n]
 };
 
 // Two waves per SIMD where the B operand, the double-buffered A operand and
 // the accumulators fit in 256 registers without spills (the instances
 // listed), one otherwise.
-template <int CT, int NKS>
+template <int CT, int NKS, int MOM>
 constexpr int gather_waves() {
-  return ((CT == 2 && NKS <= 25) || (CT == 1 && NKS <= 33)) ? 2 : 1;
+  return NKS <= 25 || (MOM == 3 && NKS <= 33) ? 2 : 1;
 }
 
-template <int CT, int NKS>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gather_waves<CT, NKS>())))
+template <int CT, int NKS, int MOM>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gather_waves<CT, NKS, MOM>())))
 k_gather_mma(GmArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -523,6 +528,9 @@ k_gather_mma(GmArgs a) {
   double ax[CT], ay[CT], az3[CT];
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) { ax[ct] = 0.0; ay[ct] = 0.0; az3[ct] = 0.0; }
+  // MOM 9: xx, yy, zz, xy, xz, yz sums of n n Re(W e); nz of this lane's first K index
+  double sec[MOM == 9 ? CT : 1][6] = {};
+  const double nz0 = (double)((g >> 1) - a.Kz);
   const int mt0 = blockIdx.y * a.mt_per_split;
   const int mt1 = min(a.mtiles, mt0 + a.mt_per_split);
   // The A operand of tile mt+1 is loaded at the top of tile mt; the
@@ -567,13 +575,19 @@ k_gather_mma(GmArgs a) {
     nyo += 4;
     while (nyo >= a.NY) { nyo -= a.NY; ++nx; }          // NY = 2 Ky + 1 may be below 4
     if (mt + 1 < mt1) load_a(mt + 1);
-    f64x4 acc[CT];
+    f64x4 acc[CT], acn[MOM == 9 ? CT : 1];
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) acc[ct] = f64x4{0.0, 0.0, 0.0, 0.0};
+    for (int ct = 0; ct < CT; ++ct) {
+      acc[ct] = f64x4{0.0, 0.0, 0.0, 0.0};
+      if (MOM == 9) acn[ct] = acc[ct];
+    }
 #pragma unroll
     for (int s = 0; s < NKS; ++s) {
 #pragma unroll
-      for (int ct = 0; ct < CT; ++ct) acc[ct] = mfma(cur[s], breg[ct][s], acc[ct]);
+      for (int ct = 0; ct < CT; ++ct) {
+        acc[ct] = mfma(cur[s], breg[ct][s], acc[ct]);
+        if (MOM == 9) acn[ct] = mfma(cur[s], (nz0 + 2.0 * s) * breg[ct][s], acn[ct]);
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -588,6 +602,17 @@ k_gather_mma(GmArgs a) {
       ax[ct] += fx * im0;
       ay[ct] += fy * im0;
       az3[ct] += im1;
+      if (MOM == 9) {
+        const double re0 = XY.re * acc[ct][0] - XY.im * acc[ct][1];
+        const double re1 = XY.re * acc[ct][2] - XY.im * acc[ct][3];
+        const double re2 = XY.re * acn[ct][2] - XY.im * acn[ct][3];
+        sec[ct][0] += fx * fx * re0;
+        sec[ct][1] += fy * fy * re0;
+        sec[ct][2] += re2;
+        sec[ct][3] += fx * fy * re0;
+        sec[ct][4] += fx * re1;
+        sec[ct][5] += fy * re1;
+      }
     }
   }
 #pragma unroll
@@ -598,9 +623,15 @@ k_gather_mma(GmArgs a) {
     ay[ct] += __shfl_xor(ay[ct], 32);
     az3[ct] += __shfl_xor(az3[ct], 16);
     az3[ct] += __shfl_xor(az3[ct], 32);
+    if (MOM == 9)
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        sec[ct][k] += __shfl_xor(sec[ct][k], 16);
+        sec[ct][k] += __shfl_xor(sec[ct][k], 32);
+      }
   }
   if (g == 0) {
-    double* o = a.out + (size_t)blockIdx.y * 3 * a.n;
+    double* o = a.out + (size_t)blockIdx.y * MOM * a.n;
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
       const int ia = atom0 + ct * 16 + col;
@@ -608,6 +639,9 @@ k_gather_mma(GmArgs a) {
         o[ia] = ax[ct];
         o[(size_t)a.n + ia] = ay[ct];
         o[(size_t)2 * a.n + ia] = az3[ct];
+        if (MOM == 9)
+#pragma unroll
+          for (int k = 0; k < 6; ++k) o[(size_t)(3 + k) * a.n + ia] = sec[ct][k];
       }
     }
   }
@@ -792,14 +826,16 @@ static int mma_bucket(int nks) {
     if (nks <= b) return b;
   return 0;
 }
-// atom tiles of 16 per wave: register budget of the B operand
-static int mma_ct(int nks) { return nks <= 25 ? 2 : 1; }
+// atom tiles of 16 per wave: register budget of the B operand and the sums
+static int mma_ct(int nks, int mom) { return mom == 3 && nks <= 25 ? 2 : 1; }
 
-// the compiled matrix-core gather for (CT, NKS), or null
-static const void* gather_kernel(int ct, int nks) {
-#define GM_CASE(CTV, NKSV) \
-  case (CTV) * 1000 + (NKSV): return reinterpret_cast<const void*>(&k_gather_mma<CTV, NKSV>);
-  switch (ct * 1000 + nks) {
+// the compiled matrix-core gather for NKS and the moments, or null
+static const void* gather_kernel(int nks, int mom) {
+#define GM_CASE(CTV, NKSV)                                                        \
+  case NKSV:                                                                      \
+    return mom == 9 ? reinterpret_cast<const void*>(&k_gather_mma<1, NKSV, 9>)    \
+                    : reinterpret_cast<const void*>(&k_gather_mma<CTV, NKSV, 3>);
+  switch (nks) {
     GM_CASE(2, 9) GM_CASE(2, 13) GM_CASE(2, 17) GM_CASE(2, 19) GM_CASE(2, 25)
     GM_CASE(1, 33) GM_CASE(1, 41) GM_CASE(1, 57)
     default: return nullptr;
@@ -932,16 +968,16 @@ int recip_setup(mdff_ctx* c) {
   // matrix-core gather: A operand and its own split count
   c->mma_nks = mma_bucket(Kz + 1);
   c->mma_mtiles = div_up(M, 4);
-  c->mma_ct = mma_ct(c->mma_nks);
   int cus = 256;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus <= 0)
     cus = 256;
-  // splits over m-tiles (gather_splits)
-  const int atom_waves = div_up(c->n, 16 * c->mma_ct);
-  const void* gfn = gather_kernel(c->mma_ct, c->mma_nks);
-  const int64_t conc = 4 * (int64_t)cus * blocks_per_cu(gfn, 0);
-  const int best_s = gather_splits(c->mma_mtiles, atom_waves, conc);
-  c->mma_splits = best_s;
+  // splits over m-tiles (gather_splits), 3 and 9 moments
+  for (int k = 0; k < 2; ++k) {
+    const int mom = k ? 9 : 3;
+    const int atom_waves = div_up(c->n, 16 * mma_ct(c->mma_nks, mom));
+    const int64_t conc = 4 * (int64_t)cus * blocks_per_cu(gather_kernel(c->mma_nks, mom), 0);
+    c->mma_splits[k] = gather_splits(c->mma_mtiles, atom_waves, conc);
+  }
   // matrix-core structure factor: atoms per staged tile within 64 KiB of
   // LDS; atom chunks chosen from the kernel's occupancy so that the blocks
   // fill whole rounds of resident blocks with the fewest tiles per block
@@ -974,7 +1010,7 @@ int recip_setup(mdff_ctx* c) {
   // block partials of the energy / stress: k-blocks of 256
   HIP_TRY(c, hipMalloc((void**)&c->rec_blk, sizeof(double) * 7 * (size_t)div_up(nb, 256)));
   HIP_TRY(c, hipMalloc((void**)&c->sk_part, sizeof(double) * 4 * (size_t)std::max(c->sk_chunks, c->sk_mma_ch) * nb));
-  c->rec_splits = std::max(splits, c->mma_splits);
+  c->rec_splits = std::max({splits, c->mma_splits[0], c->mma_splits[1]});
   HIP_TRY(c, hipMalloc((void**)&c->rec_part, sizeof(double) * 9 * (size_t)c->rec_splits * c->n));
   return MDFF_OK;
 }
@@ -1056,7 +1092,8 @@ static int rec_finish(mdff_ctx* c, const double* part, int nsplit, int moments, 
 
 int recip_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool use_mu, bool forces,
                bool field, double* ef_out, double* f_out, double* e_out) {
-  const int moments = forces && use_mu ? 9 : 3;
+  // second moments: dipole forces, and the field gradient (efg.hip)
+  const int moments = forces && (use_mu || c->d.doefg) ? 9 : 3;
   if (c->mesh) {
     const bool wanted = forces || field;
     const double* part = nullptr;
@@ -1130,7 +1167,7 @@ int recip_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool 
   }
   // the 7 energy / stress sums over the k-blocks: block partials here, the
   // final sum queued into e_out (device memory)
-  const bool mma_gather = (forces || field) && moments == 3 && c->mma_nks > 0 && c->use_mma;
+  const bool mma_gather = (forces || field) && c->mma_nks > 0 && c->use_mma;
   const int nb = div_up(c->nk_box, 256);
   MDFF_TRY(claim_partials(c, c->rec_blk));
   PROF_LAUNCH(c, PK_SKRED,
@@ -1140,6 +1177,11 @@ int recip_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool 
   if (e_out) MDFF_TRY(queue_final(c, c->rec_blk, nb, 7, e_out));
   if (!forces && !field) return MDFF_OK;
   int nsplit = 0;
+  // the longest kES(3) of dipole forces is the vector-ALU gather's
+  if ((!mma_gather || (forces && use_mu)) && gather_lds(c->K[2], 64) > lds_limit(c)) {
+    c->err = "kES(3) too large for the reciprocal gather kernel";
+    return MDFF_ERR_UNSUPPORTED;
+  }
   if (mma_gather) {
     // matrix-core path (A operand written by k_sk_reduce)
     GmArgs gm{};
@@ -1148,15 +1190,16 @@ int recip_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool 
     gm.NY = c->NYk; gm.NZ = c->NZk; gm.M = M;
     gm.nks = c->mma_nks;
     gm.mtiles = c->mma_mtiles;
-    gm.mt_per_split = div_up(c->mma_mtiles, c->mma_splits);
+    gm.mt_per_split = div_up(c->mma_mtiles, c->mma_splits[moments == 9]);
     nsplit = div_up(c->mma_mtiles, gm.mt_per_split);
     gm.tab = c->tab;
     gm.amat = c->amat;
     gm.out = c->rec_part;
-    const void* fn = gather_kernel(c->mma_ct, gm.nks);
     void* args[] = {&gm};
-    PROF_LAUNCH(c, PK_GATHER, (void)hipLaunchKernel(fn, dim3(div_up(c->n, 4 * 16 * c->mma_ct), nsplit), dim3(256), args,
-                                                    0, c->stream));
+    PROF_LAUNCH(c, PK_GATHER,
+                (void)hipLaunchKernel(gather_kernel(gm.nks, moments),
+                                      dim3(div_up(c->n, 4 * 16 * mma_ct(gm.nks, moments)), nsplit), dim3(256), args, 0,
+                                      c->stream));
   } else {
     GaArgs g{};
     g.n = c->n;
@@ -1172,10 +1215,6 @@ int recip_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool 
     int nthr = 256;
     while (nthr > 64 && gather_lds(c->K[2], nthr) > 65536) nthr -= 64;
     const size_t shm = gather_lds(c->K[2], nthr);
-    if (shm > lds_limit(c)) {
-      c->err = "kES(3) too large for the reciprocal gather kernel";
-      return MDFF_ERR_UNSUPPORTED;
-    }
     const auto fn = moments == 9 ? &k_gather<9> : &k_gather<3>;
     MDFF_TRY(allow_lds(c, reinterpret_cast<const void*>(fn), shm));
     PROF_LAUNCH(c, PK_GATHER, hipLaunchKernelGGL(fn, dim3(div_up(c->n, nthr), nsplit), dim3(nthr), shm, c->stream, g));

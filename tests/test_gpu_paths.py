@@ -6,7 +6,7 @@ of the largest force."""
 import numpy as np
 import pytest
 
-from gpu_util import note, pair, rel_force_err
+from gpu_util import note, pair, rel, rel_force_err
 from mdff_amd import capi, configs
 
 pytestmark = pytest.mark.gpu
@@ -77,6 +77,20 @@ def test_mixed_long_k_mesh(k, dip, mesh, monkeypatch):
     note(f"long mesh {k} {dip}")
     g, o = pair(s, precision=capi.PREC_MIXED)
     assert rel_force_err(g.engforce()[0], o.engforce()[0]) < TOL[capi.PREC_MIXED]
+
+
+@pytest.mark.parametrize("dip", [False, True], ids=["charges", "dipoles"])
+@pytest.mark.parametrize("kz", [1, 8, 9, 12, 16, 17, 24, 25, 32, 33, 40, 50, 56])
+def test_second_moments(kz, dip, monkeypatch):
+    """Every size of the matrix-core gather: forces and field gradient."""
+    if dip and kz > 50:
+        pytest.skip("dipole forces take kES(3) up to 50")
+    monkeypatch.setenv("MDFF_RECIP_MESH", "0")
+    s = _long_mesh((2, 3, kz), dip)
+    note(f"second moments {kz} {dip}")
+    g, o = pair(s, doefg=1)
+    assert rel_force_err(g.engforce()[0], o.engforce()[0]) < TOL[capi.PREC_FP64]
+    assert rel(g.get_efg(), o.get_efg()) < TOL[capi.PREC_FP64]
 
 
 @pytest.mark.parametrize("mesh", ["0", "1"], ids=["direct", "mesh"])
