@@ -256,7 +256,8 @@ __global__ void __launch_bounds__(256) k_sk(SkArgs a) {
 
 __host__ __device__ __forceinline__ int row_of(int ml, int comp);
 
-// S(n) = sum of chunk partials (FP64, fixed order); W(n) = A conj(S);
+// S(n) = sum of chunk partials (FP64, fixed order: a wave a quarter of the
+// chunks of 64 k, so that few k still have loads enough in flight); W(n) = A conj(S);
 // per-block sums of A|S|^2 and (delta_ab - kcoe k_a k_b) A|S|^2.  With amat,
 // also the A operand of the matrix-core gather: amat[(mtile * nks + s) * 64
 // + lane] holds, for m = 4 mtile + ml and K index kk = 4 s + lane / 16 =
@@ -269,30 +270,37 @@ __global__ void __launch_bounds__(256) k_sk_reduce(int nk_box, int nchunk, const
                                                    double* __restrict__ wk, double* __restrict__ blk,
                                                    double* __restrict__ amat, int NZ, int Kz, int nks) {
   __shared__ double sh[4 * kRedMaxCols];
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
+  __shared__ double2 quarter[4][64];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int k = blockIdx.x * 64 + lane;
   double v[kRedMaxCols];
 #pragma unroll
   for (int c = 0; c < kRedMaxCols; ++c) v[c] = 0.0;
-  if (k < nk_box) {
+  {
     // chunks in order; the loads of 8 chunks are issued before their adds
-    double re = 0.0, im = 0.0;
-    int c = 0;
-    for (; c + 8 <= nchunk; c += 8) {
-      double vr[8], vi[8];
+    double2 t = {0.0, 0.0};
+    const double2* src = reinterpret_cast<const double2*>(part) + min(k, nk_box - 1);
+    const int per = (nchunk + 3) >> 2, c1 = min(nchunk, (wave + 1) * per);
+    for (int c = wave * per; c < c1; c += 8) {
+      double2 u8[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        vr[u] = part[(size_t)(c + u) * 2 * nk_box + 2 * k];
-        vi[u] = part[(size_t)(c + u) * 2 * nk_box + 2 * k + 1];
-      }
+      for (int u = 0; u < 8; ++u) u8[u] = src[(size_t)min(c + u, c1 - 1) * nk_box];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        re += vr[u];
-        im += vi[u];
-      }
+      for (int u = 0; u < 8; ++u)
+        if (c + u < c1) {
+          t.x += u8[u].x;
+          t.y += u8[u].y;
+        }
     }
-    for (; c < nchunk; ++c) {
-      re += part[(size_t)c * 2 * nk_box + 2 * k];
-      im += part[(size_t)c * 2 * nk_box + 2 * k + 1];
+    quarter[wave][lane] = t;
+  }
+  __syncthreads();
+  if (wave == 0 && k < nk_box) {
+    double re = 0.0, im = 0.0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      re += quarter[w][lane].x;
+      im += quarter[w][lane].y;
     }
     const double Ak = kA[k];
     wk[2 * k] = Ak * re;
@@ -648,40 +656,42 @@ k_gather_mma(GmArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Matrix-core structure factor, transposed form: S^double(nz, m) = sum_i
-// Z_i(nz) P_i(m).  Rows R = (nz, Re/Im) in 7 tiles of 16 (8 nz each; 56 nz
-// per block, blockIdx.z picks the group of 56), taken straight from the Z table; columns = 16 values of m = (nx, ny); K = (atom,
-// Re/Im of P).  The generated operand P_i(m) = a_i X_i[nx] Y_i[ny] is made
-// once per lane and K step and feeds the 7 row tiles.
-//   mode 0: a = q            (charges)
-//   mode 1: a = q + i 2pi (nx m_x + ny m_y)   (charges and dipoles, first part)
-//   mode 2: a = m_z          (second part: S = S1 + i 2pi nz S2)
-// FP32/FP64 MFMA accumulation within one staged atom tile, FP64 across tiles;
-// per-chunk FP64 partials.
+// Matrix-core structure factor, transposed form: S^T(nz, m) = sum_i
+// Z_i(nz) P_i(m), m = (nx, ny).  A block's four waves take 16 columns m each
+// and RT row tiles of 16 rows (nz, Re/Im), 8 nz a tile; K = (atom, Re/Im of
+// P).  Rows come straight from the Z table; P_i(m) = a_i X_i[nx] Y_i[ny] is
+// made once per lane and K step and feeds all RT row tiles.
+//   charges: a = q
+//   dipoles: a = q + i 2pi (nx m_x + ny m_y), and the nz m_z part as a second
+//            product into the same sums, rows nz Z against i 2pi m_z X Y
+// FP64 partials per chunk of atoms.  What bounds it: the FP64 matrix rate
+// where the blocks fill the chip, below that a block's own chain of staging
+// (latency) and products, so the host weighs tile and chunk sizes (sk_plan).
+// MgO 1,440 ions, kES 9, dipoles: 9.8 us (2 x 24 + 4.5 with 7 row tiles
+// whatever kES(3), tiles of 64 atoms, and two launches and a combining one for
+// dipoles); 216 ions, kES 5: 5.4 us (2 x 23 + 4.4); NaCl 512 7.1 us (14.4).
 // ---------------------------------------------------------------------------
-struct Sm2Args {
-  int n, Kx, Ky, Kz, NY, NZ, M, mtiles, chunk, TA, mode, nk_box;
+struct SmArgs {
+  int n, Kx, Ky, Kz, NY, NZ, M, chunk, lta, nk_box;   // 1 << lta atoms a staged tile
   const double* q;
   const double* mu;
   double b[9];
   const cplx* tab;
-  double* part;                  // [chunk][2*nk_box] FP64
+  double* part;                  // [chunk][2*nk_box]
 };
 
-template <int TA>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-k_sk_mma2(Sm2Args a) {
-  constexpr int RT = 7;                                          // row tiles: 56 nz values max
-  constexpr int TAP = TA + 2;                                    // padded atom stride of a staged column
-  static_assert(256 % TA == 0 && TA % 2 == 0, "atom tile must divide the block");
+constexpr int kSkStep = 4;       // K steps unrolled: 8 atoms, the smallest tile
+
+template <int RT, bool DIP>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_sk_mma(SmArgs a) {
   extern __shared__ unsigned char smem_raw[];
   const int ncol = a.Kx + a.Ky + a.Kz + 3;
+  const int TA = 1 << a.lta, TAP = TA + 2;                       // padded atom stride of a staged column
   // staged tile, column-major: st[col * TAP + atom]; then the a-coefficients
-  // sq[c * TAP + atom], c = 0..2.  A K step advances the atom by 2, a fixed
+  // sq[c * TAP + atom], c = 0..3.  A K step advances the atom by 2, a fixed
   // byte offset, so the unrolled step loop addresses LDS with immediates.
   cplx* st = reinterpret_cast<cplx*>(smem_raw);
   double* sq = reinterpret_cast<double*>(st + (size_t)ncol * TAP);
-  const cplx* tab = a.tab;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane >> 4, col = lane & 15;
   const int kk = g & 1, ja = g >> 1;                             // K: atom 2s+ja, Re/Im kk
@@ -693,7 +703,7 @@ k_sk_mma2(Sm2Args a) {
   const bool take_im = (col & 1) ^ kk;                           // which Z component feeds A
   const double* stT = reinterpret_cast<const double*>(st);
   const double* zp[RT];
-  double zs[RT];
+  double zs[RT], zn[DIP ? RT : 1];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     const int nzi = zoff + rt * 8 + (col >> 1);
@@ -702,6 +712,7 @@ k_sk_mma2(Sm2Args a) {
     const int zc = nzi < a.NZ ? zcol + (nz < 0 ? -nz : nz) : zcol;
     const double sgn_im = nz < 0 ? -1.0 : 1.0;
     zs[rt] = part == 0 ? (kk == 0 ? 1.0 : -sgn_im) : (kk == 0 ? sgn_im : 1.0);
+    if (DIP) zn[rt] = nz;
     zp[rt] = stT + 2 * ((size_t)zc * TAP + ja) + (take_im ? 1 : 0);
   }
   // B column of this lane
@@ -715,17 +726,14 @@ k_sk_mma2(Sm2Args a) {
   const double bw = bok ? 1.0 : 0.0;                            // columns beyond M: zero B (a multiply, no branch)
   const double* qp = sq + ja;
   f64x4 acc[RT];
-  double dacc[RT][4];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) dacc[rt][r] = 0.0;
+  for (int rt = 0; rt < RT; ++rt) acc[rt] = f64x4{0.0, 0.0, 0.0, 0.0};
   const int abeg = blockIdx.y * a.chunk;
   const int aend = min(a.n, abeg + a.chunk);
   // staging: thread -> (atom sia, columns scg, scg + CG, ...); loads from
   // clamped addresses in batches of 8, so they are in flight together
-  constexpr int CG = 256 / TA;
-  const int sia = threadIdx.x % TA, scg = threadIdx.x / TA;
+  const int CG = 256 >> a.lta;
+  const int sia = threadIdx.x & (TA - 1), scg = threadIdx.x >> a.lta;
   for (int t0 = abeg; t0 < aend; t0 += TA) {
     const int nt = min(TA, aend - t0);
     const bool sok = sia < nt;
@@ -734,66 +742,70 @@ k_sk_mma2(Sm2Args a) {
     for (int c0 = scg; c0 < ncol; c0 += 8 * CG) {
       cplx v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = tab[(size_t)min(c0 + u * CG, ncol - 1) * a.n + src];
+      for (int u = 0; u < 8; ++u) v[u] = a.tab[(size_t)min(c0 + u * CG, ncol - 1) * a.n + src];
 #pragma unroll
       for (int u = 0; u < 8; ++u)
         if (c0 + u * CG < ncol) st[(size_t)(c0 + u * CG) * TAP + sia] = sok ? v[u] : cplx{0.0, 0.0};
     }
     if (threadIdx.x < TA) {
       const int ia = threadIdx.x;
-      double c0 = 0.0, c1 = 0.0, c2 = 0.0;
+      double c0 = 0.0, c1 = 0.0, c2 = 0.0, c3 = 0.0;
       if (ia < nt) {
         const int i = t0 + ia;
-        if (a.mode <= 1) c0 = a.q[i];
-        if (a.mode >= 1) {
+        c0 = a.q[i];
+        if (DIP) {
           const double u0 = a.mu[3 * i], u1 = a.mu[3 * i + 1], u2 = a.mu[3 * i + 2];
-          if (a.mode == 1) {
-            c1 = 2.0 * MDFF_PI * (u0 * a.b[0] + u1 * a.b[1] + u2 * a.b[2]);
-            c2 = 2.0 * MDFF_PI * (u0 * a.b[3] + u1 * a.b[4] + u2 * a.b[5]);
-          } else {
-            c0 = u0 * a.b[6] + u1 * a.b[7] + u2 * a.b[8];
-          }
+          c1 = 2.0 * MDFF_PI * (u0 * a.b[0] + u1 * a.b[1] + u2 * a.b[2]);
+          c2 = 2.0 * MDFF_PI * (u0 * a.b[3] + u1 * a.b[4] + u2 * a.b[5]);
+          c3 = 2.0 * MDFF_PI * (u0 * a.b[6] + u1 * a.b[7] + u2 * a.b[8]);
         }
       }
       sq[ia] = c0;
-      sq[TAP + ia] = c1;
-      sq[2 * TAP + ia] = c2;
+      if (DIP) {
+        sq[TAP + ia] = c1;
+        sq[2 * TAP + ia] = c2;
+        sq[3 * TAP + ia] = c3;
+      }
     }
     __syncthreads();
+    // K steps of 4: atoms 2s and 2s+1 (Re/Im of P).  Atoms beyond nt are the
+    // zero padding of the staged tile: no step needs a mask.
+    const int ns = (nt + 2 * kSkStep - 1) / (2 * kSkStep);
+    for (int q8 = 0; q8 < ns; ++q8) {
+      const int o = q8 * 2 * kSkStep;                            // first atom
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-      acc[rt] = f64x4{0.0, 0.0, 0.0, 0.0};
-    // K steps of 4: atoms 2s and 2s+1 (Re/Im of P).  Rows beyond nt are the
-    // zero padding of the staged tile, so every tile runs all TA/2 steps and
-    // no step needs a mask.
+      for (int s = 0; s < kSkStep; ++s) {
+        double av[RT];
 #pragma unroll
-    for (int s = 0; s < TA / 2; ++s) {
-      double av[RT];
+        for (int rt = 0; rt < RT; ++rt) av[rt] = zs[rt] * zp[rt][2 * o + 4 * s];
+        const cplx X = xp[o + 2 * s];
+        const cplx Y = yp[o + 2 * s];
+        const double yim = bneg ? -Y.im : Y.im;
+        const double xyr = X.re * Y.re - X.im * yim;
+        const double xyi = X.re * yim + X.im * Y.re;
+        const double c0 = qp[o + 2 * s];
+        double pre = c0 * xyr, pim = c0 * xyi;
+        if (DIP) {
+          // (c0 + i bb) XY, bb = 2pi (nx mx + ny my)
+          const double bb = bnxf * qp[TAP + o + 2 * s] + bnyf * qp[2 * TAP + o + 2 * s];
+          pre -= bb * xyi;
+          pim += bb * xyr;
+        }
+        const double bv = bw * (kk == 0 ? pre : pim);
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) av[rt] = zs[rt] * zp[rt][4 * s];
-      const double c0 = qp[2 * s], c1 = qp[TAP + 2 * s], c2 = qp[2 * TAP + 2 * s];
-      const cplx X = xp[2 * s];
-      const cplx Y = yp[2 * s];
-      const double yim = bneg ? -Y.im : Y.im;
-      const double xyr = X.re * Y.re - X.im * yim;
-      const double xyi = X.re * yim + X.im * Y.re;
-      // (c0 + i bb) XY, bb = 2pi (nx mx + ny my) in mode 1 (c1, c2 carry 2pi)
-      const double bb = bnxf * c1 + bnyf * c2;
-      const double pre = c0 * xyr - bb * xyi;
-      const double pim = c0 * xyi + bb * xyr;
-      const double bv = bw * (kk == 0 ? pre : pim);
+        for (int rt = 0; rt < RT; ++rt) acc[rt] = mfma(av[rt], bv, acc[rt]);
+        if (DIP) {
+          const double c3 = qp[3 * TAP + o + 2 * s];
+          const double bz = bw * (kk == 0 ? -c3 * xyi : c3 * xyr);
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-        acc[rt] = mfma(av[rt], bv, acc[rt]);
+          for (int rt = 0; rt < RT; ++rt) acc[rt] = mfma(zn[rt] * av[rt], bz, acc[rt]);
+        }
+      }
     }
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) dacc[rt][r] += acc[rt][r];
   }
+  if (!bok) return;
   // D: lane holds rows Rd(r) of column m; row Rd -> nz = rt*8 + Rd/2, part Rd%2
   double* out = a.part + (size_t)blockIdx.y * 2 * a.nk_box;
-  if (!bok) return;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -801,20 +813,8 @@ k_sk_mma2(Sm2Args a) {
       const int Rd = 4 * r + g;
       const int nzi = zoff + rt * 8 + (Rd >> 1);
       if (nzi >= a.NZ) continue;
-      out[2 * ((size_t)m * a.NZ + nzi) + (Rd & 1)] = dacc[rt][r];
+      out[2 * ((size_t)m * a.NZ + nzi) + (Rd & 1)] = acc[rt][r];
     }
-}
-
-// S = S1 + i 2pi nz S2 from two partial sets (dipole amplitude)
-__global__ void k_sk_combine(int nk_box, int NZ, int Kz, int nchunk, double* __restrict__ p1,
-                             const double* __restrict__ p2) {
-  const size_t x = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= (size_t)nchunk * nk_box) return;
-  const int k = (int)(x % nk_box);
-  const double fz = 2.0 * MDFF_PI * (double)(k % NZ - Kz);
-  const double s2r = p2[2 * x], s2i = p2[2 * x + 1];
-  p1[2 * x] -= fz * s2i;
-  p1[2 * x + 1] += fz * s2r;
 }
 
 }  // namespace
@@ -843,15 +843,15 @@ static const void* gather_kernel(int nks, int mom) {
 #undef GM_CASE
 }
 
-// the compiled matrix-core structure factor for a staged tile of TA atoms, or null
-static const void* sk_kernel(int ta) {
-  switch (ta) {
-    case 64: return reinterpret_cast<const void*>(&k_sk_mma2<64>);
-    case 32: return reinterpret_cast<const void*>(&k_sk_mma2<32>);
-    case 16: return reinterpret_cast<const void*>(&k_sk_mma2<16>);
-    case 8: return reinterpret_cast<const void*>(&k_sk_mma2<8>);
+// the compiled matrix-core structure factor of rt row tiles (1..7)
+static const void* sk_kernel(int rt, bool dip) {
+#define SK_CASE(R) \
+  case R: return dip ? reinterpret_cast<const void*>(&k_sk_mma<R, true>) : reinterpret_cast<const void*>(&k_sk_mma<R, false>);
+  switch (rt) {
+    SK_CASE(1) SK_CASE(2) SK_CASE(3) SK_CASE(4) SK_CASE(5) SK_CASE(6) SK_CASE(7)
     default: return nullptr;
   }
+#undef SK_CASE
 }
 
 // Split count of a gather over mtiles m-tiles for atom_waves waves of atoms:
@@ -885,7 +885,7 @@ static int blocks_per_cu(const void* fn, size_t lds) {
 }
 
 // LDS bytes of the matrix-core structure factor for a tile of ta atoms
-static size_t sk_lds(int ncol, int ta) { return (16 * (size_t)ncol + 24) * (size_t)(ta + 2); }
+static size_t sk_lds(int ncol, int ta) { return (16 * (size_t)ncol + 32) * (size_t)(ta + 2); }
 // ... of the vector-ALU one
 static size_t sk_valu_lds(int ncol, int ta) { return (16 * (size_t)ncol + 32) * (size_t)ta; }
 // ... and of the vector-ALU gather with nthr threads a block
@@ -901,11 +901,50 @@ static int allow_lds(mdff_ctx* c, const void* fn, size_t lds) {
   return MDFF_OK;
 }
 
+// table columns the matrix-core structure factor takes
+static int sk_cols(const mdff_ctx* c) { return c->d.precision == MDFF_PREC_MIXED ? 817 : 408; }
+
 // whether the direct kernels below take the k mesh (sums and gather both)
 static bool direct_takes(const mdff_ctx* c) {
   const bool dip = c->task_qd || c->task_dd;
   const bool gather = gather_lds(c->K[2], 64) <= lds_limit(c) || (!dip && mma_bucket(c->K[2] + 1) > 0);
-  return gather && sk_lds(c->K[0] + c->K[1] + c->K[2] + 3, 8) <= lds_limit(c);
+  return gather && c->K[0] + c->K[1] + c->K[2] + 3 <= sk_cols(c);
+}
+
+// Row tiles, staged tile and atom chunks of the matrix-core structure factor.
+// Row tiles: kES(3) spread evenly over as few blocks of at most 7 as it needs.
+// Tile and chunks: the least of a sum of what a launch waits for (us): a tile's
+// staging kStage, its products (64 cycles each on a SIMD, shared by the blocks
+// of a CU), and kChunk a chunk for the reduction that adds them up.
+static int sk_plan(mdff_ctx* c, int cus) {
+  constexpr double kStage = 1.5, kChunk = 0.08, kProduct = 64.0 / 2400.0;
+  const int ncol = c->K[0] + c->K[1] + c->K[2] + 3;
+  c->sk_mma_ch = 1;
+  if (ncol > sk_cols(c)) return MDFF_OK;          // refused at the first evaluation (sk_rt 0)
+  const bool dip = c->task_qd || c->task_dd;
+  const int nt = div_up(c->NZk, 8), zb = div_up(nt, 7);
+  c->sk_rt = div_up(nt, zb);
+  const int mblocks = div_up(div_up(c->NXk * c->NYk, 16), 4) * zb;
+  double best = 0.0;
+  for (int lta = 6; lta >= 3; --lta) {
+    const int TA = 1 << lta;
+    const size_t lds = sk_lds(ncol, TA);
+    if (lds > (lta > 3 ? 65536 : 131072)) continue;
+    for (int d = 0; d < 2; ++d) MDFF_TRY(allow_lds(c, sk_kernel(c->sk_rt, d), lds));
+    const int64_t cap = (int64_t)cus * blocks_per_cu(sk_kernel(c->sk_rt, dip), lds);
+    for (int ch = 1; ch <= 128 && (ch == 1 || div_up(c->n, ch) >= TA); ++ch) {
+      const int per = div_up(c->n, ch), nch = div_up(c->n, per), tiles = div_up(per, TA);
+      const int64_t blocks = (int64_t)mblocks * nch;
+      const double t = (double)div_up(blocks, cap) * tiles * kStage + kChunk * nch +
+                       (double)div_up(blocks, cus) * div_up(per, 8) * kSkStep * c->sk_rt * (dip ? 2 : 1) * kProduct;
+      if (best == 0.0 || t < best) {
+        best = t;
+        c->sk_mma_ch = nch;
+        c->sk_lta = lta;
+      }
+    }
+  }
+  return MDFF_OK;
 }
 
 int recip_setup(mdff_ctx* c) {
@@ -940,12 +979,14 @@ int recip_setup(mdff_ctx* c) {
   HIP_TRY(c, hipMemcpy(c->kvec, kv.data(), sizeof(double) * 4 * nb, hipMemcpyHostToDevice));
   // The direct sums cost atoms x k vectors, the transforms some 60 us of short
   // kernels and a few us per 1,000 atoms (us a step or evaluation, direct / mesh):
-  //   mixed  2.4e7 (silica 3,000) 120/132   4.3e7 (MgO 4,608 dipoles) 2906/2736   8e7 (silica 5,184) 168/143
-  //   FP64   5.4e7 (silica 4,320) 140/163   4.3e7 (MgO 4,608) 3057/3076   8e7 167/164   1.8e8 236/191
+  //   FP64   8e7 (silica 5,184) 160/164   1.5e8 (LiF 5,832) 157/145   1.8e8 (silica 8,232) 218/191
+  //   mixed  5.4e7 (silica 4,320) 136/138   4.3e7 (MgO 4,608 dipoles) 2514/2733   8e7 160/142
+  //   gradient  9e7 (NaCl 4,096) 341/323
   // The mixed form's narrower kernel (12 points, not 16) puts its line lower.
   {
     const char* ev = getenv("MDFF_RECIP_MESH");
-    const bool on = ev && ev[0] ? ev[0] != '0' : (double)c->n * nb > (c->d.precision == MDFF_PREC_MIXED ? 4e7 : 8e7);
+    const double line = c->d.doefg ? 8e7 : (c->d.precision == MDFF_PREC_MIXED ? 7e7 : 1.1e8);
+    const bool on = ev && ev[0] ? ev[0] != '0' : (double)c->n * nb > line;
     if (on && c->use_mma && direct_takes(c)) {
       MDFF_TRY(mesh_setup(c, A, kv));
       if (c->mesh) return MDFF_OK;
@@ -978,38 +1019,13 @@ int recip_setup(mdff_ctx* c) {
     const int64_t conc = 4 * (int64_t)cus * blocks_per_cu(gather_kernel(c->mma_nks, mom), 0);
     c->mma_splits[k] = gather_splits(c->mma_mtiles, atom_waves, conc);
   }
-  // matrix-core structure factor: atoms per staged tile within 64 KiB of
-  // LDS; atom chunks chosen from the kernel's occupancy so that the blocks
-  // fill whole rounds of resident blocks with the fewest tiles per block
-  {
-    int TA = 64;
-    while (TA > 8 && sk_lds(ncol, TA) > 65536) TA /= 2;
-    c->sk_ta = sk_lds(ncol, TA) <= lds_limit(c) ? TA : 0;
-    c->sk_mma_ch = 1;
-    if (c->sk_ta) {
-      const void* sfn = sk_kernel(TA);
-      MDFF_TRY(allow_lds(c, sfn, sk_lds(ncol, TA)));
-      const int64_t cap = (int64_t)cus * blocks_per_cu(sfn, sk_lds(ncol, TA));
-      const int64_t mblocks = div_up(div_up(M, 16), 4) * (int64_t)div_up(c->NZk, 56);
-      int64_t best = -1;
-      for (int ch = 1; ch <= 128 && (ch == 1 || div_up(c->n, ch) >= TA); ++ch) {
-        const int per = div_up(c->n, ch);
-        const int nch = div_up(c->n, per);
-        const int64_t rounds = (mblocks * nch + cap - 1) / cap;
-        const int64_t cost = rounds * div_up(per, TA);
-        if (best < 0 || cost < best) {
-          best = cost;
-          c->sk_mma_ch = nch;
-        }
-      }
-    }
-  }
+  MDFF_TRY(sk_plan(c, cus));
   const size_t na = (size_t)c->mma_mtiles * c->mma_nks * 64;
   HIP_TRY(c, hipMalloc((void**)&c->amat, sizeof(double) * na));
   HIP_TRY(c, hipMemset(c->amat, 0, sizeof(double) * na));
-  // block partials of the energy / stress: k-blocks of 256
-  HIP_TRY(c, hipMalloc((void**)&c->rec_blk, sizeof(double) * 7 * (size_t)div_up(nb, 256)));
-  HIP_TRY(c, hipMalloc((void**)&c->sk_part, sizeof(double) * 4 * (size_t)std::max(c->sk_chunks, c->sk_mma_ch) * nb));
+  // block partials of the energy / stress: k-blocks of 64
+  HIP_TRY(c, hipMalloc((void**)&c->rec_blk, sizeof(double) * 7 * (size_t)div_up(nb, 64)));
+  HIP_TRY(c, hipMalloc((void**)&c->sk_part, sizeof(double) * 2 * (size_t)std::max(c->sk_chunks, c->sk_mma_ch) * nb));
   c->rec_splits = std::max({splits, c->mma_splits[0], c->mma_splits[1]});
   HIP_TRY(c, hipMalloc((void**)&c->rec_part, sizeof(double) * 9 * (size_t)c->rec_splits * c->n));
   return MDFF_OK;
@@ -1104,39 +1120,28 @@ int recip_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool 
   const int M = c->NXk * c->NYk, ncol = c->K[0] + c->K[1] + c->K[2] + 3;
   int chunks = c->sk_mma_ch;
   if (c->use_mma) {
-    Sm2Args sm{};
+    SmArgs sm{};
     sm.n = c->n;
     sm.Kx = c->K[0]; sm.Ky = c->K[1]; sm.Kz = c->K[2];
     sm.NY = c->NYk; sm.NZ = c->NZk; sm.M = M;
     sm.chunk = div_up(c->n, chunks);
     chunks = div_up(c->n, sm.chunk);
+    sm.lta = c->sk_lta;
     sm.nk_box = c->nk_box;
     sm.q = use_q ? q : c->zeros;
     sm.mu = mu;
     for (int k = 0; k < 9; ++k) sm.b[k] = c->B[k];
     sm.tab = c->tab;
-    if (c->sk_ta == 0) {
+    sm.part = c->sk_part;
+    if (c->sk_rt == 0) {
       c->err = "kES too large for the structure-factor kernel";
       return MDFF_ERR_UNSUPPORTED;
     }
-    const dim3 gs(div_up(div_up(M, 16), 4), chunks, div_up(c->NZk, 56));
-    sm.part = c->sk_part;
-    // first pass: mode 0 (charges) or mode 1 (charges, zero when switched
-    // off, plus the x/y dipole phase); second pass for dipoles: mode 2
-    sm.mode = use_mu ? 1 : 0;
-    auto launch = [&](const Sm2Args& a) {
-      void* args[] = {const_cast<Sm2Args*>(&a)};
-      (void)hipLaunchKernel(sk_kernel(c->sk_ta), gs, dim3(256), args, sk_lds(ncol, c->sk_ta), c->stream);
-    };
-    PROF_LAUNCH(c, PK_SK, launch(sm));
-    if (use_mu) {
-      Sm2Args s2 = sm;
-      s2.mode = 2;
-      s2.part = c->sk_part + (size_t)2 * chunks * c->nk_box;
-      const size_t tot = (size_t)chunks * c->nk_box;
-      PROF_LAUNCH(c, PK_SK, launch(s2); hipLaunchKernelGGL(k_sk_combine, dim3(div_up(tot, 256)), dim3(256), 0, c->stream,
-                                                           c->nk_box, c->NZk, c->K[2], chunks, sm.part, s2.part));
-    }
+    void* args[] = {&sm};
+    PROF_LAUNCH(c, PK_SK,
+                (void)hipLaunchKernel(sk_kernel(c->sk_rt, use_mu),
+                                      dim3(div_up(div_up(M, 16), 4), chunks, div_up(c->NZk, 8 * c->sk_rt)), dim3(256),
+                                      args, sk_lds(ncol, 1 << c->sk_lta), c->stream));
   } else {
     SkArgs s{};
     s.n = c->n;
@@ -1168,7 +1173,7 @@ int recip_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool 
   // the 7 energy / stress sums over the k-blocks: block partials here, the
   // final sum queued into e_out (device memory)
   const bool mma_gather = (forces || field) && c->mma_nks > 0 && c->use_mma;
-  const int nb = div_up(c->nk_box, 256);
+  const int nb = div_up(c->nk_box, 64);
   MDFF_TRY(claim_partials(c, c->rec_blk));
   PROF_LAUNCH(c, PK_SKRED,
               hipLaunchKernelGGL(k_sk_reduce, dim3(nb), dim3(256), 0, c->stream, c->nk_box, chunks, c->sk_part, c->kA,
