@@ -53,6 +53,8 @@ __device__ __forceinline__ c2<T> cm(c2<T> a, c2<T> b) {
   return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
 }
 
+typedef c2<double> c2d;
+
 // parameter kinds of the fit vector
 enum { FP_A = 0, FP_RHO = 1, FP_C = 2, FP_ALPHA = 3, FP_TTB = 4, FP_TTC = 5 };
 constexpr int FIT_MAXP = 32;  // parameters
@@ -68,6 +70,21 @@ struct FitSnap {
   int npol;
   double A[9];               // cell, column-major
   double omega, rc2_sr, rc2_c, alpha;
+};
+
+// a snapshot's k box and polarisable atoms, as the iterations' matrix-core
+// kernels see them: k index (nx, ny + Ky, nz + Kz), m = (nx, ny)
+struct FitBox {
+  int np, p0;                // polarisable atoms, the first of them in pidx
+  int M, NY, NZ, nb;         // rows m, extents, k of the box
+  int mtiles, nks;           // gather: tiles of 4 m, K steps of 4 over (nz, Re/Im)
+  int chunk, nsplit, mtps;   // atoms a structure-factor chunk; gather splits, m-tiles a split
+  int nch;                   // structure-factor chunks
+  long long box0, w0;        // first k in kbox; first element in wbox (rows m padded to mtiles, nz to nks)
+  long long s0, g0;          // first record of the partial structure factors / moments
+  long long r0;              // first neighbour row (np + 1 entries)
+  long long n0;              // first neighbour entry
+  double B[9];               // reciprocal matrix, column-major
 };
 
 // per type pair (it, jt): Buckingham and the damping of the field at a
@@ -117,7 +134,6 @@ struct FitArgs {
   double* hn;                           // per snap: RMS of h (adjoint tolerance)
   double* Gs;                           // per snap: symmetric stress weight (9)
   double* gsave;                        // per snap: gradient partial sums of the pair pass (FIT_MAXP)
-  int* count;                           // snapshots still iterating (control kernel)
   const int4* gblk;                     // gather blocks: (snapshot, first atom, first k, k chunk)
   const int* snap_g0;                   // per snapshot: first gather record (atom x k chunk)
   const int* snap_nch;                  // per snapshot: k chunks
@@ -126,6 +142,22 @@ struct FitArgs {
   const int* snap_s0;                   // per snapshot: first structure-factor record (k x atom chunk)
   const int* snap_sch;                  // per snapshot: atom chunks
   double* sp;                           // structure-factor records [record][2]
+  // the iterations' matrix-core path (null boxes: the vector-ALU one)
+  const FitBox* boxes;
+  const int *pidx, *pinv;               // polarisable atoms; an atom's place among them or -1
+  const double* kbox;                   // A(k) on the boxes, 0 outside the half space
+  const int4 *mblk, *rblk, *qblk, *dblk; // blocks: structure factor, reduction, gather, real space
+  const c2d* tab64;                     // FP64 phase tables
+  double *msp, *wbox, *mgp;             // partial structure factors, W on the boxes, partial moments
+  const int *prow, *pnl;                // neighbour rows among polarisable atoms
+  int dlanes;                           // lanes an atom in the real-space field
+  // pair passes: blocks of 256 / planes atoms, their partials and the sums of a snapshot's blocks
+  const int4* pblk;
+  const int* snap_pb0;
+  double *pp, *ps;                      // [block][FIT_MAXP], [snapshot][FIT_MAXP]
+  int planes, nparam;
+  double *h_count;                      // mapped host memory: snapshots still iterating, sequence number
+  double seq;
   int ws_dst, ws_src;                   // kf_update: ws slots (3 n each) dst = alpha src
 };
 
@@ -340,7 +372,6 @@ __device__ __forceinline__ GatherStage gather_stage_of(double* lds) {
   return g;
 }
 // lanes per atom of the iteration's real-space dipole field (kf_dipreal)
-constexpr int kDipLanes = 4;
 constexpr size_t kGatherLds = sizeof(double) * 9 * FIT_KC + sizeof(int) * FIT_KC;
 
 // the block's k-vectors kb0..kb1 (kb1 - kb0 <= FIT_KC) into LDS, by every
@@ -459,10 +490,11 @@ __device__ void gather(const FitSnap& S, const c2<T>* tab, int j, int nkl, bool 
 // Real-space field passes
 // ---------------------------------------------------------------------------
 
-// static field of the charges at polarisable atoms, TT-damped (SCF), plus
+// static field of the charges at polarisable atoms, TT-damped (SCF), L lanes
+// an atom from atom ib0 of the snapshot, plus
 // the lambda . dE_stat/d(b, c) gradient terms when lam != nullptr
 template <typename T>
-__device__ void field_static(const FitArgs& a, const FitSnap& S, int ib0, int ib1, double* Es, const double* lam,
+__device__ void field_static(const FitArgs& a, const FitSnap& S, int ib0, int L, double* Es, const double* lam,
                              double* gacc) {
   const double* sx = a.sx + S.a0;
   const double* sy = a.sy + S.a0;
@@ -470,11 +502,13 @@ __device__ void field_static(const FitArgs& a, const FitSnap& S, int ib0, int ib
   const int* it = a.itype + S.a0;
   const double* q = a.q + S.a0;
   const T alpha = (T)S.alpha;
-  for (int i = ib0 + threadIdx.x; i < ib1; i += blockDim.x) {
+  const int sub = (int)threadIdx.x & (L - 1);
+  const int i = ib0 + (int)threadIdx.x / L;
+  if (i < S.n) {
     double e0 = 0, e1 = 0, e2 = 0;
     const int ti = it[i];
     if (a.alpha_t[ti] != 0.0) {
-      for (int e = a.row[S.row0 + i]; e < a.row[S.row0 + i + 1]; ++e) {
+      for (int e = a.row[S.row0 + i] + sub; e < a.row[S.row0 + i + 1]; e += L) {
         const int j = a.nl[S.nl0 + e];
         const Geo G = min_image(S, sx, sy, sz, i, j);
         if (G.r2 > S.rc2_c) continue;
@@ -489,8 +523,8 @@ __device__ void field_static(const FitArgs& a, const FitSnap& S, int ib0, int ib
           gg -= qj * (T(1) - f) * E.dm3;
           if (lam) {
             const T lr = (T)(lam[3 * i] * G.rx + lam[3 * i + 1] * G.ry + lam[3 * i + 2] * G.rz);
-            if (P.sB >= 0) gacc[P.sB] += (double)(qj * fb * E.dm3 * lr);
-            if (P.sC2 >= 0) gacc[P.sC2] += (double)(qj * fc * E.dm3 * lr);
+            if (P.sB >= 0) gacc[256 * P.sB] += (double)(qj * fb * E.dm3 * lr);
+            if (P.sC2 >= 0) gacc[256 * P.sC2] += (double)(qj * fc * E.dm3 * lr);
           }
         }
         e0 += (double)(gg * (T)G.rx);
@@ -499,6 +533,13 @@ __device__ void field_static(const FitArgs& a, const FitSnap& S, int ib0, int ib
       }
     }
     if (Es) {
+      for (int w = 1; w < L; w <<= 1) {
+        e0 += __shfl_xor(e0, w);
+        e1 += __shfl_xor(e1, w);
+        e2 += __shfl_xor(e2, w);
+      }
+    }
+    if (Es && sub == 0) {
       Es[3 * i] = e0;
       Es[3 * i + 1] = e1;
       Es[3 * i + 2] = e2;
@@ -507,24 +548,23 @@ __device__ void field_static(const FitArgs& a, const FitSnap& S, int ib0, int ib
 }
 
 // field of a dipole set v (undamped, real space only), at polarisable atoms,
-// from polarisable atoms (the mu-mu pairs of src/ewald_dir.f90:557-593)
+// from polarisable atoms (the mu-mu pairs of src/ewald_dir.f90:557-593):
+// rows of polarisable neighbours only, L lanes an atom (a power of two)
 template <typename T>
-__device__ void field_dip_real(const FitArgs& a, const FitSnap& S, int ib0, int ib1, const double* v, double* out,
-                               double* red) {
+__device__ void field_dip_real(const FitArgs& a, const FitSnap& S, const FitBox& X, int p0, int L, const double* v,
+                               double* out) {
   const double* sx = a.sx + S.a0;
   const double* sy = a.sy + S.a0;
   const double* sz = a.sz + S.a0;
-  const int* it = a.itype + S.a0;
   const T alpha = (T)S.alpha;
-  // gridDim.y lanes per atom stride its row; blockIdx.y picks the block's
-  // share of atoms (blockDim / gridDim.y of them)
-  const int L = (int)gridDim.y, sub = (int)threadIdx.x % L, per = (int)blockDim.x / L;
-  const int i = ib0 + (int)blockIdx.y * per + (int)threadIdx.x / L;
+  const int sub = (int)threadIdx.x & (L - 1);
+  const int p = p0 + (int)threadIdx.x / L;
+  const bool on = p < X.np;
+  const int i = a.pidx[X.p0 + (on ? p : 0)];
   double e0 = 0, e1 = 0, e2 = 0;
-  if (i < ib1 && a.alpha_t[it[i]] != 0.0) {
-    for (int e = a.row[S.row0 + i] + sub; e < a.row[S.row0 + i + 1]; e += L) {
-      const int j = a.nl[S.nl0 + e];
-      if (a.alpha_t[it[j]] == 0.0) continue;
+  if (on) {
+    for (int e = a.prow[X.r0 + p] + sub; e < a.prow[X.r0 + p + 1]; e += L) {
+      const int j = a.pnl[X.n0 + e];
       const Geo G = min_image(S, sx, sy, sz, i, j);
       if (G.r2 > S.rc2_c) continue;
       const T d = sqrt((T)G.r2);
@@ -538,21 +578,15 @@ __device__ void field_dip_real(const FitArgs& a, const FitSnap& S, int ib0, int 
       e2 += (double)(c3 * rz - c1 * vz);
     }
   }
-  // the L lane sums of an atom added in lane order
-  red[3 * threadIdx.x] = e0;
-  red[3 * threadIdx.x + 1] = e1;
-  red[3 * threadIdx.x + 2] = e2;
-  __syncthreads();
-  if (sub == 0 && i < ib1) {
-    double f0 = 0, f1 = 0, f2 = 0;
-    for (int l = 0; l < L; ++l) {
-      f0 += red[3 * (threadIdx.x + l)];
-      f1 += red[3 * (threadIdx.x + l) + 1];
-      f2 += red[3 * (threadIdx.x + l) + 2];
-    }
-    out[3 * i] = f0;
-    out[3 * i + 1] = f1;
-    out[3 * i + 2] = f2;
+  for (int w = 1; w < L; w <<= 1) {
+    e0 += __shfl_xor(e0, w);
+    e1 += __shfl_xor(e1, w);
+    e2 += __shfl_xor(e2, w);
+  }
+  if (on && sub == 0) {
+    out[3 * i] = e0;
+    out[3 * i + 1] = e1;
+    out[3 * i + 2] = e2;
   }
 }
 
@@ -561,9 +595,10 @@ __device__ void field_dip_real(const FitArgs& a, const FitSnap& S, int ib0, int 
 // ---------------------------------------------------------------------------
 
 // One pass over the rows.  FORCE: F (eV/A) and the real-space stress sums.
-// ADJ: h_real (into h), explicit Buckingham and TT gradients (into gacc).
+// ADJ: h_real (into h), explicit Buckingham and TT gradients (into gacc, LDS
+// of 256 threads a slot).  L lanes an atom, from atom ib0 of the snapshot.
 template <typename T, bool ADJ>
-__device__ void pair_pass(const FitArgs& a, const FitSnap& S, int ib0, int ib1, const double* mu, const double* gv,
+__device__ void pair_pass(const FitArgs& a, const FitSnap& S, int ib0, int L, const double* mu, const double* gv,
                           const double Gs[9], double* Fout, double* h, double* gacc, double st_nonb[6],
                           double st_dir[6]) {
   const double* sx = a.sx + S.a0;
@@ -574,13 +609,15 @@ __device__ void pair_pass(const FitArgs& a, const FitSnap& S, int ib0, int ib1, 
   const T alpha = (T)S.alpha;
   const double cu = a.coul_unit;
   const double sgs = 1.0 / (S.omega * a.press_unit);
-  for (int i = ib0 + threadIdx.x; i < ib1; i += blockDim.x) {
+  const int sub = (int)threadIdx.x & (L - 1);
+  const int i = ib0 + (int)threadIdx.x / L;
+  if (i < S.n) {
     const int ti = it[i];
     const T qi = (T)q[i];
     const T mix = (T)mu[3 * i], miy = (T)mu[3 * i + 1], miz = (T)mu[3 * i + 2];
     const bool dip_i = a.alpha_t[ti] != 0.0;
     double fsr[3] = {0, 0, 0}, fcl[3] = {0, 0, 0}, hh[3] = {0, 0, 0};
-    for (int e = a.row[S.row0 + i]; e < a.row[S.row0 + i + 1]; ++e) {
+    for (int e = a.row[S.row0 + i] + sub; e < a.row[S.row0 + i + 1]; e += L) {
       const int j = a.nl[S.nl0 + e];
       const int tj = it[j];
       const Geo G = min_image(S, sx, sy, sz, i, j);
@@ -618,11 +655,11 @@ __device__ void pair_pass(const FitArgs& a, const FitSnap& S, int ib0, int ib1, 
           // half (two rows per pair) of dw/dtheta [(g_i - g_j).r + r.Gs.r/(omega pu)]
           const T proj = T(0.5) * (dvx * rx + dvy * ry + dvz * rz);
           const T ex = exp(-B * d);
-          if (P.sA >= 0) gacc[P.sA] += (double)(proj * B * ex * dm1);
-          if (P.sC >= 0) gacc[P.sC] += (double)(proj * T(-6) * dm1 * dm1 * dm1 * dm1 * dm1 * dm1 * dm1 * dm1);
+          if (P.sA >= 0) gacc[256 * P.sA] += (double)(proj * B * ex * dm1);
+          if (P.sC >= 0) gacc[256 * P.sC] += (double)(proj * T(-6) * dm1 * dm1 * dm1 * dm1 * dm1 * dm1 * dm1 * dm1);
           if (P.sRho >= 0) {
             const T rho = (T)P.rho;
-            gacc[P.sRho] += (double)(proj * (-(Ab * ex * (T(1) - B * d)) * dm1 / (rho * rho)));
+            gacc[256 * P.sRho] += (double)(proj * (-(Ab * ex * (T(1) - B * d)) * dm1 / (rho * rho)));
           }
         }
       }
@@ -717,11 +754,11 @@ __device__ void pair_pass(const FitArgs& a, const FitSnap& S, int ib0, int ib1, 
             const T base3 = T(3) * E.dm5 * rmi * dr, base1 = E.dm3 * edmi;
             if (P.sB >= 0) {
               const T dF1 = -fb, dF2 = -fb + (d / T(3)) * fdb;
-              gacc[P.sB] += (double)(T(0.5) * (-qj) * (dF2 * base3 - dF1 * base1));
+              gacc[256 * P.sB] += (double)(T(0.5) * (-qj) * (dF2 * base3 - dF1 * base1));
             }
             if (P.sC2 >= 0) {
               const T dF1 = -fc, dF2 = -fc + (d / T(3)) * fdc;
-              gacc[P.sC2] += (double)(T(0.5) * (-qj) * (dF2 * base3 - dF1 * base1));
+              gacc[256 * P.sC2] += (double)(T(0.5) * (-qj) * (dF2 * base3 - dF1 * base1));
             }
           }
           if (dmp_j && (Pj.sB >= 0 || Pj.sC2 >= 0)) {
@@ -730,20 +767,31 @@ __device__ void pair_pass(const FitArgs& a, const FitSnap& S, int ib0, int ib1, 
             const T base3 = T(3) * E.dm5 * rmj * dr, base1 = E.dm3 * edmj;
             if (Pj.sB >= 0) {
               const T dF1 = -fb2, dF2 = -fb2 + (d / T(3)) * fdb2;
-              gacc[Pj.sB] += (double)(T(0.5) * qi * (dF2 * base3 - dF1 * base1));
+              gacc[256 * Pj.sB] += (double)(T(0.5) * qi * (dF2 * base3 - dF1 * base1));
             }
             if (Pj.sC2 >= 0) {
               const T dF1 = -fc2, dF2 = -fc2 + (d / T(3)) * fdc2;
-              gacc[Pj.sC2] += (double)(T(0.5) * qi * (dF2 * base3 - dF1 * base1));
+              gacc[256 * Pj.sC2] += (double)(T(0.5) * qi * (dF2 * base3 - dF1 * base1));
             }
           }
         }
       }
     }
-    if (!ADJ) {
-      for (int c = 0; c < 3; ++c) Fout[3 * i + c] = fsr[c] + cu * fcl[c];
-    } else {
-      for (int c = 0; c < 3; ++c) h[3 * i + c] = hh[c];
+    // an atom's lanes share the loop bounds' block, so all of them are here
+    for (int w = 1; w < L; w <<= 1)
+      for (int c = 0; c < 3; ++c) {
+        if (!ADJ) {
+          fsr[c] += __shfl_xor(fsr[c], w);
+          fcl[c] += __shfl_xor(fcl[c], w);
+        } else {
+          hh[c] += __shfl_xor(hh[c], w);
+        }
+      }
+    if (sub == 0) {
+      for (int c = 0; c < 3; ++c) {
+        if (!ADJ) Fout[3 * i + c] = fsr[c] + cu * fcl[c];
+        else h[3 * i + c] = hh[c];
+      }
     }
   }
 }
@@ -771,9 +819,9 @@ __device__ __forceinline__ void block_partials(double* v, int n, double* red, do
 // static field of the charges (real space, damped) at the block's atoms
 template <typename T>
 __global__ void __launch_bounds__(256) kf_static(FitArgs a) {
-  const int4 B = a.ablk[blockIdx.x];
+  const int4 B = a.pblk[blockIdx.x];
   const FitSnap S = a.snaps[B.x];
-  field_static<T>(a, S, B.y, B.z, ws_of(a, S, W_ES), nullptr, nullptr);
+  field_static<T>(a, S, B.y, a.planes, ws_of(a, S, W_ES), nullptr, nullptr);
 }
 
 // dst = alpha src at the block's atoms, for snapshots still iterating
@@ -793,11 +841,290 @@ __global__ void __launch_bounds__(256) kf_update(FitArgs a) {
 // real-space dipole field of v = ws[slot] into ws[W_TMP] (iterating snapshots)
 template <typename T>
 __global__ void __launch_bounds__(256) kf_dipreal(FitArgs a, int slot) {
-  extern __shared__ double red[];
-  const int4 B = a.ablk[blockIdx.x];
+  const int4 B = a.dblk[xcd_order(blockIdx.x, gridDim.x)];
   if (!a.active[B.x]) return;
   const FitSnap S = a.snaps[B.x];
-  field_dip_real<T>(a, S, B.y, B.z, ws_of(a, S, slot), ws_of(a, S, W_TMP), red);
+  field_dip_real<T>(a, S, a.boxes[B.x], B.y, a.dlanes, ws_of(a, S, slot), ws_of(a, S, W_TMP));
+}
+
+// ---------------------------------------------------------------------------
+// Reciprocal field of the iterations on the FP64 matrix cores, in both forms.
+// A thread a k (or an atom) over phase products was 75 % of a gradient: 404
+// us for the structure factors and 369 us for the gathers of an iteration of
+// 256 snapshots (129,000 ions, 4.7e8 ion-k terms) in FP32.  With the k box as
+// (m = (nx, ny)) x nz both are products over the polarisable ions only, on
+// the same operands as the single-configuration sums (recip.hip):
+//   S(m, nz) = sum_i i 2pi (nx m_x + ny m_y) X Y Z + nz [i 2pi m_z X Y] Z
+//   U_d(i) = sum_m X Y sum_nz W(m, nz) Z, W = A conj(S)
+// (lane layouts: A(row = l%16, k = l/16), B(k = l/16, col = l%16), D row =
+// 4 r + l/16): 126 us, 11 for the reduction and 124 (32 snapshots, FP64: 166
+// and 100 to 36, 10 and 35).
+// ---------------------------------------------------------------------------
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f64x4 mfma(double a, double b, f64x4 c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+constexpr int kSkTile = 32;      // ions of a staged tile
+constexpr int kSkRows = 4;       // row tiles (8 nz) a block at most
+
+// RT row tiles from nz index zoff, 64 columns m (16 a wave), one chunk of
+// ions: B = (snapshot, first m, chunk, first nz index)
+template <int RT>
+__device__ __forceinline__ void sk_block(const FitArgs& a, const FitSnap& S, const FitBox& X, const int4& B,
+                                         const double* v, c2d* st, double* sq) {
+  constexpr int TA = kSkTile, TAP = TA + 2;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = lane >> 4, col = lane & 15;
+  const int kk = g & 1, ja = g >> 1;                             // K: ion 2s+ja, Re/Im kk
+  const int zcol = S.Kx + S.Ky + 2;
+  const bool take_im = (col & 1) ^ kk;
+  const double* stT = reinterpret_cast<const double*>(st);
+  const double* zp[RT];
+  double zs[RT], zn[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const int nzi = B.w + rt * 8 + (col >> 1);
+    const int part = col & 1;
+    const int nz = nzi - S.Kz;
+    const int zc = nzi < X.NZ ? zcol + (nz < 0 ? -nz : nz) : zcol;   // rows beyond NZ are not stored
+    const double sgn_im = nz < 0 ? -1.0 : 1.0;
+    zs[rt] = part == 0 ? (kk == 0 ? 1.0 : -sgn_im) : (kk == 0 ? sgn_im : 1.0);
+    zn[rt] = nz;
+    zp[rt] = stT + 2 * ((size_t)zc * TAP + ja) + (take_im ? 1 : 0);
+  }
+  const int m = B.y + wave * 16 + col;
+  const bool bok = m < X.M;
+  const int nx = bok ? m / X.NY : 0, ny = bok ? m % X.NY - S.Ky : 0;
+  const c2d* xp = st + (size_t)nx * TAP + ja;
+  const c2d* yp = st + (size_t)(S.Kx + 1 + (ny >= 0 ? ny : -ny)) * TAP + ja;
+  const double bysg = ny < 0 ? -1.0 : 1.0;
+  const double bnxf = nx, bnyf = ny;
+  const double* qp = sq + ja;
+  f64x4 acc[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) acc[rt] = f64x4{0.0, 0.0, 0.0, 0.0};
+  const c2d* tab = a.tab64 + S.tab0;
+  const int pend = min(X.np, (B.z + 1) * X.chunk);
+  const int sia = threadIdx.x & (TA - 1), scg = threadIdx.x / TA;
+  constexpr int CG = 256 / TA;
+  for (int t0 = B.z * X.chunk; t0 < pend; t0 += TA) {
+    const int nt = min(TA, pend - t0);
+    const bool sok = sia < nt;
+    const int src = a.pidx[X.p0 + t0 + min(sia, nt - 1)];
+    __syncthreads();
+    for (int c0 = scg; c0 < S.ncol; c0 += 8 * CG) {
+      c2d w[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) w[u] = tab[(size_t)min(c0 + u * CG, S.ncol - 1) * S.n + src];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (c0 + u * CG < S.ncol) st[(size_t)(c0 + u * CG) * TAP + sia] = sok ? w[u] : c2d{0.0, 0.0};
+    }
+    if (scg < 3) {                                               // 2 pi (B^T v), component scg
+      const double u0 = v[3 * src], u1 = v[3 * src + 1], u2 = v[3 * src + 2];
+      const double mv = 2.0 * MDFF_PI * (u0 * X.B[3 * scg] + u1 * X.B[3 * scg + 1] + u2 * X.B[3 * scg + 2]);
+      sq[scg * TAP + sia] = sok ? mv : 0.0;
+    }
+    __syncthreads();
+    const int ns = B.y + wave * 16 < X.M ? (nt + 7) >> 3 : 0;     // a wave of columns beyond M only stages
+    for (int q8 = 0; q8 < ns; ++q8) {
+      const int o = q8 * 8;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        double av[RT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) av[rt] = zs[rt] * zp[rt][2 * o + 4 * s];
+        const c2d Xc = xp[o + 2 * s];
+        const c2d Yc = yp[o + 2 * s];
+        const double yim = bysg * Yc.im;
+        const double xyr = Xc.re * Yc.re - Xc.im * yim;
+        const double xyi = Xc.re * yim + Xc.im * Yc.re;
+        const double ixy = kk == 0 ? -xyi : xyr;                 // i X Y
+        const double bb = bnxf * qp[o + 2 * s] + bnyf * qp[TAP + o + 2 * s];
+        const double bv = bb * ixy, bz = qp[2 * TAP + o + 2 * s] * ixy;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) acc[rt] = mfma(av[rt], bv, acc[rt]);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) acc[rt] = mfma(zn[rt] * av[rt], bz, acc[rt]);
+      }
+    }
+  }
+  if (!bok) return;
+  double* out = a.msp + 2 * (X.s0 + (long long)B.z * X.nb);
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int Rd = 4 * r + g;
+      const int nzi = B.w + rt * 8 + (Rd >> 1);
+      if (nzi < X.NZ) out[2 * ((size_t)m * X.NZ + nzi) + (Rd & 1)] = acc[rt][r];
+    }
+}
+
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) kf_sk(FitArgs a, int vslot) {
+  extern __shared__ double red[];
+  const int4 B = a.mblk[blockIdx.x];
+  if (!a.active[B.x]) return;
+  const FitSnap S = a.snaps[B.x];
+  const FitBox X = a.boxes[B.x];
+  c2d* st = reinterpret_cast<c2d*>(red);
+  double* sq = red + 2 * (size_t)S.ncol * (kSkTile + 2);
+  const double* v = ws_of(a, S, vslot);
+  switch (min(kSkRows, (X.NZ - B.w + 7) >> 3)) {
+    case 1: sk_block<1>(a, S, X, B, v, st, sq); break;
+    case 2: sk_block<2>(a, S, X, B, v, st, sq); break;
+    case 3: sk_block<3>(a, S, X, B, v, st, sq); break;
+    default: sk_block<4>(a, S, X, B, v, st, sq); break;
+  }
+}
+
+// S = sum of the chunks in order; W = A conj(S) on the box
+__global__ void __launch_bounds__(256) kf_skred(FitArgs a) {
+  const int4 B = a.rblk[blockIdx.x];
+  if (!a.active[B.x]) return;
+  const FitBox& X = a.boxes[B.x];
+  const int k = B.y + threadIdx.x;
+  if (k >= X.nb) return;
+  const double2* src = reinterpret_cast<const double2*>(a.msp) + X.s0 + k;
+  double re = 0.0, im = 0.0;
+  for (int c = 0; c < X.nch; ++c) {
+    const double2 t = src[(size_t)c * X.nb];
+    re += t.x;
+    im += t.y;
+  }
+  const double Ak = a.kbox[X.box0 + k];
+  const int m = k / X.NZ;
+  *reinterpret_cast<double2*>(a.wbox + X.w0 + (size_t)m * (4 * X.nks) + 2 * (k - m * X.NZ)) = double2{Ak * re, -Ak * im};
+}
+
+// moments U of 32 polarisable ions over a share of the m-tiles, a wave a block
+// (waves of one block sit on fixed SIMDs, which small snapshots would leave idle):
+// B = (snapshot, first ion, split).  Row (comp, m_local) of the A operand is
+// the Re or Im of W(m, nz), with a sign and, for U1, nz: formed from W here, so
+// a k costs 16 bytes and not 64.  A tile's operands (W, X, Y) are loaded a
+// tile ahead of their use.
+template <int NKS>
+__device__ __forceinline__ void moments_block(const FitArgs& a, const FitSnap& S, const FitBox& X, const int4& B) {
+  constexpr int CT = 2;
+  const int lane = threadIdx.x;
+  const int g = lane >> 4, col = lane & 15;
+  const int atom0 = B.y;
+  const c2d* tab = a.tab64 + S.tab0;
+  const int comp = col >> 2;
+  // this lane's factor at K step s: f0 + s f1
+  const double sg = ((comp & 1) == 0 && (g & 1)) ? -1.0 : 1.0;
+  const double f0 = comp < 2 ? sg : sg * ((g >> 1) - S.Kz), f1 = comp < 2 ? 0.0 : 2.0 * sg;
+  const double* wb = a.wbox + X.w0 + (col & 3) * (4 * NKS) + 2 * (g >> 1) + ((comp ^ g) & 1);
+  const int zcol = S.Kx + S.Ky + 2;
+  int iac[CT];
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) iac[ct] = a.pidx[X.p0 + min(atom0 + ct * 16 + col, X.np - 1)];
+  double breg[CT][NKS];
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+    for (int s = 0; s < NKS; ++s) {
+      const int k = 4 * s + g, t = k >> 1, nz = t - S.Kz;
+      const int az = min(nz < 0 ? -nz : nz, S.Kz);
+      const double z = reinterpret_cast<const double*>(tab + (size_t)(zcol + az) * S.n + iac[ct])[k & 1];
+      breg[ct][s] = t < X.NZ ? (((k & 1) && nz < 0) ? -z : z) : 0.0;
+    }
+  double u0[CT] = {}, u1[CT] = {}, u2[CT] = {};
+  const int mt0 = B.z * X.mtps, mt1 = min(X.mtiles, mt0 + X.mtps);
+  int m = 4 * mt0 + g;
+  int nx = min(m, X.M - 1) / X.NY;
+  int nyo = min(m, X.M - 1) - nx * X.NY;                          // ny + Ky
+  double abuf[NKS];
+  c2d xbuf[CT], ybuf[CT];
+  auto load = [&](int mt) {
+    const double* wp = wb + (size_t)mt * (16 * NKS);
+#pragma unroll
+    for (int s = 0; s < NKS; ++s) abuf[s] = wp[4 * s];
+    const int ny = nyo - S.Ky;
+    const size_t xrow = (size_t)min(nx, S.Kx) * S.n, yrow = (size_t)(S.Kx + 1 + (ny >= 0 ? ny : -ny)) * S.n;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      xbuf[ct] = tab[xrow + iac[ct]];
+      ybuf[ct] = tab[yrow + iac[ct]];
+    }
+  };
+  if (mt0 < mt1) load(mt0);
+  for (int mt = mt0; mt < mt1; ++mt) {
+    double cur[NKS], fs = f0;
+    asm volatile("" : "+v"(fs));      // the factors formed anew each tile: kept, they would spill
+#pragma unroll
+    for (int s = 0; s < NKS; ++s) cur[s] = (fs + s * f1) * abuf[s];
+    c2d Xv[CT], Yv[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      Xv[ct] = xbuf[ct];
+      Yv[ct] = ybuf[ct];
+    }
+    const double mw = m < X.M ? 1.0 : 0.0;
+    const double fx = nx, fy = nyo - S.Ky, ysg = nyo < S.Ky ? -1.0 : 1.0;
+    m += 4;
+    nyo += 4;
+    while (nyo >= X.NY) { nyo -= X.NY; ++nx; }                    // NY may be below 4
+    if (mt + 1 < mt1) load(mt + 1);
+    f64x4 acc[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) acc[ct] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < NKS; ++s)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) acc[ct] = mfma(cur[s], breg[ct][s], acc[ct]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      c2d Y = Yv[ct];
+      Y.im *= ysg;
+      const c2d XY = cm(Xv[ct], Y);
+      const double im0 = mw * (XY.re * acc[ct][1] + XY.im * acc[ct][0]);
+      const double im1 = mw * (XY.re * acc[ct][3] + XY.im * acc[ct][2]);
+      u0[ct] += fx * im0;
+      u1[ct] += fy * im0;
+      u2[ct] += im1;
+    }
+  }
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) {
+    u0[ct] += __shfl_xor(u0[ct], 16);
+    u1[ct] += __shfl_xor(u1[ct], 16);
+    u2[ct] += __shfl_xor(u2[ct], 16);
+    u0[ct] += __shfl_xor(u0[ct], 32);
+    u1[ct] += __shfl_xor(u1[ct], 32);
+    u2[ct] += __shfl_xor(u2[ct], 32);
+    const int p = atom0 + ct * 16 + col;
+    if (g == 0 && p < X.np) {
+      double* o = a.mgp + X.g0 + (size_t)B.z * 3 * X.np + p;
+      o[0] = u0[ct];
+      o[X.np] = u1[ct];
+      o[2 * (size_t)X.np] = u2[ct];
+    }
+  }
+}
+
+// LONG: Z rows of 18 to 25 K steps, in a launch of their own since they leave
+// a SIMD one wave
+template <bool LONG>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LONG ? 1 : 2))) kf_moments(FitArgs a, int b0) {
+  const int4 B = a.qblk[b0 + blockIdx.x];
+  if (!a.active[B.x]) return;
+  const FitSnap S = a.snaps[B.x];
+  const FitBox X = a.boxes[B.x];
+  if (LONG) moments_block<25>(a, S, X, B);
+  else switch (X.nks) {
+    case 4: moments_block<4>(a, S, X, B); break;
+    case 6: moments_block<6>(a, S, X, B); break;
+    case 8: moments_block<8>(a, S, X, B); break;
+    case 10: moments_block<10>(a, S, X, B); break;
+    case 12: moments_block<12>(a, S, X, B); break;
+    case 13: moments_block<13>(a, S, X, B); break;
+    case 15: moments_block<15>(a, S, X, B); break;
+    default: moments_block<17>(a, S, X, B); break;
+  }
 }
 
 // structure factors of the block's k-vectors and their per-k follow-ups.
@@ -973,7 +1300,17 @@ __global__ void __launch_bounds__(256) kf_gather(FitArgs a, int vslot, int bslot
       if (al == 0.0) {
         tmp[3 * j] = tmp[3 * j + 1] = tmp[3 * j + 2] = 0.0;
       } else {
-        gather_sum(a, B.x, S, j, 3, im3, re3, re6);
+        if (a.wbox) {
+          const FitBox& X = a.boxes[B.x];
+          const double* mo = a.mgp + X.g0 + a.pinv[S.a0 + j];
+          double u[3] = {0.0, 0.0, 0.0};
+          for (int sp = 0; sp < X.nsplit; ++sp)
+            for (int c = 0; c < 3; ++c) u[c] += mo[(size_t)(3 * sp + c) * X.np];
+          for (int c = 0; c < 3; ++c)
+            im3[c] = -2.0 * MDFF_PI * (X.B[c] * u[0] + X.B[3 + c] * u[1] + X.B[6 + c] * u[2]);
+        } else {
+          gather_sum(a, B.x, S, j, 3, im3, re3, re6);
+        }
         for (int c = 0; c < 3; ++c) tmp[3 * j + c] += pre * im3[c] + self * v[3 * j + c];
       }
       for (int c = 0; c < 3; ++c) {
@@ -1031,61 +1368,109 @@ __global__ void __launch_bounds__(256) kf_gather(FitArgs a, int vslot, int bslot
   if (PH != PH_STATIC) block_partials(&part, 1, red, a.pa + (size_t)FIT_PA * blockIdx.x + (PH == PH_FORCE ? 12 : 0));
 }
 
+// v of a wave's lanes summed
+__device__ __forceinline__ double wave_sum(double v) {
+  for (int w = 1; w < 64; w <<= 1) v += __shfl_xor(v, w);
+  return v;
+}
+
+// out[c] = sums over the block's 256 threads of n values each, get(c)
+template <typename F>
+__device__ __forceinline__ void pass_partials(int n, F get, double* out) {
+  __shared__ double part[4][FIT_MAXP];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int c = 0; c < n; ++c) {
+    const double r = wave_sum(get(c));
+    if (lane == 0) part[wave][c] = r;
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < n)
+    out[threadIdx.x] = part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x];
+}
+
 // pair pass at the block's atoms.  !ADJ: forces (ws-independent) and the
 // real-space stress partials (slots 0..11); ADJ: h (real space, overwritten)
-// and the explicit gradient partials (slots 0..FIT_MAXP-1)
+// and the explicit gradient partials (a slot a parameter).  Bound by the
+// latency of the rows' scattered loads: a thread an atom left a SIMD two waves
+// (256 snapshots, 129,000 ions, FP32: 930 us and, ADJ with its sums in private
+// memory, 1640); with 4 lanes an atom and the sums in LDS 366 and 504 (32
+// snapshots FP64, 16 lanes: 658 and 1097 to 130 and 134).
 template <typename T, bool ADJ>
 __global__ void __launch_bounds__(256) kf_pair(FitArgs a) {
   extern __shared__ double red[];
-  const int4 B = a.ablk[blockIdx.x];
+  const int4 B = a.pblk[blockIdx.x];
   const FitSnap S = a.snaps[B.x];
   double stn[6] = {0, 0, 0, 0, 0, 0}, std_[6] = {0, 0, 0, 0, 0, 0};
-  double* out = a.pa + (size_t)FIT_PA * blockIdx.x;
+  double* out = a.pp + (size_t)FIT_MAXP * blockIdx.x;
   if (!ADJ) {
     const double Gdummy[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    pair_pass<T, false>(a, S, B.y, B.z, ws_of(a, S, W_MU), nullptr, Gdummy, a.F + 3 * (size_t)S.a0, nullptr,
+    pair_pass<T, false>(a, S, B.y, a.planes, ws_of(a, S, W_MU), nullptr, Gdummy, a.F + 3 * (size_t)S.a0, nullptr,
                         nullptr, stn, std_);
     double v[12];
+#pragma unroll
     for (int c = 0; c < 6; ++c) {
       v[c] = stn[c];
       v[6 + c] = std_[c];
     }
-    block_partials(v, 12, red, out);
+    pass_partials(12, [&](int c) { double r = 0.0;
+#pragma unroll
+      for (int u = 0; u < 12; ++u) r = u == c ? v[u] : r;
+      return r; }, out);
   } else {
-    double gacc[FIT_MAXP];
-    for (int p = 0; p < FIT_MAXP; ++p) gacc[p] = 0.0;
+    double* gacc = red + threadIdx.x;
+    for (int p = 0; p < a.nparam; ++p) gacc[256 * p] = 0.0;
     double Gs[9];
     for (int c = 0; c < 9; ++c) Gs[c] = a.Gs[9 * (size_t)B.x + c];
     // the non-bonded stress carries 1/press_unit, the Coulomb one coul_unit/press_unit:
     // the pair pass scales its virtual displacement by 1/(omega pu) and the
     // Coulomb terms by coul_unit itself
-    pair_pass<T, true>(a, S, B.y, B.z, ws_of(a, S, W_MU), ws_of(a, S, W_G), Gs, nullptr, ws_of(a, S, W_H), gacc,
+    pair_pass<T, true>(a, S, B.y, a.planes, ws_of(a, S, W_MU), ws_of(a, S, W_G), Gs, nullptr, ws_of(a, S, W_H), gacc,
                        stn, std_);
-    block_partials(gacc, FIT_MAXP, red, out);
+    pass_partials(a.nparam, [&](int c) { return gacc[256 * c]; }, out);
   }
 }
 
 // - lambda . dR/dtheta at the block's atoms: alpha (lambda.mu / alpha^2) and
-// TT b, c (lambda . dE_s/dtheta); gradient partials (slots 0..FIT_MAXP-1)
+// TT b, c (lambda . dE_s/dtheta); gradient partials (a slot a parameter)
 template <typename T>
 __global__ void __launch_bounds__(256) kf_lambda(FitArgs a) {
   extern __shared__ double red[];
-  const int4 B = a.ablk[blockIdx.x];
+  const int4 B = a.pblk[blockIdx.x];
   const FitSnap S = a.snaps[B.x];
   const int* it = a.itype + S.a0;
   const double* vLAM = ws_of(a, S, W_LAM);
   const double* vMU = ws_of(a, S, W_MU);
-  double gacc[FIT_MAXP];
-  for (int p = 0; p < FIT_MAXP; ++p) gacc[p] = 0.0;
-  for (int j = B.y + threadIdx.x; j < B.z; j += blockDim.x) {
+  double* gacc = red + threadIdx.x;
+  for (int p = 0; p < a.nparam; ++p) gacc[256 * p] = 0.0;
+  const int j = B.y + (int)threadIdx.x / a.planes;
+  if (((int)threadIdx.x & (a.planes - 1)) == 0 && j < S.n) {
     const int tj = it[j];
     const double al = a.alpha_t[tj];
-    if (al == 0.0 || a.s_alpha[tj] < 0) continue;
-    const double lm = vLAM[3 * j] * vMU[3 * j] + vLAM[3 * j + 1] * vMU[3 * j + 1] + vLAM[3 * j + 2] * vMU[3 * j + 2];
-    gacc[a.s_alpha[tj]] += lm / (al * al);
+    if (al != 0.0 && a.s_alpha[tj] >= 0) {
+      const double lm = vLAM[3 * j] * vMU[3 * j] + vLAM[3 * j + 1] * vMU[3 * j + 1] + vLAM[3 * j + 2] * vMU[3 * j + 2];
+      gacc[256 * a.s_alpha[tj]] += lm / (al * al);
+    }
   }
-  field_static<T>(a, S, B.y, B.z, nullptr, vLAM, gacc);
-  block_partials(gacc, FIT_MAXP, red, a.pa + (size_t)FIT_PA * blockIdx.x);
+  field_static<T>(a, S, B.y, a.planes, nullptr, vLAM, gacc);
+  pass_partials(a.nparam, [&](int c) { return gacc[256 * c]; }, a.pp + (size_t)FIT_MAXP * blockIdx.x);
+}
+
+// the pair passes' partials of a snapshot added in block order, a thread a slot
+__global__ void __launch_bounds__(64) kf_psum(FitArgs a, int n) {
+  const int s = blockIdx.x, c = threadIdx.x;
+  if (c >= n) return;
+  const int b0 = a.snap_pb0[s], b1 = a.snap_pb0[s + 1];
+  double t = 0.0;
+  int b = b0;
+  for (; b + 8 <= b1; b += 8) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = a.pp[(size_t)FIT_MAXP * (b + u) + c];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) t += v[u];
+  }
+  for (; b < b1; ++b) t += a.pp[(size_t)FIT_MAXP * b + c];
+  a.ps[(size_t)FIT_MAXP * s + c] = t;
 }
 
 // Control of every snapshot (one block, thread-strided over snapshots; each
@@ -1098,10 +1483,11 @@ __global__ void __launch_bounds__(256) kf_lambda(FitArgs a) {
 //   C_HN:     RMS of h, adjoint iterations to 0, every snapshot iterating
 //   C_ADJ:    adjoint residual; continue while above tol_adj |h|
 //   C_GRAD:   gradient = pair-pass sums + lambda-pass sums; adjoint count out
-// count = snapshots still iterating after C_START / C_SCF / C_HN / C_ADJ.
+// h_count = snapshots still iterating after C_SCF / C_ADJ, with the sequence
+// number the host waits for.
 enum { C_START = 0, C_SCF = 1, C_FORCE = 2, C_PAIRG = 3, C_HN = 4, C_ADJ = 5, C_GRAD = 6 };
-__global__ void __launch_bounds__(64) kf_ctl(FitArgs a, int what) {
-  __shared__ int cnt[64];
+__global__ void __launch_bounds__(256) kf_ctl(FitArgs a, int what) {
+  __shared__ int cnt[256];
   int mine = 0;
   for (int s = threadIdx.x; s < a.nsnap; s += blockDim.x) {
     const FitSnap S = a.snaps[s];
@@ -1125,8 +1511,8 @@ __global__ void __launch_bounds__(64) kf_ctl(FitArgs a, int what) {
     } else if (what == C_FORCE) {
       double sn[6], sd[6], sr[6];
       for (int c = 0; c < 6; ++c) {
-        sn[c] = asum(c);
-        sd[c] = asum(6 + c);
+        sn[c] = a.ps[(size_t)FIT_MAXP * s + c];
+        sd[c] = a.ps[(size_t)FIT_MAXP * s + 6 + c];
         double t = 0.0;
         for (int b = a.snap_kb0[s]; b < a.snap_kb0[s + 1]; ++b) t += a.pk[(size_t)FIT_PK * b + c];
         sr[c] = t;
@@ -1158,9 +1544,10 @@ __global__ void __launch_bounds__(64) kf_ctl(FitArgs a, int what) {
       for (int c = 0; c < 9; ++c) a.tau[9 * s + c] = tau[c];
       a.nscf[2 * s] = a.iter[s];
     } else if (what == C_PAIRG) {
-      for (int p = 0; p < FIT_MAXP; ++p) a.gsave[(size_t)FIT_MAXP * s + p] = asum(p);
+      for (int p = 0; p < a.nparam; ++p) a.gsave[(size_t)FIT_MAXP * s + p] = a.ps[(size_t)FIT_MAXP * s + p];
     } else if (what == C_GRAD) {
-      for (int p = 0; p < FIT_MAXP; ++p) a.grad[(size_t)FIT_MAXP * s + p] = a.gsave[(size_t)FIT_MAXP * s + p] + asum(p);
+      for (int p = 0; p < a.nparam; ++p)
+        a.grad[(size_t)FIT_MAXP * s + p] = a.gsave[(size_t)FIT_MAXP * s + p] + a.ps[(size_t)FIT_MAXP * s + p];
       a.nscf[2 * s + 1] = a.iter[s];
     }
     mine += a.active[s];
@@ -1170,7 +1557,11 @@ __global__ void __launch_bounds__(64) kf_ctl(FitArgs a, int what) {
   if (threadIdx.x == 0) {
     int t = 0;
     for (int x = 0; x < (int)blockDim.x; ++x) t += cnt[x];
-    a.count[0] = t;
+    if (what == C_SCF || what == C_ADJ) {
+      a.h_count[0] = t;
+      __threadfence_system();
+      a.h_count[1] = a.seq;
+    }
   }
 }
 
@@ -1224,7 +1615,22 @@ struct mdff_fit {
   // block maps for the current block size
   int nab = 0, nkb = 0;
   int4 *d_ablk = nullptr, *d_kblk = nullptr;
-  int *d_ab0 = nullptr, *d_kb0 = nullptr, *d_active = nullptr, *d_iter = nullptr, *d_count = nullptr;
+  int *d_ab0 = nullptr, *d_kb0 = nullptr, *d_active = nullptr, *d_iter = nullptr;
+  // the iterations' matrix-core path and real-space rows
+  hipStream_t stream2 = nullptr;
+  hipEvent_t ev_v = nullptr, ev_real = nullptr;
+  FitBox* d_boxes = nullptr;
+  int *d_pidx = nullptr, *d_pinv = nullptr, *d_prow = nullptr, *d_pnl = nullptr;
+  double *d_kbox = nullptr, *d_msp = nullptr, *d_wbox = nullptr, *d_mgp = nullptr;
+  int4 *d_mblk = nullptr, *d_rblk = nullptr, *d_qblk = nullptr, *d_dblk = nullptr;
+  int nmb = 0, nrb = 0, ndb = 0, nqb = 0, nql = 0, dlanes = 4;
+  // pair passes
+  int npb = 0, planes = 1;
+  int4* d_pblk = nullptr;
+  int* d_pb0 = nullptr;
+  double *d_pp = nullptr, *d_ps = nullptr;
+  double *h_count = nullptr, *d_hcount = nullptr;
+  double seq = 0.0;
   int ngb = 0;
   int4* d_gblk = nullptr;
   int nsb = 0;
@@ -1258,6 +1664,14 @@ struct mdff_fit {
   do {                                 \
     const int _rc = (call);            \
     if (_rc != MDFF_OK) return _rc;    \
+  } while (0)
+
+// a host vector to a new device array
+#define FUP(dst, vec)                                                                                   \
+  do {                                                                                                  \
+    FIT_TRY(f, hipMalloc((void**)&(dst), sizeof((vec)[0]) * std::max<size_t>(1, (vec).size())));       \
+    if (!(vec).empty())                                                                                 \
+      FIT_TRY(f, hipMemcpy((dst), (vec).data(), sizeof((vec)[0]) * (vec).size(), hipMemcpyHostToDevice)); \
   } while (0)
 
 static void fit_lattice(const double* A, double* B, double* omega, double* W) {
@@ -1359,42 +1773,204 @@ static int fit_blocks(mdff_fit* f, int block) {
   return MDFF_OK;
 }
 
+// K steps compiled for kf_moments, and the LDS of kf_sk
+static const int kFitSteps[] = {4, 6, 8, 10, 12, 13, 15, 17, 25};
+static int fit_steps(int nz) {
+  for (int b : kFitSteps)
+    if (2 * nz <= 4 * b) return b;
+  return 0;
+}
+static size_t fit_sk_lds(int ncol) { return (size_t)(kSkTile + 2) * (16 * (size_t)ncol + 24); }
+
+// Polarisable rows, k boxes and block maps of the iterations.  Every snapshot
+// on the matrix cores where kES(3) <= 24 (the ions' Z rows are held in
+// registers) and the staged columns fit 64 KiB of LDS, else all on the
+// vector-ALU kernels.  Chunks and splits: enough blocks for a wave on every
+// SIMD, and no more, since each chunk's or split's sums are added up later.
+static int fit_iter_setup(mdff_fit* f, const std::vector<int>& it, const std::vector<int>& row,
+                          const std::vector<int>& nl, const std::vector<double>& kv) {
+  const int nsnap = f->nsnap;
+  std::vector<FitBox> bx(nsnap);
+  std::vector<int> pidx, pinv(f->natm, -1), prow, pnl;
+  std::vector<char> polar(f->ntype);
+  for (int t = 0; t < f->ntype; ++t) polar[t] = f->alpha0[t] != 0.0;
+  for (int p = 0; p < f->nparam; ++p)
+    if (f->spec[3 * p] == FP_ALPHA) polar[f->spec[3 * p + 1] - 1] = 1;
+  bool mma = fit_sk_lds(f->ncol_max) <= 65536;
+  long long box = 0, wel = 0, waves = 0, mcols = 0;
+  for (int s = 0; s < nsnap; ++s) {
+    const FitSnap& S = f->snaps[s];
+    FitBox& X = bx[s];
+    X = FitBox{};
+    double om, W[3];
+    fit_lattice(S.A, X.B, &om, W);
+    X.p0 = (int)pidx.size();
+    X.r0 = (long long)prow.size();
+    X.n0 = (long long)pnl.size();
+    prow.push_back(0);
+    for (int i = 0; i < S.n; ++i) {
+      if (!polar[it[S.a0 + i]]) continue;
+      pinv[S.a0 + i] = (int)pidx.size() - X.p0;
+      pidx.push_back(i);
+      for (int e = row[S.row0 + i]; e < row[S.row0 + i + 1]; ++e)
+        if (polar[it[S.a0 + nl[S.nl0 + e]]]) pnl.push_back(nl[S.nl0 + e]);
+      prow.push_back((int)((long long)pnl.size() - X.n0));
+    }
+    X.np = (int)pidx.size() - X.p0;
+    X.NY = 2 * S.Ky + 1;
+    X.NZ = 2 * S.Kz + 1;
+    X.M = (S.Kx + 1) * X.NY;
+    X.nb = X.M * X.NZ;
+    X.mtiles = (X.M + 3) / 4;
+    X.nks = fit_steps(X.NZ);
+    mma = mma && X.nks > 0;
+    X.box0 = box;
+    X.w0 = wel;
+    wel += (long long)X.mtiles * X.nks * 16;
+    box += X.nb;
+    waves += (X.np + 31) / 32;
+    mcols += (X.np > 0) * (long long)((X.M + 63) / 64) * ((X.NZ + 8 * kSkRows - 1) / (8 * kSkRows)) * ((X.np + 127) / 128);
+  }
+  const int chunk = mcols >= 1024 ? 128 : (mcols >= 512 ? 64 : 32);
+  const int split = (int)std::max<long long>(1, 6144 / std::max<long long>(waves, 1));
+  f->dlanes = waves >= 1024 ? 8 : 32;
+  // the gradient passes hold a sum a thread and parameter in LDS (64 KiB at 32)
+  for (const void* fn : {reinterpret_cast<const void*>(&kf_pair<float, true>), reinterpret_cast<const void*>(&kf_pair<double, true>),
+                         reinterpret_cast<const void*>(&kf_lambda<float>), reinterpret_cast<const void*>(&kf_lambda<double>)})
+    FIT_TRY(f, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(double) * 256 * FIT_MAXP));
+  // lanes an atom of the pair passes: eight waves a SIMD
+  while (f->planes < 32 && (long long)f->natm * f->planes < 8192 * 64) f->planes *= 2;
+  std::vector<int4> mb, rb, db, pb;
+  std::vector<int> pb0(1, 0);
+  std::vector<int4> qb, ql;
+  std::vector<double> kb(mma ? (size_t)box : 1, 0.0);
+  long long s0 = 0, g0 = 0;
+  for (int s = 0; s < nsnap; ++s) {
+    const FitSnap& S = f->snaps[s];
+    FitBox& X = bx[s];
+    for (int i = 0; i < S.n; i += 256 / f->planes) pb.push_back(make_int4(s, i, 0, 0));
+    pb0.push_back((int)pb.size());
+    for (int p = 0; p < X.np; p += 256 / f->dlanes) db.push_back(make_int4(s, p, 0, 0));
+    X.chunk = std::max(chunk, (((X.np + 63) / 64) + kSkTile - 1) / kSkTile * kSkTile);
+    X.nch = (X.np + X.chunk - 1) / X.chunk;
+    X.mtps = std::max(4, (X.mtiles + split - 1) / split);
+    X.nsplit = (X.mtiles + X.mtps - 1) / X.mtps;
+    X.s0 = s0;
+    X.g0 = g0;
+    s0 += (long long)X.nch * X.nb;
+    g0 += (long long)X.nsplit * 3 * X.np;
+    if (!mma || X.np == 0) continue;
+    for (int c = 0; c < X.nch; ++c)
+      for (int m = 0; m < X.M; m += 64)
+        for (int z = 0; z < X.NZ; z += 8 * kSkRows) mb.push_back(make_int4(s, m, c, z));
+    for (int k = 0; k < X.nb; k += 256) rb.push_back(make_int4(s, k, 0, 0));
+    for (int sp = 0; sp < X.nsplit; ++sp)
+      for (int p = 0; p < X.np; p += 32) (X.nks > 17 ? ql : qb).push_back(make_int4(s, p, sp, 0));
+    // A of the half space on the box: the k list runs over it in the same order
+    for (int k = 0; k < S.nk; ++k) kb[X.box0 + X.nb - S.nk + k] = kv[5 * ((size_t)S.k0 + k) + 3];
+  }
+  // the longest blocks first: the rest fill up behind them
+  auto mwork = [&](const int4& b) {
+    const FitBox& X = bx[b.x];
+    return std::min(kSkRows, (X.NZ - b.w + 7) / 8) * std::min(X.chunk, X.np - b.z * X.chunk);
+  };
+  auto qwork = [&](const int4& b) { return bx[b.x].mtps * bx[b.x].nks; };
+  std::stable_sort(mb.begin(), mb.end(), [&](const int4& x, const int4& y) { return mwork(x) > mwork(y); });
+  std::stable_sort(qb.begin(), qb.end(), [&](const int4& x, const int4& y) { return qwork(x) > qwork(y); });
+  f->nqb = (int)qb.size();
+  f->nql = (int)ql.size();
+  qb.insert(qb.end(), ql.begin(), ql.end());
+  f->nmb = (int)mb.size();
+  f->nrb = (int)rb.size();
+  f->ndb = (int)db.size();
+  f->npb = (int)pb.size();
+  FUP(f->d_pblk, pb);
+  FUP(f->d_pb0, pb0);
+  FIT_TRY(f, hipMalloc((void**)&f->d_pp, sizeof(double) * FIT_MAXP * pb.size()));
+  FIT_TRY(f, hipMalloc((void**)&f->d_ps, sizeof(double) * FIT_MAXP * (size_t)nsnap));
+  FUP(f->d_boxes, bx);
+  FUP(f->d_pidx, pidx);
+  FUP(f->d_pinv, pinv);
+  FUP(f->d_prow, prow);
+  FUP(f->d_pnl, pnl);
+  FUP(f->d_dblk, db);
+  FIT_TRY(f, hipStreamCreateWithFlags(&f->stream2, hipStreamNonBlocking));
+  FIT_TRY(f, hipEventCreateWithFlags(&f->ev_v, hipEventDisableTiming));
+  FIT_TRY(f, hipEventCreateWithFlags(&f->ev_real, hipEventDisableTiming));
+  FIT_TRY(f, hipHostMalloc((void**)&f->h_count, 2 * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent));
+  FIT_TRY(f, hipHostGetDevicePointer((void**)&f->d_hcount, f->h_count, 0));
+  f->h_count[0] = f->h_count[1] = 0.0;
+  if (!mma) return MDFF_OK;
+  FUP(f->d_kbox, kb);
+  FUP(f->d_mblk, mb);
+  FUP(f->d_rblk, rb);
+  FUP(f->d_qblk, qb);
+  FIT_TRY(f, hipMalloc((void**)&f->d_msp, sizeof(double) * 2 * (size_t)std::max<long long>(s0, 1)));
+  FIT_TRY(f, hipMalloc((void**)&f->d_mgp, sizeof(double) * (size_t)std::max<long long>(g0, 1)));
+  // the padding of W stays zero
+  FIT_TRY(f, hipMalloc((void**)&f->d_wbox, sizeof(double) * (size_t)std::max<long long>(wel, 1)));
+  FIT_TRY(f, hipMemset(f->d_wbox, 0, sizeof(double) * (size_t)std::max<long long>(wel, 1)));
+  return MDFF_OK;
+}
+
 // One forward (+ adjoint gradient) evaluation: the phase kernels in order;
 // the SCF and the adjoint solve repeat their iteration's launches while the
 // control kernel counts a snapshot still iterating (read back per iteration).
 template <typename T>
 static int fit_run(mdff_fit* f, FitArgs a, size_t tsz) {
   hipStream_t st = f->stream;
-  const dim3 ga(f->nab), gk(f->nkb), gg(f->ngb), gs(f->nsb), b(f->block);
-  const size_t red = sizeof(double) * f->block;
+  const dim3 ga(f->nab), gk(f->nkb), gg(f->ngb), gs(f->nsb), gp(f->npb), b(f->block);
+  const size_t red = sizeof(double) * f->block, shm_g = sizeof(double) * 256 * (size_t)f->nparam;
   const size_t shm_sf = red + tsz * FIT_CA * f->ncol_max + sizeof(double) * 7 * FIT_CA;
-  int cnt = 0;
-  auto active_count = [&]() -> int {
-    FIT_TRY(f, hipMemcpyAsync(&cnt, f->d_count, sizeof(int), hipMemcpyDeviceToHost, st));
-    FIT_TRY(f, hipStreamSynchronize(st));
+  // snapshots still iterating, once the control kernel has said so; a launch
+  // that never does is caught by the stream
+  auto active_count = [&](int* cnt) -> int {
+    volatile const double* h = f->h_count;
+    bool seen = false;
+    for (long k = 0; k < 20000000L && !seen; ++k) seen = h[1] == f->seq;
+    if (!seen) {
+      FIT_TRY(f, hipStreamSynchronize(st));
+      if (h[1] != f->seq) return fit_fail(f, MDFF_ERR_HIP, "fit iteration signal missing");
+    }
+    *cnt = (int)h[0];
     return MDFF_OK;
   };
   auto iterate = [&](int vslot, int bslot, int what) -> int {
     for (int it = 0; it < a.max_iter; ++it) {
       a.ws_dst = vslot;
       a.ws_src = W_ET;
+      a.seq = f->seq += 1.0;
       hipLaunchKernelGGL(kf_update, ga, b, 0, st, a);
-      hipLaunchKernelGGL((kf_dipreal<T>), dim3(f->nab, kDipLanes), b, 3 * red, st, a, vslot);
-      hipLaunchKernelGGL((kf_sfpart<T>), gs, b, shm_sf, st, a, 1, vslot, -1);
-      hipLaunchKernelGGL((kf_sf<T>), gk, b, red, st, a, 1);
-      hipLaunchKernelGGL((kf_gpart<T, PH_ITER>), gg, b, kGatherLds, st, a);
+      // the real-space field beside the reciprocal one (both read v only)
+      FIT_TRY(f, hipEventRecord(f->ev_v, st));
+      FIT_TRY(f, hipStreamWaitEvent(f->stream2, f->ev_v, 0));
+      if (f->ndb) hipLaunchKernelGGL((kf_dipreal<T>), dim3(f->ndb), dim3(256), 0, f->stream2, a, vslot);
+      FIT_TRY(f, hipEventRecord(f->ev_real, f->stream2));
+      if (a.wbox) {
+        if (f->nmb) {
+          hipLaunchKernelGGL(kf_sk, dim3(f->nmb), dim3(256), fit_sk_lds(f->ncol_max), st, a, vslot);
+          hipLaunchKernelGGL(kf_skred, dim3(f->nrb), dim3(256), 0, st, a);
+          if (f->nqb) hipLaunchKernelGGL(kf_moments<false>, dim3(f->nqb), dim3(64), 0, st, a, 0);
+          if (f->nql) hipLaunchKernelGGL(kf_moments<true>, dim3(f->nql), dim3(64), 0, st, a, f->nqb);
+        }
+      } else {
+        hipLaunchKernelGGL((kf_sfpart<T>), gs, b, shm_sf, st, a, 1, vslot, -1);
+        hipLaunchKernelGGL((kf_sf<T>), gk, b, red, st, a, 1);
+        hipLaunchKernelGGL((kf_gpart<T, PH_ITER>), gg, b, kGatherLds, st, a);
+      }
+      FIT_TRY(f, hipStreamWaitEvent(st, f->ev_real, 0));
       hipLaunchKernelGGL((kf_gather<T, PH_ITER>), ga, b, red, st, a, vslot, bslot);
-      hipLaunchKernelGGL(kf_ctl, dim3(1), dim3(64), 0, st, a, what);
+      hipLaunchKernelGGL(kf_ctl, dim3(1), dim3(256), 0, st, a, what);
       FIT_TRY(f, hipGetLastError());
-      const int rc = active_count();
-      if (rc != MDFF_OK) return rc;
+      int cnt = 0;
+      FIT_RC(active_count(&cnt));
       if (cnt == 0) break;
     }
     return MDFF_OK;
   };
   // static field, SCF
-  hipLaunchKernelGGL(kf_ctl, dim3(1), dim3(64), 0, st, a, (int)C_START);
-  hipLaunchKernelGGL((kf_static<T>), ga, b, 0, st, a);
+  hipLaunchKernelGGL(kf_ctl, dim3(1), dim3(256), 0, st, a, (int)C_START);
+  hipLaunchKernelGGL((kf_static<T>), gp, dim3(256), 0, st, a);
   hipLaunchKernelGGL((kf_sfpart<T>), gs, b, shm_sf, st, a, 0, -1, -1);
   hipLaunchKernelGGL((kf_sf<T>), gk, b, red, st, a, 0);
   hipLaunchKernelGGL((kf_gpart<T, PH_STATIC>), gg, b, kGatherLds, st, a);
@@ -1402,26 +1978,29 @@ static int fit_run(mdff_fit* f, FitArgs a, size_t tsz) {
   FIT_TRY(f, hipGetLastError());
   FIT_RC(iterate(W_MU, W_ES, C_SCF));
   // forces, stress, loss
-  hipLaunchKernelGGL((kf_pair<T, false>), ga, b, red, st, a);
+  hipLaunchKernelGGL((kf_pair<T, false>), gp, dim3(256), 0, st, a);
+  hipLaunchKernelGGL(kf_psum, dim3(a.nsnap), dim3(64), 0, st, a, 12);
   hipLaunchKernelGGL((kf_sfpart<T>), gs, b, shm_sf, st, a, 2, (int)W_MU, -1);
   hipLaunchKernelGGL((kf_sf<T>), gk, b, red, st, a, 2);
   hipLaunchKernelGGL((kf_gpart<T, PH_FORCE>), gg, b, kGatherLds, st, a);
   hipLaunchKernelGGL((kf_gather<T, PH_FORCE>), ga, b, red, st, a, -1, -1);
-  hipLaunchKernelGGL(kf_ctl, dim3(1), dim3(64), 0, st, a, (int)C_FORCE);
+  hipLaunchKernelGGL(kf_ctl, dim3(1), dim3(256), 0, st, a, (int)C_FORCE);
   FIT_TRY(f, hipGetLastError());
   if (!a.want_grad) return MDFF_OK;
   // explicit pair gradients and h; adjoint solve; lambda terms
-  hipLaunchKernelGGL((kf_pair<T, true>), ga, b, red, st, a);
-  hipLaunchKernelGGL(kf_ctl, dim3(1), dim3(64), 0, st, a, (int)C_PAIRG);
+  hipLaunchKernelGGL((kf_pair<T, true>), gp, dim3(256), shm_g, st, a);
+  hipLaunchKernelGGL(kf_psum, dim3(a.nsnap), dim3(64), 0, st, a, a.nparam);
+  hipLaunchKernelGGL(kf_ctl, dim3(1), dim3(256), 0, st, a, (int)C_PAIRG);
   hipLaunchKernelGGL((kf_sfpart<T>), gs, b, shm_sf, st, a, 3, (int)W_MU, (int)W_G);
   hipLaunchKernelGGL((kf_sf<T>), gk, b, red, st, a, 3);
   hipLaunchKernelGGL((kf_gpart<T, PH_H>), gg, b, kGatherLds, st, a);
   hipLaunchKernelGGL((kf_gather<T, PH_H>), ga, b, red, st, a, -1, -1);
-  hipLaunchKernelGGL(kf_ctl, dim3(1), dim3(64), 0, st, a, (int)C_HN);
+  hipLaunchKernelGGL(kf_ctl, dim3(1), dim3(256), 0, st, a, (int)C_HN);
   FIT_TRY(f, hipGetLastError());
   FIT_RC(iterate(W_LAM, W_H, C_ADJ));
-  hipLaunchKernelGGL((kf_lambda<T>), ga, b, red, st, a);
-  hipLaunchKernelGGL(kf_ctl, dim3(1), dim3(64), 0, st, a, (int)C_GRAD);
+  hipLaunchKernelGGL((kf_lambda<T>), gp, dim3(256), shm_g, st, a);
+  hipLaunchKernelGGL(kf_psum, dim3(a.nsnap), dim3(64), 0, st, a, a.nparam);
+  hipLaunchKernelGGL(kf_ctl, dim3(1), dim3(256), 0, st, a, (int)C_GRAD);
   FIT_TRY(f, hipGetLastError());
   return MDFF_OK;
 }
@@ -1587,12 +2166,6 @@ int mdff_fit_create(const mdff_desc* d, int32_t nsnap, const int32_t* natm, cons
   f->nk = k0;
   f->tab_elems = tab0;
   FIT_TRY(f, hipStreamCreateWithFlags(&f->stream, hipStreamNonBlocking));
-#define FUP(dst, vec)                                                                                   \
-  do {                                                                                                  \
-    FIT_TRY(f, hipMalloc((void**)&(dst), sizeof((vec)[0]) * std::max<size_t>(1, (vec).size())));       \
-    if (!(vec).empty())                                                                                 \
-      FIT_TRY(f, hipMemcpy((dst), (vec).data(), sizeof((vec)[0]) * (vec).size(), hipMemcpyHostToDevice)); \
-  } while (0)
   FUP(f->d_snaps, f->snaps);
   FUP(f->d_itype, itv);
   FUP(f->d_q, q);
@@ -1603,7 +2176,6 @@ int mdff_fit_create(const mdff_desc* d, int32_t nsnap, const int32_t* natm, cons
   FUP(f->d_nl, nl);
   FUP(f->d_kv, kv);
   FUP(f->d_kn, kn);
-#undef FUP
   FIT_TRY(f, hipMalloc((void**)&f->d_pairs, sizeof(FitPair) * nt * nt));
   FIT_TRY(f, hipMalloc(&f->d_tab32, sizeof(c2<float>) * (size_t)tab0));
   FIT_TRY(f, hipMalloc(&f->d_tab64, sizeof(c2<double>) * (size_t)tab0));
@@ -1620,10 +2192,10 @@ int mdff_fit_create(const mdff_desc* d, int32_t nsnap, const int32_t* natm, cons
   FIT_TRY(f, hipMalloc((void**)&f->d_nscf, sizeof(int) * 2 * (size_t)nsnap));
   FIT_TRY(f, hipMalloc((void**)&f->d_active, sizeof(int) * (size_t)nsnap));
   FIT_TRY(f, hipMalloc((void**)&f->d_iter, sizeof(int) * (size_t)nsnap));
-  FIT_TRY(f, hipMalloc((void**)&f->d_count, sizeof(int)));
   FIT_TRY(f, hipMalloc((void**)&f->d_hn, sizeof(double) * (size_t)nsnap));
   FIT_TRY(f, hipMalloc((void**)&f->d_Gs, sizeof(double) * 9 * (size_t)nsnap));
   FIT_TRY(f, hipMalloc((void**)&f->d_gsave, sizeof(double) * FIT_MAXP * (size_t)nsnap));
+  FIT_RC(fit_iter_setup(f, itv, row, nl, kv));
   const int tg = std::min(nsnap, 1024);
   hipLaunchKernelGGL((k_fit_tables<float>), dim3(tg), dim3(256), 0, f->stream, nsnap, f->d_snaps, f->d_sx,
                      f->d_sy, f->d_sz, f->d_tab32);
@@ -1704,7 +2276,6 @@ int mdff_fit_eval(mdff_fit* f, const double* theta, int32_t precision, int32_t w
   a.hn = f->d_hn;
   a.Gs = f->d_Gs;
   a.gsave = f->d_gsave;
-  a.count = f->d_count;
   a.gblk = f->d_gblk;
   a.snap_g0 = f->d_g0;
   a.snap_nch = f->d_nch;
@@ -1713,6 +2284,28 @@ int mdff_fit_eval(mdff_fit* f, const double* theta, int32_t precision, int32_t w
   a.snap_s0 = f->d_s0;
   a.snap_sch = f->d_sch;
   a.sp = f->d_sp;
+  a.boxes = f->d_boxes;
+  a.pidx = f->d_pidx;
+  a.pinv = f->d_pinv;
+  a.kbox = f->d_kbox;
+  a.mblk = f->d_mblk;
+  a.rblk = f->d_rblk;
+  a.qblk = f->d_qblk;
+  a.dblk = f->d_dblk;
+  a.tab64 = reinterpret_cast<const c2d*>(f->d_tab64);
+  a.msp = f->d_msp;
+  a.wbox = f->d_wbox;
+  a.mgp = f->d_mgp;
+  a.prow = f->d_prow;
+  a.pnl = f->d_pnl;
+  a.dlanes = f->dlanes;
+  a.pblk = f->d_pblk;
+  a.snap_pb0 = f->d_pb0;
+  a.pp = f->d_pp;
+  a.ps = f->d_ps;
+  a.planes = f->planes;
+  a.nparam = f->nparam;
+  a.h_count = f->d_hcount;
   a.pairs = f->d_pairs;
   for (int t = 0; t < FIT_NT; ++t) a.alpha_t[t] = alpha_t[t];
   a.itype = f->d_itype;
@@ -1772,12 +2365,22 @@ int mdff_fit_eval(mdff_fit* f, const double* theta, int32_t precision, int32_t w
 int mdff_fit_destroy(mdff_fit* f) {
   if (!f) return MDFF_ERR_BAD_ARG;
   if (f->stream) (void)hipStreamSynchronize(f->stream);
+  if (f->stream2) (void)hipStreamSynchronize(f->stream2);
   void* ptrs[] = {f->d_snaps, f->d_sblk, f->d_s0, f->d_sch, f->d_sp, f->d_gblk, f->d_g0, f->d_nch, f->d_gp, f->d_ablk, f->d_kblk, f->d_ab0, f->d_kb0, f->d_pa, f->d_pk, f->d_active, f->d_iter,
-                  f->d_count, f->d_hn, f->d_Gs, f->d_gsave, f->d_pairs, f->d_itype, f->d_row, f->d_nl, f->d_kn, f->d_nscf,
+                  f->d_hn, f->d_Gs, f->d_gsave, f->d_pairs, f->d_itype, f->d_row, f->d_nl, f->d_kn, f->d_nscf,
                   f->d_q, f->d_sx, f->d_sy, f->d_sz, f->d_kv, f->d_tab32, f->d_tab64, f->d_fref,
                   f->d_tauref, f->d_ws, f->d_kws, f->d_F, f->d_tau, f->d_loss, f->d_grad};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
+  for (void* p : {(void*)f->d_boxes, (void*)f->d_pidx, (void*)f->d_pinv, (void*)f->d_prow, (void*)f->d_pnl,
+                  (void*)f->d_kbox, (void*)f->d_msp, (void*)f->d_wbox, (void*)f->d_mgp, (void*)f->d_mblk,
+                  (void*)f->d_rblk, (void*)f->d_qblk, (void*)f->d_dblk, (void*)f->d_pblk, (void*)f->d_pb0,
+                  (void*)f->d_pp, (void*)f->d_ps})
+    if (p) (void)hipFree(p);
+  if (f->h_count) (void)hipHostFree(f->h_count);
+  if (f->ev_v) (void)hipEventDestroy(f->ev_v);
+  if (f->ev_real) (void)hipEventDestroy(f->ev_real);
+  if (f->stream2) (void)hipStreamDestroy(f->stream2);
   if (f->stream) (void)hipStreamDestroy(f->stream);
   delete f;
   return MDFF_OK;

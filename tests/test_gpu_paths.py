@@ -8,6 +8,7 @@ import pytest
 
 from gpu_util import note, pair, rel, rel_force_err
 from mdff_amd import capi, configs
+from mdff_amd import fit as F
 
 pytestmark = pytest.mark.gpu
 
@@ -103,3 +104,45 @@ def test_too_long_k_mesh_refused(prec, k, dip, mesh, monkeypatch):
     g, _ = pair(s, precision=prec)
     with pytest.raises(RuntimeError, match="too large"):
         g.engforce()
+
+
+def _fit_problem(kz, params, nsnap=3):
+    snaps = configs.fit_snapshots(nsnap, nmin=64, nmax=260, seed=17)
+    for n, s in enumerate(snaps):
+        s.desc.kES[:] = [3 + n, 4, kz[n % len(kz)]]
+    return snaps, F.FitProblem(snaps, params, scf_tol=1e-12, max_iter=400)
+
+
+@pytest.mark.parametrize("kz", [(1, 4, 5), (7, 8, 9), (10, 11, 12), (13, 14, 15), (16, 17, 24), (24, 25, 3)],
+                         ids=lambda k: "-".join(map(str, k)))
+def test_fit_iterations(kz):
+    """Dipole iterations over every size of the matrix-core kernels, and the
+    vector-ALU ones where a kES(3) is above 24: forces and stress of the single
+    configurations (converged to 1e-12; bar of the fit's forward parity)."""
+    params = [("A", 1, 2), ("ALPHA", 2, 0)]
+    snaps, p = _fit_problem(kz, params)
+    note(f"fit kz {kz}")
+    f, t = F.plain_targets(snaps, scf_tol=1e-12, max_iter=400)
+    p.set_targets(f, t, 1.0)
+    r = p.eval(F.theta_of(params, configs.FIT_THETA_STAR), capi.PREC_FP64, grad=False, outputs=True)
+    assert rel(r.forces, f) < 1e-9
+    assert rel(r.stress, t) < 1e-9
+    p.close()
+
+
+def test_fit_most_parameters():
+    """32 parameters, the last of each kind and pair in force: its gradient
+    is that of the short list, and the others' is zero."""
+    short = [("A", 1, 2), ("RHO", 1, 2), ("A", 2, 2), ("RHO", 2, 2), ("C", 2, 2), ("ALPHA", 2, 0), ("TTB", 2, 1),
+             ("TTC", 2, 1)]
+    g = []
+    for params in (short, short * 4):
+        snaps, p = _fit_problem((7, 9, 8), params)
+        n = sum(s.natm for s in snaps)
+        rng = np.random.default_rng(2)
+        p.set_targets(rng.normal(size=(n, 3)), rng.normal(size=(len(snaps), 9)), 0.1)
+        note(f"fit {len(params)} parameters")
+        g.append(np.asarray(p.eval(F.theta_of(params, configs.FIT_THETA_STAR) * 1.02, capi.PREC_FP64, grad=True).grad))
+        p.close()
+    assert rel(g[1][24:], g[0]) < 1e-12
+    assert not np.any(g[1][:24])
