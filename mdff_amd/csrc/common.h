@@ -100,6 +100,7 @@ constexpr int RAW_ENVT = 30;     // extended-system energy of a Nose-Hoover chai
 constexpr int RAW_SCRATCH = 32;  // 7 moments of the SCF field (slot 0 only)
 constexpr int RAW_LJ = 40;       // 8 sums of the LJ pass beside BMHFT(D): u, vir, stress (6)
 constexpr int RAW_N = 48;
+constexpr size_t kIoMax = 32768;  // doubles handed to or from the host through mapped memory (beyond, copies)
 constexpr int RAW_SLOTS = 1024;  // evaluations held before the sums go to the host
 
 // A deferred fixed-order final sum: out[0..ncol) = sums over nb block
@@ -268,9 +269,8 @@ struct mdff_ctx {
   double *cx = nullptr, *cy = nullptr, *cz = nullptr;   // fractional coordinates of a pending list check
   double* h_chk = nullptr;                // mapped pinned host memory: block maxima of the pending check
   double* d_chk = nullptr;                // the device address of h_chk
-  hipEvent_t chk_ev = nullptr;            // the pending check's maxima are in h_chk
   int chk_pending = 0;
-  // instead of the event, the next final-sum launch writes chk_seq into
+  // the next final-sum launch writes chk_seq into
   // h_chk[2 nb] once the check kernel has completed (1: to be attached to
   // that launch, 2: attached); the host waits for the value
   int chk_seq_wait = 0;
@@ -280,6 +280,10 @@ struct mdff_ctx {
   double* h_scf = nullptr;                // mapped pinned host memory: those sums and their sequence number
   double* d_scf = nullptr;                // its device address
   double scf_seq = 0.0;
+  double* h_io = nullptr;                 // mapped pinned host memory: sequence word, kIoMax results, kIoMax inputs
+  double* d_io = nullptr;                 // its device address
+  double io_seq = 0.0;
+  int io_in_busy = 0;                     // the inputs may still be read
   double* fin_part = nullptr;             // block partials of the pair sums [0, 1024*16) and kinetic energy
   double* nhc_part = nullptr;             // Nose-Hoover chain steps: two sets of kinetic block partials
   double* nhc_st = nullptr;               // Nose-Hoover chain state (xi, vxi, Q, scale)

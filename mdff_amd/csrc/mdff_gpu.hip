@@ -4,6 +4,8 @@
 // setup chain that feeds it (src/read_pos.f90:160-234,
 // src/non_bonded.f90:455-644, src/coulomb.f90:363-493, src/pim.f90:147-240).
 #include <algorithm>
+#include <atomic>
+#include <initializer_list>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -416,14 +418,6 @@ __global__ void k_kick(int n, double dt2, const double* __restrict__ m, double* 
   vz[i] = vz[i] + fz[i] * dt2 / m[i];
 }
 
-__global__ void k_scale_v(int n, double s, double sx, double sy, double sz, double* vx, double* vy, double* vz) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  vx[i] = vx[i] * s - sx;
-  vy[i] = vy[i] * s - sy;
-  vz[i] = vz[i] * s - sz;
-}
-
 // kinetic energy column and velocity sums
 __global__ void k_kin(int n, const double* __restrict__ m, const double* vx, const double* vy, const double* vz,
                       double* __restrict__ out) {
@@ -436,6 +430,99 @@ __global__ void k_kin(int n, const double* __restrict__ m, const double* vx, con
 }
 
 inline int nblk(int n) { return div_up(n, 256); }
+
+// Small results to the host: up to four arrays into mapped host memory by one
+// block, then the sequence number that the host waits for.  A copy and a stream
+// synchronisation take 8 to 10 us each whatever the size: a 64-ion frame
+// (positions in, list check, forces out) took 172 us with nine of them, now 106.
+// Up to kIoMax doubles: 3 x 2,048 out 55 and 25 us, 3 x 8,788 59 and 51, level
+// at about 3 x 14,000.
+struct HandArgs {
+  const double* src[4];
+  int cnt[4];
+  double* out;                   // the arrays one after the other
+  double* word;
+  double seq;
+};
+__global__ void __launch_bounds__(1024) k_hand_over(HandArgs a) {
+  double* o = a.out;
+  for (int k = 0; k < 4; ++k) {
+    for (int i = threadIdx.x; i < a.cnt[k]; i += 1024) o[i] = a.src[k][i];
+    o += a.cnt[k];
+  }
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) *reinterpret_cast<volatile double*>(a.word) = a.seq;
+}
+
+// three arrays from mapped host memory
+__global__ void __launch_bounds__(256) k_hand_in(int n, const double* __restrict__ in, double* __restrict__ x,
+                                                 double* __restrict__ y, double* __restrict__ z) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  x[i] = in[i];
+  y[i] = in[(size_t)n + i];
+  z[i] = in[(size_t)2 * n + i];
+}
+
+// Velocity rescale (rescale_velocities, src/kinetic.f90:122-198) in three
+// launches without a host round trip: block partials of sum m v^2; every block
+// adds them up, scales its atoms and leaves its velocity sums; every block adds
+// those and takes the mean off.
+struct RescaleArgs {
+  int n, nb, ndeg, csvr;         // csvr 0: the factor lambda
+  double lambda;
+  double sigma, factor, r1, sumnoise;
+  const double* m;
+  double *vx, *vy, *vz;
+  double *pk, *pv;               // partials: kinetic [nb], velocities [nb][3]
+  double* out;                   // kinetic energy before and after (csvr)
+};
+__global__ void __launch_bounds__(256) k_rescale_kin(RescaleArgs a) {
+  __shared__ double sh[4 * kRedMaxCols];
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  double v[kRedMaxCols] = {};
+  if (i < a.n) v[0] = (a.vx[i] * a.vx[i] + a.vy[i] * a.vy[i] + a.vz[i] * a.vz[i]) * a.m[i];
+  const double r = block_sum_cols(v, 1, sh);
+  if (threadIdx.x == 0) a.pk[blockIdx.x] = r;
+}
+__global__ void __launch_bounds__(256) k_rescale_v(RescaleArgs a) {
+  __shared__ double sh[4 * kRedMaxCols];
+  __shared__ double tot;
+  double s = a.lambda;
+  if (a.csvr) {
+    sum_block_partials(a.nb, 1, a.pk, &tot, sh);
+    __syncthreads();
+    const double ekin = tot * 0.5;
+    const double knew = ekin + (1.0 - a.factor) * (a.sigma * (a.sumnoise + a.r1 * a.r1) / a.ndeg - ekin) +
+                        2.0 * a.r1 * sqrt(ekin * a.sigma / a.ndeg * (1.0 - a.factor) * a.factor);
+    s = sqrt(knew / ekin);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      a.out[0] = ekin;
+      a.out[1] = knew;
+    }
+  }
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  double v[kRedMaxCols] = {};
+  if (i < a.n) {
+    a.vx[i] = v[0] = a.vx[i] * s;
+    a.vy[i] = v[1] = a.vy[i] * s;
+    a.vz[i] = v[2] = a.vz[i] * s;
+  }
+  const double r = block_sum_cols(v, 3, sh);
+  if (threadIdx.x < 3) a.pv[3 * (size_t)blockIdx.x + threadIdx.x] = r;
+}
+__global__ void __launch_bounds__(256) k_rescale_mean(RescaleArgs a) {
+  __shared__ double sh[4 * kRedMaxCols];
+  __shared__ double tot[3];
+  sum_block_partials(a.nb, 3, a.pv, tot, sh);
+  __syncthreads();
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= a.n) return;
+  a.vx[i] -= tot[0] / a.n;
+  a.vy[i] -= tot[1] / a.n;
+  a.vz[i] -= tot[2] / a.n;
+}
 
 // ---- Nose-Hoover chain steps on the device (nose_hoover_chain_n,
 // src/integration.f90:538-701).  The chain state lives in device memory
@@ -576,12 +663,48 @@ static int fail(mdff_ctx* c, int code, const char* msg) {
   return code;
 }
 
+// Arrays to host memory the caller reads at the returned address until its
+// next hand-over; null where they are more than fits (kIoMax doubles).
+struct HandSeg {
+  const double* src;
+  size_t cnt;
+};
+static int hand_over(mdff_ctx* c, std::initializer_list<HandSeg> segs, const double** out) {
+  *out = nullptr;
+  HandArgs a{};
+  size_t tot = 0;
+  int k = 0;
+  for (const HandSeg& g : segs) {
+    tot += g.cnt;
+    if (tot > kIoMax) return MDFF_OK;
+    a.src[k] = g.src;
+    a.cnt[k++] = (int)g.cnt;
+  }
+  a.out = c->d_io + 8;
+  a.word = c->d_io;
+  a.seq = c->io_seq += 1.0;
+  hipLaunchKernelGGL(k_hand_over, dim3(1), dim3(1024), 0, c->stream, a);
+  HIP_TRY(c, hipGetLastError());
+  // spin on the mapped word; a launch that never posts is caught by the stream
+  volatile const double* word = c->h_io;
+  bool seen = false;
+  for (long t = 0; t < 20000000L && !seen; ++t) seen = *word == a.seq;
+  if (!seen) {
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    if (*word != a.seq) return fail(c, MDFF_ERR_HIP, "hand-over signal missing");
+  }
+  std::atomic_thread_fence(std::memory_order_acquire);
+  c->io_in_busy = 0;             // whatever the stream held before is done
+  *out = c->h_io + 8;
+  return MDFF_OK;
+}
+
 // deterministic column sums of a [ncol][n] device array; result on the host
 int reduce_cols(mdff_ctx* c, const double* in, int ncol, double* host_out) {
   MDFF_TRY(reduce_cols_dev(c, in, ncol, c->red));
-  HIP_TRY(c, hipMemcpyAsync(c->h_red, c->red, sizeof(double) * ncol, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  for (int k = 0; k < ncol; ++k) host_out[k] = c->h_red[k];
+  const double* h = nullptr;
+  MDFF_TRY(hand_over(c, {{c->red, (size_t)ncol}}, &h));
+  for (int k = 0; k < ncol; ++k) host_out[k] = h[k];
   return MDFF_OK;
 }
 
@@ -832,7 +955,6 @@ static int ctx_init(mdff_ctx* c, const mdff_desc* d, const int32_t* itype) {
                            hipHostMallocMapped | hipHostMallocCoherent));
   HIP_TRY(c, hipHostGetDevicePointer((void**)&c->d_chk, c->h_chk, 0));
   memset(c->h_chk, 0, sizeof(double) * (2 * (size_t)nblk(n) + 2));
-  HIP_TRY(c, hipEventCreateWithFlags(&c->chk_ev, hipEventDisableTiming));
   HIP_TRY(c, hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking));
   HIP_TRY(c, hipEventCreateWithFlags(&c->ov_tab, hipEventDisableTiming));
   HIP_TRY(c, hipEventCreateWithFlags(&c->ov_pair, hipEventDisableTiming));
@@ -846,6 +968,10 @@ static int ctx_init(mdff_ctx* c, const mdff_desc* d, const int32_t* itype) {
   HIP_TRY(c, hipHostMalloc((void**)&c->h_red, sizeof(double) * nred));
   DMALLOC(c->red_part, nred);
   DMALLOC(c->scf_part, 2 * (size_t)nblk(n));
+  // mapped hand-over memory: the sequence word, results, and incoming arrays
+  HIP_TRY(c, hipHostMalloc((void**)&c->h_io, sizeof(double) * (8 + 2 * kIoMax), hipHostMallocMapped | hipHostMallocCoherent));
+  HIP_TRY(c, hipHostGetDevicePointer((void**)&c->d_io, c->h_io, 0));
+  c->h_io[0] = 0.0;
   HIP_TRY(c, hipHostMalloc((void**)&c->h_scf, sizeof(double) * 4, hipHostMallocMapped | hipHostMallocCoherent));
   HIP_TRY(c, hipHostGetDevicePointer((void**)&c->d_scf, c->h_scf, 0));
   memset(c->h_scf, 0, sizeof(double) * 4);
@@ -1426,18 +1552,56 @@ static void engforce_finish(const mdff_ctx* c, const double* raw, mdff_terms* t)
   }
 }
 
-// sums of one or more evaluations to the host: raw slots [0, nslots)
-static int fetch_raw(mdff_ctx* c, int nslots) {
+// sums of one or more evaluations on the host: raw slots [0, nslots)
+static int copy_raw(mdff_ctx* c, int nslots, const double** h) {
   HIP_TRY(c, hipMemcpyAsync(c->h_raw, c->raw, sizeof(double) * RAW_N * nslots, hipMemcpyDeviceToHost,
                             c->stream));
+  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  *h = c->h_raw;
+  return MDFF_OK;
+}
+static int fetch_raw(mdff_ctx* c, int nslots, const double** h) {
+  MDFF_TRY(hand_over(c, {{c->raw, (size_t)RAW_N * nslots}}, h));
+  return *h ? MDFF_OK : copy_raw(c, nslots, h);
+}
+
+static int copy3_out(mdff_ctx* c, const double* dx, const double* dy, const double* dz, double* x, double* y,
+                     double* z) {
+  if (!c || !x || !y || !z) return MDFF_ERR_BAD_ARG;
+  const size_t n = c->n, b = sizeof(double) * n;
+  const double* h = nullptr;
+  MDFF_TRY(hand_over(c, {{dx, n}, {dy, n}, {dz, n}}, &h));
+  if (h) {
+    memcpy(x, h, b);
+    memcpy(y, h + n, b);
+    memcpy(z, h + 2 * n, b);
+    return MDFF_OK;
+  }
+  HIP_TRY(c, hipMemcpyAsync(x, dx, b, hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(c, hipMemcpyAsync(y, dy, b, hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(c, hipMemcpyAsync(z, dz, b, hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   return MDFF_OK;
 }
 
-static int engforce(mdff_ctx* c, mdff_terms* t) {
+// f: 3 host arrays for the forces, or null
+static int engforce(mdff_ctx* c, mdff_terms* t, double* const* f) {
   MDFF_TRY(engforce_launch(c, c->raw, t, false));
-  MDFF_TRY(fetch_raw(c, 1));
-  engforce_finish(c, c->h_raw, t);
+  const size_t n = c->n, b = sizeof(double) * n;
+  const double* h = nullptr;
+  if (!f) {
+    MDFF_TRY(fetch_raw(c, 1, &h));
+  } else {
+    MDFF_TRY(hand_over(c, {{c->raw, RAW_N}, {c->fx, n}, {c->fy, n}, {c->fz, n}}, &h));
+    if (h) {
+      for (int k = 0; k < 3; ++k) memcpy(f[k], h + RAW_N + k * n, b);
+    } else {
+      // (copies start faster on a stream that has been waited for)
+      MDFF_TRY(copy_raw(c, 1, &h));
+      MDFF_TRY(copy3_out(c, c->fx, c->fy, c->fz, f[0], f[1], f[2]));
+    }
+  }
+  engforce_finish(c, h, t);
   c->last_terms = *t;
   return MDFF_OK;
 }
@@ -1537,7 +1701,7 @@ int mdff_ctx_destroy(mdff_ctx* c) {
   if (c->h_raw) (void)hipHostFree(c->h_raw);
   if (c->h_chk) (void)hipHostFree(c->h_chk);
   if (c->h_scf) (void)hipHostFree(c->h_scf);
-  if (c->chk_ev) (void)hipEventDestroy(c->chk_ev);
+  if (c->h_io) (void)hipHostFree(c->h_io);
   if (c->ov_tab) (void)hipEventDestroy(c->ov_tab);
   if (c->ov_pair) (void)hipEventDestroy(c->ov_pair);
   if (c->stream2) (void)hipStreamDestroy(c->stream2);
@@ -1554,21 +1718,23 @@ int mdff_ctx_destroy(mdff_ctx* c) {
 static int copy3_in(mdff_ctx* c, double* dx, double* dy, double* dz, const double* x, const double* y,
                     const double* z) {
   if (!c || !x || !y || !z) return MDFF_ERR_BAD_ARG;
-  const size_t b = sizeof(double) * c->n;
+  const size_t n = c->n, b = sizeof(double) * n;
+  if (3 * n <= kIoMax) {
+    // staged in mapped memory and read from there; the staging is free again
+    // once a later hand-over has come back
+    if (c->io_in_busy) HIP_TRY(c, hipStreamSynchronize(c->stream));
+    double* in = c->h_io + 8 + kIoMax;
+    memcpy(in, x, b);
+    memcpy(in + n, y, b);
+    memcpy(in + 2 * n, z, b);
+    c->io_in_busy = 1;
+    hipLaunchKernelGGL(k_hand_in, dim3(nblk(c->n)), dim3(256), 0, c->stream, c->n, c->d_io + 8 + kIoMax, dx, dy, dz);
+    HIP_TRY(c, hipGetLastError());
+    return MDFF_OK;
+  }
   HIP_TRY(c, hipMemcpyAsync(dx, x, b, hipMemcpyHostToDevice, c->stream));
   HIP_TRY(c, hipMemcpyAsync(dy, y, b, hipMemcpyHostToDevice, c->stream));
   HIP_TRY(c, hipMemcpyAsync(dz, z, b, hipMemcpyHostToDevice, c->stream));
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  return MDFF_OK;
-}
-
-static int copy3_out(mdff_ctx* c, const double* dx, const double* dy, const double* dz, double* x, double* y,
-                     double* z) {
-  if (!c || !x || !y || !z) return MDFF_ERR_BAD_ARG;
-  const size_t b = sizeof(double) * c->n;
-  HIP_TRY(c, hipMemcpyAsync(x, dx, b, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(c, hipMemcpyAsync(y, dy, b, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(c, hipMemcpyAsync(z, dz, b, hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   return MDFF_OK;
 }
@@ -1614,7 +1780,7 @@ int mdff_vnlistcheck(mdff_ctx* c, int32_t* rebuilt) {
   if (!c) return MDFF_ERR_BAD_ARG;
   int rb = 0;
   MDFF_TRY(nl_check(c, &rb));
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  if (rb) HIP_TRY(c, hipStreamSynchronize(c->stream));
   if (rebuilt) *rebuilt = rb;
   return MDFF_OK;
 }
@@ -1627,9 +1793,9 @@ int mdff_get_pairs(mdff_ctx* c, int32_t which, int32_t* point, int32_t* list, in
 int mdff_engforce(mdff_ctx* c, double* fx, double* fy, double* fz, mdff_terms* terms) {
   if (!c) return MDFF_ERR_BAD_ARG;
   mdff_terms t;
-  MDFF_TRY(engforce(c, &t));
+  double* const f[3] = {fx, fy, fz};
+  MDFF_TRY(engforce(c, &t, fx && fy && fz ? f : nullptr));
   if (terms) *terms = t;
-  if (fx && fy && fz) MDFF_TRY(mdff_get_forces(c, fx, fy, fz));
   return MDFF_OK;
 }
 
@@ -1641,7 +1807,14 @@ int mdff_last_terms(mdff_ctx* c, mdff_terms* terms) {
 
 int mdff_get_dipoles(mdff_ctx* c, double* mu, double* ef) {
   if (!c) return MDFF_ERR_BAD_ARG;
-  const size_t b = 3 * sizeof(double) * c->n;
+  const size_t n3 = 3 * (size_t)c->n, b = sizeof(double) * n3;
+  const double* h = nullptr;
+  MDFF_TRY(hand_over(c, {{c->mu, mu ? n3 : 0}, {c->efield, ef ? n3 : 0}}, &h));
+  if (h) {
+    if (mu) memcpy(mu, h, b);
+    if (ef) memcpy(ef, h + (mu ? n3 : 0), b);
+    return MDFF_OK;
+  }
   if (mu) HIP_TRY(c, hipMemcpyAsync(mu, c->mu, b, hipMemcpyDeviceToHost, c->stream));
   if (ef) HIP_TRY(c, hipMemcpyAsync(ef, c->efield, b, hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(c, hipStreamSynchronize(c->stream));
@@ -1652,6 +1825,12 @@ int mdff_get_efg(mdff_ctx* c, double* efg) {
   if (!c || !efg) return MDFF_ERR_BAD_ARG;
   const size_t b = 9 * sizeof(double) * c->n;
   if (c->efg) {
+    const double* h = nullptr;
+    MDFF_TRY(hand_over(c, {{c->efg, 9 * (size_t)c->n}}, &h));
+    if (h) {
+      memcpy(efg, h, b);
+      return MDFF_OK;
+    }
     HIP_TRY(c, hipMemcpyAsync(efg, c->efg, b, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
   } else {
@@ -1688,9 +1867,10 @@ int mdff_md_vv(mdff_ctx* c, int32_t nsteps, double dt, double* ekin, double* upo
     // tables), or here before the sums go to the host
     if (slot == RAW_SLOTS - 1 || st == nsteps - 1) MDFF_TRY(flush_finals(c));
     if (slot == RAW_SLOTS - 1 || st == nsteps - 1) {
-      MDFF_TRY(fetch_raw(c, slot + 1));
+      const double* h_raw = nullptr;
+      MDFF_TRY(fetch_raw(c, slot + 1, &h_raw));
       for (int k = 0; k <= slot; ++k) {
-        const double* h = c->h_raw + (size_t)RAW_N * k;
+        const double* h = h_raw + (size_t)RAW_N * k;
         engforce_finish(c, h, &held[k]);
         c->last_terms = held[k];
         if (ekin) ekin[st0 + k] = 0.5 * h[RAW_EKIN];
@@ -1796,9 +1976,10 @@ int mdff_md_nhcn(mdff_ctx* c, int32_t nsteps, double dt, double temp, double tim
     if (c->d.lvnlist) MDFF_TRY(nl_check_launch(c));
     if (slot == RAW_SLOTS - 1 || step == nsteps - 1) {
       MDFF_TRY(flush_finals(c));
-      MDFF_TRY(fetch_raw(c, slot + 1));
+      const double* h_raw = nullptr;
+      MDFF_TRY(fetch_raw(c, slot + 1, &h_raw));
       for (int k = 0; k <= slot; ++k) {
-        const double* h = c->h_raw + (size_t)RAW_N * k;
+        const double* h = h_raw + (size_t)RAW_N * k;
         engforce_finish(c, h, &held[k]);
         c->last_terms = held[k];
         if (ekin) ekin[st0 + k] = 0.5 * h[RAW_EKIN];
@@ -1819,39 +2000,48 @@ int mdff_md_nhcn(mdff_ctx* c, int32_t nsteps, double dt, double temp, double tim
   return MDFF_OK;
 }
 
+// one velocity rescale; e: kinetic energy before and after (csvr)
+static int rescale(mdff_ctx* c, RescaleArgs a, double e[2]) {
+  const int nb = nblk(c->n);
+  a.n = c->n;
+  a.nb = nb;
+  a.m = c->mass;
+  a.vx = c->vx; a.vy = c->vy; a.vz = c->vz;
+  a.pk = extra(c);
+  a.pv = extra(c) + nb;
+  a.out = c->red;
+  if (a.csvr) hipLaunchKernelGGL(k_rescale_kin, dim3(nb), dim3(256), 0, c->stream, a);
+  hipLaunchKernelGGL(k_rescale_v, dim3(nb), dim3(256), 0, c->stream, a);
+  hipLaunchKernelGGL(k_rescale_mean, dim3(nb), dim3(256), 0, c->stream, a);
+  const double* h = nullptr;
+  MDFF_TRY(hand_over(c, {{c->red, 2}}, &h));
+  e[0] = h[0];
+  e[1] = h[1];
+  return MDFF_OK;
+}
+
 int mdff_csvr_rescale(mdff_ctx* c, double temp, double taut, double r1, double sumnoise, double* conint) {
   if (!c) return MDFF_ERR_BAD_ARG;
   const int n = c->n;
-  double ekin;
-  MDFF_TRY(kinetic(c, &ekin, nullptr));
-  const int ndeg = 3 * n - 3;
-  const double sigma = ndeg * temp * 0.5;
-  const double factor = taut > 0.1 ? exp(-1.0 / taut) : 0.0;
-  const double knew = ekin + (1.0 - factor) * (sigma * (sumnoise + r1 * r1) / ndeg - ekin) +
-                      2.0 * r1 * sqrt(ekin * sigma / ndeg * (1.0 - factor) * factor);
-  if (conint) *conint = *conint - (knew - ekin);
-  const double lambda = sqrt(knew / ekin);
-  hipLaunchKernelGGL(k_scale_v, dim3(nblk(n)), dim3(256), 0, c->stream, n, lambda, 0.0, 0.0, 0.0, c->vx, c->vy,
-                     c->vz);
-  double k2, vs[3];
-  MDFF_TRY(kinetic(c, &k2, vs));
-  hipLaunchKernelGGL(k_scale_v, dim3(nblk(n)), dim3(256), 0, c->stream, n, 1.0, vs[0] / n, vs[1] / n, vs[2] / n,
-                     c->vx, c->vy, c->vz);
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  RescaleArgs a{};
+  a.csvr = 1;
+  a.ndeg = 3 * n - 3;
+  a.sigma = a.ndeg * temp * 0.5;
+  a.factor = taut > 0.1 ? exp(-1.0 / taut) : 0.0;
+  a.r1 = r1;
+  a.sumnoise = sumnoise;
+  double e[2];
+  MDFF_TRY(rescale(c, a, e));
+  if (conint) *conint = *conint - (e[1] - e[0]);
   return MDFF_OK;
 }
 
 int mdff_rescale_velocities(mdff_ctx* c, double lambda) {
   if (!c || !(lambda >= 0.0)) return MDFF_ERR_BAD_ARG;
-  const int n = c->n;
-  hipLaunchKernelGGL(k_scale_v, dim3(nblk(n)), dim3(256), 0, c->stream, n, lambda, 0.0, 0.0, 0.0, c->vx, c->vy,
-                     c->vz);
-  double k2, vs[3];
-  MDFF_TRY(kinetic(c, &k2, vs));
-  hipLaunchKernelGGL(k_scale_v, dim3(nblk(n)), dim3(256), 0, c->stream, n, 1.0, vs[0] / n, vs[1] / n, vs[2] / n,
-                     c->vx, c->vy, c->vz);
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  return MDFF_OK;
+  RescaleArgs a{};
+  a.lambda = lambda;
+  double e[2];
+  return rescale(c, a, e);
 }
 
 int mdff_calc_temp(mdff_ctx* c, double boltz_unit, double* temp, double* ekin) {

@@ -697,19 +697,16 @@ static CheckArgs check_args(mdff_ctx* c) {
   return k;
 }
 
-// the check's block maxima are written straight into mapped host memory
-// (h_chk); the event says when they are there
-static int check_posted(mdff_ctx* c) {
-  HIP_TRY(c, hipEventRecord(c->chk_ev, c->stream));
-  c->chk_pending = 1;
-  return MDFF_OK;
-}
-
 int nl_check_launch(mdff_ctx* c) {
   const int nb = div_up(c->n, 256);
   hipLaunchKernelGGL(k_disp_top2, dim3(nb), dim3(256), 0, c->stream, check_args(c), c->rx, c->ry, c->rz);
   HIP_TRY(c, hipGetLastError());
-  return check_posted(c);
+  // the check's block maxima are written straight into mapped host memory
+  // (h_chk); the next final-sum launch posts the word that says they are there
+  c->chk_seq += 1.0;
+  c->chk_seq_wait = 1;
+  c->chk_pending = 1;
+  return MDFF_OK;
 }
 
 int vv_pos_launch(mdff_ctx* c, double dt) {
@@ -750,23 +747,19 @@ int nl_check_finish(mdff_ctx* c, int* rebuilt) {
   c->chk_pending = 0;
   const int n = c->n;
   const int nb = div_up(n, 256);
-  if (c->chk_seq_wait) {
-    // the check's maxima are in h_chk once the sequence value is: spin on the
-    // mapped word, then (if the signal was never attached or is slow) wait
-    // for the stream and look again
-    volatile const double* sig = c->h_chk + 2 * nb;
-    bool seen = false;
-    if (c->chk_seq_wait == 2)
-      for (long k = 0; k < 20000000L && !seen; ++k) seen = (*sig == c->chk_seq);
-    if (!seen) {
-      if (c->chk_seq_wait == 1) MDFF_TRY(flush_finals(c));
-      HIP_TRY(c, hipStreamSynchronize(c->stream));
-      if (*sig != c->chk_seq) { c->err = "skin check signal missing"; return MDFF_ERR_HIP; }
-    }
-    c->chk_seq_wait = 0;
-  } else {
-    HIP_TRY(c, hipEventSynchronize(c->chk_ev));
+  // the check's maxima are in h_chk once the sequence value is: spin on the
+  // mapped word, then (if the signal was never attached or is slow) wait for
+  // the stream and look again
+  volatile const double* sig = c->h_chk + 2 * nb;
+  bool seen = false;
+  if (c->chk_seq_wait == 2)
+    for (long k = 0; k < 20000000L && !seen; ++k) seen = (*sig == c->chk_seq);
+  if (!seen) {
+    if (c->chk_seq_wait == 1) MDFF_TRY(flush_finals(c));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    if (*sig != c->chk_seq) { c->err = "skin check signal missing"; return MDFF_ERR_HIP; }
   }
+  c->chk_seq_wait = 0;
   double m1 = 0.0, m2 = 0.0;
   for (int b = 0; b < nb; ++b) {
     double v[2] = {c->h_chk[2 * b], c->h_chk[2 * b + 1]};
@@ -786,6 +779,7 @@ int nl_check_finish(mdff_ctx* c, int* rebuilt) {
 
 int nl_check(mdff_ctx* c, int* rebuilt) {
   MDFF_TRY(nl_check_launch(c));
+  MDFF_TRY(flush_finals(c));
   return nl_check_finish(c, rebuilt);
 }
 

@@ -146,3 +146,22 @@ def test_fit_most_parameters():
         p.close()
     assert rel(g[1][24:], g[0]) < 1e-12
     assert not np.any(g[1][:24])
+
+
+@pytest.mark.parametrize("ncell", [3, 13, 14])
+def test_arrays_through_mapped_memory(ncell):
+    """108 and 8,788 atoms: arrays go through mapped memory; 10,976: copies.
+    Two positions in a row before the device has read the first."""
+    s = _lj(ncell)
+    note(f"arrays n={s.natm}")
+    g, o = pair(s)
+    for k in range(3):
+        g.set_positions(s.pos + 0.1 * k)
+        v = s.pos * (k + 1.0)
+        g.set_velocities(v)
+    assert np.array_equal(g.get_positions(), s.pos + 0.2)
+    assert np.array_equal(g.get_velocities(), v)
+    o.set_positions(s.pos + 0.2)
+    f = g.engforce()[0]
+    assert rel_force_err(f, o.engforce()[0]) < TOL[capi.PREC_FP64]
+    assert not np.any(g.get_dipoles()[0])
