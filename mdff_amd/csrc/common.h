@@ -303,7 +303,8 @@ struct mdff_ctx {
 
   // neighbour list (full rows, cut = max(rc_vdw, rc_coul) + skin)
   int32_t* cell_of = nullptr;             // cell index per atom
-  int32_t* cell_key = nullptr;            // sorted keys
+  int32_t* cell_slot = nullptr;           // an atom's place in its cell, as counted
+  int32_t* cell_cnt = nullptr;            // atoms a cell, zero between builds (ncell_alloc)
   int32_t* cell_atoms = nullptr;          // atoms sorted by cell
   int32_t* cell_atoms_in = nullptr;
   int32_t* cell_start = nullptr;          // ncell + 1
@@ -328,6 +329,9 @@ struct mdff_ctx {
   int nb_lo[3] = {0, 0, 0}, nb_hi[3] = {0, 0, 0}, nb_all[3] = {1, 1, 1};  // neighbour cell offsets
   float4* bf = nullptr;                   // wrapped single-precision copy of (bx, by, bz)
   int ncell_alloc = 0;
+  double* h_nl = nullptr;                 // mapped pinned host memory: a build's overflow flag, sequence number
+  double* d_nl = nullptr;
+  double nl_seq = 0.0;
   void* sort_tmp = nullptr;
   size_t sort_tmp_bytes = 0;
   int lists_valid = 0;

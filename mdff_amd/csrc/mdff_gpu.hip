@@ -931,7 +931,7 @@ static int ctx_init(mdff_ctx* c, const mdff_desc* d, const int32_t* itype) {
   DMALLOC(c->d_pp, c->pp.size());
   HIP_TRY(c, hipMemcpy(c->d_pp, c->pp.data(), sizeof(PairParam) * c->pp.size(), hipMemcpyHostToDevice));
   DMALLOC(c->cell_of, n);
-  DMALLOC(c->cell_key, n);
+  DMALLOC(c->cell_slot, n);
   DMALLOC(c->cell_atoms, n);
   DMALLOC(c->cell_atoms_in, n);
   DMALLOC(c->nl_count, n + 1);
@@ -968,6 +968,9 @@ static int ctx_init(mdff_ctx* c, const mdff_desc* d, const int32_t* itype) {
   HIP_TRY(c, hipHostMalloc((void**)&c->h_red, sizeof(double) * nred));
   DMALLOC(c->red_part, nred);
   DMALLOC(c->scf_part, 2 * (size_t)nblk(n));
+  HIP_TRY(c, hipHostMalloc((void**)&c->h_nl, sizeof(double) * 2, hipHostMallocMapped | hipHostMallocCoherent));
+  HIP_TRY(c, hipHostGetDevicePointer((void**)&c->d_nl, c->h_nl, 0));
+  c->h_nl[0] = c->h_nl[1] = 0.0;
   // mapped hand-over memory: the sequence word, results, and incoming arrays
   HIP_TRY(c, hipHostMalloc((void**)&c->h_io, sizeof(double) * (8 + 2 * kIoMax), hipHostMallocMapped | hipHostMallocCoherent));
   HIP_TRY(c, hipHostGetDevicePointer((void**)&c->d_io, c->h_io, 0));
@@ -1687,7 +1690,7 @@ int mdff_ctx_destroy(mdff_ctx* c) {
   void* ps[] = {c->rx, c->ry, c->rz, c->vx, c->vy, c->vz, c->fx, c->fy, c->fz, c->fsx, c->fsy, c->fsz,
                 c->sx, c->sy, c->sz, c->xs, c->ys, c->zs, c->bx, c->by, c->bz, c->bf, c->itype, c->q, c->mass,
                 c->pol, c->invpol, c->dipia, c->mu, c->mu_ind, c->efield, c->e_stat, c->e_tot, c->e_ind,
-                c->hist, c->frec, c->zeros, c->arec, c->ameta, c->peratom, c->red, c->red_part, c->d_pp, c->cell_of, c->cell_key,
+                c->hist, c->frec, c->zeros, c->arec, c->ameta, c->peratom, c->red, c->red_part, c->d_pp, c->cell_of, c->cell_slot, c->cell_cnt,
                 c->cell_atoms, c->cell_atoms_in, c->cell_start, c->nl_count, c->nl_start, c->nl_j,
                 c->nl_flag, c->nl_count_in, c->nl_j_tmp, c->nl_flag_tmp, c->sort_tmp, c->d_flag, c->raw,
                 c->cx, c->cy, c->cz, c->fin_part, c->nhc_part, c->nhc_st, c->peratom_lj, c->f_lj, c->lj_part, c->scf_part};
@@ -1702,6 +1705,7 @@ int mdff_ctx_destroy(mdff_ctx* c) {
   if (c->h_chk) (void)hipHostFree(c->h_chk);
   if (c->h_scf) (void)hipHostFree(c->h_scf);
   if (c->h_io) (void)hipHostFree(c->h_io);
+  if (c->h_nl) (void)hipHostFree(c->h_nl);
   if (c->ov_tab) (void)hipEventDestroy(c->ov_tab);
   if (c->ov_pair) (void)hipEventDestroy(c->ov_pair);
   if (c->stream2) (void)hipStreamDestroy(c->stream2);

@@ -18,7 +18,6 @@
 #include <algorithm>
 #include <cstring>
 
-#include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_reduce.hpp>
 #include <rocprim/device/device_scan.hpp>
 
@@ -71,43 +70,102 @@ __device__ __forceinline__ int wrap_cell(double s, int nc) {
   return k < 0 ? 0 : (k >= nc ? nc - 1 : k);
 }
 
-__global__ void k_cell_assign(int n, const double* __restrict__ sx, const double* __restrict__ sy,
-                              const double* __restrict__ sz, int nx, int ny, int nz,
-                              int32_t* __restrict__ cell_of, int32_t* __restrict__ iota) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+// Atoms into cells, in the order of their indices within each: count, scan,
+// scatter, and ranks within a cell counted out by k_cell_order (a cell holds a
+// few atoms).  Four short launches; the radix sort of (cell, index) and what
+// it needed around it were eight, 45 us of a build of 24,000 atoms.
+__global__ void k_cell_count(int n, const double* __restrict__ sx, const double* __restrict__ sy,
+                             const double* __restrict__ sz, int nx, int ny, int nz, int32_t* __restrict__ cell_of,
+                             int32_t* __restrict__ slot, int32_t* __restrict__ cnt) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  int cx = wrap_cell(sx[i], nx), cy = wrap_cell(sy[i], ny), cz = wrap_cell(sz[i], nz);
-  cell_of[i] = (cx * ny + cy) * nz + cz;
-  iota[i] = i;
+  const int cx = wrap_cell(sx[i], nx), cy = wrap_cell(sy[i], ny), cz = wrap_cell(sz[i], nz);
+  const int k = (cx * ny + cy) * nz + cz;
+  cell_of[i] = k;
+  slot[i] = atomicAdd(cnt + k, 1);
 }
 
-// start offset of every cell from the sorted keys (empty cells included)
-__global__ void k_cell_start(int n, int ncell, const int32_t* __restrict__ key,
-                             int32_t* __restrict__ start) {
-  int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  int k = key[p];
-  int prev = (p == 0) ? -1 : key[p - 1];
-  for (int c = prev + 1; c <= k; ++c) start[c] = p;
-  if (p == n - 1)
-    for (int c = k + 1; c <= ncell; ++c) start[c] = n;
+// start[k] = atoms before cell k, start[ncell] = n; the counts and the overflow
+// flag back to zero.  One block, a run of cells a thread.
+constexpr int kScanRun = 16;
+__global__ void __launch_bounds__(1024) k_cell_scan(int n, int ncell, int32_t* __restrict__ cnt,
+                                                    int32_t* __restrict__ start, int32_t* __restrict__ overflow) {
+  __shared__ int wsum[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int base = 0;
+  // kScanRun cells a thread and round (4 would leave 64,000 cells 48 us of rounds)
+  for (int c0 = 0; c0 < ncell; c0 += 1024 * kScanRun) {
+    const int k = c0 + kScanRun * (int)threadIdx.x;
+    int v[kScanRun], sum = 0;
+#pragma unroll
+    for (int u = 0; u < kScanRun; ++u) {
+      v[u] = k + u < ncell ? cnt[k + u] : 0;
+      sum += v[u];
+    }
+    int incl = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += t;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    int before = base, all = base;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      before += w < wave ? wsum[w] : 0;
+      all += wsum[w];
+    }
+    int at = before + incl - sum;
+#pragma unroll
+    for (int u = 0; u < kScanRun; ++u)
+      if (k + u < ncell) {
+        start[k + u] = at;
+        cnt[k + u] = 0;
+        at += v[u];
+      }
+    base = all;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    start[ncell] = n;
+    *overflow = 0;
+  }
 }
 
-// fractional coordinates in cell order: the doubles, and a wrapped
-// single-precision copy (s - floor(s), exact in double, then rounded) for
-// the sweep's prefilter
-__global__ void k_gather_sorted(int n, const int32_t* __restrict__ order, const double* __restrict__ sx,
-                                const double* __restrict__ sy, const double* __restrict__ sz,
-                                double* __restrict__ ox, double* __restrict__ oy, double* __restrict__ oz,
-                                float4* __restrict__ of) {
-  int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  int i = order[p];
+__global__ void k_cell_scatter(int n, const int32_t* __restrict__ cell_of, const int32_t* __restrict__ slot,
+                               const int32_t* __restrict__ start, int32_t* __restrict__ out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[start[cell_of[i]] + slot[i]] = i;
+}
+
+// atoms of a cell in the order of their indices, and their fractional
+// coordinates in cell order: the doubles, and a wrapped single-precision copy
+// (s - floor(s), exact in double, then rounded) for the sweep's prefilter;
+// with save, also kept per atom (xs, ys, zs)
+__global__ void k_cell_order(int n, const int32_t* __restrict__ in, const int32_t* __restrict__ cell_of,
+                             const int32_t* __restrict__ start, const double* __restrict__ sx,
+                             const double* __restrict__ sy, const double* __restrict__ sz,
+                             int32_t* __restrict__ order, double* __restrict__ ox, double* __restrict__ oy,
+                             double* __restrict__ oz, float4* __restrict__ of, int save, double* __restrict__ xs,
+                             double* __restrict__ ys, double* __restrict__ zs) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const int i = in[t];
+  const int k = cell_of[i], b = start[k], e = start[k + 1];
+  int p = b;
+  for (int u = b; u < e; ++u) p += in[u] < i ? 1 : 0;
   const double x = sx[i], y = sy[i], z = sz[i];
+  order[p] = i;
   ox[p] = x;
   oy[p] = y;
   oz[p] = z;
   of[p] = make_float4((float)(x - floor(x)), (float)(y - floor(y)), (float)(z - floor(z)), 0.f);
+  if (save) {
+    xs[i] = x;
+    ys[i] = y;
+    zs[i] = z;
+  }
 }
 
 struct NLArgs {
@@ -123,6 +181,11 @@ struct NLArgs {
   // neighbour cells: offsets ox0..ox1 (x), oy0..oy1 (y) around the atom's
   // cell; in z either oz0..oz1 around it or, zall != 0, every z cell
   int ox0, ox1, oy0, oy1, oz0, oz1, zall;
+  // orthogonal cells: the columns and z cells farther than the cutoff from the
+  // atom itself are left out (trim); an axis whose cells are all visited has no
+  // nearer side (xall, yall)
+  int trim, xall, yall;
+  double lx, ly, lz, cut2_trim;
   // prefilter: r^2 in single precision; decided exactly (FP64, reference
   // rounding) when within marg of a cutoff or when prefilter == 0
   int prefilter;
@@ -157,13 +220,20 @@ __device__ __forceinline__ double min_image_r2(const NLArgs& a, double dx, doubl
 
 // Candidate index v of the wave's concatenated ranges -> sorted position:
 // range k holds v in [pref[k], pref[k + 1]) starting at position st[k];
-// unused entries hold pref = total, so the branch-free search over 64
+// unused entries hold pref = total, so the branch-free search over 128
 // entries ends on the range that holds v.
 __device__ __forceinline__ int range_pos(const int* pref, const int* st, int v) {
   int k = 0;
 #pragma unroll
-  for (int step = 32; step > 0; step >>= 1) k += (pref[k + step] <= v) ? step : 0;
+  for (int step = 64; step > 0; step >>= 1) k += (pref[k + step] <= v) ? step : 0;
   return st[k] + (v - pref[k]);
+}
+
+// distance from a fraction f, in cell k of nc, to the cell at offset d (0 in
+// its own)
+__device__ __forceinline__ double cell_gap(double f, int k, int d, int nc) {
+  const double g = d > 0 ? (double)(k + d) / nc - f : f - (double)(k + d + 1) / nc;
+  return d == 0 || g < 0.0 ? 0.0 : g;
 }
 
 // One wave per atom (atoms in cell order).  The neighbour cells form, per
@@ -174,9 +244,13 @@ __device__ __forceinline__ int range_pos(const int* pref, const int* st, int v) 
 // (wrapped coordinates, rint minimum image); one whose r^2 lies within marg
 // of a cutoff is tested again in FP64 exactly as the reference does, so the
 // accepted set and the flags equal the reference's bit for bit.
+// VALU-bound, some 80 instructions per 64 candidates, so what counts is the
+// candidates: cells of a third of the cutoff, and those beyond the atom's own
+// sphere left out, 62 us for 24,000 atoms at 11 A and 445 for 195,112 at 10 (109
+// and 690 with cells of half the cutoff, all 125 of them).
 template <bool FILL>
 __global__ void __launch_bounds__(256) k_nl_sweep(NLArgs a) {
-  __shared__ int rpref[4][66], rst[4][65];
+  __shared__ int rpref[4][130], rst[4][129];
   const int lane = threadIdx.x & 63;
   const int wl = threadIdx.x >> 6;
   const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -189,21 +263,38 @@ __global__ void __launch_bounds__(256) k_nl_sweep(NLArgs a) {
   const int64_t base = FILL ? (a.row_w ? (int64_t)i * a.row_w : (int64_t)a.row_start[i]) : 0;
   const int64_t lim = a.row_w ? base + a.row_w : a.cap;
   const int ncx = a.ox1 - a.ox0 + 1, ncy = a.oy1 - a.oy0 + 1;
-  const int ncol = ncx * ncy;              // <= 25 columns, <= 2 ranges each
+  const int ncol = ncx * ncy;              // <= 49 columns, <= 2 ranges each
   int b0 = 0, e0 = 0, b1 = 0, e1 = 0;
   if (lane < ncol) {
     const int dy = a.oy0 + lane % ncy, dx = a.ox0 + lane / ncy;
     const int xx = (cx + dx + a.nx) % a.nx, yy = (cy + dy + a.ny) % a.ny;
     const int c0 = (xx * a.ny + yy) * a.nz;  // cell (xx, yy, 0)
     int z0 = 0, z1 = a.nz - 1, w0 = 0, w1 = -1;   // [z0, z1] and the wrapped [w0, w1]
-    if (!a.zall) {
+    double rem = a.cut2_trim;              // what the column's distance leaves of the cutoff
+    if (a.trim) {
+      const double gx = a.xall ? 0.0 : a.lx * cell_gap(si - floor(si), cx, dx, a.nx);
+      const double gy = a.yall ? 0.0 : a.ly * cell_gap(ti - floor(ti), cy, dy, a.ny);
+      rem -= gx * gx + gy * gy;
+    }
+    if (rem < 0.0) {
+      z1 = -1;
+    } else if (!a.zall) {
       z0 = cz + a.oz0;
       z1 = cz + a.oz1;
-      if (z0 < 0) { w0 = z0 + a.nz; w1 = a.nz - 1; z0 = 0; }
+      if (a.trim) {
+        const double f = (ui - floor(ui)) * a.nz, h = sqrt(rem) / a.lz * a.nz + 1e-6;
+        z0 = max(z0, (int)floor(f - h));
+        z1 = min(z1, (int)floor(f + h));
+      }
+      if (z1 < 0) { z0 += a.nz; z1 += a.nz; }
+      else if (z0 >= a.nz) { z0 -= a.nz; z1 -= a.nz; }
+      else if (z0 < 0) { w0 = z0 + a.nz; w1 = a.nz - 1; z0 = 0; }
       else if (z1 >= a.nz) { w0 = 0; w1 = z1 - a.nz; z1 = a.nz - 1; }
     }
-    b0 = a.cell_start[c0 + z0];
-    e0 = a.cell_start[c0 + z1 + 1];
+    if (z1 >= z0) {
+      b0 = a.cell_start[c0 + z0];
+      e0 = a.cell_start[c0 + z1 + 1];
+    }
     if (w1 >= w0) {
       b1 = a.cell_start[c0 + w0];
       e1 = a.cell_start[c0 + w1 + 1];
@@ -219,40 +310,37 @@ __global__ void __launch_bounds__(256) k_nl_sweep(NLArgs a) {
   }
   const int total = __shfl(incl, 63, 64);
   const int excl = incl - len;
-  // range 2l: [b0, e0), range 2l+1: [b1, e1); 64 entries (2 * 25 + pad)
-  if (lane < 32) {
-    rpref[wl][2 * lane] = lane < ncol ? excl : total;
-    rpref[wl][2 * lane + 1] = lane < ncol ? excl + (e0 - b0) : total;
-    rst[wl][2 * lane] = b0;
-    rst[wl][2 * lane + 1] = b1;
-  }
-  if (lane < 2) rpref[wl][64 + lane] = total;
+  // range 2l: [b0, e0), range 2l+1: [b1, e1); 128 entries (2 * 49 + pad)
+  rpref[wl][2 * lane] = lane < ncol ? excl : total;
+  rpref[wl][2 * lane + 1] = lane < ncol ? excl + (e0 - b0) : total;
+  rst[wl][2 * lane] = b0;
+  rst[wl][2 * lane + 1] = b1;
+  if (lane < 2) rpref[wl][128 + lane] = total;
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   const int* pref = rpref[wl];
   const int* st = rst[wl];
   int found = 0, found_in = 0;
-  // chunk loads: candidate sorted position, its atom and coordinates (clamped)
-  int qn = 0, jn = -1;
+  // chunk loads: candidate sorted position and coordinates; the atom itself is
+  // at position `wave`
+  int qn = 0;
   float4 fn = make_float4(0.f, 0.f, 0.f, 0.f);
   if (lane < total) {
     qn = range_pos(pref, st, lane);
-    jn = a.cell_atoms[qn];
     fn = a.pf[qn];
   }
   for (int v0 = 0; v0 < total; v0 += 64) {
-    const int q = qn, j = jn;
+    const int q = qn;
     const float4 f = fn;
     const bool live = v0 + lane < total;
     if (v0 + 64 + lane < total) {
       qn = range_pos(pref, st, v0 + 64 + lane);
-      jn = a.cell_atoms[qn];
       fn = a.pf[qn];
     }
     bool ok = false, inner = false;
     uint8_t flag = 0;
-    if (live && j != i) {
+    if (live && q != wave) {
       float dx = sif - f.x, dy = tif - f.y, dz = uif - f.z;
       dx -= rintf(dx);
       dy -= rintf(dy);
@@ -261,8 +349,8 @@ __global__ void __launch_bounds__(256) k_nl_sweep(NLArgs a) {
       const float ry = fmaf(dx, a.a21f, fmaf(dy, a.a22f, dz * a.a23f));
       const float rz = fmaf(dx, a.a31f, fmaf(dy, a.a32f, dz * a.a33f));
       const float r2f = fmaf(rx, rx, fmaf(ry, ry, rz * rz));
-      const bool near = fabsf(r2f - a.c2f_max) <= a.marg || fabsf(r2f - a.c2f_v) <= a.marg ||
-                        fabsf(r2f - a.c2f_c) <= a.marg;
+      // (the largest cutoff is one of the two)
+      const bool near = fabsf(r2f - a.c2f_v) <= a.marg || fabsf(r2f - a.c2f_c) <= a.marg;
       if (!a.prefilter || near) {
         const double r2 = min_image_r2(a, si - a.px[q], ti - a.py[q], ui - a.pz[q]);
         ok = (r2 <= a.cut2_max);
@@ -299,7 +387,7 @@ __global__ void __launch_bounds__(256) k_nl_sweep(NLArgs a) {
 // first, count_in of them, both parts in their sweep order.  One wave per
 // row; the rows are read from (sj, sf) and written to (dj, df) at the same
 // row starts.
-__global__ void __launch_bounds__(256) k_nl_partition(int n, const int32_t* __restrict__ start,
+__global__ void __launch_bounds__(256) k_nl_partition(int n, int row_w, const int32_t* __restrict__ start,
                                                       const int32_t* __restrict__ count,
                                                       const int32_t* __restrict__ count_in,
                                                       const int32_t* __restrict__ sj, const uint8_t* __restrict__ sf,
@@ -308,7 +396,8 @@ __global__ void __launch_bounds__(256) k_nl_partition(int n, const int32_t* __re
   const int i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   if (i >= n) return;                      // whole waves
   const int64_t base = start[i];
-  const int cnt = count[i], nin = count_in[i];
+  // a row that overflowed its width is rebuilt by the counting pass
+  const int cnt = min(count[i], row_w), nin = min(count_in[i], cnt);
   const uint64_t below = (1ull << lane) - 1ull;
   int oin = 0, oout = 0;
   for (int v0 = 0; v0 < cnt; v0 += 64) {
@@ -324,12 +413,21 @@ __global__ void __launch_bounds__(256) k_nl_partition(int n, const int32_t* __re
     const uint64_t mi = __ballot(in), mo = __ballot(live && !in);
     if (live) {
       const int64_t d = in ? base + oin + __popcll(mi & below) : base + nin + oout + __popcll(mo & below);
-      dj[d] = j;
-      df[d] = f;
+      if (d < base + cnt) {
+        dj[d] = j;
+        df[d] = f;
+      }
     }
     oin += __popcll(mi);
     oout += __popcll(mo);
   }
+}
+
+__global__ void k_post_flag(const int32_t* flag, double* out, double seq) {
+  if (threadIdx.x != 0) return;
+  out[0] = (double)*flag;
+  __threadfence_system();
+  *reinterpret_cast<volatile double*>(out + 1) = seq;
 }
 
 static int ensure(mdff_ctx* c, void** p, size_t& have, size_t need) {
@@ -367,6 +465,11 @@ static NLArgs make_args(mdff_ctx* c) {
   a.oy0 = c->nb_lo[1]; a.oy1 = c->nb_hi[1];
   a.oz0 = c->nb_lo[2]; a.oz1 = c->nb_hi[2];
   a.zall = c->nb_all[2];
+  a.trim = A[1] == 0.0 && A[2] == 0.0 && A[3] == 0.0 && A[5] == 0.0 && A[6] == 0.0 && A[7] == 0.0;
+  a.xall = c->nb_all[0];
+  a.yall = c->nb_all[1];
+  a.lx = std::fabs(A[0]); a.ly = std::fabs(A[4]); a.lz = std::fabs(A[8]);
+  a.cut2_trim = a.cut2_max * (1.0 + 1e-6);
   // Single-precision prefilter.  The wrapped coordinates carry an error of
   // at most 2^-24, the difference, the minimum image and each Cartesian
   // component add a few units of 2^-24 relative to |A| (row sums of |A|),
@@ -407,22 +510,39 @@ static NLArgs make_args(mdff_ctx* c) {
   return a;
 }
 
+// the sweep's overflow flag on the host; `next` is launched before the wait
+template <typename F>
+static int nl_overflow(mdff_ctx* c, F next, bool* over) {
+  c->h_nl[1] = 0.0;
+  c->nl_seq += 1.0;
+  hipLaunchKernelGGL(k_post_flag, dim3(1), dim3(64), 0, c->stream, c->d_flag + 1, c->d_nl, c->nl_seq);
+  next();
+  volatile const double* h = c->h_nl;
+  bool seen = false;
+  for (long k = 0; k < 20000000L && !seen; ++k) seen = h[1] == c->nl_seq;
+  if (!seen) {
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    if (h[1] != c->nl_seq) { c->err = "list overflow signal missing"; return MDFF_ERR_HIP; }
+  }
+  *over = h[0] != 0.0;
+  return MDFF_OK;
+}
+
 // vnlist_pbc: rebuild the rows from the current positions.
 // list build from the fractional coordinates (px, py, pz) of the build
-static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const double* pz) {
+static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const double* pz, bool save) {
   const int n = c->n;
-  // cells: width >= cutoff / 2 in a reciprocal direction with room for at
-  // least 5 of them (partners within +-2 cells), else width >= cutoff
-  // (partners within +-1 cell); 1e-9 margin against rounding of the wrapped
+  // cells: width >= cutoff / 3 in a reciprocal direction with room for at
+  // least 7 of them (partners within +-3 cells), else cutoff / 2 (5, +-2),
+  // else the cutoff (+-1); 1e-9 margin against rounding of the wrapped
   // coordinates.  With fewer cells than the reach covers, every cell of that
   // direction is visited once.
   double rmax = std::max(c->rc_vdw, c->rc_coul) + c->d.skindiff;
   for (int d = 0; d < 3; ++d) {
-    const int k2 = (int)floor(c->W[d] / (0.5 * rmax * (1.0 + 1e-9)));
-    int reach = 2, k = k2;
-    if (k2 < 5) {
-      reach = 1;
-      k = (int)floor(c->W[d] / (rmax * (1.0 + 1e-9)));
+    int reach = 3, k = 0;
+    for (; reach >= 1; --reach) {
+      k = (int)floor(c->W[d] * reach / (rmax * (1.0 + 1e-9)));
+      if (k >= 2 * reach + 1 || reach == 1) break;
     }
     c->ncell[d] = k < 1 ? 1 : k;
     const bool all = c->ncell[d] < 2 * reach + 1;
@@ -433,30 +553,22 @@ static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const 
   int ncell = c->ncell[0] * c->ncell[1] * c->ncell[2];
   if (ncell + 1 > c->ncell_alloc) {
     if (c->cell_start) HIP_TRY(c, hipFree(c->cell_start));
+    if (c->cell_cnt) HIP_TRY(c, hipFree(c->cell_cnt));
+    c->cell_cnt = nullptr;
     HIP_TRY(c, hipMalloc((void**)&c->cell_start, sizeof(int32_t) * (ncell + 1)));
+    HIP_TRY(c, hipMalloc((void**)&c->cell_cnt, sizeof(int32_t) * (ncell + 1)));
+    HIP_TRY(c, hipMemsetAsync(c->cell_cnt, 0, sizeof(int32_t) * (ncell + 1), c->stream));   // zero between builds
     c->ncell_alloc = ncell + 1;
   }
-  hipLaunchKernelGGL(k_cell_assign, dim3(div_up(n, 256)), dim3(256), 0, c->stream, n, px, py, pz,
-                     c->ncell[0], c->ncell[1], c->ncell[2], c->cell_of, c->cell_atoms_in);
-  int bits = 1;
-  while ((1 << bits) <= ncell) ++bits;
-  size_t tmp = 0;
-  HIP_TRY(c, rocprim::radix_sort_pairs(nullptr, tmp, c->cell_of, c->cell_key, c->cell_atoms_in,
-                                       c->cell_atoms, (unsigned)n, 0u, (unsigned)bits, c->stream));
-  size_t tmp2 = 0, tmp3 = 0;
-  HIP_TRY(c, rocprim::exclusive_scan(nullptr, tmp2, c->nl_count, c->nl_start, 0, (size_t)n + 1,
-                                     rocprim::plus<int32_t>(), c->stream));
-  HIP_TRY(c, rocprim::reduce(nullptr, tmp3, c->nl_count, c->d_flag + 2, 0, (size_t)n,
-                             rocprim::maximum<int32_t>(), c->stream));
-  MDFF_TRY(ensure(c, &c->sort_tmp, c->sort_tmp_bytes, std::max(tmp, std::max(tmp2, tmp3))));
-  HIP_TRY(c, rocprim::radix_sort_pairs(c->sort_tmp, tmp, c->cell_of, c->cell_key, c->cell_atoms_in,
-                                       c->cell_atoms, (unsigned)n, 0u, (unsigned)bits, c->stream));
-  hipLaunchKernelGGL(k_cell_start, dim3(div_up(n, 256)), dim3(256), 0, c->stream, n, ncell, c->cell_key,
-                     c->cell_start);
+  const dim3 ga(div_up(n, 256)), b256(256);
+  hipLaunchKernelGGL(k_cell_count, ga, b256, 0, c->stream, n, px, py, pz, c->ncell[0], c->ncell[1], c->ncell[2],
+                     c->cell_of, c->cell_slot, c->cell_cnt);
+  hipLaunchKernelGGL(k_cell_scan, dim3(1), dim3(1024), 0, c->stream, n, ncell, c->cell_cnt, c->cell_start, c->d_flag + 1);
+  hipLaunchKernelGGL(k_cell_scatter, ga, b256, 0, c->stream, n, c->cell_of, c->cell_slot, c->cell_start, c->cell_atoms_in);
   // fractional coordinates in cell order (coalesced candidate loads); they
   // are kept as the positions of this build
-  hipLaunchKernelGGL(k_gather_sorted, dim3(div_up(n, 256)), dim3(256), 0, c->stream, n, c->cell_atoms,
-                     px, py, pz, c->bx, c->by, c->bz, c->bf);
+  hipLaunchKernelGGL(k_cell_order, ga, b256, 0, c->stream, n, c->cell_atoms_in, c->cell_of, c->cell_start, px, py, pz,
+                     c->cell_atoms, c->bx, c->by, c->bz, c->bf, save ? 1 : 0, c->xs, c->ys, c->zs);
   NLArgs a = make_args(c);
   a.sx = px; a.sy = py; a.sz = pz;
   a.px = c->bx; a.py = c->by; a.pz = c->bz;
@@ -466,7 +578,8 @@ static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const 
   const bool split = c->rc_inner > 0.0;
   auto partition = [&]() {
     if (split)
-      PROF_LAUNCH(c, PK_NLIST, hipLaunchKernelGGL(k_nl_partition, grid, dim3(256), 0, c->stream, n, c->nl_start,
+      PROF_LAUNCH(c, PK_NLIST, hipLaunchKernelGGL(k_nl_partition, grid, dim3(256), 0, c->stream, n,
+                                                  a.row_w ? a.row_w : INT32_MAX, c->nl_start,
                                                   c->nl_count, c->nl_count_in, c->nl_j_tmp, c->nl_flag_tmp,
                                                   c->nl_j, c->nl_flag));
   };
@@ -478,18 +591,25 @@ static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const 
     // one pass into rows of the width sized at an earlier build; a row that
     // does not fit sends the build through the counting pass below
     a.row_w = c->nl_row_w;
-    HIP_TRY(c, hipMemsetAsync(c->d_flag + 1, 0, sizeof(int32_t), c->stream));
     PROF_LAUNCH(c, PK_NLIST, hipLaunchKernelGGL(k_nl_sweep<true>, grid, dim3(256), 0, c->stream, a));
-    HIP_TRY(c, hipMemcpyAsync(c->h_flag + 1, c->d_flag + 1, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    if (c->h_flag[1] == 0) {
-      partition();
+    // the partition is queued before the host looks at the flag, so that the
+    // device has work while it does
+    bool over = false;
+    MDFF_TRY(nl_overflow(c, partition, &over));
+    if (!over) {
       HIP_TRY(c, hipGetLastError());
       c->lists_valid = 1;
       return MDFF_OK;
     }
+    HIP_TRY(c, hipMemsetAsync(c->d_flag + 1, 0, sizeof(int32_t), c->stream));
     a.row_w = 0;
   }
+  size_t tmp2 = 0, tmp3 = 0;
+  HIP_TRY(c, rocprim::exclusive_scan(nullptr, tmp2, c->nl_count, c->nl_start, 0, (size_t)n + 1,
+                                     rocprim::plus<int32_t>(), c->stream));
+  HIP_TRY(c, rocprim::reduce(nullptr, tmp3, c->nl_count, c->d_flag + 2, 0, (size_t)n,
+                             rocprim::maximum<int32_t>(), c->stream));
+  MDFF_TRY(ensure(c, &c->sort_tmp, c->sort_tmp_bytes, std::max(tmp2, tmp3)));
   HIP_TRY(c, hipMemsetAsync(c->nl_count + n, 0, sizeof(int32_t), c->stream));
   PROF_LAUNCH(c, PK_NLIST, hipLaunchKernelGGL(k_nl_sweep<false>, grid, dim3(256), 0, c->stream, a));
   HIP_TRY(c, rocprim::exclusive_scan(c->sort_tmp, tmp2, c->nl_count, c->nl_start, 0, (size_t)n + 1,
@@ -534,7 +654,6 @@ static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const 
   a.cap = c->nl_cap;
   a.row_w = (int)w;
   c->nl_row_w = (int)w;
-  HIP_TRY(c, hipMemsetAsync(c->d_flag + 1, 0, sizeof(int32_t), c->stream));
   PROF_LAUNCH(c, PK_NLIST, hipLaunchKernelGGL(k_nl_sweep<true>, grid, dim3(256), 0, c->stream, a));
   partition();
   HIP_TRY(c, hipGetLastError());
@@ -544,7 +663,7 @@ static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const 
 
 int nl_build(mdff_ctx* c) {
   launch_kardir(c);
-  return nl_build_from(c, c->sx, c->sy, c->sz);
+  return nl_build_from(c, c->sx, c->sy, c->sz, false);
 }
 
 // the two largest of the block's values m1 (m2 = 0 on entry) -> out[2 * block]
@@ -669,15 +788,6 @@ __global__ void __launch_bounds__(256) k_vv_end(VvEndArgs e) {
   if (e.check) block_top2(m1, 0.0, s1, s2, e.k.out);
 }
 
-__global__ void k_copy3(int n, const double* a, const double* b, const double* cc, double* x, double* y,
-                        double* z) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  x[i] = a[i];
-  y[i] = b[i];
-  z[i] = cc[i];
-}
-
 // vnlistcheck: rebuild when (largest + second largest displacement) > skindiff,
 // then save the fractional coordinates (src/tools.f90:513-526).  Split in two
 // halves so that a caller can queue more work between them: the launch half
@@ -769,9 +879,7 @@ int nl_check_finish(mdff_ctx* c, int* rebuilt) {
     }
   }
   if (m1 + m2 > c->d.skindiff) {
-    MDFF_TRY(nl_build_from(c, c->cx, c->cy, c->cz));
-    hipLaunchKernelGGL(k_copy3, dim3(nb), dim3(256), 0, c->stream, n, c->cx, c->cy, c->cz, c->xs, c->ys,
-                       c->zs);
+    MDFF_TRY(nl_build_from(c, c->cx, c->cy, c->cz, true));
     *rebuilt = 1;
   }
   return MDFF_OK;

@@ -165,3 +165,31 @@ def test_arrays_through_mapped_memory(ncell):
     f = g.engforce()[0]
     assert rel_force_err(f, o.engforce()[0]) < TOL[capi.PREC_FP64]
     assert not np.any(g.get_dipoles()[0])
+
+
+@pytest.mark.parametrize("rc", [3.3, 5.0, 7.0, 9.0])
+@pytest.mark.parametrize("shape", ["perfect", "displaced", "unwrapped", "sheared", "mirrored"])
+def test_pair_sets_over_cell_widths(rc, shape):
+    """Cells of a third, half and all of the cutoff and axes swept whole, in one
+    box of 12.6 x 21.1 x 37.9 A; ions on cell boundaries, far outside the box, a
+    box that is not orthogonal and one with a negative axis."""
+    s = configs.mgo_pim(cells=(3, 5, 9), rcut=rc, kmax=2, skin=0.4, sigma=0.0 if shape == "perfect" else 0.1)
+    A = np.array(s.desc.cell[:]).reshape(3, 3, order="F")
+    if shape == "unwrapped":
+        s.pos = s.pos + (np.random.default_rng(4).integers(-3, 4, s.pos.shape) @ A.T)
+    elif shape == "sheared":
+        m = np.array([[1.0, 0.18, -0.07], [0.0, 1.0, 0.11], [0.0, 0.0, 1.0]])
+        s.desc.cell[:] = list((m @ A).reshape(-1, order="F"))
+        s.pos = s.pos @ m.T
+    elif shape == "mirrored":
+        m = np.diag([1.0, -1.0, 1.0])
+        s.desc.cell[:] = list((A @ m).reshape(-1, order="F"))
+        s.pos = s.pos @ m
+    note(f"pair sets rc {rc} {shape}")
+    g, o = pair(s)
+    g.vnlist_build()
+    o.vnlist_build()
+    for which in (0, 1):
+        (pg, lg), (po, lo) = g.get_pairs(which), o.get_pairs(which)
+        assert np.array_equal(pg, po) and np.array_equal(lg, lo)
+        assert lg.size > 0
