@@ -276,8 +276,8 @@ struct mdff_ctx {
   int chk_seq_wait = 0;
   double chk_seq = 0.0;
   double* red_part = nullptr;             // reduction block partials
-  double* scf_part = nullptr;             // block partials of a dipole iteration's two sums
-  double* h_scf = nullptr;                // mapped pinned host memory: those sums and their sequence number
+  double* mu_next = nullptr;              // the next dipole iteration's mu_ind (3n)
+  double* h_scf = nullptr;                // mapped pinned host memory: a dipole iteration's sums, a slot a block
   double* d_scf = nullptr;                // its device address
   double scf_seq = 0.0;
   double* h_io = nullptr;                 // mapped pinned host memory: sequence word, kIoMax results, kIoMax inputs

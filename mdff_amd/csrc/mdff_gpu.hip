@@ -184,18 +184,29 @@ __global__ void k_upol(int n, const double* __restrict__ invpol, const double* _
   upol[i] = u;
 }
 
-// One SCF iteration is two of these small kernels around the two field sums
-// (real space beside the reciprocal chain).  An iteration of few ions is bound
-// by launches and waits: 12 small launches and two copies with a wait each took
-// 40 us of it; now four and one wait on a word in host memory (216 ions
-// converged 2432 -> 2114 us FP64, 2073 -> 1662 mixed; 1,440 ions 3094 -> 2645
-// and 2499 -> 2109).
-// Start of an iteration: mu = alpha E (induced_moment; or, INDUCE = false, the
-// predicted mu as it is) and the block partials of mu.alpha^-1.mu.
+// An SCF iteration ends in one small kernel after the two field sums; it also
+// starts the next (mu = alpha E) and hands the host its sums, a block a slot of
+// mapped memory: residual, mu.alpha^-1.mu of the next mu, sequence number, and
+// that sum of the first mu.  An iteration of few ions is bound by its launches
+// and waits (converged MgO, 216 ions FP64: 2432 us with 12 small launches and
+// two copies with a wait each, 1225 with four, the real-space field on a second
+// stream and one wait, now 770; 1,440 ions 3094, 1516, 1135).
+constexpr int kScfSlot = 4;
+
+// mu.alpha^-1.mu of one ion
+__device__ __forceinline__ double scf_upol(const double* ip, const double m[3]) {
+  double u = 0.0;
+  for (int a = 0; a < 3; ++a)
+    for (int b = 0; b < 3; ++b) u = u + m[a] * ip[a + 3 * b] * m[b];
+  return u;
+}
+
+// The first mu: alpha E (induced_moment; or, INDUCE = false, the predicted mu
+// as it is), and the sums of mu.alpha^-1.mu.
 template <bool INDUCE>
 __global__ void __launch_bounds__(256) k_scf_begin(int n, const double* __restrict__ pol,
                                                    const double* __restrict__ invpol, const double* __restrict__ E,
-                                                   double* __restrict__ mu, double* __restrict__ part) {
+                                                   double* __restrict__ mu, double* __restrict__ slot) {
   __shared__ double sh[4 * kRedMaxCols];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   double v[kRedMaxCols] = {};
@@ -212,36 +223,34 @@ __global__ void __launch_bounds__(256) k_scf_begin(int n, const double* __restri
     } else {
       for (int a = 0; a < 3; ++a) m[a] = mu[3 * i + a];
     }
-    const double* ip = invpol + 9 * (size_t)i;
-    double u = 0.0;
-    for (int a = 0; a < 3; ++a)
-      for (int b = 0; b < 3; ++b) u = u + m[a] * ip[a + 3 * b] * m[b];
-    v[0] = u;
+    v[0] = scf_upol(invpol + 9 * (size_t)i, m);
   }
   const double r = block_sum_cols(v, 1, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = r;
+  if (threadIdx.x == 0) slot[kScfSlot * blockIdx.x + 3] = r;
 }
 
 // End of an iteration: E = E_stat + E_ind, E_ind = real space + reciprocal
 // (from the moments, rec_final_field) + surface + self term of mu; correct:
-// mu = aspc alpha E + (1 - aspc) mu (:579-583); then the block
-// partials of the residual (mu / alpha - E)^2 (get_rmsd_mu, :998-1027).
+// mu = aspc alpha E + (1 - aspc) mu (:579-583); the sums of the residual
+// (mu / alpha - E)^2 (get_rmsd_mu, :998-1027); and the next mu.
 struct ScfEndArgs {
   int n, lsurf;
   RecFinal rf;
-  const double *edir, *estat, *pol;
+  const double *edir, *estat, *pol, *invpol;
   const int32_t* polar;
   int correct;                   // the ASPC corrector with weight aspc
   double self2, fpi_3V, aspc;
   const double* mom;             // device moments (lsurf)
-  double *mu, *E, *part;
+  double *mu, *E, *next;
+  double* slot;
+  double seq;
 };
 __global__ void __launch_bounds__(256) k_scf_end(ScfEndArgs a) {
   __shared__ double sh[4 * kRedMaxCols];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   double v[kRedMaxCols] = {};
   if (i < a.n) {
-    double s[9], g[3], er[3], E[3], m[3];
+    double s[9], g[3], er[3], E[3], m[3], t[3];
     rec_final_moments(a.rf, i, s, g);
     rec_final_field(a.rf, g, er);
     for (int k = 0; k < 3; ++k) {
@@ -253,19 +262,18 @@ __global__ void __launch_bounds__(256) k_scf_end(ScfEndArgs a) {
       a.E[3 * i + k] = E[k];
     }
     const double* p = a.pol + 9 * (size_t)i;
-    if (a.correct) {
-      const double w = a.aspc;
-      double t[3];
-      for (int k = 0; k < 3; ++k) {
-        double x = 0.0;
-        for (int b = 0; b < 3; ++b) x = x + p[k + 3 * b] * E[b];
-        t[k] = w * x + (1.0 - w) * m[k];
-      }
-      for (int k = 0; k < 3; ++k) {
-        m[k] = t[k];
-        a.mu[3 * i + k] = t[k];
-      }
+    for (int k = 0; k < 3; ++k) {
+      double x = 0.0;
+      for (int b = 0; b < 3; ++b) x = x + p[k + 3 * b] * E[b];
+      t[k] = x;
+      a.next[3 * i + k] = x;
     }
+    v[1] = scf_upol(a.invpol + 9 * (size_t)i, t);
+    if (a.correct)
+      for (int k = 0; k < 3; ++k) {
+        m[k] = a.aspc * t[k] + (1.0 - a.aspc) * m[k];
+        a.mu[3 * i + k] = m[k];
+      }
     if (a.polar[i])
       for (int k = 0; k < 3; ++k) {
         const double pk = p[k + 3 * k];
@@ -274,25 +282,14 @@ __global__ void __launch_bounds__(256) k_scf_end(ScfEndArgs a) {
         v[0] = v[0] + x * x;
       }
   }
-  const double r = block_sum_cols(v, 1, sh);
-  if (threadIdx.x == 0) a.part[blockIdx.x] = r;
-}
-
-// both sums of an iteration to the host: out[0] = sum pu, out[1] = sum pr
-// (mapped memory), then the sequence number the host waits for
-__global__ void __launch_bounds__(256) k_scf_sums(int nb, const double* __restrict__ pu, const double* __restrict__ pr,
-                                                  double* __restrict__ out, double seq) {
-  __shared__ double sh[4 * kRedMaxCols];
-  __shared__ double tot[2];
-  sum_block_partials(nb, 1, pu, tot, sh);
-  sum_block_partials(nb, 1, pr, tot + 1, sh);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    out[0] = tot[0];
-    out[1] = tot[1];
+  const double r = block_sum_cols(v, 2, sh);
+  double* o = a.slot + kScfSlot * blockIdx.x;
+  if (threadIdx.x < 2) {
+    o[threadIdx.x] = r;
     __threadfence_system();
-    out[2] = seq;
   }
+  __syncthreads();
+  if (threadIdx.x == 0) *reinterpret_cast<volatile double*>(o + 2) = a.seq;
 }
 
 // ASPC predictor (src/moment_from_pola.f90:566-575) and history shift
@@ -912,6 +909,7 @@ static int ctx_init(mdff_ctx* c, const mdff_desc* d, const int32_t* itype) {
   DMALLOC(c->dipia, 3 * (size_t)n);
   DMALLOC(c->mu, 3 * (size_t)n);
   DMALLOC(c->mu_ind, 3 * (size_t)n);
+  DMALLOC(c->mu_next, 3 * (size_t)n);
   DMALLOC(c->efield, 3 * (size_t)n);
   DMALLOC(c->e_stat, 3 * (size_t)n);
   DMALLOC(c->e_tot, 3 * (size_t)n);
@@ -959,15 +957,17 @@ static int ctx_init(mdff_ctx* c, const mdff_desc* d, const int32_t* itype) {
   HIP_TRY(c, hipEventCreateWithFlags(&c->ov_tab, hipEventDisableTiming));
   HIP_TRY(c, hipEventCreateWithFlags(&c->ov_pair, hipEventDisableTiming));
   {
-    // MDFF_PAIR_OVERLAP=0 keeps every kernel on the one stream
+    // MDFF_PAIR_OVERLAP=0 keeps every kernel on the one stream, =1 overlaps
+    // them at any size.  The events cost some 10 us, which a short pair kernel
+    // does not hide (us a step, overlapped / in line: NaCl 512 67/65, silica
+    // 648 92/85, 3,000 100/104, NaCl 4,096 118/123, silica 24,000 232/239)
     const char* ov = getenv("MDFF_PAIR_OVERLAP");
-    c->overlap = (ov && ov[0] == '0') ? 0 : 1;
+    c->overlap = ov && ov[0] ? ov[0] != '0' : n > 2048;
   }
   HIP_TRY(c, hipHostMalloc((void**)&c->h_flag, sizeof(int32_t) * 4));
   const size_t nred = std::max<size_t>(64 * 1024, 2 * (size_t)nblk(n) + 2);
   HIP_TRY(c, hipHostMalloc((void**)&c->h_red, sizeof(double) * nred));
   DMALLOC(c->red_part, nred);
-  DMALLOC(c->scf_part, 2 * (size_t)nblk(n));
   HIP_TRY(c, hipHostMalloc((void**)&c->h_nl, sizeof(double) * 2, hipHostMallocMapped | hipHostMallocCoherent));
   HIP_TRY(c, hipHostGetDevicePointer((void**)&c->d_nl, c->h_nl, 0));
   c->h_nl[0] = c->h_nl[1] = 0.0;
@@ -975,9 +975,9 @@ static int ctx_init(mdff_ctx* c, const mdff_desc* d, const int32_t* itype) {
   HIP_TRY(c, hipHostMalloc((void**)&c->h_io, sizeof(double) * (8 + 2 * kIoMax), hipHostMallocMapped | hipHostMallocCoherent));
   HIP_TRY(c, hipHostGetDevicePointer((void**)&c->d_io, c->h_io, 0));
   c->h_io[0] = 0.0;
-  HIP_TRY(c, hipHostMalloc((void**)&c->h_scf, sizeof(double) * 4, hipHostMallocMapped | hipHostMallocCoherent));
+  HIP_TRY(c, hipHostMalloc((void**)&c->h_scf, sizeof(double) * kScfSlot * (size_t)nblk(n), hipHostMallocMapped | hipHostMallocCoherent));
   HIP_TRY(c, hipHostGetDevicePointer((void**)&c->d_scf, c->h_scf, 0));
-  memset(c->h_scf, 0, sizeof(double) * 4);
+  memset(c->h_scf, 0, sizeof(double) * kScfSlot * (size_t)nblk(n));
   DMALLOC(c->red, 64);
   DMALLOC(c->fin_part, 1024 * 16 + (size_t)nblk(n) + 16);
   DMALLOC(c->nhc_part, 2 * (size_t)nblk(n));
@@ -1085,39 +1085,30 @@ static int scf(mdff_ctx* c, mdff_terms* t) {
   const int nb = nblk(n);
   const double alpha2 = c->alpha * c->alpha;
   const double selfa = c->alpha / sqrt(MDFF_PI), selfa2 = 2.0 * selfa * alpha2 / 3.0;
-  double* pu = c->scf_part;        // block partials: mu.alpha^-1.mu, then the residual
-  double* pr = c->scf_part + nb;
-  while ((iscf < d.max_scf_pol_iter && rmsd > d.conv_tol_ind) || iscf < d.min_scf_pol_iter) {
+  double unext = 0.0;            // mu.alpha^-1.mu of the next mu
+  bool again = (iscf < d.max_scf_pol_iter && rmsd > d.conv_tol_ind) || iscf < d.min_scf_pol_iter;
+  while (again) {
     iscf++;
     const bool predict = iscf == 1 && d.calc_md;
     if (predict)
       hipLaunchKernelGGL(k_aspc_predict, dim3(div_up(n3, 256)), dim3(256), 0, c->stream, n3, ext, Bc[0], Bc[1],
                          Bc[2], Bc[3], Bc[4], c->hist, c->mu_ind);
-    hipLaunchKernelGGL(predict ? &k_scf_begin<false> : &k_scf_begin<true>, dim3(nb), dim3(256), 0, c->stream, n, c->pol,
-                       c->invpol, c->e_tot, c->mu_ind, pu);
-    // the real-space field beside the reciprocal sums (both read mu only);
-    // off with MDFF_PAIR_OVERLAP=0 and while the event profiler runs
-    const bool ov = c->overlap && !c->prof_on;
-    hipStream_t s0 = c->stream;
-    if (ov) {
-      HIP_TRY(c, hipEventRecord(c->ov_tab, c->stream));
-      HIP_TRY(c, hipStreamWaitEvent(c->stream2, c->ov_tab, 0));
-      c->stream = c->stream2;
-    }
-    const int rc = realspace_field(c, 1, c->mu_ind, ef_dir(c));
-    c->stream = s0;
-    MDFF_TRY(rc);
-    if (ov) HIP_TRY(c, hipEventRecord(c->ov_pair, c->stream2));
+    if (iscf == 1)
+      hipLaunchKernelGGL(predict ? &k_scf_begin<false> : &k_scf_begin<true>, dim3(nb), dim3(256), 0, c->stream, n, c->pol,
+                         c->invpol, c->e_tot, c->mu_ind, c->d_scf);
+    // (beside the reciprocal sums on a second stream the field costs more in
+    // events than it hides: 216 ions 1225 us and 875 in line, 12,000 3329 and 3157)
+    MDFF_TRY(realspace_field(c, 1, c->mu_ind, ef_dir(c)));
     ScfEndArgs a{};
     MDFF_TRY(recip_moments(c, c->mu_ind, &a.rf));
     a.mom = c->raw + RAW_SCRATCH;
     if (d.lsurf) MDFF_TRY(moments_dev(c, c->q, c->mu_ind, c->raw + RAW_SCRATCH));
-    if (ov) HIP_TRY(c, hipStreamWaitEvent(c->stream, c->ov_pair, 0));
     a.n = n;
     a.lsurf = d.lsurf;
     a.edir = ef_dir(c);
     a.estat = c->e_stat;
     a.pol = c->pol;
+    a.invpol = c->invpol;
     a.polar = polar;
     a.self2 = 2.0 * selfa2;
     a.fpi_3V = 2.0 * (2.0 * MDFF_PI / c->omega / 3.0);
@@ -1125,22 +1116,33 @@ static int scf(mdff_ctx* c, mdff_terms* t) {
     a.aspc = w;
     a.mu = c->mu_ind;
     a.E = c->e_tot;
-    a.part = pr;
+    a.next = c->mu_next;
+    a.slot = c->d_scf;
+    a.seq = c->scf_seq += 1.0;
     hipLaunchKernelGGL(k_scf_end, dim3(nb), dim3(256), 0, c->stream, a);
-    c->scf_seq += 1.0;
-    hipLaunchKernelGGL(k_scf_sums, dim3(1), dim3(256), 0, c->stream, nb, pu, pr, c->d_scf, c->scf_seq);
     HIP_TRY(c, hipGetLastError());
-    // wait for the sequence number; a launch that never reports is caught by
-    // the stream
+    // wait for every block's sequence number; a launch that never reports is
+    // caught by the stream
     volatile const double* h = c->h_scf;
-    bool seen = false;
-    for (long k = 0; k < 20000000L && !seen; ++k) seen = h[2] == c->scf_seq;
-    if (!seen) {
-      HIP_TRY(c, hipStreamSynchronize(c->stream));
-      if (h[2] != c->scf_seq) return fail(c, MDFF_ERR_HIP, "dipole iteration signal missing");
+    double res = 0.0, u0 = 0.0, un = 0.0;
+    long spins = 0;
+    for (int b = 0; b < nb; ++b) {
+      const volatile double* o = h + kScfSlot * b;
+      while (o[2] != a.seq && spins < 20000000L) ++spins;
+      if (o[2] != a.seq) {
+        HIP_TRY(c, hipStreamSynchronize(c->stream));
+        if (o[2] != a.seq) return fail(c, MDFF_ERR_HIP, "dipole iteration signal missing");
+      }
+      std::atomic_thread_fence(std::memory_order_acquire);
+      res += o[0];
+      un += o[1];
+      u0 += o[3];
     }
-    upol = 0.5 * h[0];
-    rmsd = sqrt(h[1] / (double)npol);
+    upol = 0.5 * (iscf == 1 ? u0 : unext);
+    unext = un;
+    rmsd = sqrt(res / (double)npol);
+    again = (iscf < d.max_scf_pol_iter && rmsd > d.conv_tol_ind) || iscf < d.min_scf_pol_iter;
+    if (again) std::swap(c->mu_ind, c->mu_next);
   }
   HIP_TRY(c, hipMemcpyAsync(c->hist, c->mu_ind, sizeof(double) * n3, hipMemcpyDeviceToDevice, c->stream));
   t->u_pol = upol;
@@ -1693,7 +1695,7 @@ int mdff_ctx_destroy(mdff_ctx* c) {
                 c->hist, c->frec, c->zeros, c->arec, c->ameta, c->peratom, c->red, c->red_part, c->d_pp, c->cell_of, c->cell_slot, c->cell_cnt,
                 c->cell_atoms, c->cell_atoms_in, c->cell_start, c->nl_count, c->nl_start, c->nl_j,
                 c->nl_flag, c->nl_count_in, c->nl_j_tmp, c->nl_flag_tmp, c->sort_tmp, c->d_flag, c->raw,
-                c->cx, c->cy, c->cz, c->fin_part, c->nhc_part, c->nhc_st, c->peratom_lj, c->f_lj, c->lj_part, c->scf_part};
+                c->cx, c->cy, c->cz, c->fin_part, c->nhc_part, c->nhc_st, c->peratom_lj, c->f_lj, c->lj_part, c->mu_next};
   for (void* p : ps)
     if (p) (void)hipFree(p);
   if (c->polar) (void)hipFree(c->polar);
@@ -1883,9 +1885,10 @@ int mdff_md_vv(mdff_ctx* c, int32_t nsteps, double dt, double* ekin, double* upo
       st0 = st + 1;
     }
   }
+  // (the sums have come back behind everything else the stream held)
   int rb = 0;
   MDFF_TRY(nl_check_finish(c, &rb));
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  if (rb) HIP_TRY(c, hipStreamSynchronize(c->stream));
   return MDFF_OK;
 }
 
