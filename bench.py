@@ -52,7 +52,7 @@ BOUND_OF = {"k_sk": ("mfma", "fp64"), "k_gather": ("valu", "fp64"), "k_pair_forc
 # WRITE_SIZE x 0.996 (KiB per dispatch x 1024; the factors calibrate the
 # counters on a 256 MiB device-to-device copy), measured with
 # mdff_amd.profile_workload (profiles/engforce_sio2_24k_hbm_traffic.md)
-TRAFFIC = {"k_pair_force": 63.92e6}
+TRAFFIC = {"k_pair_force": 63.39e6, "k_sk": 32.49e6, "k_gather": 8.48e6}
 
 
 NKINDS = 8  # kernel classes of the library's event profiler (mdff_profile_name)
@@ -251,18 +251,19 @@ def fit_leg(nsnap: int, reps: int) -> dict:
     # operator application (SCF and adjoint iterations) and the four other
     # passes (static field, forces, h, its reciprocal part), at the
     # structure-factor and gather figures of the engforce (11 + 10 flops per
-    # (k, atom)); pairs left out (under a tenth of the work).  FP32 VALU peak.
+    # (k, atom)); pairs left out (under a tenth of the work).  FP64 matrix peak
+    # (the iterations' reciprocal field runs there in both forms).
     def nk_of(k):
         return k[2] + k[1] * (2 * k[2] + 1) + k[0] * (2 * k[1] + 1) * (2 * k[2] + 1)
     nkn = np.array([s.natm * nk_of(list(s.desc.kES)) for s in snaps], float)
     passes = r32.nscf[:, 0] + r32.nscf[:, 1] + 4
     fit_flops = float(np.sum(passes * nkn) * 21.0)
-    fit_roof = {"kernel": "kf_* phase kernels (FP32)", "bound": "valu", "achieved": round(fit_flops / sec / 1e12, 3),
-                "peak": PEAK["fp32"], "unit": "TFLOP/s", "frac": round(fit_flops / sec / 1e12 / PEAK["fp32"], 4),
+    fit_roof = {"kernel": "kf_* phase kernels (iterations: kf_sk, kf_moments)", "bound": "mfma", "achieved": round(fit_flops / sec / 1e12, 3),
+                "peak": PEAK["fp64"], "unit": "TFLOP/s", "frac": round(fit_flops / sec / 1e12 / PEAK["fp64"], 4),
                 "algorithmic_flops_per_launch": fit_flops, "flops_per_unit": 21.0,
                 "units_per_launch": float(np.sum(passes * nkn)), "traffic": None,
                 "note": "phase launches over (snapshot, block of atoms or k-vectors); launches per "
-                        "evaluation: 12 + 5 per SCF or adjoint iteration of the slowest snapshot"}
+                        "evaluation: 22 + 7 per SCF or adjoint iteration of the slowest snapshot"}
     return {"metric": "fit-gradients/s", "value": round(1.0 / sec, 3), "seconds_per_gradient": sec,
             "roofline": fit_roof,
             "fp64_seconds_per_gradient": sec64, "snapshots": nsnap, "ions": natm,
