@@ -648,20 +648,29 @@ PairArgs make_args(mdff_ctx* c) {
   return a;
 }
 
-// Lanes of an atom's group.  Force rows: 16, but 32 for few atoms, whose 16
-// would leave SIMDs with a wave each (4,000 LJ atoms: 81 against 103 us a step;
-// from 5,000 atoms on 16 is as good, at 24,000 better: 312 against 317, with 64
-// lanes 332).  Field rows: 64, a wave an atom, while that fills the chip (a
-// converged 12,000-ion MgO evaluation 4.2 against 4.4 ms, 1,440 ions 2.5
-// against 2.9).
-inline int force_lanes(int n) { return n < 4608 ? 32 : 16; }
+// Lanes of an atom's group.  Force rows: 16, more where that would leave the
+// SIMDs with a wave or two: 64 below 2,048 atoms, 32 below 4,608, and 32 to
+// 16,384 where a row is long (us a step with 16, 32, 64 lanes: LJ 864 87/69/60,
+// silica 648 95/85/80, 3,000 110/103/102, LJ 4,000 101/78/79, NaCl 4,096
+// 118/118/123, LJ 8,788 (1,100 in a row) 123/115/114, silica 8,232 174/175/179).
+// By the mean row of the cell's density, so that it is the same in every run.
+// Field rows: 64, a wave an atom, while that fills the chip (a converged
+// 12,000-ion MgO evaluation 4.2 against 4.4 ms, 1,440 ions 2.5 against 2.9).
+inline int force_lanes(const mdff_ctx* c) {
+  const double r = std::max(c->rc_vdw, c->rc_coul) + c->d.skindiff;
+  const double row = 4.0 / 3.0 * MDFF_PI * r * r * r * c->n / c->omega;
+  if (c->n < 2048) return 64;
+  return c->n < 4608 || (c->n < 16384 && row > 700.0) ? 32 : 16;
+}
 inline int field_lanes(int n) { return n < 32768 ? 64 : 16; }
 
 template <typename T, bool DIP, int SRM>
 void launch_force_lanes(mdff_ctx* c, const PairArgs& a) {
-  const int lpa = force_lanes(c->n);
+  const int lpa = force_lanes(c);
   const dim3 grid(div_up((int64_t)c->n * lpa, 256));
-  if (lpa == 32)
+  if (lpa == 64)
+    PROF_LAUNCH(c, PK_PAIR, hipLaunchKernelGGL((k_pair_force<T, DIP, 64, SRM>), grid, dim3(256), 0, c->stream, a));
+  else if (lpa == 32)
     PROF_LAUNCH(c, PK_PAIR, hipLaunchKernelGGL((k_pair_force<T, DIP, 32, SRM>), grid, dim3(256), 0, c->stream, a));
   else
     PROF_LAUNCH(c, PK_PAIR, hipLaunchKernelGGL((k_pair_force<T, DIP, 16, SRM>), grid, dim3(256), 0, c->stream, a));

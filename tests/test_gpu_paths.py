@@ -38,10 +38,11 @@ def test_lj_exponents(p, q, prec):
 
 
 @PRECS
-@pytest.mark.parametrize("ncell", [10, 11])
-def test_lj_lanes(ncell, prec):
-    """4,000 and 5,324 atoms: 32 and 16 lanes an atom."""
-    s = _lj(ncell)
+@pytest.mark.parametrize("ncell,rc", [(7, 2.5), (10, 2.5), (11, 2.5), (11, 5.4)])
+def test_lj_lanes(ncell, rc, prec):
+    """1,372, 4,000 and 5,324 atoms, the last with short and long rows: 64, 32,
+    16 and 32 lanes an atom."""
+    s = _lj(ncell, rc=rc)
     note(f"lj n={s.natm}")
     g, o = pair(s, precision=prec)
     assert rel_force_err(g.engforce()[0], o.engforce()[0]) < TOL[prec]
