@@ -1086,6 +1086,7 @@ static int scf(mdff_ctx* c, mdff_terms* t) {
   const double alpha2 = c->alpha * c->alpha;
   const double selfa = c->alpha / sqrt(MDFF_PI), selfa2 = 2.0 * selfa * alpha2 / 3.0;
   double unext = 0.0;            // mu.alpha^-1.mu of the next mu
+  bool field_queued = false;
   bool again = (iscf < d.max_scf_pol_iter && rmsd > d.conv_tol_ind) || iscf < d.min_scf_pol_iter;
   while (again) {
     iscf++;
@@ -1098,7 +1099,7 @@ static int scf(mdff_ctx* c, mdff_terms* t) {
                          c->invpol, c->e_tot, c->mu_ind, c->d_scf);
     // (beside the reciprocal sums on a second stream the field costs more in
     // events than it hides: 216 ions 1225 us and 875 in line, 12,000 3329 and 3157)
-    MDFF_TRY(realspace_field(c, 1, c->mu_ind, ef_dir(c)));
+    if (!field_queued) MDFF_TRY(realspace_field(c, 1, c->mu_ind, ef_dir(c)));
     ScfEndArgs a{};
     MDFF_TRY(recip_moments(c, c->mu_ind, &a.rf));
     a.mom = c->raw + RAW_SCRATCH;
@@ -1121,6 +1122,12 @@ static int scf(mdff_ctx* c, mdff_terms* t) {
     a.seq = c->scf_seq += 1.0;
     hipLaunchKernelGGL(k_scf_end, dim3(nb), dim3(256), 0, c->stream, a);
     HIP_TRY(c, hipGetLastError());
+    // the next iteration's real-space field, before the host has seen whether
+    // there is one: the device works while the host waits, decides and queues
+    // the rest (the last one is of no use; 216 ions 770 -> 707 us, 1,440 1135 ->
+    // 1042, 12,000 3010 -> 2960)
+    field_queued = iscf < d.max_scf_pol_iter;
+    if (field_queued) MDFF_TRY(realspace_field(c, 1, c->mu_next, ef_dir(c)));
     // wait for every block's sequence number; a launch that never reports is
     // caught by the stream
     volatile const double* h = c->h_scf;
