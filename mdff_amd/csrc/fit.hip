@@ -187,6 +187,38 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
   return r;
 }
 
+// v[0..n) of each atom's L lanes added in lane order, in its first lane's v; lx:
+// 256 n doubles of LDS.  Called by the whole block of 256 threads.
+__device__ __forceinline__ void lane_sums(double* v, int n, int L, double* lx) {
+  const int t = threadIdx.x;
+  for (int c = 0; c < n; ++c) lx[256 * c + t] = v[c];
+  __syncthreads();
+  if ((t & (L - 1)) == 0)
+    for (int c = 0; c < n; ++c) {
+      double r = 0.0;
+      for (int l = 0; l < L; ++l) r += lx[256 * c + t + l];
+      v[c] = r;
+    }
+  __syncthreads();
+}
+
+// out[c] = sums over the block's 256 threads of the n <= 32 values lx[256 c + t]
+__device__ __forceinline__ void slot_sums(int n, double* lx, double* out) {
+  const int t = threadIdx.x, slot = t >> 3, part = t & 7;
+  __syncthreads();
+  double r = 0.0;
+  if (slot < n)
+    for (int k = 0; k < 32; ++k) r += lx[256 * slot + part + 8 * k];
+  __syncthreads();
+  if (slot < n) lx[256 * slot + part] = r;
+  __syncthreads();
+  if (t < n) {
+    double v = 0.0;
+    for (int k = 0; k < 8; ++k) v += lx[256 * t + k];
+    out[t] = v;
+  }
+}
+
 // Tang-Toennies f, f' and their derivatives with respect to b and c
 // (f = 1 - c e^{-x} sum_{k<=K} x^k/k!, x = b r; d f/d b = r f'/b,
 // d f'/d b = f' (1 + K - x)/b, d f/d c = (f - 1)/c, d f'/d c = f'/c)
@@ -494,7 +526,7 @@ __device__ void gather(const FitSnap& S, const c2<T>* tab, int j, int nkl, bool 
 // an atom from atom ib0 of the snapshot, plus
 // the lambda . dE_stat/d(b, c) gradient terms when lam != nullptr
 template <typename T>
-__device__ void field_static(const FitArgs& a, const FitSnap& S, int ib0, int L, double* Es, const double* lam,
+__device__ void field_static(const FitArgs& a, const FitSnap& S, int ib0, int L, double* lx, double* Es, const double* lam,
                              double* gacc) {
   const double* sx = a.sx + S.a0;
   const double* sy = a.sy + S.a0;
@@ -504,6 +536,7 @@ __device__ void field_static(const FitArgs& a, const FitSnap& S, int ib0, int L,
   const T alpha = (T)S.alpha;
   const int sub = (int)threadIdx.x & (L - 1);
   const int i = ib0 + (int)threadIdx.x / L;
+  double ev[3] = {0, 0, 0};
   if (i < S.n) {
     double e0 = 0, e1 = 0, e2 = 0;
     const int ti = it[i];
@@ -532,18 +565,14 @@ __device__ void field_static(const FitArgs& a, const FitSnap& S, int ib0, int L,
         e2 += (double)(gg * (T)G.rz);
       }
     }
-    if (Es) {
-      for (int w = 1; w < L; w <<= 1) {
-        e0 += __shfl_xor(e0, w);
-        e1 += __shfl_xor(e1, w);
-        e2 += __shfl_xor(e2, w);
-      }
-    }
-    if (Es && sub == 0) {
-      Es[3 * i] = e0;
-      Es[3 * i + 1] = e1;
-      Es[3 * i + 2] = e2;
-    }
+    ev[0] = e0;
+    ev[1] = e1;
+    ev[2] = e2;
+  }
+  if (Es) {
+    lane_sums(ev, 3, L, lx);
+    if (sub == 0 && i < S.n)
+      for (int c = 0; c < 3; ++c) Es[3 * i + c] = ev[c];
   }
 }
 
@@ -552,7 +581,7 @@ __device__ void field_static(const FitArgs& a, const FitSnap& S, int ib0, int L,
 // rows of polarisable neighbours only, L lanes an atom (a power of two)
 template <typename T>
 __device__ void field_dip_real(const FitArgs& a, const FitSnap& S, const FitBox& X, int p0, int L, const double* v,
-                               double* out) {
+                               double* out, double* lx) {
   const double* sx = a.sx + S.a0;
   const double* sy = a.sy + S.a0;
   const double* sz = a.sz + S.a0;
@@ -578,16 +607,10 @@ __device__ void field_dip_real(const FitArgs& a, const FitSnap& S, const FitBox&
       e2 += (double)(c3 * rz - c1 * vz);
     }
   }
-  for (int w = 1; w < L; w <<= 1) {
-    e0 += __shfl_xor(e0, w);
-    e1 += __shfl_xor(e1, w);
-    e2 += __shfl_xor(e2, w);
-  }
-  if (on && sub == 0) {
-    out[3 * i] = e0;
-    out[3 * i + 1] = e1;
-    out[3 * i + 2] = e2;
-  }
+  double ev[3] = {e0, e1, e2};
+  lane_sums(ev, 3, L, lx);
+  if (on && sub == 0)
+    for (int c = 0; c < 3; ++c) out[3 * i + c] = ev[c];
 }
 
 // ---------------------------------------------------------------------------
@@ -598,7 +621,7 @@ __device__ void field_dip_real(const FitArgs& a, const FitSnap& S, const FitBox&
 // ADJ: h_real (into h), explicit Buckingham and TT gradients (into gacc, LDS
 // of 256 threads a slot).  L lanes an atom, from atom ib0 of the snapshot.
 template <typename T, bool ADJ>
-__device__ void pair_pass(const FitArgs& a, const FitSnap& S, int ib0, int L, const double* mu, const double* gv,
+__device__ void pair_pass(const FitArgs& a, const FitSnap& S, int ib0, int L, double* lx, const double* mu, const double* gv,
                           const double Gs[9], double* Fout, double* h, double* gacc, double st_nonb[6],
                           double st_dir[6]) {
   const double* sx = a.sx + S.a0;
@@ -611,6 +634,7 @@ __device__ void pair_pass(const FitArgs& a, const FitSnap& S, int ib0, int L, co
   const double sgs = 1.0 / (S.omega * a.press_unit);
   const int sub = (int)threadIdx.x & (L - 1);
   const int i = ib0 + (int)threadIdx.x / L;
+  double sums[6] = {0, 0, 0, 0, 0, 0};
   if (i < S.n) {
     const int ti = it[i];
     const T qi = (T)q[i];
@@ -777,23 +801,17 @@ __device__ void pair_pass(const FitArgs& a, const FitSnap& S, int ib0, int L, co
         }
       }
     }
-    // an atom's lanes share the loop bounds' block, so all of them are here
-    for (int w = 1; w < L; w <<= 1)
-      for (int c = 0; c < 3; ++c) {
-        if (!ADJ) {
-          fsr[c] += __shfl_xor(fsr[c], w);
-          fcl[c] += __shfl_xor(fcl[c], w);
-        } else {
-          hh[c] += __shfl_xor(hh[c], w);
-        }
-      }
-    if (sub == 0) {
-      for (int c = 0; c < 3; ++c) {
-        if (!ADJ) Fout[3 * i + c] = fsr[c] + cu * fcl[c];
-        else h[3 * i + c] = hh[c];
-      }
+    for (int c = 0; c < 3; ++c) {
+      sums[c] = ADJ ? hh[c] : fsr[c];
+      sums[3 + c] = fcl[c];
     }
   }
+  lane_sums(sums, ADJ ? 3 : 6, L, lx);
+  if (sub == 0 && i < S.n)
+    for (int c = 0; c < 3; ++c) {
+      if (!ADJ) Fout[3 * i + c] = sums[c] + cu * sums[3 + c];
+      else h[3 * i + c] = sums[c];
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -819,9 +837,10 @@ __device__ __forceinline__ void block_partials(double* v, int n, double* red, do
 // static field of the charges (real space, damped) at the block's atoms
 template <typename T>
 __global__ void __launch_bounds__(256) kf_static(FitArgs a) {
+  extern __shared__ double red[];
   const int4 B = a.pblk[blockIdx.x];
   const FitSnap S = a.snaps[B.x];
-  field_static<T>(a, S, B.y, a.planes, ws_of(a, S, W_ES), nullptr, nullptr);
+  field_static<T>(a, S, B.y, a.planes, red, ws_of(a, S, W_ES), nullptr, nullptr);
 }
 
 // dst = alpha src at the block's atoms, for snapshots still iterating
@@ -841,12 +860,17 @@ __global__ void __launch_bounds__(256) kf_update(FitArgs a) {
 // real-space dipole field of v = ws[slot] into ws[W_TMP] (iterating snapshots)
 template <typename T>
 __global__ void __launch_bounds__(256) kf_dipreal(FitArgs a, int slot) {
-  const int4 B = a.dblk[xcd_order(blockIdx.x, gridDim.x)];
+  extern __shared__ double red[];
+  const int4 B = a.dblk[blockIdx.x];
   if (!a.active[B.x]) return;
   const FitSnap S = a.snaps[B.x];
-  field_dip_real<T>(a, S, a.boxes[B.x], B.y, a.dlanes, ws_of(a, S, slot), ws_of(a, S, W_TMP));
+  field_dip_real<T>(a, S, a.boxes[B.x], B.y, a.dlanes, ws_of(a, S, slot), ws_of(a, S, W_TMP), red);
 }
 
+constexpr int kSkTile = 32;      // ions of a staged tile of kf_sk
+constexpr int kSkRows = 4;       // row tiles (8 nz) of its blocks at most
+
+#ifdef __HIPCC__   // (the kernels' host build for the tests goes without)
 // ---------------------------------------------------------------------------
 // Reciprocal field of the iterations on the FP64 matrix cores, in both forms.
 // A thread a k (or an atom) over phase products was 75 % of a gradient: 404
@@ -865,9 +889,6 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ f64x4 mfma(double a, double b, f64x4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
-
-constexpr int kSkTile = 32;      // ions of a staged tile
-constexpr int kSkRows = 4;       // row tiles (8 nz) a block at most
 
 // RT row tiles from nz index zoff, 64 columns m (16 a wave), one chunk of
 // ions: B = (snapshot, first m, chunk, first nz index)
@@ -1127,6 +1148,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LONG ? 
   }
 }
 
+#endif
+
 // structure factors of the block's k-vectors and their per-k follow-ups.
 // mode 0: q -> K_SQ, C1 = A S; 1: i k.v -> K_S, C1 = A S (iterating
 // snapshots only); 2: q + i k.mu -> K_S, C1 = A S and the reciprocal stress
@@ -1368,26 +1391,6 @@ __global__ void __launch_bounds__(256) kf_gather(FitArgs a, int vslot, int bslot
   if (PH != PH_STATIC) block_partials(&part, 1, red, a.pa + (size_t)FIT_PA * blockIdx.x + (PH == PH_FORCE ? 12 : 0));
 }
 
-// v of a wave's lanes summed
-__device__ __forceinline__ double wave_sum(double v) {
-  for (int w = 1; w < 64; w <<= 1) v += __shfl_xor(v, w);
-  return v;
-}
-
-// out[c] = sums over the block's 256 threads of n values each, get(c)
-template <typename F>
-__device__ __forceinline__ void pass_partials(int n, F get, double* out) {
-  __shared__ double part[4][FIT_MAXP];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int c = 0; c < n; ++c) {
-    const double r = wave_sum(get(c));
-    if (lane == 0) part[wave][c] = r;
-  }
-  __syncthreads();
-  if ((int)threadIdx.x < n)
-    out[threadIdx.x] = part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x];
-}
-
 // pair pass at the block's atoms.  !ADJ: forces (ws-independent) and the
 // real-space stress partials (slots 0..11); ADJ: h (real space, overwritten)
 // and the explicit gradient partials (a slot a parameter).  Bound by the
@@ -1404,18 +1407,13 @@ __global__ void __launch_bounds__(256) kf_pair(FitArgs a) {
   double* out = a.pp + (size_t)FIT_MAXP * blockIdx.x;
   if (!ADJ) {
     const double Gdummy[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    pair_pass<T, false>(a, S, B.y, a.planes, ws_of(a, S, W_MU), nullptr, Gdummy, a.F + 3 * (size_t)S.a0, nullptr,
+    pair_pass<T, false>(a, S, B.y, a.planes, red, ws_of(a, S, W_MU), nullptr, Gdummy, a.F + 3 * (size_t)S.a0, nullptr,
                         nullptr, stn, std_);
-    double v[12];
-#pragma unroll
     for (int c = 0; c < 6; ++c) {
-      v[c] = stn[c];
-      v[6 + c] = std_[c];
+      red[256 * c + threadIdx.x] = stn[c];
+      red[256 * (6 + c) + threadIdx.x] = std_[c];
     }
-    pass_partials(12, [&](int c) { double r = 0.0;
-#pragma unroll
-      for (int u = 0; u < 12; ++u) r = u == c ? v[u] : r;
-      return r; }, out);
+    slot_sums(12, red, out);
   } else {
     double* gacc = red + threadIdx.x;
     for (int p = 0; p < a.nparam; ++p) gacc[256 * p] = 0.0;
@@ -1424,9 +1422,9 @@ __global__ void __launch_bounds__(256) kf_pair(FitArgs a) {
     // the non-bonded stress carries 1/press_unit, the Coulomb one coul_unit/press_unit:
     // the pair pass scales its virtual displacement by 1/(omega pu) and the
     // Coulomb terms by coul_unit itself
-    pair_pass<T, true>(a, S, B.y, a.planes, ws_of(a, S, W_MU), ws_of(a, S, W_G), Gs, nullptr, ws_of(a, S, W_H), gacc,
+    pair_pass<T, true>(a, S, B.y, a.planes, red + 256 * a.nparam, ws_of(a, S, W_MU), ws_of(a, S, W_G), Gs, nullptr, ws_of(a, S, W_H), gacc,
                        stn, std_);
-    pass_partials(a.nparam, [&](int c) { return gacc[256 * c]; }, out);
+    slot_sums(a.nparam, red, out);
   }
 }
 
@@ -1451,8 +1449,8 @@ __global__ void __launch_bounds__(256) kf_lambda(FitArgs a) {
       gacc[256 * a.s_alpha[tj]] += lm / (al * al);
     }
   }
-  field_static<T>(a, S, B.y, a.planes, nullptr, vLAM, gacc);
-  pass_partials(a.nparam, [&](int c) { return gacc[256 * c]; }, a.pp + (size_t)FIT_MAXP * blockIdx.x);
+  field_static<T>(a, S, B.y, a.planes, nullptr, nullptr, vLAM, gacc);
+  slot_sums(a.nparam, red, a.pp + (size_t)FIT_MAXP * blockIdx.x);
 }
 
 // the pair passes' partials of a snapshot added in block order, a thread a slot
@@ -1559,7 +1557,9 @@ __global__ void __launch_bounds__(256) kf_ctl(FitArgs a, int what) {
     for (int x = 0; x < (int)blockDim.x; ++x) t += cnt[x];
     if (what == C_SCF || what == C_ADJ) {
       a.h_count[0] = t;
+#ifdef __HIPCC__
       __threadfence_system();
+#endif
       a.h_count[1] = a.seq;
     }
   }
@@ -1833,9 +1833,13 @@ static int fit_iter_setup(mdff_fit* f, const std::vector<int>& it, const std::ve
   const int split = (int)std::max<long long>(1, 6144 / std::max<long long>(waves, 1));
   f->dlanes = waves >= 1024 ? 8 : 32;
   // the gradient passes hold a sum a thread and parameter in LDS (64 KiB at 32)
+#ifdef __HIPCC__
   for (const void* fn : {reinterpret_cast<const void*>(&kf_pair<float, true>), reinterpret_cast<const void*>(&kf_pair<double, true>),
                          reinterpret_cast<const void*>(&kf_lambda<float>), reinterpret_cast<const void*>(&kf_lambda<double>)})
-    FIT_TRY(f, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(double) * 256 * FIT_MAXP));
+    FIT_TRY(f, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(double) * 256 * (FIT_MAXP + 3)));
+#else
+  mma = false;
+#endif
   // lanes an atom of the pair passes: eight waves a SIMD
   while (f->planes < 32 && (long long)f->natm * f->planes < 8192 * 64) f->planes *= 2;
   std::vector<int4> mb, rb, db, pb;
@@ -1892,8 +1896,13 @@ static int fit_iter_setup(mdff_fit* f, const std::vector<int>& it, const std::ve
   FUP(f->d_prow, prow);
   FUP(f->d_pnl, pnl);
   FUP(f->d_dblk, db);
+#ifdef __HIPCC__
   FIT_TRY(f, hipHostMalloc((void**)&f->h_count, 2 * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent));
   FIT_TRY(f, hipHostGetDevicePointer((void**)&f->d_hcount, f->h_count, 0));
+#else
+  FIT_TRY(f, hipMalloc((void**)&f->h_count, 2 * sizeof(double)));
+  f->d_hcount = f->h_count;
+#endif
   f->h_count[0] = f->h_count[1] = 0.0;
   if (!mma) return MDFF_OK;
   FUP(f->d_kbox, kb);
@@ -1942,7 +1951,8 @@ static int fit_run(mdff_fit* f, FitArgs a, size_t tsz) {
       hipLaunchKernelGGL(kf_update, ga, b, 0, st, a);
       // (beside the reciprocal kernels on a second stream: 256 snapshots 17.44 ms
       // and 17.53 in line, 32 FP64 7.42 and 6.74, 4 3.74 and 3.11)
-      if (f->ndb) hipLaunchKernelGGL((kf_dipreal<T>), dim3(f->ndb), dim3(256), 0, st, a, vslot);
+      if (f->ndb) hipLaunchKernelGGL((kf_dipreal<T>), dim3(f->ndb), dim3(256), 3 * 2048, st, a, vslot);
+#ifdef __HIPCC__
       if (a.wbox) {
         if (f->nmb) {
           hipLaunchKernelGGL(kf_sk, dim3(f->nmb), dim3(256), fit_sk_lds(f->ncol_max), st, a, vslot);
@@ -1950,7 +1960,9 @@ static int fit_run(mdff_fit* f, FitArgs a, size_t tsz) {
           if (f->nqb) hipLaunchKernelGGL(kf_moments<false>, dim3(f->nqb), dim3(64), 0, st, a, 0);
           if (f->nql) hipLaunchKernelGGL(kf_moments<true>, dim3(f->nql), dim3(64), 0, st, a, f->nqb);
         }
-      } else {
+      } else
+#endif
+      {
         hipLaunchKernelGGL((kf_sfpart<T>), gs, b, shm_sf, st, a, 1, vslot, -1);
         hipLaunchKernelGGL((kf_sf<T>), gk, b, red, st, a, 1);
         hipLaunchKernelGGL((kf_gpart<T, PH_ITER>), gg, b, kGatherLds, st, a);
@@ -1967,7 +1979,7 @@ static int fit_run(mdff_fit* f, FitArgs a, size_t tsz) {
   };
   // static field, SCF
   hipLaunchKernelGGL(kf_ctl, dim3(1), dim3(256), 0, st, a, (int)C_START);
-  hipLaunchKernelGGL((kf_static<T>), gp, dim3(256), 0, st, a);
+  hipLaunchKernelGGL((kf_static<T>), gp, dim3(256), 3 * 2048, st, a);
   hipLaunchKernelGGL((kf_sfpart<T>), gs, b, shm_sf, st, a, 0, -1, -1);
   hipLaunchKernelGGL((kf_sf<T>), gk, b, red, st, a, 0);
   hipLaunchKernelGGL((kf_gpart<T, PH_STATIC>), gg, b, kGatherLds, st, a);
@@ -1975,7 +1987,7 @@ static int fit_run(mdff_fit* f, FitArgs a, size_t tsz) {
   FIT_TRY(f, hipGetLastError());
   FIT_RC(iterate(W_MU, W_ES, C_SCF));
   // forces, stress, loss
-  hipLaunchKernelGGL((kf_pair<T, false>), gp, dim3(256), 0, st, a);
+  hipLaunchKernelGGL((kf_pair<T, false>), gp, dim3(256), 12 * 2048, st, a);
   hipLaunchKernelGGL(kf_psum, dim3(a.nsnap), dim3(64), 0, st, a, 12);
   hipLaunchKernelGGL((kf_sfpart<T>), gs, b, shm_sf, st, a, 2, (int)W_MU, -1);
   hipLaunchKernelGGL((kf_sf<T>), gk, b, red, st, a, 2);
@@ -1985,7 +1997,7 @@ static int fit_run(mdff_fit* f, FitArgs a, size_t tsz) {
   FIT_TRY(f, hipGetLastError());
   if (!a.want_grad) return MDFF_OK;
   // explicit pair gradients and h; adjoint solve; lambda terms
-  hipLaunchKernelGGL((kf_pair<T, true>), gp, dim3(256), shm_g, st, a);
+  hipLaunchKernelGGL((kf_pair<T, true>), gp, dim3(256), shm_g + 3 * 2048, st, a);
   hipLaunchKernelGGL(kf_psum, dim3(a.nsnap), dim3(64), 0, st, a, a.nparam);
   hipLaunchKernelGGL(kf_ctl, dim3(1), dim3(256), 0, st, a, (int)C_PAIRG);
   hipLaunchKernelGGL((kf_sfpart<T>), gs, b, shm_sf, st, a, 3, (int)W_MU, (int)W_G);
@@ -2373,7 +2385,11 @@ int mdff_fit_destroy(mdff_fit* f) {
                   (void*)f->d_rblk, (void*)f->d_qblk, (void*)f->d_dblk, (void*)f->d_pblk, (void*)f->d_pb0,
                   (void*)f->d_pp, (void*)f->d_ps})
     if (p) (void)hipFree(p);
+#ifdef __HIPCC__
   if (f->h_count) (void)hipHostFree(f->h_count);
+#else
+  if (f->h_count) (void)hipFree(f->h_count);
+#endif
   if (f->stream) (void)hipStreamDestroy(f->stream);
   delete f;
   return MDFF_OK;
