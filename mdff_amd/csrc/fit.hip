@@ -31,8 +31,9 @@
 // extra structure factors' worth of gathers (see k_fit, phase 6).
 //
 // Precision: T = double (FP64 form, used for the finite-difference checks) or
-// float (pair arithmetic and phase-table products in FP32); minimum image,
-// phase angles, every accumulation, the SCF and adjoint residuals in FP64.
+// float (pair arithmetic and, outside the iterations, phase-table products in
+// FP32); minimum image, phase angles, the iterations' reciprocal field, every
+// accumulation, the SCF and adjoint residuals in FP64.
 #include "common.h"
 
 #include <algorithm>

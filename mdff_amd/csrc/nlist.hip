@@ -3,9 +3,9 @@
 // Replaces vnlist_pbc (src/tools.f90:273-368) and vnlistcheck
 // (src/tools.f90:444-537).  The reference tests every ordered pair of the
 // O(N^2) sweep with the ownership rule; here atoms are binned into cells in
-// fractional space (cell width >= cutoff / perpendicular width, so every
-// partner lies in the 27 neighbouring cells) and one wavefront per atom
-// sweeps those cells.  Each device row holds ALL partners j != i with
+// fractional space (cells of a third of the cutoff where they fit, so every
+// partner lies within three cells) and one wavefront per atom sweeps those
+// cells.  Each device row holds ALL partners j != i with
 // r^2 <= (max cut + skin)^2, plus a flag byte saying which of the two
 // reference lists (vdw, coul) accepts the pair.  The reference half lists are
 // the ownership-filtered rows; r^2(i,j) and r^2(j,i) are bitwise equal (the
@@ -154,7 +154,10 @@ __global__ void k_cell_order(int n, const int32_t* __restrict__ in, const int32_
   const int i = in[t];
   const int k = cell_of[i], b = start[k], e = start[k + 1];
   int p = b;
-  for (int u = b; u < e; ++u) p += in[u] < i ? 1 : 0;
+  for (int u = b; u < e; u += 8) {       // eight loads in flight (few cells can hold many atoms)
+#pragma unroll
+    for (int v = 0; v < 8; ++v) p += u + v < e && in[min(u + v, e - 1)] < i ? 1 : 0;
+  }
   const double x = sx[i], y = sy[i], z = sz[i];
   order[p] = i;
   ox[p] = x;
