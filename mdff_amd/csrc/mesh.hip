@@ -1085,9 +1085,22 @@ bool choose_grid(const int* K, const double* aL, int w, double tol, int* G, doub
         g[d] = g[d - 1];
       } else {
         const int lo = std::max(w, 2 * K[d] + 1), hi = 4 * lo + 2 * kTile;
+        // the other directions have at least this one's size or their smallest
+        // grid: no size is tried that could not beat the best
+        double rest = 1.0;
+        bool cube = true;
+        for (int e = d + 1; e < 3; ++e) {
+          cube = cube && K[e] == K[d] && aL[e] == aL[d];
+          if (!cube) rest *= div_up(std::max(w, 2 * K[e] + 1), kTile) * kTile;
+        }
+        auto beaten = [&](int gd) {
+          double c = cells * gd * rest;
+          for (int e = d + 1; e < 3 && K[e] == K[d] && aL[e] == aL[d]; ++e) c *= gd;
+          return best > 0.0 && c >= best;
+        };
         g[d] = div_up(lo, kTile) * kTile;
-        while (g[d] <= hi && mesh_error(K[d], aL[d], g[d], w, r * w, tol) > tol) g[d] += kTile;
-        if (g[d] > hi) cells = 0.0;
+        while (g[d] <= hi && !beaten(g[d]) && mesh_error(K[d], aL[d], g[d], w, r * w, tol) > tol) g[d] += kTile;
+        if (g[d] > hi || beaten(g[d])) cells = 0.0;
       }
       cells *= g[d];
       if (best > 0.0 && cells > best) cells = 0.0;
@@ -1110,19 +1123,22 @@ void kernel_pieces(int w, double beta, std::vector<double>& coef) {
   T[1][1] = 1;
   for (int k = 2; k < M; ++k)
     for (int c = 0; c < M; ++c) T[k][c] = (c ? 2 * T[k - 1][c - 1] : 0) - T[k - 2][c];
+  ld cs[M][M];                             // cos(k (a + 1/2) pi / M)
+  for (int k = 0; k < M; ++k)
+    for (int a = 0; a < M; ++a) cs[k][a] = cosl(k * (a + 0.5L) * kPiL / M);
   const ld top = bessel_xi1(beta);
   coef.assign((size_t)(w / 2) * M, 0.0);
   for (int j = 0; j < w / 2; ++j) {
     ld y[M], mono[M] = {};
     for (int a = 0; a < M; ++a) {
-      const ld v = cosl((a + 0.5L) * kPiL / M);
+      const ld v = cs[1][a];
       const ld x = (j - (ld)w / 2 + (v + 1) / 2) / ((ld)w / 2);
       const ld s2 = 1 - x * x;
       y[a] = s2 > 0 ? bessel_xi1((ld)beta * sqrtl(s2)) / top : 0;
     }
     for (int k = 0; k < M; ++k) {
       ld ck = 0;
-      for (int a = 0; a < M; ++a) ck += y[a] * cosl(k * (a + 0.5L) * kPiL / M);
+      for (int a = 0; a < M; ++a) ck += y[a] * cs[k][a];
       ck *= (k ? 2.0L : 1.0L) / M;
       for (int c = 0; c <= k; ++c) mono[c] += ck * T[k][c];
     }
