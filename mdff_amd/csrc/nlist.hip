@@ -21,6 +21,7 @@
 #include <rocprim/device/device_reduce.hpp>
 #include <rocprim/device/device_scan.hpp>
 
+#include "cells.h"
 #include "common.h"
 #include "reduce.h"
 
@@ -535,25 +536,19 @@ static int nl_overflow(mdff_ctx* c, F next, bool* over) {
 // list build from the fractional coordinates (px, py, pz) of the build
 static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const double* pz, bool save) {
   const int n = c->n;
-  // cells: width >= cutoff / 3 in a reciprocal direction with room for at
-  // least 7 of them (partners within +-3 cells), else cutoff / 2 (5, +-2),
-  // else the cutoff (+-1); 1e-9 margin against rounding of the wrapped
-  // coordinates.  With fewer cells than the reach covers, every cell of that
-  // direction is visited once.
-  double rmax = std::max(c->rc_vdw, c->rc_coul) + c->d.skindiff;
+  // with fewer cells than the reach covers, every cell of that direction is
+  // visited once
+  const double rmax = std::max(c->rc_vdw, c->rc_coul) + c->d.skindiff;
+  const CellGrid cells = choose_cells(c->W, rmax, n);
   for (int d = 0; d < 3; ++d) {
-    int reach = 3, k = 0;
-    for (; reach >= 1; --reach) {
-      k = (int)floor(c->W[d] * reach / (rmax * (1.0 + 1e-9)));
-      if (k >= 2 * reach + 1 || reach == 1) break;
-    }
-    c->ncell[d] = k < 1 ? 1 : k;
-    const bool all = c->ncell[d] < 2 * reach + 1;
+    const int reach = cells.reach[d];
+    c->ncell[d] = cells.n[d];
+    const bool all = cells.n[d] < 2 * reach + 1;
     c->nb_lo[d] = all ? 0 : -reach;
-    c->nb_hi[d] = all ? c->ncell[d] - 1 : reach;
+    c->nb_hi[d] = all ? cells.n[d] - 1 : reach;
     c->nb_all[d] = all ? 1 : 0;
   }
-  int ncell = c->ncell[0] * c->ncell[1] * c->ncell[2];
+  const int ncell = cells.total();
   if (ncell + 1 > c->ncell_alloc) {
     if (c->cell_start) HIP_TRY(c, hipFree(c->cell_start));
     if (c->cell_cnt) HIP_TRY(c, hipFree(c->cell_cnt));

@@ -1,0 +1,84 @@
+"""Cell grids of the neighbour-list build (mdff_amd/csrc/cells.h) on the CPU:
+their number fits an int and is bounded by the atoms, and two atoms within the
+cutoff are never further apart than the cells that a sweep visits; and the pair
+sets of a few atoms in very wide boxes on the GPU."""
+import copy
+import ctypes as C
+import shutil
+import subprocess
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+from mdff_amd import configs
+
+ROOT = Path(__file__).resolve().parents[1]
+
+
+@pytest.fixture(scope="module")
+def choose(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not available")
+    tmp = tmp_path_factory.mktemp("cells")
+    (tmp / "c.cpp").write_text(
+        '#include "cells.h"\nextern "C" void choose(const double* W, double r, int n, int* out) {\n'
+        "  const CellGrid g = choose_cells(W, r, n);\n"
+        "  for (int d = 0; d < 3; ++d) { out[d] = g.n[d]; out[3 + d] = g.reach[d]; }\n}\n")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", f"-I{ROOT / 'mdff_amd' / 'csrc'}", "-o",
+                    str(tmp / "c.so"), str(tmp / "c.cpp")], check=True)
+    lib = C.CDLL(str(tmp / "c.so"))
+
+    def f(W, r, n):
+        out = (C.c_int * 6)()
+        lib.choose((C.c_double * 3)(*W), C.c_double(r), C.c_int(n), out)
+        return list(out[:3]), list(out[3:])
+    return f
+
+
+@pytest.mark.parametrize("natm", [1, 64, 4000, 200000])
+@pytest.mark.parametrize("W", [(0.5, 0.5, 0.5), (2.4, 2.4, 2.4), (7, 7, 7), (7, 20, 3), (25, 26, 24), (58, 58, 58),
+                               (111, 111, 111), (450, 450, 450), (700, 700, 700), (2000, 2000, 2000), (1e6, 1, 1),
+                               (1e9, 1e9, 1e9), (1e5, 1e5, 2.0)])
+def test_cells_are_bounded_and_cover_the_cutoff(choose, W, natm):
+    r = 9.3
+    n, reach = choose([w * r for w in W], r, natm)
+    assert n[0] * n[1] * n[2] <= max(16384, 4 * natm)
+    for d in range(3):
+        assert n[d] >= 1 and 1 <= reach[d] <= 3
+        # all cells are visited, or those of +-reach hold every partner
+        assert n[d] < 2 * reach[d] + 1 or W[d] * r / n[d] * reach[d] >= r
+        # the reach is as long as it was where the cells are few enough
+        k = int(W[d] * 3 / (1 + 1e-9))
+        if k >= 7 and np.prod([w * 3.0 for w in W]) <= 16384:
+            assert (n[d], reach[d]) == (k, 3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ratio", [40, 100, 460, 1000])
+def test_pair_sets_in_wide_boxes(ratio):
+    """Forty atoms in clumps, some across the faces, in a box of 40 to 1,000
+    reaches: both lists as the oracle's, and the forces."""
+    import gpu_util as G
+    G.note(f"wide box {ratio}")
+    rng = np.random.default_rng(ratio)
+    rc = 4.0
+    L = ratio * rc
+    centres = np.concatenate([rng.uniform(0, L, (6, 3)), [[0.0, 0.0, 0.0], [L, L / 2, 0.0]]])
+    pos = np.concatenate([c + np.stack(np.meshgrid(*[[0.0, 1.1]] * 3), -1).reshape(-1, 3)[:5] + rng.normal(0, 0.05, (5, 3))
+                          for c in centres])
+    s = configs.fcc_lj(ncell=2)
+    d = copy.deepcopy(s.desc)
+    d.natm = len(pos)
+    d.cell[:] = [L, 0, 0, 0, L, 0, 0, 0, L]
+    d.cutshortrange, d.skindiff = rc - 0.3, 0.3
+    w = configs.System("wide", d, np.ones(len(pos), np.int32), pos, np.zeros_like(pos))
+    g, o = G.pair(w)
+    for e in (g, o):
+        e.vnlist_build()
+    for a, b in zip(g.get_pairs(0), o.get_pairs(0)):
+        assert np.array_equal(a, b)
+    assert len(g.get_pairs(0)[1]) >= 10 * len(centres)
+    fg, fo = g.engforce()[0], o.engforce()[0]
+    assert G.rel_force_err(fg, fo) < 1e-10
+    g.close()
