@@ -357,6 +357,7 @@ struct mdff_ctx {
   int mma_nks = 0, mma_mtiles = 0;
   int mma_splits[2] = {1, 1};             // of the gathers of 3 and 9 moments
   int use_mma = 1;                        // matrix-core reciprocal kernels
+  int rec_wide = 0;                       // transforms to FP64 accuracy (recip_wide)
   int sk_rt = 0, sk_lta = 6;              // structure factor: row tiles a block, log2 of a staged tile's atoms
   int sk_mma_ch = 1;                      // atom chunks of the matrix-core structure factor
   double* kO_ws = nullptr;                // scf_kO_v2 work vectors (11 x 3n)

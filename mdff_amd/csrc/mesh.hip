@@ -1244,8 +1244,7 @@ void mesh_free(mdff_ctx* c) {
 // the half space).  Leaves c->mesh null where no grid meets the error bound.
 int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<double>& kv) {
   const int n = c->n;
-  const bool mixed = c->d.precision == MDFF_PREC_MIXED;
-  const bool wide = !mixed || c->d.doefg;   // the gradient is FP64 in both forms
+  const bool wide = c->rec_wide != 0;
   const int w = wide ? 16 : 12;
   // the gradient's second derivatives weigh the alias error by k^2: with
   // 4e-15 its error at 1,728 ions would be 4e-14, with 5e-16 it is 1.3e-14, the

@@ -947,6 +947,25 @@ static int sk_plan(mdff_ctx* c, int cus) {
   return MDFF_OK;
 }
 
+// Whether the transforms are to hold FP64 accuracy: the FP64 form; the field
+// gradient, which is FP64 in both; and of the mixed form the dipole systems that
+// ask for it (MDFF_DIP_RECIP_FP64=1, read at context creation) or are large
+// enough in x, y or z that the form has always summed them to FP64 rounding
+// (more than 1,024 columns (nx, ny), or nz beyond 31, within |k| <= 2.5 alpha).
+static bool recip_wide(const mdff_ctx* c) {
+  if (c->d.precision != MDFF_PREC_MIXED || c->d.doefg) return true;
+  if (!c->task_qd && !c->task_dd) return false;
+  const char* ev = getenv("MDFF_DIP_RECIP_FP64");
+  if (ev && ev[0] == '1') return true;
+  int kin[3];
+  for (int d = 0; d < 3; ++d) {
+    const double* a = c->A + 3 * d;
+    const double len = sqrt(a[0] * a[0] + a[1] * a[1] + a[2] * a[2]);
+    kin[d] = std::min(c->K[d], (int)ceil(2.5 * c->alpha * len / (2.0 * MDFF_PI)));
+  }
+  return !c->task_qq || std::min({kin[0], kin[1], kin[2]}) < 1 || kin[2] > 31 || (kin[0] + 1) * (2 * kin[1] + 1) > 1024;
+}
+
 int recip_setup(mdff_ctx* c) {
   const int Kx = c->d.kES[0], Ky = c->d.kES[1], Kz = c->d.kES[2];
   c->K[0] = Kx; c->K[1] = Ky; c->K[2] = Kz;
@@ -985,7 +1004,8 @@ int recip_setup(mdff_ctx* c) {
   // The mixed form's narrower kernel (12 points, not 16) puts its line lower.
   {
     const char* ev = getenv("MDFF_RECIP_MESH");
-    const double line = c->d.doefg ? 8e7 : (c->d.precision == MDFF_PREC_MIXED ? 7e7 : 1.1e8);
+    c->rec_wide = recip_wide(c) ? 1 : 0;
+    const double line = c->d.doefg ? 8e7 : (c->rec_wide ? 1.1e8 : 7e7);
     const bool on = ev && ev[0] ? ev[0] != '0' : (double)c->n * nb > line;
     if (on && c->use_mma && direct_takes(c)) {
       MDFF_TRY(mesh_setup(c, A, kv));
