@@ -448,7 +448,7 @@ int recip_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool 
 int recip_moments(mdff_ctx* c, const double* mu, RecFinal* rf);
 void recip_free(mdff_ctx* c);
 // the same sums as non-uniform fast transforms (mesh.hip)
-int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<double>& kv);
+int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<double>& kv, double most_us);
 int mesh_bin(mdff_ctx* c, bool from_r, bool pack);
 int mesh_eval(mdff_ctx* c, const double* mu, bool use_q, bool use_mu, int mom, double* e_out, const double** out);
 void mesh_free(mdff_ctx* c);

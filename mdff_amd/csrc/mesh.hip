@@ -1240,9 +1240,22 @@ void mesh_free(mdff_ctx* c) {
   c->mesh = nullptr;
 }
 
+// Time (us) of an evaluation's transforms beyond their launches: by the
+// operations of their products, and the grid's points.  Fitted over grids of
+// 64^3 to 1104 x 144 x 96 (FP64, 64 to 4,096 ions: 160^3 154 of 156 us measured,
+// 208 x 208 x 192 365 of 353, 272 x 272 x 224 732 of 698, 736 x 272 x 112 1074 of
+// 1070; the longest, 1104 x 144 x 96, 790 of 1126).
+static double mesh_transform_us(const int* G, const int* K) {
+  const double NX = 2 * K[0] + 1, NY = 2 * K[1] + 1, CN = K[2] + 1, cp = 16 * div_up(K[2] + 1, 16);
+  const double points = (double)G[0] * G[1] * G[2];
+  const double ops = 2.0 * (4.0 * points * cp + 8.0 * G[0] * G[1] * NY * cp + 8.0 * G[0] * NX * NY * CN);
+  return 30e-9 * ops + 8e-6 * points;
+}
+
 // A and kvec: the k mesh of recip_setup ([nx][ny][nz], nx >= 0, A = 0 outside
-// the half space).  Leaves c->mesh null where no grid meets the error bound.
-int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<double>& kv) {
+// the half space).  Leaves c->mesh null where no grid meets the error bound, or
+// the transforms of the one that does would take more than most_us.
+int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<double>& kv, double most_us) {
   const int n = c->n;
   const bool wide = c->rec_wide != 0;
   const int w = wide ? 16 : 12;
@@ -1258,6 +1271,7 @@ int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<doub
   }
   if (!choose_grid(c->K, aL, w, tol, G, beta)) return MDFF_OK;
   if ((double)G[0] * G[1] * G[2] > 536870912.0) return MDFF_OK;   // 4 GiB of grid
+  if (mesh_transform_us(G, c->K) > most_us) return MDFF_OK;
   // LDS of the transforms (doubles: planes and the waves' exchange)
   const int nyp = (2 * c->K[1] + 16) & ~15, nxp = (2 * c->K[0] + 16) & ~15;
   const int ctiles = div_up(c->K[2] + 1, 16), yld = 32 * ctiles + 2;

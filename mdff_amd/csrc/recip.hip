@@ -1002,13 +1002,20 @@ int recip_setup(mdff_ctx* c) {
   //   mixed  5.4e7 (silica 4,320) 136/138   4.3e7 (MgO 4,608 dipoles) 2514/2733   8e7 160/142
   //   gradient  9e7 (NaCl 4,096) 341/323
   // The mixed form's narrower kernel (12 points, not 16) puts its line lower.
+  // Few atoms in a large k mesh are another matter: the transforms' own work goes
+  // with the mesh alone, and has to be less than what the direct sums spend on
+  // atoms and k vectors (28 us a 1e8 terms, 220 us a 1e6 k vectors, fitted like
+  // mesh_transform_us; FP64, us an evaluation, direct / mesh: 256 ions at kES 48
+  // 248/507, 512 at 40 232/306, 128 at 200, 60, 20 442/1219, 1,728 at 28 224/183).
+  // Not so for kES(3) > 56, whose direct gather is the vector-ALU one.
   {
     const char* ev = getenv("MDFF_RECIP_MESH");
     c->rec_wide = recip_wide(c) ? 1 : 0;
     const double line = c->d.doefg ? 8e7 : (c->rec_wide ? 1.1e8 : 7e7);
-    const bool on = ev && ev[0] ? ev[0] != '0' : (double)c->n * nb > line;
+    const bool asked = ev && ev[0], on = asked ? ev[0] != '0' : (double)c->n * nb > line;
+    const double direct_us = asked || mma_bucket(Kz + 1) == 0 ? INFINITY : 28e-8 * c->n * nb + 220e-6 * nb;
     if (on && c->use_mma && direct_takes(c)) {
-      MDFF_TRY(mesh_setup(c, A, kv));
+      MDFF_TRY(mesh_setup(c, A, kv, direct_us));
       if (c->mesh) return MDFF_OK;
     }
   }

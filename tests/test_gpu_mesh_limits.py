@@ -7,6 +7,7 @@ largest force (alias error 4e-15 a direction, measured at three times that,
 rounding below 1e-13 on either side); the mixed form's cut-off of 1e-9 shows
 in the energy at 1e-10 and above."""
 import copy
+import ctypes as C
 
 import numpy as np
 import pytest
@@ -46,3 +47,47 @@ def test_mixed_dipoles_in_fp64(charges, mesh, monkeypatch):
         monkeypatch.setenv("MDFF_DIP_RECIP_FP64", "1")
     u = _engine(s, capi.PREC_MIXED).engforce()[1]["u_rec"]
     assert abs(u - u64) < 1e-12 * abs(u64)
+
+
+def _table_launches(e):
+    """Launches of the phase tables (direct sums: one) or of the kernel values
+    (transforms: three) of an evaluation."""
+    lib = capi.gpu_lib()
+    ms, count = (C.c_double * 16)(), (C.c_int32 * 16)()
+    lib.mdff_profile_name.restype = C.c_char_p
+    lib.mdff_profile(e.h, 1)
+    e.engforce()
+    lib.mdff_profile_read(e.h, ms, count, 16)
+    lib.mdff_profile(e.h, 0)
+    return count[[lib.mdff_profile_name(k) for k in range(16)].index(b"k_tables")]
+
+
+@pytest.mark.parametrize("ncell,k,fp64,mixed", [
+    (3, (50, 50, 50), 0, 1),                 # 216 ions: 275/447 us in FP64, 275/247 in the mixed form
+    (4, (40, 40, 40), 0, 1),                 # 512: 232/306, 232/205
+    (6, (28, 28, 28), 1, 1),                 # 1,728: 224/183, 224/144
+    (2, (80, 80, 50), 0, 0),                 # 64: 434/1198, 434/640
+    (2, (100, 100, 57), None, 1),            # (mixed only) no matrix-core gather of the direct sums: 1457 at kES 60, 64 ions
+])
+def test_route_of_few_ions_in_a_large_mesh(ncell, k, fp64, mixed, monkeypatch):
+    """The rule weighs the transforms' own work; either way the forces are those of
+    both kernels (to the forms' parity bars: splittings this sharp round at 1e-15
+    of alpha^2 q^2, a thousand times the forces)."""
+    s = configs.nacl(ncell=ncell, alpha=max(0.3, 0.15 * max(k) / ncell))
+    s.desc.kES[:] = list(k)
+    s.desc.cutshortrange = s.desc.cutlongrange = 5.0
+    G.note(f"route {ncell} {k}")
+    for prec, mesh in ((capi.PREC_FP64, fp64), (capi.PREC_MIXED, mixed)):
+        if mesh is None:
+            continue
+        monkeypatch.delenv("MDFF_RECIP_MESH", raising=False)
+        e = _engine(s, prec)
+        f = e.engforce()[0]
+        assert (_table_launches(e) > 1) == bool(mesh)
+        e.close()
+        for mode in ("0", "1"):
+            monkeypatch.setenv("MDFF_RECIP_MESH", mode)
+            e = _engine(s, prec)
+            err = G.rel_force_err(e.engforce()[0], f)
+            assert err < (1e-10 if prec == capi.PREC_FP64 else 1e-5)
+            e.close()
