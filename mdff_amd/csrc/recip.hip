@@ -858,17 +858,21 @@ static const void* sk_kernel(int rt, bool dip) {
 // every wave first loads its atoms' B operand (a prologue worth about
 // kGatherPrologue m-tiles), then runs its share of the m-tiles; the time is
 // taken as rounds of resident waves x (prologue + m-tiles per wave).  At
-// least 4 m-tiles per wave; fewer splits win ties.
-constexpr double kGatherPrologue = 4.0;
-static int gather_splits(int mtiles, int64_t atom_waves, int64_t conc) {
+// least 4 m-tiles per wave; fewer splits win ties.  More than 64 only up to a
+// block a CU, and where they pay for the longer sum over splits in the force
+// kernel, kSplitCost m-tiles a split of one K step (few atoms in a large k mesh: 64
+// at kES 80, 80, 50 192 -> 68 us).
+constexpr double kGatherPrologue = 4.0, kSplitCost = 4.6;
+static int gather_splits(int mtiles, int64_t atom_waves, int64_t conc, int cus, int nks) {
   int best_s = 1;
   double best = -1.0;
-  for (int sp = 1; sp <= std::min(mtiles, 64); ++sp) {
+  const int most = (int)std::min<int64_t>(256, std::max<int64_t>(64, cus / div_up(atom_waves, 4)));
+  for (int sp = 1; sp <= std::min(mtiles, most); ++sp) {
     if (sp > 1 && mtiles / sp < 4) break;
     const int mps = div_up(mtiles, sp);
     const int nsp = div_up(mtiles, mps);
     const int64_t rounds = (atom_waves * nsp + conc - 1) / conc;
-    const double cost = (double)rounds * (kGatherPrologue + mps);
+    const double cost = (double)rounds * (kGatherPrologue + mps) + (nsp > 64 ? kSplitCost / nks * (nsp - 64) : 0.0);
     if (best < 0.0 || cost < best - 1e-9) {
       best = cost;
       best_s = nsp;
@@ -915,9 +919,11 @@ static bool direct_takes(const mdff_ctx* c) {
 // Row tiles: kES(3) spread evenly over as few blocks of at most 7 as it needs.
 // Tile and chunks: the least of a sum of what a launch waits for (us): a tile's
 // staging kStage, its products (64 cycles each on a SIMD, shared by the blocks
-// of a CU), and kChunk a chunk for the reduction that adds them up.
+// of a CU), kChunk a chunk for the reduction that adds them up, and for partial
+// sums beyond the L2s' 32 MB their way to memory and back (kByte; 64 ions at kES
+// 80, 80, 50, 21 MB a chunk: sums and reduction 141 -> 126 us; 512 at 40 101 -> 77).
 static int sk_plan(mdff_ctx* c, int cus) {
-  constexpr double kStage = 1.5, kChunk = 0.08, kProduct = 64.0 / 2400.0;
+  constexpr double kStage = 1.5, kChunk = 0.08, kProduct = 64.0 / 2400.0, kByte = 2.0 / 4e6, kCached = 32e6;
   const int ncol = c->K[0] + c->K[1] + c->K[2] + 3;
   c->sk_mma_ch = 1;
   if (ncol > sk_cols(c)) return MDFF_OK;          // refused at the first evaluation (sk_rt 0)
@@ -936,6 +942,7 @@ static int sk_plan(mdff_ctx* c, int cus) {
       const int per = div_up(c->n, ch), nch = div_up(c->n, per), tiles = div_up(per, TA);
       const int64_t blocks = (int64_t)mblocks * nch;
       const double t = (double)div_up(blocks, cap) * tiles * kStage + kChunk * nch +
+                       kByte * std::max(0.0, 16.0 * c->nk_box * nch - kCached) +
                        (double)div_up(blocks, cus) * div_up(per, 8) * kSkStep * c->sk_rt * (dip ? 2 : 1) * kProduct;
       if (best == 0.0 || t < best) {
         best = t;
@@ -1006,7 +1013,7 @@ int recip_setup(mdff_ctx* c) {
   // with the mesh alone, and has to be less than what the direct sums spend on
   // atoms and k vectors (28 us a 1e8 terms, 220 us a 1e6 k vectors, fitted like
   // mesh_transform_us; FP64, us an evaluation, direct / mesh: 256 ions at kES 48
-  // 248/507, 512 at 40 232/306, 128 at 200, 60, 20 442/1219, 1,728 at 28 224/183).
+  // 247/508, 512 at 40 208/306, 128 at 200, 60, 20 341/1219, 1,728 at 28 224/183).
   // Not so for kES(3) > 56, whose direct gather is the vector-ALU one.
   {
     const char* ev = getenv("MDFF_RECIP_MESH");
@@ -1044,7 +1051,7 @@ int recip_setup(mdff_ctx* c) {
     const int mom = k ? 9 : 3;
     const int atom_waves = div_up(c->n, 16 * mma_ct(c->mma_nks, mom));
     const int64_t conc = 4 * (int64_t)cus * blocks_per_cu(gather_kernel(c->mma_nks, mom), 0);
-    c->mma_splits[k] = gather_splits(c->mma_mtiles, atom_waves, conc);
+    c->mma_splits[k] = gather_splits(c->mma_mtiles, atom_waves, conc, cus, std::max(c->mma_nks, 1));
   }
   MDFF_TRY(sk_plan(c, cus));
   const size_t na = (size_t)c->mma_mtiles * c->mma_nks * 64;
