@@ -527,12 +527,17 @@ __global__ void __launch_bounds__(1024) k_mesh_spread(SpreadArgs a) {
 //    + (R & 3) and part (R >> 2) & 1, so a lane ends with re and im of its two
 //    n.  The re and im inputs go to neighbouring waves, which halves the chain
 //    of a wave; their sums meet in LDS.
+// The rows that a product sums over are staged all at once where they fit the
+// block's LDS, else (Gy or Gx + NX beyond 576: LiF of 53 cells and more in a
+// row) a slice of them at a time: the sums of the slices before are read back by
+// the threads that wrote them (y and x forward, x back) or kept in registers (y
+// back).  The direct sums, the alternative, took 2960 us for LiF 66 x 8 x 8
+// (33,792 ions, mixed) and 10.06 s for 46^3 (778,688); in slices 541 us and 10 ms.
 constexpr int kFtThreads = 1024, kFtWaves = 16;
 
-// the tile's operand (e, es doubles between steps of 4 l) times the LDS rows v
-// over L (operand and rows up to the next 16)
-__device__ __forceinline__ f64x4 mid_chain(const double* e, size_t es, const double* v, int L) {
-  f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+// acc + the tile's operand (e, es doubles between steps of 4 l) times the LDS
+// rows v over L (operand and rows up to the next 16)
+__device__ __forceinline__ f64x4 mid_chain(const double* e, size_t es, const double* v, int L, f64x4 acc) {
   for (int l = 0; l < L; l += 16) {
     double ev[4], vv[4];
 #pragma unroll
@@ -557,7 +562,7 @@ __device__ __forceinline__ void mid_product(const double* in, int lrows, int L, 
   for (int t0 = 0; t0 < ntiles; t0 += kFtWaves / 2) {
     const int t = t0 + (wave >> 1);
     f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-    if (t < ntiles) acc = mid_chain(E + ((size_t)t * 2 + sp) * 64 + lane, (size_t)ntiles * 128, v, L);
+    if (t < ntiles) acc = mid_chain(E + ((size_t)t * 2 + sp) * 64 + lane, (size_t)ntiles * 128, v, L, acc);
     if (sp == 1) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) x[64 * r] = acc[r];
@@ -576,6 +581,7 @@ __device__ __forceinline__ void mid_product(const double* in, int lrows, int L, 
 
 struct ZyArgs {
   int Gy, Gz, CN, NY, ctiles;
+  int slice;                     // SLICED: y rows in LDS (a multiple of 16)
   size_t sstride;                // between the shares of the grid, which are added
   const double* grid;
   const double* zf;              // row operand: column tile 2 ct + part
@@ -585,62 +591,71 @@ struct ZyArgs {
 
 // Block (nz tile, x): z transform of the plane's rows at 16 nz into LDS, then
 // their y transform.  SH: shares of the grid
-template <int SH>
+template <int SH, bool SLICED>
 __global__ void __launch_bounds__(kFtThreads) k_mesh_zy(ZyArgs a) {
   extern __shared__ double lds[];
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15, wave = wave_id();
   const int ct = blockIdx.x, x = blockIdx.y;
-  const int ytiles = a.Gy / 16;
-  double* pl = lds;                                       // [part][Gy][16]
-  double* xb = lds + 2 * (size_t)a.Gy * 16;
-  for (int u = wave; u < 2 * ytiles; u += kFtWaves) {
-    const int rt = u >> 1, part = u & 1;
-    const double* in = a.grid + ((size_t)x * a.Gy + 16 * rt + c) * a.Gz + 4 * g;
-    const double* m = a.zf + ((size_t)2 * ct + part) * 256 + lane;
-    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-    for (int k0 = 0; k0 < a.Gz; k0 += 32) {
-      // the second of the two steps repeats a valid one when Gz ends before it
-      const int kk[2] = {k0, min(k0 + 16, a.Gz - 16)};
-      double2 v[2][SH][2];
-      double b[2][4];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-#pragma unroll
-        for (int s = 0; s < SH; ++s) {
-          v[h][s][0] = *reinterpret_cast<const double2*>(in + s * a.sstride + kk[h]);
-          v[h][s][1] = *reinterpret_cast<const double2*>(in + s * a.sstride + kk[h] + 2);
-        }
-#pragma unroll
-        for (int s = 0; s < 4; ++s) b[h][s] = m[(size_t)(kk[h] / 16) * a.ctiles * 512 + 64 * s];
-      }
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        if (h == 1 && k0 + 16 >= a.Gz) break;
-        double2 v0 = v[h][0][0], v1 = v[h][0][1];
-#pragma unroll
-        for (int s = 1; s < SH; ++s) {
-          v0.x += v[h][s][0].x; v0.y += v[h][s][0].y;
-          v1.x += v[h][s][1].x; v1.y += v[h][s][1].y;
-        }
-        acc = mma64(v0.x, b[h][0], acc);
-        acc = mma64(v0.y, b[h][1], acc);
-        acc = mma64(v1.x, b[h][2], acc);
-        acc = mma64(v1.y, b[h][3], acc);
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) pl[((size_t)part * a.Gy + 16 * rt + 4 * r + g) * 16 + c] = acc[r];
-  }
-  __syncthreads();
+  const int slice = SLICED ? a.slice : a.Gy;
+  double* pl = lds;                                       // [part][slice][16]
+  double* xb = lds + 2 * (size_t)slice * 16;
   double2* out = a.out + (size_t)x * a.NY * a.CN;
-  const int cc = 16 * ct + c;
-  mid_product(pl, a.Gy, a.Gy, div_up_dev(a.NY, 8), a.NY, a.yf, xb, [&](int n, int, double re, double im) {
-    if (cc < a.CN) out[(size_t)n * a.CN + cc] = make_double2(re, im);
-  });
+  const int cc = 16 * ct + c, ntiles = div_up_dev(a.NY, 8);
+  int y0 = 0;
+  do {
+    const int ny = SLICED ? min(slice, a.Gy - y0) : a.Gy;
+    for (int u = wave; u < ny / 8; u += kFtWaves) {
+      const int rt = u >> 1, part = u & 1;
+      const double* in = a.grid + ((size_t)x * a.Gy + y0 + 16 * rt + c) * a.Gz + 4 * g;
+      const double* m = a.zf + ((size_t)2 * ct + part) * 256 + lane;
+      f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+      for (int k0 = 0; k0 < a.Gz; k0 += 32) {
+        // the second of the two steps repeats a valid one when Gz ends before it
+        const int kk[2] = {k0, min(k0 + 16, a.Gz - 16)};
+        double2 v[2][SH][2];
+        double b[2][4];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+          for (int s = 0; s < SH; ++s) {
+            v[h][s][0] = *reinterpret_cast<const double2*>(in + s * a.sstride + kk[h]);
+            v[h][s][1] = *reinterpret_cast<const double2*>(in + s * a.sstride + kk[h] + 2);
+          }
+#pragma unroll
+          for (int s = 0; s < 4; ++s) b[h][s] = m[(size_t)(kk[h] / 16) * a.ctiles * 512 + 64 * s];
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          if (h == 1 && k0 + 16 >= a.Gz) break;
+          double2 v0 = v[h][0][0], v1 = v[h][0][1];
+#pragma unroll
+          for (int s = 1; s < SH; ++s) {
+            v0.x += v[h][s][0].x; v0.y += v[h][s][0].y;
+            v1.x += v[h][s][1].x; v1.y += v[h][s][1].y;
+          }
+          acc = mma64(v0.x, b[h][0], acc);
+          acc = mma64(v0.y, b[h][1], acc);
+          acc = mma64(v1.x, b[h][2], acc);
+          acc = mma64(v1.y, b[h][3], acc);
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) pl[((size_t)part * slice + 16 * rt + 4 * r + g) * 16 + c] = acc[r];
+    }
+    __syncthreads();
+    mid_product(pl, slice, ny, ntiles, a.NY, a.yf + (size_t)(y0 / 4) * ntiles * 128, xb,
+                [&](int n, int, double re, double im) {
+                  if (cc >= a.CN) return;
+                  double2* o = out + (size_t)n * a.CN + cc;
+                  *o = SLICED && y0 > 0 ? make_double2(o->x + re, o->y + im) : make_double2(re, im);
+                });
+  } while (SLICED && (y0 += slice) < a.Gy);
 }
 
 struct XArgs {
   int Gx, NX, C, back;           // C = NY CN columns
+  int slice;                     // SLICED: rows in LDS (a multiple of 16)
+  double2* s;                    // SLICED: S, then W, [nx][C]
   const double* xf;
   const double* xb;
   double2* t;                    // [x][C], in place
@@ -651,48 +666,72 @@ struct XArgs {
 
 // Block: 16 columns (ny, nz).  S(n); W = A conj(S); the energy and stress
 // partials ((delta_ab - kcoe k_a k_b) A |S|^2, src/ewald_rec.f90:173-174,
-// 252-263); W's x transform back in place (back).
+// 252-263); W's x transform back in place (back).  S and W stay in LDS, or
+// (SLICED) in global memory.
+template <bool SLICED>
 __global__ void __launch_bounds__(kFtThreads) k_mesh_x(XArgs a) {
   extern __shared__ double lds[];
   const int lane = threadIdx.x & 63, wave = wave_id(), c = lane & 15;
-  const int nxp = (a.NX + 15) & ~15;
-  double* pl = lds;                                       // [part][Gx][16]
-  double* wl = pl + 2 * (size_t)a.Gx * 16;                // [part][nxp][16]
-  double* xb = wl + 2 * (size_t)nxp * 16;
-  const int c0 = blockIdx.x * 16;
-  for (int k = threadIdx.x; k < a.Gx * 16; k += kFtThreads) {
-    const double2 v = a.t[(size_t)(k >> 4) * a.C + min(c0 + (k & 15), a.C - 1)];
-    pl[k] = v.x;
-    pl[(size_t)a.Gx * 16 + k] = v.y;
-  }
-  for (int k = a.NX * 16 + threadIdx.x; k < nxp * 16; k += kFtThreads) {
-    wl[k] = 0.0;
-    wl[(size_t)nxp * 16 + k] = 0.0;
-  }
-  __syncthreads();
-  double sum[7] = {0, 0, 0, 0, 0, 0, 0};
-  const int cc = c0 + c;
-  mid_product(pl, a.Gx, a.Gx, div_up_dev(a.NX, 8), a.NX, a.xf, xb, [&](int n, int, double re, double im) {
-    double wr = 0.0, wi = 0.0;
-    if (cc < a.C) {
-      const size_t at = (size_t)n * a.C + cc;
-      const double Ak = a.A[at];
-      const double* k = a.kvec + 4 * at;
-      const double str = (re * re + im * im) * Ak;
-      const double kx = k[0], ky = k[1], kz = k[2], kc = k[3];
-      sum[0] += str;
-      sum[1] += (1.0 - kc * kx * kx) * str;
-      sum[2] += (1.0 - kc * ky * ky) * str;
-      sum[3] += (1.0 - kc * kz * kz) * str;
-      sum[4] += -kc * kx * ky * str;
-      sum[5] += -kc * kx * kz * str;
-      sum[6] += -kc * ky * kz * str;
-      wr = Ak * re;
-      wi = -Ak * im;
+  const int nxp = (a.NX + 15) & ~15, ntiles = div_up_dev(a.NX, 8);
+  const int rows = SLICED ? a.slice : a.Gx;
+  double* pl = lds;                                       // [part][rows][16]
+  double* wl = pl + 2 * (size_t)rows * 16;                // [part][nxp][16]
+  double* xb = wl + (SLICED ? 0 : 2 * (size_t)nxp * 16);
+  const int c0 = blockIdx.x * 16, cc = c0 + c;
+  // rows from..from + cnt of src into LDS, zero beyond cnt up to the next 16
+  auto stage = [&](const double2* src, int from, int cnt) {
+    for (int k = threadIdx.x; k < ((cnt + 15) & ~15) * 16; k += kFtThreads) {
+      double2 v = src[(size_t)(from + min(k >> 4, cnt - 1)) * a.C + min(c0 + (k & 15), a.C - 1)];
+      if ((k >> 4) >= cnt) v = make_double2(0.0, 0.0);
+      pl[k] = v.x;
+      pl[(size_t)rows * 16 + k] = v.y;
     }
-    wl[n * 16 + c] = wr;
-    wl[(size_t)nxp * 16 + n * 16 + c] = wi;
-  });
+  };
+  if constexpr (!SLICED)
+    for (int k = a.NX * 16 + threadIdx.x; k < nxp * 16; k += kFtThreads) {
+      wl[k] = 0.0;
+      wl[(size_t)nxp * 16 + k] = 0.0;
+    }
+  double sum[7] = {0, 0, 0, 0, 0, 0, 0};
+  // A conj(S) of entry (n, cc), and its part of the sums
+  auto weigh = [&](int n, double re, double im) {
+    const size_t at = (size_t)n * a.C + cc;
+    const double Ak = a.A[at];
+    const double* k = a.kvec + 4 * at;
+    const double str = (re * re + im * im) * Ak;
+    const double kx = k[0], ky = k[1], kz = k[2], kc = k[3];
+    sum[0] += str;
+    sum[1] += (1.0 - kc * kx * kx) * str;
+    sum[2] += (1.0 - kc * ky * ky) * str;
+    sum[3] += (1.0 - kc * kz * kz) * str;
+    sum[4] += -kc * kx * ky * str;
+    sum[5] += -kc * kx * kz * str;
+    sum[6] += -kc * ky * kz * str;
+    return make_double2(Ak * re, -Ak * im);
+  };
+  int g0 = 0;
+  do {
+    const int cnt = SLICED ? min(rows, a.Gx - g0) : a.Gx;
+    stage(a.t, g0, cnt);
+    __syncthreads();
+    mid_product(pl, rows, cnt, ntiles, a.NX, a.xf + (size_t)(g0 / 4) * ntiles * 128, xb,
+                [&](int n, int, double re, double im) {
+                  if constexpr (SLICED) {
+                    if (cc >= a.C) return;
+                    double2* o = a.s + (size_t)n * a.C + cc;
+                    if (g0 > 0) {
+                      re += o->x;
+                      im += o->y;
+                    }
+                    *o = g0 + rows < a.Gx ? make_double2(re, im) : weigh(n, re, im);
+                  } else {
+                    double2 w = {0.0, 0.0};
+                    if (cc < a.C) w = weigh(n, re, im);
+                    wl[n * 16 + c] = w.x;
+                    wl[(size_t)nxp * 16 + n * 16 + c] = w.y;
+                  }
+                });
+  } while (SLICED && (g0 += rows) < a.Gx);
   // wave sums, then the waves in order
 #pragma unroll
   for (int k = 0; k < 7; ++k) {
@@ -708,15 +747,30 @@ __global__ void __launch_bounds__(kFtThreads) k_mesh_x(XArgs a) {
   }
   if (!a.back) return;
   __syncthreads();
-  mid_product(wl, nxp, a.NX, a.Gx / 8, a.Gx, a.xb, xb, [&](int n, int, double re, double im) {
-    if (cc < a.C) a.t[(size_t)n * a.C + cc] = make_double2(re, im);
-  });
+  if constexpr (SLICED) {
+    for (int n0 = 0; n0 < a.NX; n0 += rows) {
+      const int cnt = min(rows, a.NX - n0);
+      stage(a.s, n0, cnt);
+      __syncthreads();
+      mid_product(pl, rows, cnt, a.Gx / 8, a.Gx, a.xb + (size_t)(n0 / 4) * (a.Gx / 8) * 128, xb,
+                  [&](int n, int, double re, double im) {
+                    if (cc >= a.C) return;
+                    double2* o = a.t + (size_t)n * a.C + cc;
+                    *o = n0 > 0 ? make_double2(o->x + re, o->y + im) : make_double2(re, im);
+                  });
+    }
+  } else {
+    mid_product(wl, nxp, a.NX, a.Gx / 8, a.Gx, a.xb, xb, [&](int n, int, double re, double im) {
+      if (cc < a.C) a.t[(size_t)n * a.C + cc] = make_double2(re, im);
+    });
+  }
 }
 
 constexpr int kYzRows = 32;      // y rows of a k_mesh_yz block
 
 struct YzArgs {
   int Gy, Gz, CN, NY, ctiles, ld;
+  int slice;                     // SLICED: ny rows in LDS (a multiple of 16)
   const double2* in;             // [x][ny][nz]
   const double* yb;
   const double* zb;
@@ -725,11 +779,12 @@ struct YzArgs {
 
 // Block (32 y, x): y transform back of those rows, 16 nz at a time, into LDS
 // rows of (nz, re / im), then their z transform back
+template <bool SLICED>
 __global__ void __launch_bounds__(kFtThreads) k_mesh_yz(YzArgs a) {
   extern __shared__ double lds[];
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15, wave = wave_id();
   const int y0 = blockIdx.x * kYzRows, x = blockIdx.y;
-  const int nyp = (a.NY + 15) & ~15;
+  const int nyp = SLICED ? a.slice : (a.NY + 15) & ~15;
   const int ny = min(kYzRows, a.Gy - y0);
   double* rows = lds;                                     // [kYzRows][ld]
   double* pl = rows + (size_t)kYzRows * a.ld;             // [nz tile][part][nyp][16]
@@ -741,24 +796,28 @@ __global__ void __launch_bounds__(kFtThreads) k_mesh_yz(YzArgs a) {
   double* xw = xb + (wave >> 1) * 256 + lane;
   for (int ct0 = 0; ct0 < a.ctiles; ct0 += 2) {
     const int nct = min(2, a.ctiles - ct0);
-    for (int k = threadIdx.x; k < nct * nyp * 16; k += kFtThreads) {
-      const int h = k >= nyp * 16 ? 1 : 0, kk = k - h * nyp * 16;
-      const int cc = 16 * (ct0 + h) + (kk & 15), l = kk >> 4;
-      double2 v = in[(size_t)min(l, a.NY - 1) * a.CN + min(cc, a.CN - 1)];
-      if (l >= a.NY || cc >= a.CN) v = make_double2(0.0, 0.0);
-      pl[(size_t)(2 * h) * nyp * 16 + kk] = v.x;
-      pl[(size_t)(2 * h + 1) * nyp * 16 + kk] = v.y;
-    }
-    __syncthreads();
     f64x4 acc = {0.0, 0.0, 0.0, 0.0};
     const bool on = 8 * t < ny && half < nct;
-    if (on) {
-      acc = mid_chain(a.yb + ((size_t)(y0 / 8 + t) * 2 + sp) * 64 + lane, (size_t)(a.Gy / 8) * 128,
-                      pl + (size_t)(2 * half + sp) * nyp * 16 + 16 * g + c, a.NY);
-      if (sp == 1) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) xw[64 * r] = acc[r];
+    int l0 = 0;
+    do {
+      for (int k = threadIdx.x; k < nct * nyp * 16; k += kFtThreads) {
+        const int h = k >= nyp * 16 ? 1 : 0, kk = k - h * nyp * 16;
+        const int cc = 16 * (ct0 + h) + (kk & 15), l = l0 + (kk >> 4);
+        double2 v = in[(size_t)min(l, a.NY - 1) * a.CN + min(cc, a.CN - 1)];
+        if (l >= a.NY || cc >= a.CN) v = make_double2(0.0, 0.0);
+        pl[(size_t)(2 * h) * nyp * 16 + kk] = v.x;
+        pl[(size_t)(2 * h + 1) * nyp * 16 + kk] = v.y;
       }
+      __syncthreads();
+      if (on)
+        acc = mid_chain(a.yb + (size_t)(l0 / 4) * (a.Gy / 8) * 128 + ((size_t)(y0 / 8 + t) * 2 + sp) * 64 + lane,
+                        (size_t)(a.Gy / 8) * 128, pl + (size_t)(2 * half + sp) * nyp * 16 + 16 * g + c,
+                        SLICED ? min(nyp, a.NY - l0) : a.NY, acc);
+      if (SLICED && l0 + nyp < a.NY) __syncthreads();
+    } while (SLICED && (l0 += nyp) < a.NY);
+    if (on && sp == 1) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) xw[64 * r] = acc[r];
     }
     __syncthreads();
     if (sp == 0 && on) {
@@ -1216,6 +1275,7 @@ struct MeshRecip {
   MeshGrid m{};
   int K[3] = {0, 0, 0}, CN = 0;            // CN = Kz + 1 complex columns
   int nbins = 0, shares = 1, X = 8, nblk = 0, ctiles = 0, ld = 0;
+  int slice_zy = 0, slice_x = 0, slice_yz = 0;   // rows staged at a time, 0: all
   size_t lds_zy = 0, lds_x = 0, lds_yz = 0;
   int sorted = 0;                          // bins and phi belong to the current coordinates
   int counted = 0;                         // k_mesh_bin has run and the scan has not
@@ -1228,6 +1288,21 @@ struct MeshRecip {
   double *phi = nullptr, *grid = nullptr, *mom = nullptr, *blk = nullptr;
   double2* t = nullptr;
 };
+
+// the transforms' kernels
+static const void* zy_kernel(int shares, bool sliced) {
+  switch (shares) {
+    case 1: return sliced ? reinterpret_cast<const void*>(&k_mesh_zy<1, true>) : reinterpret_cast<const void*>(&k_mesh_zy<1, false>);
+    case 2: return sliced ? reinterpret_cast<const void*>(&k_mesh_zy<2, true>) : reinterpret_cast<const void*>(&k_mesh_zy<2, false>);
+    default: return sliced ? reinterpret_cast<const void*>(&k_mesh_zy<4, true>) : reinterpret_cast<const void*>(&k_mesh_zy<4, false>);
+  }
+}
+static const void* x_kernel(bool sliced) {
+  return sliced ? reinterpret_cast<const void*>(&k_mesh_x<true>) : reinterpret_cast<const void*>(&k_mesh_x<false>);
+}
+static const void* yz_kernel(bool sliced) {
+  return sliced ? reinterpret_cast<const void*>(&k_mesh_yz<true>) : reinterpret_cast<const void*>(&k_mesh_yz<false>);
+}
 
 void mesh_free(mdff_ctx* c) {
   MeshRecip* m = c->mesh;
@@ -1272,24 +1347,29 @@ int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<doub
   if (!choose_grid(c->K, aL, w, tol, G, beta)) return MDFF_OK;
   if ((double)G[0] * G[1] * G[2] > 536870912.0) return MDFF_OK;   // 4 GiB of grid
   if (mesh_transform_us(G, c->K) > most_us) return MDFF_OK;
-  // LDS of the transforms (doubles: planes and the waves' exchange)
+  // LDS of the transforms (doubles: planes and the waves' exchange), and the
+  // rows that fit
   const int nyp = (2 * c->K[1] + 16) & ~15, nxp = (2 * c->K[0] + 16) & ~15;
   const int ctiles = div_up(c->K[2] + 1, 16), yld = 32 * ctiles + 2;
-  const size_t xch = (size_t)kFtWaves / 2 * 256;
-  const size_t lds_zy = 8 * (2 * (size_t)G[1] * 16 + xch), lds_x = 8 * (32 * ((size_t)G[0] + nxp) + xch),
-               lds_yz = 8 * ((size_t)kYzRows * yld + 4 * (size_t)nyp * 16 + xch);
   int maxlds = 0;
   HIP_TRY(c, hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device));
-  if (std::max({lds_zy, lds_x, lds_yz}) > (size_t)maxlds) return MDFF_OK;
-  for (const void* fn : {reinterpret_cast<const void*>(&k_mesh_zy<1>), reinterpret_cast<const void*>(&k_mesh_zy<2>),
-                         reinterpret_cast<const void*>(&k_mesh_zy<4>), reinterpret_cast<const void*>(&k_mesh_x),
-                         reinterpret_cast<const void*>(&k_mesh_yz)})
-    HIP_TRY(c, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, maxlds));
+  const int xch = kFtWaves / 2 * 256, room = maxlds / 8 - xch;
+  const int fit = (room / 32) & ~15, fit_yz = std::max(0, room - kYzRows * yld) / 64 & ~15;
+  if (fit_yz < 16) return MDFF_OK;         // kES(3) beyond 270
+  const int slice_zy = G[1] <= fit ? 0 : fit, slice_x = G[0] + nxp <= fit ? 0 : fit, slice_yz = nyp <= fit_yz ? 0 : fit_yz;
+  const size_t lds_zy = 8 * (32 * (size_t)std::min(G[1], fit) + xch), lds_x = 8 * (32 * (size_t)std::min(G[0] + nxp, fit) + xch),
+               lds_yz = 8 * ((size_t)kYzRows * yld + 64 * (size_t)std::min(nyp, fit_yz) + xch);
+  for (int sl = 0; sl < 2; ++sl)
+    for (const void* fn : {zy_kernel(1, sl), zy_kernel(2, sl), zy_kernel(4, sl), x_kernel(sl), yz_kernel(sl)})
+      HIP_TRY(c, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, maxlds));
   MeshRecip* m = new MeshRecip();
   c->mesh = m;
   m->w = w;
   m->ctiles = ctiles;
   m->ld = yld;
+  m->slice_zy = slice_zy;
+  m->slice_x = slice_x;
+  m->slice_yz = slice_yz;
   m->lds_zy = lds_zy;
   m->lds_x = lds_x;
   m->lds_yz = lds_yz;
@@ -1513,31 +1593,41 @@ int mesh_eval(mdff_ctx* c, const double* mu, bool use_q, bool use_mu, int mom, d
   ZyArgs za{};
   za.Gy = Gy; za.Gz = Gz; za.CN = CN; za.NY = NY;
   za.ctiles = m->ctiles;
+  za.slice = m->slice_zy;
   za.sstride = (size_t)Gx * Gy * Gz;
   za.grid = m->grid;
   za.zf = m->zf; za.yf = m->yf;
   za.out = m->t;
-  const auto zy = m->shares == 1 ? &k_mesh_zy<1> : (m->shares == 2 ? &k_mesh_zy<2> : &k_mesh_zy<4>);
-  PROF_LAUNCH(c, PK_SKRED, hipLaunchKernelGGL(zy, dim3(m->ctiles, Gx), dim3(kFtThreads), m->lds_zy, c->stream, za));
+  void* zargs[] = {&za};
+  PROF_LAUNCH(c, PK_SKRED, (void)hipLaunchKernel(zy_kernel(m->shares, m->slice_zy > 0), dim3(m->ctiles, Gx), dim3(kFtThreads),
+                                                 zargs, m->lds_zy, c->stream));
   MDFF_TRY(claim_partials(c, m->blk));
   XArgs xa{};
   xa.Gx = Gx; xa.NX = NX; xa.C = NY * CN;
   xa.back = mom > 0 ? 1 : 0;
+  xa.slice = m->slice_x;
+  // (the grid is free between the plane transforms, and at least as large:
+  // NX <= Gx, NY <= Gy, 2 CN <= Gz)
+  xa.s = reinterpret_cast<double2*>(m->grid);
   xa.xf = m->xf; xa.xb = m->xb;
   xa.t = m->t;
   xa.A = m->A; xa.kvec = m->kvec; xa.blk = m->blk;
-  PROF_LAUNCH(c, PK_SKRED, hipLaunchKernelGGL(k_mesh_x, dim3(m->nblk), dim3(kFtThreads), m->lds_x, c->stream, xa));
+  void* xargs[] = {&xa};
+  PROF_LAUNCH(c, PK_SKRED, (void)hipLaunchKernel(x_kernel(m->slice_x > 0), dim3(m->nblk), dim3(kFtThreads), xargs, m->lds_x,
+                                                 c->stream));
   if (e_out) MDFF_TRY(queue_final(c, m->blk, m->nblk, 7, e_out));
   if (mom > 0) {
     YzArgs ya{};
     ya.Gy = Gy; ya.Gz = Gz; ya.CN = CN; ya.NY = NY;
     ya.ctiles = m->ctiles;
     ya.ld = m->ld;
+    ya.slice = m->slice_yz;
     ya.in = m->t;
     ya.yb = m->yb; ya.zb = m->zb;
     ya.grid = m->grid;
-    PROF_LAUNCH(c, PK_SKRED, hipLaunchKernelGGL(k_mesh_yz, dim3(div_up(Gy, kYzRows), Gx), dim3(kFtThreads), m->lds_yz,
-                                                c->stream, ya));
+    void* yargs[] = {&ya};
+    PROF_LAUNCH(c, PK_SKRED, (void)hipLaunchKernel(yz_kernel(m->slice_yz > 0), dim3(div_up(Gy, kYzRows), Gx), dim3(kFtThreads),
+                                                   yargs, m->lds_yz, c->stream));
     GatherArgs ga{};
     ga.n = n;
     ga.X = m->X;

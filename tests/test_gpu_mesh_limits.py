@@ -91,3 +91,69 @@ def test_route_of_few_ions_in_a_large_mesh(ncell, k, fp64, mixed, monkeypatch):
             err = G.rel_force_err(e.engforce()[0], f)
             assert err < (1e-10 if prec == capi.PREC_FP64 else 1e-5)
             e.close()
+
+
+def _stretched(f, k, dip=False):
+    """NaCl with the cell's axes stretched (no two ions nearer than before),
+    so that the k mesh's far entries still carry weight."""
+    s = configs.nacl(ncell=2, alpha=0.9)
+    d = s.desc
+    cell = np.array(d.cell[:]).reshape(3, 3)
+    s.pos = s.pos @ np.linalg.inv(cell) @ (cell * np.array(f)[:, None])
+    d.cell[:] = list((cell * np.array(f)[:, None]).reshape(9))
+    d.kES[:] = list(k)
+    if dip:
+        d.dip[0 + 16 * 0], d.dip[0 + 16 * 1], d.dip[0 + 16 * 2] = 0.11, -0.05, 0.07
+        d.dip[1 + 16 * 0], d.dip[1 + 16 * 1], d.dip[1 + 16 * 2] = -0.04, 0.09, 0.13
+    return s
+
+
+@pytest.mark.parametrize("f,k,dip", [
+    ((8, 1, 1), (90, 8, 9), False),          # x: all staged at once
+    ((24, 1, 1), (260, 8, 9), False),        # x: two slices of the grid and of the modes
+    ((27, 1, 1), (290, 8, 9), True),
+    ((1, 27, 1), (9, 290, 8), False),        # y: slices of the grid and of the modes
+    ((1, 24, 1), (9, 260, 8), True),
+    ((2, 14, 5), (20, 160, 50), True),       # y, with four tiles of nz
+    ((1, 16, 16), (9, 170, 56), False),
+], ids=["x_whole", "x", "x_dip", "y", "y_dip", "yz_dip", "yz"])
+def test_sliced_planes_match_direct_sums(f, k, dip, monkeypatch):
+    """Meshes too long for LDS: energy, forces, stress and the field of the
+    transforms against the direct sums and the oracle, and in the mixed form
+    against the oracle."""
+    s = _stretched(f, k, dip)
+    G.note(f"sliced {f} {k} {dip}")
+    out = []
+    for mesh in ("0", "1"):
+        monkeypatch.setenv("MDFF_RECIP_MESH", mesh)
+        e = _engine(s, capi.PREC_FP64, doefield=1)
+        out.append((*e.engforce(), e.get_dipoles()[1]))
+        again = e.engforce()
+        assert np.array_equal(out[-1][0], again[0]) and out[-1][1]["u_rec"] == again[1]["u_rec"]
+        e.close()
+    (fd, td, ed), (fm, tm, em) = out
+    assert np.abs(fm - fd).max() < 1e-12 * np.abs(fd).max()
+    assert np.abs(em - ed).max() < 1e-12 * np.abs(ed).max()
+    assert abs(tm["u_rec"] - td["u_rec"]) < 1e-12 * abs(td["u_rec"])
+    assert np.abs(tm["tau_coul"] - td["tau_coul"]).max() < 1e-12 * np.abs(td["tau_coul"]).max()
+    _, o = G.pair(s)
+    fo, to = o.engforce()
+    assert G.rel_force_err(fm, fo) < 1e-10
+    assert not G.compare_terms(tm, to, 1e-10)
+    e = _engine(s, capi.PREC_MIXED)
+    assert G.rms_force_err(e.engforce()[0], fo) < 1e-5
+    e.close()
+
+
+def test_sliced_planes_take_a_mixed_mesh_beyond_the_fp64_form(monkeypatch):
+    """Two slices of the modes in x and three in y."""
+    monkeypatch.setenv("MDFF_RECIP_MESH", "1")
+    s = _stretched((30, 24, 1), (330, 260, 8))
+    G.note("sliced mixed")
+    e = _engine(s, capi.PREC_MIXED)
+    _, o = G.pair(s)
+    fo, to = o.engforce()
+    fm, tm = e.engforce()
+    assert G.rms_force_err(fm, fo) < 1e-5
+    assert abs(tm["u_rec"] - to["u_rec"]) < 1e-8 * abs(to["u_rec"])
+    e.close()
