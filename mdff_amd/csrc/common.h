@@ -267,7 +267,8 @@ struct mdff_ctx {
   double* red = nullptr;                  // reduction outputs
   int mu_static = 0;                      // mu holds the static dipoles (no induced dipoles)
   double *cx = nullptr, *cy = nullptr, *cz = nullptr;   // fractional coordinates of a pending list check
-  double* h_chk = nullptr;                // mapped pinned host memory: block maxima of the pending check
+  double* h_mapped = nullptr;             // one block of mapped pinned host memory, the h_ arrays its parts
+  double* h_chk = nullptr;                // block maxima of the pending check
   double* d_chk = nullptr;                // the device address of h_chk
   int chk_pending = 0;
   // the next final-sum launch writes chk_seq into
@@ -277,10 +278,10 @@ struct mdff_ctx {
   double chk_seq = 0.0;
   double* red_part = nullptr;             // reduction block partials
   double* mu_next = nullptr;              // the next dipole iteration's mu_ind (3n)
-  double* h_scf = nullptr;                // mapped pinned host memory: a dipole iteration's sums, a slot a block
+  double* h_scf = nullptr;                // a dipole iteration's sums, a slot a block
   double* d_scf = nullptr;                // its device address
   double scf_seq = 0.0;
-  double* h_io = nullptr;                 // mapped pinned host memory: sequence word, kIoMax results, kIoMax inputs
+  double* h_io = nullptr;                 // sequence word, kIoMax results, kIoMax inputs
   double* d_io = nullptr;                 // its device address
   double io_seq = 0.0;
   int io_in_busy = 0;                     // the inputs may still be read
@@ -329,17 +330,16 @@ struct mdff_ctx {
   int nb_lo[3] = {0, 0, 0}, nb_hi[3] = {0, 0, 0}, nb_all[3] = {1, 1, 1};  // neighbour cell offsets
   float4* bf = nullptr;                   // wrapped single-precision copy of (bx, by, bz)
   int ncell_alloc = 0;
-  double* h_nl = nullptr;                 // mapped pinned host memory: a build's overflow flag, sequence number
+  double* h_nl = nullptr;                 // a build's overflow flag, sequence number
   double* d_nl = nullptr;
   double nl_seq = 0.0;
   void* sort_tmp = nullptr;
   size_t sort_tmp_bytes = 0;
   int lists_valid = 0;
   int32_t* d_flag = nullptr;              // device flags: [0] rebuild, [1] overflow
-  int32_t* h_flag = nullptr;              // pinned host mirror
-  double* h_red = nullptr;                // pinned host reduction mirror
+  int32_t* h_flag = nullptr;              // host mirror of d_flag
   double* raw = nullptr;                  // device sums of evaluations: RAW_SLOTS x RAW_N
-  double* h_raw = nullptr;                // pinned host mirror of raw
+  double* h_raw = nullptr;                // host mirror of raw
   int timings_pending = 0;
 
   // reciprocal space

@@ -947,12 +947,37 @@ static int ctx_init(mdff_ctx* c, const mdff_desc* d, const int32_t* itype) {
   }
   DMALLOC(c->d_flag, 4);
   DMALLOC(c->cx, n); DMALLOC(c->cy, n); DMALLOC(c->cz, n);
-  // written by the check kernels over the bus, read by the host after the
-  // check's event: mapped, coherent (uncached on the device side)
-  HIP_TRY(c, hipHostMalloc((void**)&c->h_chk, sizeof(double) * (2 * (size_t)nblk(n) + 2),
-                           hipHostMallocMapped | hipHostMallocCoherent));
-  HIP_TRY(c, hipHostGetDevicePointer((void**)&c->d_chk, c->h_chk, 0));
-  memset(c->h_chk, 0, sizeof(double) * (2 * (size_t)nblk(n) + 2));
+  {
+    // what kernels write over the bus for the host, and copies land in: one
+    // block of mapped, coherent memory (uncached on the device side), since an
+    // allocation of pinned memory costs some 20 us, and as much to give back
+    struct Part {
+      double **h, **d;
+      size_t count;
+      bool zero;
+    };
+    const size_t nb = nblk(n);
+    const Part parts[] = {{&c->h_chk, &c->d_chk, 2 * nb + 2, true},
+                          {&c->h_scf, &c->d_scf, kScfSlot * nb, true},
+                          {&c->h_nl, &c->d_nl, 2, true},
+                          {&c->h_io, &c->d_io, 8 + 2 * kIoMax, false},   // sequence word, results, incoming arrays
+                          {&c->h_raw, nullptr, (size_t)RAW_N * RAW_SLOTS, false},
+                          {(double**)&c->h_flag, nullptr, 2, false}};
+    auto padded = [](size_t k) { return (k + 7) & ~(size_t)7; };
+    size_t total = 0;
+    for (const Part& p : parts) total += padded(p.count);
+    HIP_TRY(c, hipHostMalloc((void**)&c->h_mapped, sizeof(double) * total, hipHostMallocMapped | hipHostMallocCoherent));
+    double* dev = nullptr;
+    HIP_TRY(c, hipHostGetDevicePointer((void**)&dev, c->h_mapped, 0));
+    size_t at = 0;
+    for (const Part& p : parts) {
+      *p.h = c->h_mapped + at;
+      if (p.d) *p.d = dev + at;
+      if (p.zero) memset(*p.h, 0, sizeof(double) * p.count);
+      at += padded(p.count);
+    }
+    c->h_io[0] = 0.0;
+  }
   HIP_TRY(c, hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking));
   HIP_TRY(c, hipEventCreateWithFlags(&c->ov_tab, hipEventDisableTiming));
   HIP_TRY(c, hipEventCreateWithFlags(&c->ov_pair, hipEventDisableTiming));
@@ -964,26 +989,12 @@ static int ctx_init(mdff_ctx* c, const mdff_desc* d, const int32_t* itype) {
     const char* ov = getenv("MDFF_PAIR_OVERLAP");
     c->overlap = ov && ov[0] ? ov[0] != '0' : n > 2048;
   }
-  HIP_TRY(c, hipHostMalloc((void**)&c->h_flag, sizeof(int32_t) * 4));
-  const size_t nred = std::max<size_t>(64 * 1024, 2 * (size_t)nblk(n) + 2);
-  HIP_TRY(c, hipHostMalloc((void**)&c->h_red, sizeof(double) * nred));
-  DMALLOC(c->red_part, nred);
-  HIP_TRY(c, hipHostMalloc((void**)&c->h_nl, sizeof(double) * 2, hipHostMallocMapped | hipHostMallocCoherent));
-  HIP_TRY(c, hipHostGetDevicePointer((void**)&c->d_nl, c->h_nl, 0));
-  c->h_nl[0] = c->h_nl[1] = 0.0;
-  // mapped hand-over memory: the sequence word, results, and incoming arrays
-  HIP_TRY(c, hipHostMalloc((void**)&c->h_io, sizeof(double) * (8 + 2 * kIoMax), hipHostMallocMapped | hipHostMallocCoherent));
-  HIP_TRY(c, hipHostGetDevicePointer((void**)&c->d_io, c->h_io, 0));
-  c->h_io[0] = 0.0;
-  HIP_TRY(c, hipHostMalloc((void**)&c->h_scf, sizeof(double) * kScfSlot * (size_t)nblk(n), hipHostMallocMapped | hipHostMallocCoherent));
-  HIP_TRY(c, hipHostGetDevicePointer((void**)&c->d_scf, c->h_scf, 0));
-  memset(c->h_scf, 0, sizeof(double) * kScfSlot * (size_t)nblk(n));
+  DMALLOC(c->red_part, std::max<size_t>(64 * 1024, 2 * (size_t)nblk(n) + 2));
   DMALLOC(c->red, 64);
   DMALLOC(c->fin_part, 1024 * 16 + (size_t)nblk(n) + 16);
   DMALLOC(c->nhc_part, 2 * (size_t)nblk(n));
   DMALLOC(c->nhc_st, NHC_N);
   DMALLOC(c->raw, (size_t)RAW_N * RAW_SLOTS);
-  HIP_TRY(c, hipHostMalloc((void**)&c->h_raw, sizeof(double) * RAW_N * RAW_SLOTS));
   HIP_TRY(c, hipMemcpy(c->itype, it0.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
   HIP_TRY(c, hipMemcpy(c->q, q.data(), sizeof(double) * n, hipMemcpyHostToDevice));
   HIP_TRY(c, hipMemcpy(c->mass, m.data(), sizeof(double) * n, hipMemcpyHostToDevice));
@@ -1708,13 +1719,7 @@ int mdff_ctx_destroy(mdff_ctx* c) {
   if (c->polar) (void)hipFree(c->polar);
   recip_free(c);
   efg_free(c);
-  if (c->h_flag) (void)hipHostFree(c->h_flag);
-  if (c->h_red) (void)hipHostFree(c->h_red);
-  if (c->h_raw) (void)hipHostFree(c->h_raw);
-  if (c->h_chk) (void)hipHostFree(c->h_chk);
-  if (c->h_scf) (void)hipHostFree(c->h_scf);
-  if (c->h_io) (void)hipHostFree(c->h_io);
-  if (c->h_nl) (void)hipHostFree(c->h_nl);
+  if (c->h_mapped) (void)hipHostFree(c->h_mapped);
   if (c->ov_tab) (void)hipEventDestroy(c->ov_tab);
   if (c->ov_pair) (void)hipEventDestroy(c->ov_pair);
   if (c->stream2) (void)hipStreamDestroy(c->stream2);
