@@ -1449,7 +1449,9 @@ int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<doub
   HIP_TRY(c, hipMalloc((void**)&m->slot, sizeof(int32_t) * n));
   HIP_TRY(c, hipMalloc((void**)&m->order, sizeof(BinAtom) * n));
   HIP_TRY(c, hipMalloc((void**)&m->cnt, sizeof(int32_t) * m->nbins));
-  HIP_TRY(c, hipMemset(m->cnt, 0, sizeof(int32_t) * m->nbins));
+  // (on the context's stream: hipMemset may return before the null stream has done
+  // it, and this stream does not wait for that one)
+  HIP_TRY(c, hipMemsetAsync(m->cnt, 0, sizeof(int32_t) * m->nbins, c->stream));
   HIP_TRY(c, hipMalloc((void**)&m->start, sizeof(int32_t) * (m->nbins + 1)));
   HIP_TRY(c, hipMalloc((void**)&m->at, sizeof(int4) * n));
   HIP_TRY(c, hipMalloc((void**)&m->phi, sizeof(double) * nr * w * (size_t)n));

@@ -1056,7 +1056,8 @@ int recip_setup(mdff_ctx* c) {
   MDFF_TRY(sk_plan(c, cus));
   const size_t na = (size_t)c->mma_mtiles * c->mma_nks * 64;
   HIP_TRY(c, hipMalloc((void**)&c->amat, sizeof(double) * na));
-  HIP_TRY(c, hipMemset(c->amat, 0, sizeof(double) * na));
+  // (on the context's stream, as the kernels: it does not wait for the null stream)
+  HIP_TRY(c, hipMemsetAsync(c->amat, 0, sizeof(double) * na, c->stream));
   // block partials of the energy / stress: k-blocks of 64
   HIP_TRY(c, hipMalloc((void**)&c->rec_blk, sizeof(double) * 7 * (size_t)div_up(nb, 64)));
   HIP_TRY(c, hipMalloc((void**)&c->sk_part, sizeof(double) * 2 * (size_t)std::max(c->sk_chunks, c->sk_mma_ch) * nb));
