@@ -133,6 +133,25 @@ __device__ __forceinline__ int xcd_order(int bid, int nbk) {
   return (xcd < ext ? xcd * (per + 1) : ext * (per + 1) + (xcd - ext) * per) + slot;
 }
 
+// Weight A of mode n = (x, y, z), 0 for n = 0, its k vector and kcoe
+// (src/kspace.f90:162-191); B: reciprocal matrix, column-major
+struct KWeight {
+  double A, kx, ky, kz, kc;
+};
+__device__ __forceinline__ KWeight k_weight(const double* B, double alpha2, double x, double y, double z) {
+  const double tpi = 2.0 * MDFF_PI;
+  KWeight w{};
+  w.kx = tpi * (x * B[0] + y * B[3] + z * B[6]);
+  w.ky = tpi * (x * B[1] + y * B[4] + z * B[7]);
+  w.kz = tpi * (x * B[2] + y * B[5] + z * B[8]);
+  const double kk = w.kx * w.kx + w.ky * w.ky + w.kz * w.kz;
+  if (kk != 0.0) {
+    w.A = exp(-(kk * 0.25) / alpha2) / kk;
+    w.kc = 2.0 * (1.0 / kk + 1.0 / alpha2 / 4.0);
+  }
+  return w;
+}
+
 // Last step of the reciprocal gather for one atom: the per-split partial
 // moments part[(s * moments + c) * n + i] summed over the splits, then the
 // Cartesian field and force (src/ewald_rec.f90:196-233, scaled as :300-358:
@@ -448,7 +467,7 @@ int recip_eval(mdff_ctx* c, const double* q, const double* mu, bool use_q, bool 
 int recip_moments(mdff_ctx* c, const double* mu, RecFinal* rf);
 void recip_free(mdff_ctx* c);
 // the same sums as non-uniform fast transforms (mesh.hip)
-int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<double>& kv, double most_us);
+int mesh_setup(mdff_ctx* c, double most_us);
 int mesh_bin(mdff_ctx* c, bool from_r, bool pack);
 int mesh_eval(mdff_ctx* c, const double* mu, bool use_q, bool use_mu, int mom, double* e_out, const double** out);
 void mesh_free(mdff_ctx* c);

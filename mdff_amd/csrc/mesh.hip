@@ -22,7 +22,7 @@
 // which the derivatives need.  Its transform is elementary
 // (2 h beta (z cosh z - sinh z) / z^3, z^2 = beta^2 - (2 pi f h)^2, h = w/2).
 // The grid G and beta are chosen per direction from the alias error weighted
-// with the decay of A(k) (mesh_error): below 4e-15 with w = 16 in the FP64
+// with the decay of A(k) (mesh_error_above): below 4e-15 with w = 16 in the FP64
 // form, which measured 1e-14 of the reciprocal force (its rounding), below
 // 1e-9 with w = 12 in the mixed form, whose FP32 pair terms carry 1e-7.
 //
@@ -1106,19 +1106,22 @@ R kernel_hat(int w, R beta, R f) {
   const R h = (R)w / 2, a = 2 * (R)kPiL * f * h, z2 = beta * beta - a * a;
   if (std::fabs(z2) < (R)1e-6) return (R)1 / 3 + z2 / 30;
   const R z = std::sqrt(std::fabs(z2));
-  if (z2 > 0) return (z * std::cosh(z) - std::sinh(z)) / (z * z2);
+  if (z2 > 0) {
+    const R e = std::exp(z);     // z cosh z - sinh z
+    return ((z - 1) * e + (z + 1) / e) / (2 * z * z2);
+  }
   return (std::sin(z) - z * std::cos(z)) / (z * -z2);
 }
 
-// The alias error of the gradient of V from one direction, relative to the
-// terms that carry the force: mode n of weight a(n) >= A(n)/A(0) comes with
-// modes n + jG of weight phih(n + jG) / phih(n), each differentiated.  The
-// force itself sits at n* = alpha |a| / (pi sqrt 2).  Measured errors are
-// about 3 times this.  Stops where it exceeds `enough`.
-double mesh_error(int K, double aL, int G, int w, double beta, double enough) {
-  const double pi = MDFF_PI, nstar = std::max(1.0, aL / (pi * sqrt(2.0)));
-  double worst = 0.0;
-  for (int n = K; n >= 0 && worst <= enough * nstar; --n) {
+// Whether the alias error of the gradient of V from one direction, relative to
+// the terms that carry the force, is above tol: mode n of weight a(n) >= A(n)/A(0)
+// comes with modes n + jG of weight phih(n + jG) / phih(n), each differentiated.
+// The force itself sits at n* = alpha |a| / (pi sqrt 2).  Measured errors are
+// about 3 times this.  `first`: the mode looked at first, left at the one that was
+// above, which is the likeliest to be so again.
+bool mesh_error_above(int K, double aL, int G, int w, double beta, double tol, int& first) {
+  const double pi = MDFF_PI, most = tol * std::max(1.0, aL / (pi * sqrt(2.0)));
+  auto above = [&](int n) {
     double e = 0.0;
     for (int j = 1; j <= 2; ++j)
       for (int sg = -1; sg <= 1; sg += 2) {
@@ -1126,9 +1129,15 @@ double mesh_error(int K, double aL, int G, int w, double beta, double enough) {
         e += fabs(kernel_hat<double>(w, beta, m / G)) * fabs(m);
       }
     const double an = exp(-(pi * n / aL) * (pi * n / aL));
-    worst = std::max(worst, an * e / kernel_hat<double>(w, beta, (double)n / G));
-  }
-  return worst / nstar;
+    return an * e / kernel_hat<double>(w, beta, (double)n / G) > most;
+  };
+  if (above(first)) return true;
+  for (int n = K; n >= 0; --n)
+    if (above(n)) {
+      first = n;
+      return true;
+    }
+  return false;
 }
 
 // Grids (multiples of the tile, at least the 2K + 1 modes and w) and the beta
@@ -1136,6 +1145,7 @@ double mesh_error(int K, double aL, int G, int w, double beta, double enough) {
 // grids have the fewest points.  false: none up to 4 (2K + 1) points.
 bool choose_grid(const int* K, const double* aL, int w, double tol, int* G, double& beta) {
   double best = 0.0;
+  int first[3] = {K[0], K[1], K[2]};
   for (double r = 1.5; r < 3.0; r += 0.05) {
     int g[3];
     double cells = 1.0;
@@ -1158,7 +1168,7 @@ bool choose_grid(const int* K, const double* aL, int w, double tol, int* G, doub
           return best > 0.0 && c >= best;
         };
         g[d] = div_up(lo, kTile) * kTile;
-        while (g[d] <= hi && !beaten(g[d]) && mesh_error(K[d], aL[d], g[d], w, r * w, tol) > tol) g[d] += kTile;
+        while (g[d] <= hi && !beaten(g[d]) && mesh_error_above(K[d], aL[d], g[d], w, r * w, tol, first[d])) g[d] += kTile;
         if (g[d] > hi || beaten(g[d])) cells = 0.0;
       }
       cells *= g[d];
@@ -1205,67 +1215,117 @@ void kernel_pieces(int w, double beta, std::vector<double>& coef) {
   }
 }
 
-// 1 / phih(n) for n = 0..K, phi as the pieces have it (x I1(x) over its top)
-std::vector<ld> deconv(int w, double beta, int K, int G) {
-  std::vector<ld> d(K + 1);
-  const ld h = (ld)w / 2, b = beta;
-  for (int n = 0; n <= K; ++n) d[n] = bessel_xi1(b) / (2 * h * b * b * kernel_hat<ld>(w, b, (ld)n / G));
-  return d;
+// x as the sum of two doubles
+void push_split(std::vector<double>& v, ld x) {
+  v.push_back((double)x);
+  v.push_back((double)(x - (ld)(double)x));
 }
 
-// e^{2 pi i a / G} for every a
-struct Roots {
-  std::vector<ld> c, s;
-  explicit Roots(int G) : c(G), s(G) {
-    for (int a = 0; a < G; ++a) {
-      c[a] = cosl(2 * kPiL * a / G);
-      s[a] = sinl(2 * kPiL * a / G);
-    }
+// 1 / phih(n) for n = 0..K, phi as the pieces have it (x I1(x) over its top)
+void push_deconv(std::vector<double>& v, int w, double beta, int K, int G) {
+  const ld b = beta, top = bessel_xi1(b) / (w * b * b);
+  for (int n = 0; n <= K; ++n) push_split(v, top / kernel_hat<ld>(w, b, (ld)n / G));
+}
+
+// e^{2 pi i a / G} for every a, as (cos, its rest, sin, its rest); G is a
+// multiple of 16, so an eighth of the circle holds them all
+void push_roots(std::vector<double>& v, int G) {
+  std::vector<ld> c(G / 4 + 1), s(G / 4 + 1);
+  for (int a = 0; a <= G / 8; ++a) {
+    c[a] = s[G / 4 - a] = cosl(2 * kPiL * a / G);
+    s[a] = c[G / 4 - a] = sinl(2 * kPiL * a / G);
   }
-  size_t at(long long a) const {
-    const long long G = (long long)c.size();
-    return (size_t)(((a % G) + G) % G);
+  for (int a = 0; a < G; ++a) {
+    const int q = a / (G / 4), r = a % (G / 4);
+    push_split(v, q == 0 ? c[r] : q == 1 ? -s[r] : q == 2 ? -c[r] : s[r]);
+    push_split(v, q == 0 ? s[r] : q == 1 ? c[r] : q == 2 ? -s[r] : -c[r]);
   }
+}
+
+// ---- the matrices, made on the device: they and A(k) have as many entries as
+// the k mesh, and made on the host they were most of a context's creation (LiF
+// 195,112 24.5 ms, now 8.6; silica 24,000 FP64 3.2 ms, now 0.8).
+
+struct TableArgs {
+  int G[3], K[3], CN, ctiles;
+  const double4* root[3];        // push_roots
+  const double2* dec[3];         // 1 / phih(n), n = 0..K, as two doubles
+  double *zf, *zb, *f[2], *b[2]; // f, b: x and y
+  double *A, *kvec;
+  double cell[9], alpha2;        // reciprocal matrix, column-major
 };
 
-// operand order of a row product for an M of K rows and N columns
-template <typename F>
-std::vector<double> row_operand(int K, int N, F value) {
-  const int kc = div_up(K, 16), nt = div_up(N, 16);
-  std::vector<double> m((size_t)kc * nt * 256, 0.0);
-  for (int k = 0; k < K; ++k)
-    for (int n = 0; n < N; ++n) {
-      const int g = (k & 15) >> 2, s = k & 3;
-      m[(((size_t)(k / 16) * nt + n / 16) * 4 + s) * 64 + 16 * g + (n & 15)] = value(k, n);
-    }
-  return m;
+// (x + its rest) times (d + its rest), rounded once
+__device__ __forceinline__ double split_product(double x, double xl, double2 d) {
+  const double p = x * d.x;
+  return p + (fma(x, d.x, -p) + (x * d.y + xl * d.x));
 }
 
-// operand order of a mid product for E of N rows and L columns (zero up to
-// the next 16 of L)
-template <typename F>
-std::vector<double> mid_operand(int N, int L, F value) {
-  const int lc = 4 * div_up(L, 16), nt = div_up(N, 8);
-  std::vector<double> m((size_t)lc * nt * 128, 0.0);
-  for (int l = 0; l < L; ++l)
-    for (int n = 0; n < N; ++n) {
-      ld re, im;
-      value(n, l, re, im);
-      const int nl = n & 7, g = l & 3;
-      double* t = m.data() + ((size_t)(l / 4) * nt + n / 8) * 128;
-      for (int part = 0; part < 2; ++part) {
-        const int R = 8 * (nl >> 2) + 4 * part + (nl & 3);
-        t[16 * g + R] = (double)(part ? im : re);
-        t[64 + 16 * g + R] = (double)(part ? re : -im);
+// cos and sin of 2 pi a b / G over phih
+__device__ __forceinline__ double2 table_entry(const TableArgs& a, int d, int mode, int point) {
+  const long long G = a.G[d];
+  const double4 r = a.root[d][(((long long)mode * point) % G + G) % G];
+  const double2 w = a.dec[d][mode < 0 ? -mode : mode];
+  return make_double2(split_product(r.x, r.y, w), split_product(r.z, r.w, w));
+}
+
+// blockIdx.y: 0 z forward, 1 z back, 2 and 3 x, 4 and 5 y forward and back, 6 the
+// weights
+__global__ void __launch_bounds__(256) k_mesh_tables(TableArgs a) {
+  const int what = blockIdx.y, i0 = blockIdx.x * 256 + threadIdx.x, step = gridDim.x * 256;
+  const int Gz = a.G[2];
+  if (what < 2) {
+    // operand order of a row product: [k / 16][column tile][step][lane].  Forward:
+    // column tile 2 ct + part holds that part of nz = 16 ct ..; back: row k = 2 nz + part
+    const int rows = what == 0 ? Gz : 32 * a.ctiles, nt = what == 0 ? 2 * a.ctiles : Gz / 16;
+    double* out = what == 0 ? a.zf : a.zb;
+    for (int i = i0; i < rows * nt * 16; i += step) {
+      const int lane = i & 63, s = (i >> 6) & 3, tile = i >> 8;
+      const int k = 16 * (tile / nt) + 4 * (lane >> 4) + s, col = 16 * (tile % nt) + (lane & 15);
+      double v = 0.0;
+      if (what == 0) {
+        const int nz = 16 * (col >> 5) + (col & 15);
+        if (nz < a.CN) {
+          const double2 e = table_entry(a, 2, nz, k);
+          v = (col & 16) ? e.y : e.x;
+        }
+      } else if (k < 2 * a.CN) {
+        const double2 e = table_entry(a, 2, k >> 1, col);
+        v = (k & 1) ? -e.y : e.x;
       }
+      out[i] = v;
     }
-  return m;
-}
-
-int upload(mdff_ctx* c, const std::vector<double>& v, double** p) {
-  HIP_TRY(c, hipMalloc((void**)p, sizeof(double) * v.size()));
-  HIP_TRY(c, hipMemcpy(*p, v.data(), sizeof(double) * v.size(), hipMemcpyHostToDevice));
-  return MDFF_OK;
+  } else if (what < 6) {
+    // operand order of a mid product: [l / 4][n tile of 8][re in, im in][lane]
+    const int d = (what - 2) >> 1, G = a.G[d], K = a.K[d], M = 2 * K + 1;
+    const bool back = what & 1;
+    const int N = back ? G : M, L = back ? M : G, nt = (N + 7) / 8, lt = 4 * ((L + 15) / 16);
+    double* out = back ? a.b[d] : a.f[d];
+    for (int i = i0; i < lt * nt * 128; i += step) {
+      const int lane = i & 63, im_in = (i >> 6) & 1, tile = i >> 7;
+      const int R = lane & 15, part = (R >> 2) & 1;
+      const int l = 4 * (tile / nt) + (lane >> 4), n = 8 * (tile % nt) + 4 * (R >> 3) + (R & 3);
+      double v = 0.0;
+      if (n < N && l < L) {
+        const double2 e = table_entry(a, d, (back ? l : n) - K, back ? n : l);
+        v = im_in ? (part ? e.x : -e.y) : (part ? e.y : e.x);
+      }
+      out[i] = v;
+    }
+  } else {
+    // A and k on nz >= 0: an entry and its opposite are one term, so nz = 0 keeps
+    // half of each of the two
+    const int NX = 2 * a.K[0] + 1, NY = 2 * a.K[1] + 1;
+    for (int i = i0; i < NX * NY * a.CN; i += step) {
+      const int z = i % a.CN, xy = i / a.CN, y = xy % NY - a.K[1], x = xy / NY - a.K[0];
+      const KWeight w = k_weight(a.cell, a.alpha2, x, y, z);
+      a.A[i] = z == 0 ? 0.5 * w.A : w.A;
+      a.kvec[4 * (size_t)i] = w.kx;
+      a.kvec[4 * (size_t)i + 1] = w.ky;
+      a.kvec[4 * (size_t)i + 2] = w.kz;
+      a.kvec[4 * (size_t)i + 3] = w.kc;
+    }
+  }
 }
 
 }  // namespace
@@ -1280,6 +1340,7 @@ struct MeshRecip {
   int sorted = 0;                          // bins and phi belong to the current coordinates
   int counted = 0;                         // k_mesh_bin has run and the scan has not
   double *zf = nullptr, *zb = nullptr, *yf = nullptr, *yb = nullptr, *xf = nullptr, *xb = nullptr;
+  void* mem = nullptr;                     // one allocation, the arrays its parts
   double *coef = nullptr, *A = nullptr, *kvec = nullptr;
   int32_t *key = nullptr, *slot = nullptr, *cnt = nullptr, *start = nullptr;
   BinAtom* order = nullptr;
@@ -1307,10 +1368,7 @@ static const void* yz_kernel(bool sliced) {
 void mesh_free(mdff_ctx* c) {
   MeshRecip* m = c->mesh;
   if (!m) return;
-  void* ps[] = {m->zf, m->zb, m->yf, m->yb, m->xf, m->xb, m->coef, m->A, m->kvec, m->key, m->slot, m->cnt, m->start,
-                m->order, m->at, m->amp, m->vt, m->phi, m->grid, m->mom, m->blk, m->t};
-  for (void* p : ps)
-    if (p) (void)hipFree(p);
+  if (m->mem) (void)hipFree(m->mem);
   delete m;
   c->mesh = nullptr;
 }
@@ -1327,10 +1385,9 @@ static double mesh_transform_us(const int* G, const int* K) {
   return 30e-9 * ops + 8e-6 * points;
 }
 
-// A and kvec: the k mesh of recip_setup ([nx][ny][nz], nx >= 0, A = 0 outside
-// the half space).  Leaves c->mesh null where no grid meets the error bound, or
-// the transforms of the one that does would take more than most_us.
-int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<double>& kv, double most_us) {
+// Leaves c->mesh null where no grid meets the error bound, or the transforms of
+// the one that does would take more than most_us.
+int mesh_setup(mdff_ctx* c, double most_us) {
   const int n = c->n;
   const bool wide = c->rec_wide != 0;
   const int w = wide ? 16 : 12;
@@ -1390,78 +1447,80 @@ int mesh_setup(mdff_ctx* c, const std::vector<double>& A, const std::vector<doub
   const int flight = kGatherThreads / 16 * kGatherAtoms;
   m->X = std::max(2, std::min(16, (int)(0.9 * flight / std::max(per_x, 1e-3))));
   m->CN = c->K[2] + 1;
-  const int Kx = c->K[0], Ky = c->K[1], Kz = c->K[2], CN = m->CN, NX = 2 * Kx + 1, NY = 2 * Ky + 1;
-  std::vector<double> coef;
-  kernel_pieces(w, beta, coef);
-  MDFF_TRY(upload(c, coef, &m->coef));
-  const std::vector<ld> dx = deconv(w, beta, Kx, G[0]), dy = deconv(w, beta, Ky, G[1]),
-                        dz = deconv(w, beta, Kz, G[2]);
-  const Roots rz(G[2]);
-  // z: column tile 2 ct + part holds that part of nz = 16 ct ..; back, row
-  // k = 2 nz + part
-  MDFF_TRY(upload(c, row_operand(G[2], 32 * ctiles, [&](int k, int col) {
-                    const int nz = 16 * (col / 32) + (col & 15);
-                    if (nz >= CN) return 0.0;
-                    const size_t a = rz.at((long long)nz * k);
-                    return (double)(((col & 16) ? rz.s[a] : rz.c[a]) * dz[nz]);
-                  }), &m->zf));
-  MDFF_TRY(upload(c, row_operand(32 * ctiles, G[2], [&](int k, int z) {
-                    if (k >= 2 * CN) return 0.0;
-                    const size_t a = rz.at((long long)(k >> 1) * z);
-                    return (double)(((k & 1) ? -rz.s[a] : rz.c[a]) * dz[k >> 1]);
-                  }), &m->zb));
-  auto mid = [&](int K, int g, const std::vector<ld>& dd, double** f, double** b) -> int {
-    const Roots r(g);
-    auto value = [&](int nn, int l, ld& re, ld& im) {
-      const size_t a = r.at((long long)(nn - K) * l);
-      re = r.c[a] * dd[std::abs(nn - K)];
-      im = r.s[a] * dd[std::abs(nn - K)];
-    };
-    MDFF_TRY(upload(c, mid_operand(2 * K + 1, g, value), f));
-    return upload(c, mid_operand(g, 2 * K + 1, [&](int l, int nn, ld& re, ld& im) { value(nn, l, re, im); }), b);
-  };
-  MDFF_TRY(mid(Ky, G[1], dy, &m->yf, &m->yb));
-  MDFF_TRY(mid(Kx, G[0], dx, &m->xf, &m->xb));
-  // A and k on nz >= 0: an entry and its opposite are one term, so nz = 0
-  // keeps half of each of the two
-  const size_t nk = (size_t)NX * NY * CN;
-  std::vector<double> Am(nk), km(4 * nk);
-  for (int x = -Kx; x <= Kx; ++x)
-    for (int y = -Ky; y <= Ky; ++y)
-      for (int z = 0; z <= Kz; ++z) {
-        const size_t o = ((size_t)(x + Kx) * NY + (y + Ky)) * CN + z;
-        auto src = [&](int a, int b, int e) { return ((size_t)a * c->NYk + (b + Ky)) * c->NZk + (e + Kz); };
-        double v, sg = 1.0;
-        size_t at;
-        if (x >= 0 && A[src(x, y, z)] != 0.0) at = src(x, y, z);
-        else if (x <= 0) { at = src(-x, -y, -z); sg = -1.0; }
-        else at = src(x, y, z);
-        v = A[at];
-        Am[o] = z == 0 ? 0.5 * v : v;
-        for (int k = 0; k < 3; ++k) km[4 * o + k] = sg * kv[4 * at + k];
-        km[4 * o + 3] = kv[4 * at + 3];
-      }
-  MDFF_TRY(upload(c, Am, &m->A));
-  MDFF_TRY(upload(c, km, &m->kvec));
+  const int CN = m->CN, NX = 2 * c->K[0] + 1, NY = 2 * c->K[1] + 1;
+  // what the host makes: the pieces of phi, roots and deconvolution, one copy
+  std::vector<double> small;
+  kernel_pieces(w, beta, small);
+  size_t root_at[3], dec_at[3];
+  for (int d = 0; d < 3; ++d) {
+    int same = 0;
+    while (same < d && G[same] != G[d]) ++same;
+    root_at[d] = same < d ? root_at[same] : small.size();
+    if (same == d) push_roots(small, G[d]);
+  }
+  for (int d = 0; d < 3; ++d) {
+    int same = 0;
+    while (same < d && (G[same] != G[d] || c->K[same] != c->K[d])) ++same;
+    dec_at[d] = same < d ? dec_at[same] : small.size();
+    if (same == d) push_deconv(small, w, beta, c->K[d], G[d]);
+  }
+  m->nblk = div_up((int64_t)NY * CN, 16);
+  std::vector<std::pair<void**, size_t>> parts;
+  auto part = [&](auto** p, size_t count) { parts.push_back({(void**)p, (sizeof(**p) * count + 255) & ~(size_t)255}); };
   const int nr = m->dip ? 6 : 3;
-  const size_t gcells = (size_t)G[0] * G[1] * G[2];
-  HIP_TRY(c, hipMalloc((void**)&m->key, sizeof(int32_t) * n));
-  HIP_TRY(c, hipMalloc((void**)&m->slot, sizeof(int32_t) * n));
-  HIP_TRY(c, hipMalloc((void**)&m->order, sizeof(BinAtom) * n));
-  HIP_TRY(c, hipMalloc((void**)&m->cnt, sizeof(int32_t) * m->nbins));
+  const size_t nk = (size_t)NX * NY * CN, zt = (size_t)32 * ctiles * G[2];
+  auto mid_size = [](int N, int L) { return (size_t)4 * div_up(L, 16) * div_up(N, 8) * 128; };
+  part(&m->coef, small.size());
+  part(&m->zf, zt);
+  part(&m->zb, zt);
+  part(&m->yf, mid_size(NY, G[1]));
+  part(&m->yb, mid_size(G[1], NY));
+  part(&m->xf, mid_size(NX, G[0]));
+  part(&m->xb, mid_size(G[0], NX));
+  part(&m->A, nk);
+  part(&m->kvec, 4 * nk);
+  part(&m->key, n);
+  part(&m->slot, n);
+  part(&m->order, n);
+  part(&m->cnt, m->nbins);
+  part(&m->start, m->nbins + 1);
+  part(&m->at, n);
+  part(&m->phi, (size_t)nr * w * n);
+  part(&m->vt, n);
+  if (m->dip) part(&m->amp, n);
+  part(&m->grid, (size_t)G[0] * G[1] * G[2] * m->shares);
+  part(&m->t, (size_t)G[0] * NY * CN);
+  part(&m->mom, 9 * (size_t)n);
+  part(&m->blk, 7 * (size_t)m->nblk);
+  size_t total = 0;
+  for (const auto& p : parts) total += p.second;
+  HIP_TRY(c, hipMalloc(&m->mem, total));
+  total = 0;
+  for (const auto& p : parts) {
+    *p.first = (char*)m->mem + total;
+    total += p.second;
+  }
+  HIP_TRY(c, hipMemcpy(m->coef, small.data(), sizeof(double) * small.size(), hipMemcpyHostToDevice));
   // (on the context's stream: hipMemset may return before the null stream has done
   // it, and this stream does not wait for that one)
   HIP_TRY(c, hipMemsetAsync(m->cnt, 0, sizeof(int32_t) * m->nbins, c->stream));
-  HIP_TRY(c, hipMalloc((void**)&m->start, sizeof(int32_t) * (m->nbins + 1)));
-  HIP_TRY(c, hipMalloc((void**)&m->at, sizeof(int4) * n));
-  HIP_TRY(c, hipMalloc((void**)&m->phi, sizeof(double) * nr * w * (size_t)n));
-  HIP_TRY(c, hipMalloc((void**)&m->vt, sizeof(double4) * n));
-  if (m->dip) HIP_TRY(c, hipMalloc((void**)&m->amp, sizeof(double4) * n));
-  HIP_TRY(c, hipMalloc((void**)&m->grid, sizeof(double) * gcells * m->shares));
-  HIP_TRY(c, hipMalloc((void**)&m->t, sizeof(double2) * (size_t)G[0] * NY * CN));
-  HIP_TRY(c, hipMalloc((void**)&m->mom, sizeof(double) * 9 * (size_t)n));
-  m->nblk = div_up((int64_t)NY * CN, 16);
-  HIP_TRY(c, hipMalloc((void**)&m->blk, sizeof(double) * 7 * m->nblk));
+  TableArgs ta{};
+  for (int d = 0; d < 3; ++d) {
+    ta.G[d] = G[d];
+    ta.K[d] = c->K[d];
+    ta.root[d] = reinterpret_cast<const double4*>(m->coef + root_at[d]);
+    ta.dec[d] = reinterpret_cast<const double2*>(m->coef + dec_at[d]);
+  }
+  ta.CN = CN;
+  ta.ctiles = ctiles;
+  ta.zf = m->zf; ta.zb = m->zb;
+  ta.f[0] = m->xf; ta.b[0] = m->xb;
+  ta.f[1] = m->yf; ta.b[1] = m->yb;
+  ta.A = m->A; ta.kvec = m->kvec;
+  for (int k = 0; k < 9; ++k) ta.cell[k] = c->B[k];
+  ta.alpha2 = c->alpha * c->alpha;
+  hipLaunchKernelGGL(k_mesh_tables, dim3(std::min(256, div_up(nk, 256)), 7), dim3(256), 0, c->stream, ta);
+  HIP_TRY(c, hipGetLastError());
   return MDFF_OK;
 }
 

@@ -144,6 +144,27 @@ __global__ void __launch_bounds__(256) k_tables_r(TabRArgs a, FinalBatch fb, int
   table_run(s, r, a.n, i, a.tab);
 }
 
+// A, k vector and kcoe on the box, A = 0 outside the half space (n_x > 0, or 0 and
+// n_y > 0, or both 0 and n_z > 0)
+struct BoxArgs {
+  int K[3];
+  double b[9], alpha2;
+  double *A, *kvec;
+};
+__global__ void __launch_bounds__(256) k_box_weights(BoxArgs a) {
+  const int NY = 2 * a.K[1] + 1, NZ = 2 * a.K[2] + 1;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= (a.K[0] + 1) * NY * NZ) return;
+  const int z = i % NZ - a.K[2], xy = i / NZ, y = xy % NY - a.K[1], x = xy / NY;
+  const bool half = x > 0 || (x == 0 && y > 0) || (x == 0 && y == 0 && z > 0);
+  const KWeight w = k_weight(a.b, a.alpha2, x, y, z);
+  a.A[i] = half ? w.A : 0.0;
+  a.kvec[4 * (size_t)i] = w.kx;
+  a.kvec[4 * (size_t)i + 1] = w.ky;
+  a.kvec[4 * (size_t)i + 2] = w.kz;
+  a.kvec[4 * (size_t)i + 3] = half ? w.kc : 0.0;
+}
+
 struct SkArgs {
   int n, Kx, Ky, Kz, NY, NZ, M, NG, GZ;
   int use_q, use_mu;
@@ -980,29 +1001,6 @@ int recip_setup(mdff_ctx* c) {
   c->nk_box = c->NXk * c->NYk * c->NZk;
   c->nk = Kz + Ky * (2 * Kz + 1) + Kx * (2 * Ky + 1) * (2 * Kz + 1);
   const int nb = c->nk_box;
-  std::vector<double> A(nb, 0.0), kv(4 * (size_t)nb, 0.0);
-  const double tpi = 2.0 * MDFF_PI, alpha2 = c->alpha * c->alpha;
-  const double* B = c->B;
-  for (int nx = 0; nx <= Kx; ++nx)
-    for (int ny = -Ky; ny <= Ky; ++ny)
-      for (int nz = -Kz; nz <= Kz; ++nz) {
-        bool half = (nx > 0) || (nx == 0 && ny > 0) || (nx == 0 && ny == 0 && nz > 0);
-        int idx = (nx * c->NYk + (ny + Ky)) * c->NZk + (nz + Kz);
-        double fx = nx, fy = ny, fz = nz;
-        double kx = tpi * (fx * B[0] + fy * B[3] + fz * B[6]);
-        double ky = tpi * (fx * B[1] + fy * B[4] + fz * B[7]);
-        double kz = tpi * (fx * B[2] + fy * B[5] + fz * B[8]);
-        double kk = kx * kx + ky * ky + kz * kz;
-        kv[4 * idx] = kx; kv[4 * idx + 1] = ky; kv[4 * idx + 2] = kz;
-        if (half && kk != 0.0) {
-          A[idx] = exp(-(kk * 0.25) / alpha2) / kk;
-          kv[4 * idx + 3] = 2.0 * (1.0 / kk + 1.0 / alpha2 / 4.0);
-        }
-      }
-  HIP_TRY(c, hipMalloc((void**)&c->kA, sizeof(double) * nb));
-  HIP_TRY(c, hipMalloc((void**)&c->kvec, sizeof(double) * 4 * nb));
-  HIP_TRY(c, hipMemcpy(c->kA, A.data(), sizeof(double) * nb, hipMemcpyHostToDevice));
-  HIP_TRY(c, hipMemcpy(c->kvec, kv.data(), sizeof(double) * 4 * nb, hipMemcpyHostToDevice));
   // The direct sums cost atoms x k vectors, the transforms some 60 us of short
   // kernels and a few us per 1,000 atoms (us a step or evaluation, direct / mesh):
   //   FP64   8e7 (silica 5,184) 160/164   1.5e8 (LiF 5,832) 157/145   1.8e8 (silica 8,232) 218/191
@@ -1022,9 +1020,21 @@ int recip_setup(mdff_ctx* c) {
     const bool asked = ev && ev[0], on = asked ? ev[0] != '0' : (double)c->n * nb > line;
     const double direct_us = asked || mma_bucket(Kz + 1) == 0 ? INFINITY : 28e-8 * c->n * nb + 220e-6 * nb;
     if (on && c->use_mma && direct_takes(c)) {
-      MDFF_TRY(mesh_setup(c, A, kv, direct_us));
+      MDFF_TRY(mesh_setup(c, direct_us));
       if (c->mesh) return MDFF_OK;
     }
+  }
+  {
+    HIP_TRY(c, hipMalloc((void**)&c->kA, sizeof(double) * nb));
+    HIP_TRY(c, hipMalloc((void**)&c->kvec, sizeof(double) * 4 * (size_t)nb));
+    BoxArgs a{};
+    for (int d = 0; d < 3; ++d) a.K[d] = c->K[d];
+    for (int k = 0; k < 9; ++k) a.b[k] = c->B[k];
+    a.alpha2 = c->alpha * c->alpha;
+    a.A = c->kA;
+    a.kvec = c->kvec;
+    hipLaunchKernelGGL(k_box_weights, dim3(div_up(nb, 256)), dim3(256), 0, c->stream, a);
+    HIP_TRY(c, hipGetLastError());
   }
   const int ncol = Kx + Ky + Kz + 3;
   HIP_TRY(c, hipMalloc((void**)&c->tab, sizeof(cplx) * ncol * (size_t)c->n));
