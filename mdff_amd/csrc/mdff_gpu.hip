@@ -465,7 +465,10 @@ __global__ void __launch_bounds__(256) k_hand_in(int n, const double* __restrict
 // Velocity rescale (rescale_velocities, src/kinetic.f90:122-198) in three
 // launches without a host round trip: block partials of sum m v^2; every block
 // adds them up, scales its atoms and leaves its velocity sums; every block adds
-// those and takes the mean off.
+// those and takes the mean off.  At most kRescaleBlocks, since each block reads
+// the others' partials (4.0e6 atoms 70 us, with a block for every 256 of them
+// 319; 1.0e7 151 and 1565; in four launches and two waits 160 and 410).
+constexpr int kRescaleBlocks = 1024;
 struct RescaleArgs {
   int n, nb, ndeg, csvr;         // csvr 0: the factor lambda
   double lambda;
@@ -477,9 +480,9 @@ struct RescaleArgs {
 };
 __global__ void __launch_bounds__(256) k_rescale_kin(RescaleArgs a) {
   __shared__ double sh[4 * kRedMaxCols];
-  const int i = blockIdx.x * 256 + threadIdx.x;
   double v[kRedMaxCols] = {};
-  if (i < a.n) v[0] = (a.vx[i] * a.vx[i] + a.vy[i] * a.vy[i] + a.vz[i] * a.vz[i]) * a.m[i];
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < a.n; i += gridDim.x * 256)
+    v[0] += (a.vx[i] * a.vx[i] + a.vy[i] * a.vy[i] + a.vz[i] * a.vz[i]) * a.m[i];
   const double r = block_sum_cols(v, 1, sh);
   if (threadIdx.x == 0) a.pk[blockIdx.x] = r;
 }
@@ -499,12 +502,15 @@ __global__ void __launch_bounds__(256) k_rescale_v(RescaleArgs a) {
       a.out[1] = knew;
     }
   }
-  const int i = blockIdx.x * 256 + threadIdx.x;
   double v[kRedMaxCols] = {};
-  if (i < a.n) {
-    a.vx[i] = v[0] = a.vx[i] * s;
-    a.vy[i] = v[1] = a.vy[i] * s;
-    a.vz[i] = v[2] = a.vz[i] * s;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < a.n; i += gridDim.x * 256) {
+    const double x = a.vx[i] * s, y = a.vy[i] * s, z = a.vz[i] * s;
+    a.vx[i] = x;
+    a.vy[i] = y;
+    a.vz[i] = z;
+    v[0] += x;
+    v[1] += y;
+    v[2] += z;
   }
   const double r = block_sum_cols(v, 3, sh);
   if (threadIdx.x < 3) a.pv[3 * (size_t)blockIdx.x + threadIdx.x] = r;
@@ -514,11 +520,11 @@ __global__ void __launch_bounds__(256) k_rescale_mean(RescaleArgs a) {
   __shared__ double tot[3];
   sum_block_partials(a.nb, 3, a.pv, tot, sh);
   __syncthreads();
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= a.n) return;
-  a.vx[i] -= tot[0] / a.n;
-  a.vy[i] -= tot[1] / a.n;
-  a.vz[i] -= tot[2] / a.n;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < a.n; i += gridDim.x * 256) {
+    a.vx[i] -= tot[0] / a.n;
+    a.vy[i] -= tot[1] / a.n;
+    a.vz[i] -= tot[2] / a.n;
+  }
 }
 
 // ---- Nose-Hoover chain steps on the device (nose_hoover_chain_n,
@@ -2021,7 +2027,7 @@ int mdff_md_nhcn(mdff_ctx* c, int32_t nsteps, double dt, double temp, double tim
 
 // one velocity rescale; e: kinetic energy before and after (csvr)
 static int rescale(mdff_ctx* c, RescaleArgs a, double e[2]) {
-  const int nb = nblk(c->n);
+  const int nb = std::min(nblk(c->n), kRescaleBlocks);
   a.n = c->n;
   a.nb = nb;
   a.m = c->mass;
