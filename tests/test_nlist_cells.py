@@ -82,3 +82,31 @@ def test_pair_sets_in_wide_boxes(ratio):
     fg, fo = g.engforce()[0], o.engforce()[0]
     assert G.rel_force_err(fg, fo) < 1e-10
     g.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("skew", [0.0, 0.12])
+@pytest.mark.parametrize("cells", [25, 32, 35])
+def test_pair_sets_over_many_cells(cells, skew):
+    """15,625 cells (one block of the scan), 32,768 (two full ones) and 42,875
+    (three) of 10,976 atoms; a second build gives the same."""
+    import gpu_util as G
+    G.note(f"many cells {cells} {skew}")
+    s = configs.fcc_lj(ncell=14, L=1.5414361 * 14)
+    d = s.desc
+    s.pos = s.pos + np.random.default_rng(cells).normal(0.0, 0.05, s.pos.shape)
+    L = d.cell[0]
+    s.pos[:, 1] += skew * s.pos[:, 0]
+    d.cell[:] = [L, skew * L, 0, 0, L, 0, 0, 0, L]
+    width = 1.0 / np.linalg.norm(np.linalg.inv(np.array(d.cell[:]).reshape(3, 3)), axis=0).max()
+    d.skindiff = 0.15
+    d.cutshortrange = 3.0 * width / (cells + 0.5) - d.skindiff
+    g, o = G.pair(s)
+    for e in (g, o):
+        e.vnlist_build()
+    for a, b in zip(g.get_pairs(0), o.get_pairs(0)):
+        assert np.array_equal(a, b)
+    g.vnlist_build()
+    for a, b in zip(g.get_pairs(0), o.get_pairs(0)):
+        assert np.array_equal(a, b)
+    g.close()
