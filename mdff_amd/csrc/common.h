@@ -327,7 +327,7 @@ struct mdff_ctx {
   int32_t* cell_cnt = nullptr;            // atoms a cell, zero between builds (ncell_alloc)
   int32_t* cell_atoms = nullptr;          // atoms sorted by cell
   int32_t* cell_atoms_in = nullptr;
-  int32_t* cell_start = nullptr;          // ncell + 1
+  int32_t* cell_start = nullptr;          // ncell + 1 (ncell_alloc)
   int32_t* nl_count = nullptr;            // n (+1): row lengths
   int32_t* nl_start = nullptr;            // n + 1: row starts
   int32_t* nl_j = nullptr;                // capacity entries

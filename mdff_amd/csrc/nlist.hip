@@ -86,13 +86,16 @@ __global__ void k_cell_count(int n, const double* __restrict__ sx, const double*
   slot[i] = atomicAdd(cnt + k, 1);
 }
 
-// start[k] = atoms before cell k, start[ncell] = n; the counts and the overflow
-// flag back to zero.  A run of kScanRun cells a thread, kScanBlock a block; with
-// more than one block the sums of each first (k_cell_sums), which every block adds
-// up for itself (one block over all of them was most of a build of a large system of
-// short cutoff: 4 million LJ atoms at 2.5, 4.5e6 cells, 10.9 ms a build, now 4.8;
-// 256,000 716 us, now 392).
-constexpr int kScanRun = 16, kScanBlock = 1024 * kScanRun;
+// start[k] = atoms before cell k, and n from ncell on; the overflow flag back to
+// zero.  Cells in whole runs of kScanRun (beyond ncell they are empty), a run a
+// thread, kScanBlock a block.  A block adds up the cells before its own: up to
+// kScanDirect blocks from their counts, beyond that from the blocks' sums
+// (k_cell_sums), a launch more.  One block over all cells, 16 loads a run, was
+// most of a build of a large system of short cutoff (4 million LJ atoms at 2.5,
+// 4.5e6 cells, 10.9 ms a build, now 4.8; 256,000 716 us, now 374; LiF
+// 13,248 at 5.4, 1.9e4 cells, 77 us, now 52).
+constexpr int kScanRun = 16, kScanBlock = 1024 * kScanRun, kScanDirect = 8;
+static int scan_cells(int ncell) { return (ncell + kScanRun) / kScanRun * kScanRun; }   // at least one beyond ncell
 
 // sums over the block's waves of each wave's value
 __device__ __forceinline__ int scan_block_sum(int v, int* wsum) {
@@ -107,35 +110,46 @@ __device__ __forceinline__ int scan_block_sum(int v, int* wsum) {
   return all;
 }
 
-__global__ void __launch_bounds__(1024) k_cell_sums(int ncell, const int32_t* __restrict__ cnt, int32_t* __restrict__ sums) {
+__device__ __forceinline__ int sum4(int4 v) { return (v.x + v.y) + (v.z + v.w); }
+
+// cells: a multiple of kScanRun
+__global__ void __launch_bounds__(1024) k_cell_sums(int cells, const int32_t* __restrict__ cnt, int32_t* __restrict__ sums) {
   __shared__ int wsum[16];
-  const int c0 = blockIdx.x * kScanBlock;
+  const int4* c = reinterpret_cast<const int4*>(cnt) + blockIdx.x * (kScanBlock / 4);
+  const int m = min(kScanBlock, cells - (int)blockIdx.x * kScanBlock) / 4;
   int v = 0;
 #pragma unroll
-  for (int u = 0; u < kScanRun; ++u) {
-    const int k = c0 + 1024 * u + (int)threadIdx.x;
-    v += k < ncell ? cnt[k] : 0;
+  for (int u = 0; u < kScanBlock / 4096; ++u) {
+    const int k = 1024 * u + (int)threadIdx.x;
+    if (k < m) v += sum4(c[k]);
   }
   const int all = scan_block_sum(v, wsum);
   if (threadIdx.x == 0) sums[blockIdx.x] = all;
 }
 
-__global__ void __launch_bounds__(1024) k_cell_scan(int n, int ncell, int32_t* __restrict__ cnt,
-                                                    int32_t* __restrict__ start, int32_t* __restrict__ overflow,
-                                                    const int32_t* __restrict__ sums) {
+__global__ void __launch_bounds__(1024) k_cell_scan(int cells, const int32_t* __restrict__ cnt, int32_t* __restrict__ start,
+                                                    int32_t* __restrict__ overflow, const int32_t* __restrict__ sums) {
   __shared__ int wsum[16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int k = blockIdx.x * kScanBlock + kScanRun * (int)threadIdx.x;
-  int v[kScanRun], sum = 0;
+  const bool on = k < cells;
+  const int4* c = reinterpret_cast<const int4*>(cnt + (on ? k : 0));
+  int4 v[kScanRun / 4];
+  int sum = 0, before = 0;
 #pragma unroll
-  for (int u = 0; u < kScanRun; ++u) {
-    v[u] = k + u < ncell ? cnt[k + u] : 0;
-    sum += v[u];
+  for (int u = 0; u < kScanRun / 4; ++u) {
+    v[u] = c[u];
+    if (on) sum += sum4(v[u]);
   }
-  int before = 0;
   if (blockIdx.x > 0) {
     int s = 0;
-    for (int b = threadIdx.x; b < (int)blockIdx.x; b += 1024) s += sums[b];
+    if (sums) {
+      for (int b = threadIdx.x; b < (int)blockIdx.x; b += 1024) s += sums[b];
+    } else {
+      const int4* all = reinterpret_cast<const int4*>(cnt);
+#pragma unroll 4
+      for (int b = threadIdx.x; b < (int)blockIdx.x * (kScanBlock / 4); b += 1024) s += sum4(all[b]);
+    }
     before = scan_block_sum(s, wsum);
     __syncthreads();
   }
@@ -150,23 +164,25 @@ __global__ void __launch_bounds__(1024) k_cell_scan(int n, int ncell, int32_t* _
 #pragma unroll
   for (int w = 0; w < 16; ++w) before += w < wave ? wsum[w] : 0;
   int at = before + incl - sum;
+  if (on) {
+    int4* o = reinterpret_cast<int4*>(start + k);
 #pragma unroll
-  for (int u = 0; u < kScanRun; ++u)
-    if (k + u < ncell) {
-      start[k + u] = at;
-      cnt[k + u] = 0;
-      at += v[u];
+    for (int u = 0; u < kScanRun / 4; ++u) {
+      const int4 w = make_int4(at, at + v[u].x, at + v[u].x + v[u].y, at + v[u].x + v[u].y + v[u].z);
+      at = w.w + v[u].w;
+      o[u] = w;
     }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    start[ncell] = n;
-    *overflow = 0;
   }
+  if (blockIdx.x == 0 && threadIdx.x == 0) *overflow = 0;
 }
 
+// and the counts back to zero
 __global__ void k_cell_scatter(int n, const int32_t* __restrict__ cell_of, const int32_t* __restrict__ slot,
-                               const int32_t* __restrict__ start, int32_t* __restrict__ out) {
+                               const int32_t* __restrict__ start, int32_t* __restrict__ out, int cells,
+                               int32_t* __restrict__ cnt) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) out[start[cell_of[i]] + slot[i]] = i;
+  for (int k = i; k < cells / 4; k += gridDim.x * blockDim.x) reinterpret_cast<int4*>(cnt)[k] = make_int4(0, 0, 0, 0);
 }
 
 // atoms of a cell in the order of their indices, and their fractional
@@ -568,36 +584,35 @@ static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const 
   // with fewer cells than the reach covers, every cell of that direction is
   // visited once
   const double rmax = std::max(c->rc_vdw, c->rc_coul) + c->d.skindiff;
-  const CellGrid cells = choose_cells(c->W, rmax, n);
+  const CellGrid cg = choose_cells(c->W, rmax, n);
   for (int d = 0; d < 3; ++d) {
-    const int reach = cells.reach[d];
-    c->ncell[d] = cells.n[d];
-    const bool all = cells.n[d] < 2 * reach + 1;
+    const int reach = cg.reach[d];
+    c->ncell[d] = cg.n[d];
+    const bool all = cg.n[d] < 2 * reach + 1;
     c->nb_lo[d] = all ? 0 : -reach;
-    c->nb_hi[d] = all ? cells.n[d] - 1 : reach;
+    c->nb_hi[d] = all ? cg.n[d] - 1 : reach;
     c->nb_all[d] = all ? 1 : 0;
   }
-  const int ncell = cells.total();
-  if (ncell + 1 > c->ncell_alloc) {
+  const int cells = scan_cells(cg.total()), sblk = div_up(cells, kScanBlock);
+  if (cells > c->ncell_alloc) {
     if (c->cell_start) HIP_TRY(c, hipFree(c->cell_start));
     if (c->cell_cnt) HIP_TRY(c, hipFree(c->cell_cnt));
     c->cell_start = c->cell_cnt = nullptr;
     c->ncell_alloc = 0;
-    HIP_TRY(c, hipMalloc((void**)&c->cell_start, sizeof(int32_t) * (ncell + 1)));
+    HIP_TRY(c, hipMalloc((void**)&c->cell_start, sizeof(int32_t) * cells));
     // counts, zero between builds, and the scan's block sums behind them
-    HIP_TRY(c, hipMalloc((void**)&c->cell_cnt, sizeof(int32_t) * (ncell + 1 + div_up(ncell, kScanBlock))));
-    HIP_TRY(c, hipMemsetAsync(c->cell_cnt, 0, sizeof(int32_t) * (ncell + 1), c->stream));
-    c->ncell_alloc = ncell + 1;
+    HIP_TRY(c, hipMalloc((void**)&c->cell_cnt, sizeof(int32_t) * ((size_t)cells + sblk)));
+    HIP_TRY(c, hipMemsetAsync(c->cell_cnt, 0, sizeof(int32_t) * cells, c->stream));
+    c->ncell_alloc = cells;
   }
   const dim3 ga(div_up(n, 256)), b256(256);
   hipLaunchKernelGGL(k_cell_count, ga, b256, 0, c->stream, n, px, py, pz, c->ncell[0], c->ncell[1], c->ncell[2],
                      c->cell_of, c->cell_slot, c->cell_cnt);
-  const int sblk = div_up(ncell, kScanBlock);
-  int32_t* sums = c->cell_cnt + c->ncell_alloc;
-  if (sblk > 1)
-    hipLaunchKernelGGL(k_cell_sums, dim3(sblk), dim3(1024), 0, c->stream, ncell, c->cell_cnt, sums);
-  hipLaunchKernelGGL(k_cell_scan, dim3(sblk), dim3(1024), 0, c->stream, n, ncell, c->cell_cnt, c->cell_start, c->d_flag + 1, sums);
-  hipLaunchKernelGGL(k_cell_scatter, ga, b256, 0, c->stream, n, c->cell_of, c->cell_slot, c->cell_start, c->cell_atoms_in);
+  int32_t* sums = sblk > kScanDirect ? c->cell_cnt + c->ncell_alloc : nullptr;
+  if (sums) hipLaunchKernelGGL(k_cell_sums, dim3(sblk), dim3(1024), 0, c->stream, cells, c->cell_cnt, sums);
+  hipLaunchKernelGGL(k_cell_scan, dim3(sblk), dim3(1024), 0, c->stream, cells, c->cell_cnt, c->cell_start, c->d_flag + 1, sums);
+  hipLaunchKernelGGL(k_cell_scatter, ga, b256, 0, c->stream, n, c->cell_of, c->cell_slot, c->cell_start, c->cell_atoms_in,
+                     cells, c->cell_cnt);
   // fractional coordinates in cell order (coalesced candidate loads); they
   // are kept as the positions of this build
   hipLaunchKernelGGL(k_cell_order, ga, b256, 0, c->stream, n, c->cell_atoms_in, c->cell_of, c->cell_start, px, py, pz,
