@@ -10,12 +10,17 @@ struct CellGrid {
   int total() const { return n[0] * n[1] * n[2]; }
 };
 
-// Most cells of a grid: one round of the one-block scan over them (16,384), or
-// four an atom.  More would be empty ones, which a build still clears, scans
-// and holds in memory: 108 atoms in 1000 A at a reach of 9 A made 3.7e7 cells,
-// 300 MB, and builds of 48 ms (60 us with the limit), and from 430 reaches a side on
-// their number no longer fits an int.
-inline double cell_limit(int natm) { return std::max(16384.0, 4.0 * natm); }
+// Most cells of a grid: 256 an atom up to 2^24, four an atom beyond, and 16,384 for
+// the fewest.  A build clears and scans its cells and holds 8 bytes for each:
+// nothing at 16,384, some 60 us and 128 MB at 2^24; 108 atoms in 1000 A at a reach
+// of 9 A made 3.7e7 and builds of 48 ms (60 us with the limit), and from 430 reaches
+// a side on their number no longer fits an int.  Coarser cells would cost more where
+// atoms sit close in a wide box, candidates by the cube of their width (a droplet of
+// 4,000 atoms builds in 82 us in a box of 100 reaches, 75 in one of 20).
+inline double cell_limit(int natm) {
+  const double n = natm;
+  return std::max({16384.0, 4.0 * n, std::min(256.0 * n, 16777216.0)});
+}
 
 // Cells for partners within rmax between planes W[d] apart: of a third of rmax
 // where at least 7 of them fit (partners within +-3 cells), else of a half (5,

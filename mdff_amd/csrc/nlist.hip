@@ -72,18 +72,43 @@ __device__ __forceinline__ int wrap_cell(double s, int nc) {
 }
 
 // Atoms into cells, in the order of their indices within each: count, scan,
-// scatter, and ranks within a cell counted out by k_cell_order (a cell holds a
-// few atoms).  Four short launches; the radix sort of (cell, index) and what
-// it needed around it were eight, 45 us of a build of 24,000 atoms.
-__global__ void k_cell_count(int n, const double* __restrict__ sx, const double* __restrict__ sy,
-                             const double* __restrict__ sz, int nx, int ny, int nz, int32_t* __restrict__ cell_of,
-                             int32_t* __restrict__ slot, int32_t* __restrict__ cnt) {
+// scatter, and ranks within a cell counted out by k_cell_order.  Four short
+// launches; the radix sort of (cell, index) and what it needed around it were
+// eight, 45 us of a build of 24,000 atoms.
+// CROWD: few cells of many atoms (more than 32 on average, in a box of a few
+// cutoffs).  Then a block first counts in LDS, so that a cell's counter sees an
+// addition a block and not one an atom, and 16 lanes count an atom's rank (LJ
+// 4,000 at 7.0, eight cells: build 92 us, 159 like the others; 10,976 at 9.2, 599
+// and 790).
+constexpr int kCrowdCells = 4096;
+template <bool CROWD>
+__global__ void __launch_bounds__(256) k_cell_count(int n, const double* __restrict__ sx, const double* __restrict__ sy,
+                                                    const double* __restrict__ sz, int nx, int ny, int nz,
+                                                    int32_t* __restrict__ cell_of, int32_t* __restrict__ slot,
+                                                    int32_t* __restrict__ cnt) {
+  __shared__ int h[CROWD ? kCrowdCells : 1];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int ncell = nx * ny * nz;
+  if (CROWD) {
+    for (int k = threadIdx.x; k < ncell; k += 256) h[k] = 0;
+    __syncthreads();
+  }
+  int k = 0, s = 0;
+  if (i < n) {
+    const int cx = wrap_cell(sx[i], nx), cy = wrap_cell(sy[i], ny), cz = wrap_cell(sz[i], nz);
+    k = (cx * ny + cy) * nz + cz;
+    s = atomicAdd(CROWD ? h + k : cnt + k, 1);
+  }
+  if (CROWD) {
+    __syncthreads();
+    for (int c = threadIdx.x; c < ncell; c += 256)
+      if (h[c] > 0) h[c] = atomicAdd(cnt + c, h[c]);
+    __syncthreads();
+    s += h[k];
+  }
   if (i >= n) return;
-  const int cx = wrap_cell(sx[i], nx), cy = wrap_cell(sy[i], ny), cz = wrap_cell(sz[i], nz);
-  const int k = (cx * ny + cy) * nz + cz;
   cell_of[i] = k;
-  slot[i] = atomicAdd(cnt + k, 1);
+  slot[i] = s;
 }
 
 // start[k] = atoms before cell k, and n from ncell on; the overflow flag back to
@@ -188,22 +213,28 @@ __global__ void k_cell_scatter(int n, const int32_t* __restrict__ cell_of, const
 // atoms of a cell in the order of their indices, and their fractional
 // coordinates in cell order: the doubles, and a wrapped single-precision copy
 // (s - floor(s), exact in double, then rounded) for the sweep's prefilter;
-// with save, also kept per atom (xs, ys, zs)
+// with save, also kept per atom (xs, ys, zs).  An atom's rank is the number of
+// smaller indices in its cell, counted by L lanes.
+template <int L>
 __global__ void k_cell_order(int n, const int32_t* __restrict__ in, const int32_t* __restrict__ cell_of,
                              const int32_t* __restrict__ start, const double* __restrict__ sx,
                              const double* __restrict__ sy, const double* __restrict__ sz,
                              int32_t* __restrict__ order, double* __restrict__ ox, double* __restrict__ oy,
                              double* __restrict__ oz, float4* __restrict__ of, int save, double* __restrict__ xs,
                              double* __restrict__ ys, double* __restrict__ zs) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
+  const int tid = blockIdx.x * blockDim.x + threadIdx.x, t = tid / L, lane = tid % L;
+  if (t >= n) return;                    // whole groups
   const int i = in[t];
   const int k = cell_of[i], b = start[k], e = start[k + 1];
-  int p = b;
-  for (int u = b; u < e; u += 8) {       // eight loads in flight (few cells can hold many atoms)
+  int rank = 0;
+  for (int u = b + lane; u < e; u += 8 * L) {       // eight loads in flight
 #pragma unroll
-    for (int v = 0; v < 8; ++v) p += u + v < e && in[min(u + v, e - 1)] < i ? 1 : 0;
+    for (int v = 0; v < 8; ++v) rank += u + v * L < e && in[min(u + v * L, e - 1)] < i ? 1 : 0;
   }
+#pragma unroll
+  for (int o = L / 2; o > 0; o >>= 1) rank += __shfl_xor(rank, o, L);
+  if (lane > 0) return;
+  const int p = b + rank;
   const double x = sx[i], y = sy[i], z = sz[i];
   order[p] = i;
   ox[p] = x;
@@ -606,7 +637,8 @@ static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const 
     c->ncell_alloc = cells;
   }
   const dim3 ga(div_up(n, 256)), b256(256);
-  hipLaunchKernelGGL(k_cell_count, ga, b256, 0, c->stream, n, px, py, pz, c->ncell[0], c->ncell[1], c->ncell[2],
+  const bool crowd = n > 32 * (int64_t)cg.total() && cg.total() <= kCrowdCells;
+  hipLaunchKernelGGL(crowd ? &k_cell_count<true> : &k_cell_count<false>, ga, b256, 0, c->stream, n, px, py, pz, c->ncell[0], c->ncell[1], c->ncell[2],
                      c->cell_of, c->cell_slot, c->cell_cnt);
   int32_t* sums = sblk > kScanDirect ? c->cell_cnt + c->ncell_alloc : nullptr;
   if (sums) hipLaunchKernelGGL(k_cell_sums, dim3(sblk), dim3(1024), 0, c->stream, cells, c->cell_cnt, sums);
@@ -615,7 +647,7 @@ static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const 
                      cells, c->cell_cnt);
   // fractional coordinates in cell order (coalesced candidate loads); they
   // are kept as the positions of this build
-  hipLaunchKernelGGL(k_cell_order, ga, b256, 0, c->stream, n, c->cell_atoms_in, c->cell_of, c->cell_start, px, py, pz,
+  hipLaunchKernelGGL(crowd ? &k_cell_order<16> : &k_cell_order<1>, dim3(div_up((int64_t)n * (crowd ? 16 : 1), 256)), b256, 0, c->stream, n, c->cell_atoms_in, c->cell_of, c->cell_start, px, py, pz,
                      c->cell_atoms, c->bx, c->by, c->bz, c->bf, save ? 1 : 0, c->xs, c->ys, c->zs);
   NLArgs a = make_args(c);
   a.sx = px; a.sy = py; a.sz = pz;

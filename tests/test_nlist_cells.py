@@ -43,7 +43,7 @@ def choose(tmp_path_factory):
 def test_cells_are_bounded_and_cover_the_cutoff(choose, W, natm):
     r = 9.3
     n, reach = choose([w * r for w in W], r, natm)
-    assert n[0] * n[1] * n[2] <= max(16384, 4 * natm)
+    assert n[0] * n[1] * n[2] <= max(16384, 4 * natm, min(256 * natm, 1 << 24))
     for d in range(3):
         assert n[d] >= 1 and 1 <= reach[d] <= 3
         # all cells are visited, or those of +-reach hold every partner
@@ -112,4 +112,27 @@ def test_pair_sets_over_many_cells(m, cells, skew):
     g.vnlist_build()
     for a, b in zip(g.get_pairs(0), o.get_pairs(0)):
         assert np.array_equal(a, b)
+    g.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,rc", [(10, 8.5), (10, 7.0), (10, 4.6), (10, 3.8), (10, 2.8), (7, 5.0), (5, 2.9), (12, 6.0)])
+def test_pair_sets_of_crowded_cells(m, rc):
+    """From one cell of 4,000 atoms to 125 of 32, the line, and beyond it."""
+    import gpu_util as G
+    G.note(f"crowded {m} {rc}")
+    s = configs.fcc_lj(ncell=m, L=1.5414361 * m)
+    s.pos = s.pos + np.random.default_rng(m).normal(0.0, 0.05, s.pos.shape)
+    s.desc.cutshortrange, s.desc.skindiff = rc, 0.2
+    g, o = G.pair(s)
+    for e in (g, o):
+        e.vnlist_build()
+    for a, b in zip(g.get_pairs(0), o.get_pairs(0)):
+        assert np.array_equal(a, b)
+    f = []
+    for _ in range(2):
+        g.vnlist_build()
+        f.append(g.engforce()[0])
+    assert np.array_equal(f[0], f[1])                        # rows in the same order every time
+    assert G.rel_force_err(f[0], o.engforce()[0]) < 1e-10
     g.close()
