@@ -590,9 +590,20 @@ static NLArgs make_args(mdff_ctx* c) {
   return a;
 }
 
-// the sweep's overflow flag on the host; `next` is launched before the wait
+// the sweep's overflow flag on the host.  `next`, if any, is launched before the
+// wait, which then ends on a word in mapped memory and not behind `next`.
+// Without one a copy and a stream synchronisation: the runtime takes back the
+// launches before it there, and the ones after it cost the host 3 us each and
+// not 6 (LJ rebuilt every step, 108 atoms 70 us a step, 2,048 76, 10,976 at
+// 5.0 155; 85-92, 92 and 163 with the word).
 template <typename F>
-static int nl_overflow(mdff_ctx* c, F next, bool* over) {
+static int nl_overflow(mdff_ctx* c, bool more, F next, bool* over) {
+  if (!more) {
+    HIP_TRY(c, hipMemcpyAsync(c->h_flag + 1, c->d_flag + 1, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    *over = c->h_flag[1] != 0;
+    return MDFF_OK;
+  }
   c->h_nl[1] = 0.0;
   c->nl_seq += 1.0;
   hipLaunchKernelGGL(k_post_flag, dim3(1), dim3(64), 0, c->stream, c->d_flag + 1, c->d_nl, c->nl_seq);
@@ -657,11 +668,10 @@ static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const 
   // pass writes the final ones
   const bool split = c->rc_inner > 0.0;
   auto partition = [&]() {
-    if (split)
-      PROF_LAUNCH(c, PK_NLIST, hipLaunchKernelGGL(k_nl_partition, grid, dim3(256), 0, c->stream, n,
-                                                  a.row_w ? a.row_w : INT32_MAX, c->nl_start,
-                                                  c->nl_count, c->nl_count_in, c->nl_j_tmp, c->nl_flag_tmp,
-                                                  c->nl_j, c->nl_flag));
+    PROF_LAUNCH(c, PK_NLIST, hipLaunchKernelGGL(k_nl_partition, grid, dim3(256), 0, c->stream, n,
+                                                a.row_w ? a.row_w : INT32_MAX, c->nl_start,
+                                                c->nl_count, c->nl_count_in, c->nl_j_tmp, c->nl_flag_tmp,
+                                                c->nl_j, c->nl_flag));
   };
   if (split) {
     a.nl_j = c->nl_j_tmp;
@@ -675,7 +685,7 @@ static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const 
     // the partition is queued before the host looks at the flag, so that the
     // device has work while it does
     bool over = false;
-    MDFF_TRY(nl_overflow(c, partition, &over));
+    MDFF_TRY(nl_overflow(c, split, partition, &over));
     if (!over) {
       HIP_TRY(c, hipGetLastError());
       c->lists_valid = 1;
@@ -735,7 +745,7 @@ static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const 
   a.row_w = (int)w;
   c->nl_row_w = (int)w;
   PROF_LAUNCH(c, PK_NLIST, hipLaunchKernelGGL(k_nl_sweep<true>, grid, dim3(256), 0, c->stream, a));
-  partition();
+  if (split) partition();
   HIP_TRY(c, hipGetLastError());
   c->lists_valid = 1;
   return MDFF_OK;

@@ -136,3 +136,29 @@ def test_pair_sets_of_crowded_cells(m, rc):
     assert np.array_equal(f[0], f[1])                        # rows in the same order every time
     assert G.rel_force_err(f[0], o.engforce()[0]) < 1e-10
     g.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [3, 6])
+def test_rows_outgrow_their_width_without_inner_entries(m):
+    """LJ alone: no inner entries, so the build waits for the flag by a copy."""
+    import gpu_util as G
+    G.note(f"outgrown rows {m}")
+    s = configs.fcc_lj(ncell=m, L=1.5414361 * m)
+    s.desc.cutshortrange, s.desc.skindiff = 1.6, 0.2
+    g, o = G.pair(s)
+    half = s.pos.copy()
+    half[:, 0] *= 0.25                                       # four times as dense, and a row as long
+    for pos in (s.pos, half, s.pos):
+        for e in (g, o):
+            e.set_positions(pos)
+            e.vnlist_build()
+        for a, b in zip(g.get_pairs(0), o.get_pairs(0)):
+            assert np.array_equal(a, b)
+    g.set_positions(half)
+    assert g.vnlistcheck()                                   # the check's own build
+    o.set_positions(half)
+    o.vnlist_build()
+    for a, b in zip(g.get_pairs(0), o.get_pairs(0)):
+        assert np.array_equal(a, b)
+    g.close()
