@@ -871,7 +871,7 @@ __global__ void __launch_bounds__(256) kf_dipreal(FitArgs a, int slot) {
 constexpr int kSkTile = 32;      // ions of a staged tile of kf_sk
 constexpr int kSkRows = 4;       // row tiles (8 nz) of its blocks at most
 
-#ifdef __HIPCC__   // (the kernels' host build for the tests goes without)
+#ifdef __HIPCC__   // a host build without matrix instructions goes without
 // ---------------------------------------------------------------------------
 // Reciprocal field of the iterations on the FP64 matrix cores, in both forms.
 // A thread a k (or an atom) over phase products was 75 % of a gradient: 404

@@ -190,7 +190,7 @@ __global__ void k_upol(int n, const double* __restrict__ invpol, const double* _
 // that sum of the first mu.  An iteration of few ions is bound by its launches
 // and waits (converged MgO, 216 ions FP64: 2432 us with 12 small launches and
 // two copies with a wait each, 1225 with four, the real-space field on a second
-// stream and one wait, now 770; 1,440 ions 3094, 1516, 1135).
+// stream and one wait, now 655; 1,440 ions 3094, 1516 and 1065).
 constexpr int kScfSlot = 4;
 
 // mu.alpha^-1.mu of one ion
@@ -431,7 +431,7 @@ inline int nblk(int n) { return div_up(n, 256); }
 // Small results to the host: up to four arrays into mapped host memory by one
 // block, then the sequence number that the host waits for.  A copy and a stream
 // synchronisation take 8 to 10 us each whatever the size: a 64-ion frame
-// (positions in, list check, forces out) took 172 us with nine of them, now 106.
+// (positions in, list check, forces out) took 172 us with nine of them, now 84.
 // Up to kIoMax doubles: 3 x 2,048 out 55 and 25 us, 3 x 8,788 59 and 51, level
 // at about 3 x 14,000.
 struct HandArgs {
@@ -1141,8 +1141,8 @@ static int scf(mdff_ctx* c, mdff_terms* t) {
     HIP_TRY(c, hipGetLastError());
     // the next iteration's real-space field, before the host has seen whether
     // there is one: the device works while the host waits, decides and queues
-    // the rest (the last one is of no use; 216 ions 770 -> 707 us, 1,440 1135 ->
-    // 1042, 12,000 3010 -> 2960)
+    // the rest (the last one is of no use; FP64, 216 ions 727 us without, 655 with,
+    // 1,440 1151 and 1067, 12,000 mixed 3383 and 3308)
     field_queued = iscf < d.max_scf_pol_iter;
     if (field_queued) MDFF_TRY(realspace_field(c, 1, c->mu_next, ef_dir(c)));
     // wait for every block's sequence number; a launch that never reports is

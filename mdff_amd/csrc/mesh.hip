@@ -24,13 +24,16 @@
 // The grid G and beta are chosen per direction from the alias error weighted
 // with the decay of A(k) (mesh_error_above): below 4e-15 with w = 16 in the FP64
 // form, which measured 1e-14 of the reciprocal force (its rounding), below
-// 1e-9 with w = 12 in the mixed form, whose FP32 pair terms carry 1e-7.
+// 1e-9 with w = 12 in the mixed form, whose FP32 pair terms carry 1e-7 (16 points
+// there too where recip_wide, recip.hip, asks for them).
 //
 // Launches of one evaluation: k_mesh_bin (s = B^T r, count per bin),
 // k_mesh_scan, k_mesh_scatter, k_mesh_phi (order within the bins, phi
 // values), k_mesh_spread, k_mesh_zy (z and y transforms), k_mesh_x (x
 // transform, W, energy and stress, x transform back), k_mesh_yz, k_mesh_gather.
-// Every sum has a fixed order.
+// Planes longer than LDS holds are transformed in slices (SLICED).  Every sum has
+// a fixed order.  What an evaluation reads besides the atoms (weights, twiddles,
+// deconvolution, A(k)) is formed on the device at creation (k_mesh_tables).
 #include <algorithm>
 #include <cmath>
 

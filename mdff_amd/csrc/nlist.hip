@@ -4,7 +4,7 @@
 // (src/tools.f90:444-537).  The reference tests every ordered pair of the
 // O(N^2) sweep with the ownership rule; here atoms are binned into cells in
 // fractional space (cells of a third of the cutoff where they fit, so every
-// partner lies within three cells) and one wavefront per atom sweeps those
+// partner lies within three cells; cells.h) and one wavefront per atom sweeps those
 // cells.  Each device row holds ALL partners j != i with
 // r^2 <= (max cut + skin)^2, plus a flag byte saying which of the two
 // reference lists (vdw, coul) accepts the pair.  The reference half lists are

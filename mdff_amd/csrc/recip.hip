@@ -916,9 +916,11 @@ static size_t sk_valu_lds(int ncol, int ta) { return (16 * (size_t)ncol + 32) * 
 // ... and of the vector-ALU gather with nthr threads a block
 static size_t gather_lds(int Kz, int nthr) { return 16 * ((size_t)(Kz + 1) * nthr + 8 * (2 * (size_t)Kz + 1)); }
 
-// LDS a block may take where no smaller tile fits: 64 KiB, 128 KiB for the
-// mixed form, whose tables were once FP32 and which takes k meshes of twice
-// the FP64 form's extent.  Smaller tiles are used long before that.
+// LDS a block may take where no smaller tile fits: 64 KiB, 128 KiB in the mixed
+// form.  This is what decides which k meshes a context is created for
+// (direct_takes), the mixed form's reaching to twice the FP64 form's extent; it
+// stays where it is so that the same ones are taken and refused.  Smaller tiles
+// are used long before that.
 static size_t lds_limit(const mdff_ctx* c) { return c->d.precision == MDFF_PREC_MIXED ? 131072 : 65536; }
 static int allow_lds(mdff_ctx* c, const void* fn, size_t lds) {
   if (lds > 65536)
@@ -1004,8 +1006,10 @@ int recip_setup(mdff_ctx* c) {
   // The direct sums cost atoms x k vectors, the transforms some 60 us of short
   // kernels and a few us per 1,000 atoms (us a step or evaluation, direct / mesh):
   //   FP64   8e7 (silica 5,184) 160/164   1.5e8 (LiF 5,832) 157/145   1.8e8 (silica 8,232) 218/191
-  //   mixed  5.4e7 (silica 4,320) 136/138   4.3e7 (MgO 4,608 dipoles) 2514/2733   8e7 160/142
-  //   gradient  9e7 (NaCl 4,096) 341/323
+  //          dipoles, MgO 5,832 2662/2869   6,480 2834/2872   8,000 3379/2965
+  //   mixed  5.4e7 (silica 4,320) 136/138   8e7 160/142
+  //          dipoles, 4.3e7 (MgO 4,608) 1994/2407   5,832 2561/2458   8,000 3240/2898
+  //   gradient  4e7 (NaCl 2,744) 162/164   9e7 (4,096) 207/184   (5,832) 320/194
   // The mixed form's narrower kernel (12 points, not 16) puts its line lower.
   // Few atoms in a large k mesh are another matter: the transforms' own work goes
   // with the mesh alone, and has to be less than what the direct sums spend on
