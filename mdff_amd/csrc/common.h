@@ -437,7 +437,7 @@ static inline int div_up(int64_t a, int64_t b) { return (int)((a + b - 1) / b); 
 int nl_build(mdff_ctx* c);
 int nl_check(mdff_ctx* c, int* rebuilt);
 int nl_check_launch(mdff_ctx* c);
-int nl_check_finish(mdff_ctx* c, int* rebuilt);
+int nl_check_finish(mdff_ctx* c, int* rebuilt, bool queued = false);   // queued: work ahead of a rebuild
 // velocity Verlet: position update; step end + list check (+ the next
 // step's position update)
 int vv_pos_launch(mdff_ctx* c, double dt);

@@ -1413,7 +1413,7 @@ static int engforce_launch(mdff_ctx* c, double* raw, mdff_terms* t, bool defer_f
   }
   ev_rec(c, 2 * EVS_LIST);
   int rb = 0;
-  MDFF_TRY(nl_check_finish(c, &rb));
+  MDFF_TRY(nl_check_finish(c, &rb, recip_first));
   if (!d.lvnlist || !c->lists_valid) {
     MDFF_TRY(nl_build(c));
     t->list_rebuilt = 1;

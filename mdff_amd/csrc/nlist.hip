@@ -590,15 +590,17 @@ static NLArgs make_args(mdff_ctx* c) {
   return a;
 }
 
-// the sweep's overflow flag on the host.  `next`, if any, is launched before the
-// wait, which then ends on a word in mapped memory and not behind `next`.
-// Without one a copy and a stream synchronisation: the runtime takes back the
-// launches before it there, and the ones after it cost the host 3 us each and
-// not 6 (LJ rebuilt every step, 108 atoms 70 us a step, 2,048 76, 10,976 at
-// 5.0 155; 85-92, 92 and 163 with the word).
+// the sweep's overflow flag on the host.  `next`, if any (split), is launched
+// before the wait, which then ends on a word in mapped memory and not behind it.
+// Without one, and with nothing queued ahead of the build, a copy and a stream
+// synchronisation: the runtime takes back the launches before it there, and the
+// ones after it cost the host 3 us each and not 6 (LJ rebuilt every step, 108 atoms
+// 70 us a step, 2,048 76, 10,976 at 5.0 155; 85-92, 92 and 163 with the word).  Behind
+// a step's reciprocal sums the word is ahead (NaCl 512 rebuilt every step 87 us,
+// 91 with the copy).
 template <typename F>
-static int nl_overflow(mdff_ctx* c, bool more, F next, bool* over) {
-  if (!more) {
+static int nl_overflow(mdff_ctx* c, bool split, bool queued, F next, bool* over) {
+  if (!split && !queued) {
     HIP_TRY(c, hipMemcpyAsync(c->h_flag + 1, c->d_flag + 1, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     *over = c->h_flag[1] != 0;
@@ -607,7 +609,7 @@ static int nl_overflow(mdff_ctx* c, bool more, F next, bool* over) {
   c->h_nl[1] = 0.0;
   c->nl_seq += 1.0;
   hipLaunchKernelGGL(k_post_flag, dim3(1), dim3(64), 0, c->stream, c->d_flag + 1, c->d_nl, c->nl_seq);
-  next();
+  if (split) next();
   volatile const double* h = c->h_nl;
   bool seen = false;
   for (long k = 0; k < 20000000L && !seen; ++k) seen = h[1] == c->nl_seq;
@@ -621,7 +623,7 @@ static int nl_overflow(mdff_ctx* c, bool more, F next, bool* over) {
 
 // vnlist_pbc: rebuild the rows from the current positions.
 // list build from the fractional coordinates (px, py, pz) of the build
-static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const double* pz, bool save) {
+static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const double* pz, bool save, bool queued) {
   const int n = c->n;
   // with fewer cells than the reach covers, every cell of that direction is
   // visited once
@@ -685,7 +687,7 @@ static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const 
     // the partition is queued before the host looks at the flag, so that the
     // device has work while it does
     bool over = false;
-    MDFF_TRY(nl_overflow(c, split, partition, &over));
+    MDFF_TRY(nl_overflow(c, split, queued, partition, &over));
     if (!over) {
       HIP_TRY(c, hipGetLastError());
       c->lists_valid = 1;
@@ -753,7 +755,7 @@ static int nl_build_from(mdff_ctx* c, const double* px, const double* py, const 
 
 int nl_build(mdff_ctx* c) {
   launch_kardir(c);
-  return nl_build_from(c, c->sx, c->sy, c->sz, false);
+  return nl_build_from(c, c->sx, c->sy, c->sz, false, false);
 }
 
 // the two largest of the block's values m1 (m2 = 0 on entry) -> out[2 * block]
@@ -941,7 +943,7 @@ int vv_end_launch(mdff_ctx* c, double dt, bool next, double* ke_part) {
   return MDFF_OK;
 }
 
-int nl_check_finish(mdff_ctx* c, int* rebuilt) {
+int nl_check_finish(mdff_ctx* c, int* rebuilt, bool queued) {
   *rebuilt = 0;
   if (!c->chk_pending) return MDFF_OK;
   c->chk_pending = 0;
@@ -969,7 +971,7 @@ int nl_check_finish(mdff_ctx* c, int* rebuilt) {
     }
   }
   if (m1 + m2 > c->d.skindiff) {
-    MDFF_TRY(nl_build_from(c, c->cx, c->cy, c->cz, true));
+    MDFF_TRY(nl_build_from(c, c->cx, c->cy, c->cz, true, queued));
     *rebuilt = 1;
   }
   return MDFF_OK;
